@@ -201,11 +201,11 @@ def work(case: dict) -> dict:
 
 
 def tolerance(case: dict) -> dict:
-    """About four times the distance measured between the path and the same mathematics in 64 bits.  bf16:
-    attention 1.3e-3 to 1.6e-3 (probabilities rounded before PV), layer 1.8e-3 to 2.2e-3, FFN 2.9e-3 to 3.4e-3 (2.8e-4 at the
-    same rounding points); fp16: attention 1.8e-4, layer 2.5e-4, FFN 4.2e-4.  The e4m3 FFN at the same rounding points: 1.4e-3 in
-    norm and 0.10 in a single value, since a value of h that moves by an ulp takes another code; an appended e4m3
-    cache row: 0.06 in a single value, one code."""
+    """About four times the distance measured between the path and the same mathematics in 64 bits.
+    bf16: attention 1.3e-3 to 1.6e-3 (probabilities rounded before PV), layer 1.8e-3 to 2.2e-3, FFN 2.9e-3
+    to 3.4e-3 (2.8e-4 at the same rounding points); fp16: attention 1.8e-4, layer 2.5e-4, FFN 4.2e-4.  The
+    e4m3 FFN at the same rounding points: 1.4e-3 in norm and 0.10 in a single value, since a value of h that
+    moves by an ulp takes another code; an appended e4m3 cache row: 0.06 in a single value, one code."""
     bf16 = case["dtype"] == "bf16"
     if case["kind"] == "ffn":
         return {"rel": 6e-3, "max": 0.4} if case["weights"] == "e4m3" else {"rel": 1.2e-2 if bf16 else 1.7e-3}
