@@ -25,7 +25,8 @@ namespace gemm8 {
 typedef int v8i __attribute__((ext_vector_type(8)));
 typedef __attribute__((__vector_size__(16 * sizeof(float)))) float f32x16;
 typedef __attribute__((__vector_size__(4 * sizeof(uint32_t)))) uint32_t u32x4;
-typedef __attribute__((address_space(3))) uint8_t lds_u8;
+typedef __attribute__((address_space(3))) const char lds_cchar;
+typedef __attribute__((address_space(3))) const u32x4 lds_cu32x4;
 
 constexpr int BK = 128;   // k extent of one LDS tile row, in codes (= bytes)
 constexpr int BN = 256;   // B rows (output channels) per tile
@@ -55,35 +56,10 @@ struct Params {
 // 64 of them per lane while the matrix pipes idle.
 __device__ __forceinline__ float silu(float g) { return g * __builtin_amdgcn_rcpf(1.f + __expf(-g)); }
 
-// 4 x 4 transpose across the four lanes of a quad.  In: v[k] = the value of row R + k at this lane's
-// column.  Out: v[k] = the value of row R + (lane % 4) at column 4 * (this lane's column / 4) + k.
-// An MFMA accumulator holds four consecutive rows of ONE column per lane; after the transpose a lane
-// holds four consecutive columns of one row, which is a single 8- or 16-byte store instead of four
-// 2- or 4-byte ones - the epilogue is bound by the number of store instructions, not by bytes.
-__device__ __forceinline__ float quad_xor1(float x) {
-  return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, x), 0xB1, 0xF, 0xF, true));  // quad_perm 1,0,3,2
-}
-__device__ __forceinline__ float quad_xor2(float x) {
-  return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, x), 0x4E, 0xF, 0xF, true));  // quad_perm 2,3,0,1
-}
-__device__ __forceinline__ void quad_transpose(float (&v)[4], int lane) {
-  const bool b0 = (lane & 1) != 0, b1 = (lane & 2) != 0;
-  const float r01 = quad_xor1(b0 ? v[0] : v[1]), r23 = quad_xor1(b0 ? v[2] : v[3]);
-  if (b0) {
-    v[0] = r01;
-    v[2] = r23;
-  } else {
-    v[1] = r01;
-    v[3] = r23;
-  }
-  const float r02 = quad_xor2(b1 ? v[0] : v[2]), r13 = quad_xor2(b1 ? v[1] : v[3]);
-  if (b1) {
-    v[0] = r02;
-    v[1] = r13;
-  } else {
-    v[2] = r02;
-    v[3] = r13;
-  }
+// two outputs rounded to the 16-bit type, packed
+template <typename OutT>
+__device__ __forceinline__ uint32_t pack2(float a, float b) {
+  return (uint32_t)__builtin_bit_cast(uint16_t, (OutT)a) | ((uint32_t)__builtin_bit_cast(uint16_t, (OutT)b) << 16);
 }
 
 // four consecutive outputs of one row as one store
@@ -92,10 +68,7 @@ __device__ __forceinline__ void store4(OutT* dst, const float (&v)[4]) {
   if constexpr (sizeof(OutT) == 4) {
     *reinterpret_cast<float4*>(dst) = float4{v[0], v[1], v[2], v[3]};
   } else {
-    const OutT a = (OutT)v[0], b = (OutT)v[1], c = (OutT)v[2], d = (OutT)v[3];
-    uint2 w;
-    w.x = (uint32_t)__builtin_bit_cast(uint16_t, a) | ((uint32_t)__builtin_bit_cast(uint16_t, b) << 16);
-    w.y = (uint32_t)__builtin_bit_cast(uint16_t, c) | ((uint32_t)__builtin_bit_cast(uint16_t, d) << 16);
+    const uint2 w = {pack2<OutT>(v[0], v[1]), pack2<OutT>(v[2], v[3])};
     *reinterpret_cast<uint2*>(dst) = w;
   }
 }
@@ -107,302 +80,404 @@ __device__ __forceinline__ int xcd_remap(int pid, int nwg) {
   return base + local;
 }
 
-// Tile (32*MT*WM) x 256 x 128 with WM x WN wavefronts; wavefront (wm, wn) owns (32*MT) x (32*NT) as
-// MT x NT accumulators of 32x32, NT = 8 / WN.  In the gate/up pass the 256 B rows of a tile are 128
-// gate channels followed by the 128 up channels of the same outputs, and accumulator columns
-// jn / jn + NT/2 of a wavefront are gate / up of the same 32 outputs, so SiLU(g) * u is applied on
-// the accumulators.
-// Both tiles have 128-byte rows and go global -> LDS directly (1 KB per wavefront instruction =
-// 8 rows); the hardware fixes where a lane's 16 bytes land, so instead of padding, the lane whose
-// bytes land in slot s of row r fetches logical chunk s ^ ((r / 2) % 8) and the fragment reads apply
-// the same XOR: the 16 lanes the LDS checks together for bank conflicts (16 consecutive rows, one
-// logical chunk, 256 bytes = all 64 banks) then hit 16 different slots of 8 row pairs.
-// A wavefront reads (32*MT + 32*NT) x 128 bytes of fragments per k-tile: eight wavefronts of 128 x 64
-// read 192 KB per k-tile next to 64 KB of tile writes, which at the LDS's ~128 bytes a clock is as
-// many LDS clocks as the k-tile has MFMA clocks (2048 per SIMD).
-template <int MT, int NT, int WM, int WN, bool DUAL, typename OutT>
-__global__ __launch_bounds__(64 * WM * WN) void gemm8_kernel(Params p) {
-  constexpr int T = 64 * WM * WN;
-  constexpr int BM = 32 * MT * WM;
-  static_assert(32 * NT * WN == BN && (!DUAL || NT % 2 == 0), "wavefront grid must cover 256 B rows");
-  constexpr int RPR = T / 8;       // tile rows one round of 16-byte requests covers
-  constexpr int NA = BM / RPR;     // rounds (= requests per thread) for the A tile
-  constexpr int NB = BN / RPR;
-  static_assert(RPR % 16 == 0, "the swizzle key of a thread's row must not change from round to round");
-  constexpr int A_BYTES = BM * BK, B_BYTES = BN * BK;
-  extern __shared__ __attribute__((aligned(16))) uint8_t smem8[];
-  uint8_t* sa = smem8;                 // [2][BM][128]
-  uint8_t* sb = smem8 + 2 * A_BYTES;   // [2][256][128]
-  float* s_rows = reinterpret_cast<float*>(smem8 + 2 * A_BYTES + 2 * B_BYTES);  // [BM] row scales of this tile
+// One direct request: 16 bytes per lane from sbase + voff to the KB of LDS at lds_w + OFF (wave-uniform).
+// The instruction is written out: told that a load writes LDS, the compiler waits for every such
+// load in flight before each later LDS read, whatever buffer that read addresses.  (s_nop: a write
+// of m0 needs one wait state before a load that reads it.)
+template <int OFF>
+__device__ __forceinline__ void to_lds(uint32_t voff, const uint8_t* sbase, uint32_t lds_w) {
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"  // m0 is named as clobbered on purpose
+  asm volatile("s_add_u32 m0, %2, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(voff), "s"(sbase), "s"(lds_w), "n"(OFF)
+               : "memory", "m0", "scc");
+#pragma clang diagnostic pop
+}
+
+template <int N>
+struct Const {
+  static constexpr int value = N;
+};
+
+// Tile (128*MH) x 256 x 128 on four wavefronts, one per SIMD, in a 2 x 2 grid; a wavefront owns
+// (64*MH) x 128 as four quadrants of MH x 2 accumulators (32 x 32 each).  Row and column halves of a
+// tile are the unit of everything: the operand tiles are cut into quarters A0, A1 (64*MH rows) and
+// B0, B1 (128 channels) of whole 128-byte rows, and a k-tile is four phases
+//     P1 (A0,B0)   P2 (A0,B1)   P3 (A1,B1)   P4 (A1,B0)
+// of 4*MH MFMAs per wavefront.  The fragments of one quarter are read from LDS in the phase before
+// their first use (P1 reads B1, P2 A1, P3 the next tile's A0, P4 its B0), so after each phase's barrier
+// one quarter's slot is free and is requested again at once, RING tiles ahead: a request has
+// 4*RING - 1 phases to land, and the waits (vmcnt counted, never 0) leave all but the oldest quarter
+// in flight.  What bounds it: with whole tiles double-buffered instead (eight wavefronts of 128 x 64, one
+// barrier and one full wait a k-tile), a k-tile took the 1.3-1.4 us that its 64 KB need to arrive,
+// whatever its height, against 0.86 us of MFMA at the full clock; now the matrix pipes are busy in 75 % of
+// the clocks of the tall tile's loop and epilogue and the shader clock drops to 2.0 GHz under the load.
+// Weights of three blocks in turn, LLaMA-7B shape at 2048 tokens: gate/up pass 171 -> 148 us (2.5 PFLOP/s), down
+// pass 119 -> 92 us, block 313 -> 264 us; at 300 / 512 / 1024 / 4000 tokens 129 -> 107, 148 -> 125, 193 -> 174,
+// 527 -> 491 us.  Holding a whole tile's fragments (A0, A1, B0, B1) takes 96-128 registers next to 256
+// accumulators: hence one wavefront per SIMD, which also reads a third less from LDS per MFMA than
+// two of 128 x 64 would.
+// The weights are the MFMA's first operand, so that an accumulator register holds four consecutive channels of
+// one row: rows are stored 16 bytes at a time without a transpose (the epilogue of a tile, which the matrix
+// pipes wait out: 23 thousand clocks with quad transposes and an address per store, 11 thousand so).
+// In the gate/up pass a B quarter is 64 gate channels followed by the 64 up channels of the same
+// outputs, and the two accumulator columns of a quadrant are gate / up of the same 32 outputs, so
+// SiLU(g) * u is applied on the accumulators.
+// The tiles go global -> LDS directly (1 KB per wavefront instruction = 8 rows); the hardware fixes
+// where a lane's 16 bytes land, so instead of padding, the lane whose bytes land in slot s of row r
+// fetches logical chunk s ^ ((r / 2) % 8) and the fragment reads apply the same XOR: the 16 lanes the
+// LDS checks together for bank conflicts (16 consecutive rows, one logical chunk, 256 bytes = all 64
+// banks) then hit 16 different slots of 8 row pairs.
+template <int MH, int RING, bool DUAL, bool SPLIT, typename OutT>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) void gemm8_kernel(Params p) {
+  constexpr int BM = 128 * MH;
+  constexpr int QA = 64 * MH * BK, QB = 128 * BK;  // bytes of an A and of a B quarter
+  constexpr int TILE = 2 * (QA + QB);
+  constexpr int NA = 2 * MH, NB = 4;               // requests of one wavefront for an A and for a B quarter
+  extern __shared__ __attribute__((aligned(16))) uint8_t smem8[];  // [RING][A0 | A1 | B0 | B1], then the row and channel scales
+  lds_cchar* lds0 = (lds_cchar*)smem8;
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int wm = wave % WM, wn = wave / WM;
+  const int wm = wave & 1, wn = wave >> 1;
   const int ntiles = p.tiles_m * p.tiles_n;
   const int logical = xcd_remap(blockIdx.x, ntiles * p.splits);
-  const int split = logical / ntiles, tile = logical % ntiles;
+  const int split = logical / ntiles, tile_id = logical % ntiles;
   // bands of eight row tiles, rows first: an XCD's 32 consecutive ids are 8 row tiles x 4 column tiles
   // whatever the height of the problem (walking whole columns would pull all of A through its L2 per column tile)
   const int per_band = 8 * p.tiles_n;
-  const int band = tile / per_band, idx = tile - band * per_band;
+  const int band = tile_id / per_band, idx = tile_id - band * per_band;
   const int band_rows = min(8, p.tiles_m - band * 8);
   const int tn = idx / band_rows, tm = band * 8 + (idx - tn * band_rows);
   const int k_begin = split * p.k_per_split;  // this workgroup's k range: [k_begin, k_begin + nk * BK)
+  const int nk = (min(p.k, k_begin + p.k_per_split) - k_begin) / BK;
   const int m0 = tm * BM;
   const int n0 = tn * (DUAL ? BN / 2 : BN);
 
-  // the tile's row scales go to LDS once (rows past m clamped): the epilogue reads them four at a time
-  for (int r = tid; r < BM; r += T) s_rows[r] = p.sa[min(m0 + r, p.m - 1)];
-
-  // ---- global -> LDS requests ----------------------------------------------------------------
-  const int row_in_round = tid >> 3;
-  const int chunk = (tid & 7) ^ ((row_in_round >> 1) & 7);  // logical chunk whose slot this thread fills
-  const uint8_t* a_ptr[NA];
-#pragma unroll
-  for (int i = 0; i < NA; ++i) {
-    const int r = min(m0 + i * RPR + row_in_round, p.m - 1);
-    a_ptr[i] = p.a + (int64_t)r * p.lda + k_begin + chunk * 16;
-  }
-  const uint8_t* b_ptr[NB];
-#pragma unroll
-  for (int i = 0; i < NB; ++i) {
-    const int tr = i * RPR + row_in_round;  // row of the B tile
-    const uint8_t* src = (DUAL && tr >= BN / 2) ? p.b1 : p.b0;
-    const int ch = min(n0 + (DUAL ? tr % (BN / 2) : tr), p.n - 1);
-    b_ptr[i] = src + (int64_t)ch * p.ldb + k_begin + chunk * 16;
-  }
-  // The instruction is written out: told that a load writes LDS, the compiler waits for every such
-  // load in flight before each later LDS read, whatever buffer that read addresses.
-  auto to_lds = [&](const void* src, const uint8_t* dst) {
-    const uint32_t lds_base = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(const lds_u8*)dst);
-#pragma clang diagnostic push
-#pragma clang diagnostic ignored "-Winline-asm"  // m0 is named as clobbered on purpose
-    asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(src), "s"(lds_base) : "memory", "m0");
-#pragma clang diagnostic pop
-  };
-  auto request = [&](int buf, int k0, int e) {  // e < NA: A round e, else B round e - NA
-    if (e < NA) to_lds(a_ptr[e] + k0, sa + buf * A_BYTES + (e * RPR + wave * 8) * BK);
-    else to_lds(b_ptr[e - NA] + k0, sb + buf * B_BYTES + ((e - NA) * RPR + wave * 8) * BK);
-  };
-
-  // ---- fragments -------------------------------------------------------------------------------
-  // lane l: row/column l % 32, logical chunks 4*ks + 2*(l/32) and the next; every fragment starts at
-  // a row that is a multiple of 32, so the swizzle key is (l / 2) % 8 for all of them.
-  const int key = (lane >> 1) & 7;
-  const int frag_row = (lane & 31) * BK;
-  const int c_lane = (lane >> 5) * 2;
-  v8i fa[MT], fb[NT];
-  auto read16 = [&](const uint8_t* tile_base, int row_off, int c) -> u32x4 {
-    return *reinterpret_cast<const u32x4*>(tile_base + row_off + frag_row + ((c ^ key) << 4));
-  };
-  auto read_a = [&](int buf, int ks, int i) {
-    const uint8_t* base = sa + buf * A_BYTES;
-    const int row_off = (wm * MT * 32 + i * 32) * BK;
-    const u32x4 lo = read16(base, row_off, 4 * ks + c_lane), hi = read16(base, row_off, 4 * ks + c_lane + 1);
-    fa[i] = v8i{(int)lo[0], (int)lo[1], (int)lo[2], (int)lo[3], (int)hi[0], (int)hi[1], (int)hi[2], (int)hi[3]};
-  };
-  auto read_b = [&](int buf, int ks, int jn) {
-    const uint8_t* base = sb + buf * B_BYTES;
-    const int row = DUAL ? (jn / (NT / 2)) * (BN / 2) + wn * (16 * NT) + (jn % (NT / 2)) * 32 : wn * (32 * NT) + jn * 32;
-    const u32x4 lo = read16(base, row * BK, 4 * ks + c_lane), hi = read16(base, row * BK, 4 * ks + c_lane + 1);
-    fb[jn] = v8i{(int)lo[0], (int)lo[1], (int)lo[2], (int)lo[3], (int)hi[0], (int)hi[1], (int)hi[2], (int)hi[3]};
-  };
-
-  // this lane's output columns and their channel scales (fetched now, used in the epilogue)
-  int col[NT];
-  float sc[NT];
-#pragma unroll
-  for (int jn = 0; jn < NT; ++jn) {
-    col[jn] = DUAL ? n0 + wn * (16 * NT) + (jn % (NT / 2)) * 32 + (lane & 31) : n0 + wn * (32 * NT) + jn * 32 + (lane & 31);
-    const float* s = (DUAL && jn >= NT / 2) ? p.sb1 : p.sb0;
-    sc[jn] = col[jn] < p.n ? s[col[jn]] : 0.f;
-  }
-
-  f32x16 acc[MT][NT];
-#pragma unroll
-  for (int i = 0; i < MT; ++i)
-#pragma unroll
-    for (int jn = 0; jn < NT; ++jn)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) acc[i][jn][r] = 0.f;
-
-  // One k-step (64 codes): MT x NT MFMAs, column by column.  A fragment register is reloaded for the
-  // next k-step right after its last use - fb[jn] after column jn, fa[i] after MFMA (i, NT-1) - so one
-  // set of fragment registers serves as its own double buffer and every fragment is requested at
-  // least MT - 1 MFMAs (200 cycles and more) ahead of its first use.
-  // `mid` runs once after column 0, before the first reload; per_slot(q) after MFMA number q.
-  auto k_step = [&](int next_buf, int next_ks, auto&& mid, auto&& per_slot) {
-#pragma unroll
-    for (int jn = 0; jn < NT; ++jn) {
-#pragma unroll
-      for (int i = 0; i < MT; ++i) {
-        acc[i][jn] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(fa[i], fb[jn], acc[i][jn], 0, 0, 0, 0, 0, 0);
-        if (jn == NT - 1) read_a(next_buf, next_ks, i);
-        per_slot(jn * MT + i);
-        __builtin_amdgcn_sched_barrier(0);
-      }
-      if (jn == 0) mid();
-      read_b(next_buf, next_ks, jn);
-      __builtin_amdgcn_sched_barrier(0);
-    }
-  };
-
-  const int nk = (min(p.k, k_begin + p.k_per_split) - k_begin) / BK;
-  // Tiles kt (being multiplied), kt+1 (landed in the other buffer) and kt+2 (in flight into the
-  // buffer of kt) are live at once.  The one barrier of a k-tile sits in its second k-step, after
-  // column 0: by then this wavefront has read the last fragment of tile kt (the wait for it is
-  // covered by those MFMAs) and waits for its own requests of tile kt+1; past the barrier every
-  // wavefront has done both, so tile kt+1 may be read and the buffer of tile kt refilled.
+  // The tile's row and channel scales go to LDS now (clamped past the end): fetched after the loop they
+  // would cost two memory round trips with the matrix pipes idle.
+  float* s_rows = reinterpret_cast<float*>(smem8 + RING * TILE);  // [BM]
+  float* s_cols = s_rows + BM;                                    // [256], in the order of the tile's B rows
+  for (int r = tid; r < BM; r += 256) s_rows[r] = p.sa[min(m0 + r, p.m - 1)];
   {
+    const int h = tid >> 7, r = tid & 127;
+    const int ch = min(n0 + (DUAL ? h * 64 + (r & 63) : tid), p.n - 1);
+    s_cols[tid] = (DUAL && r >= 64 ? p.sb1 : p.sb0)[ch];
+  }
+
+  // ---- requests: instruction e of a quarter brings its rows 32 e + 8 wave + lane / 8; rows and channels
+  // past the end are clamped (their products are not stored) ----
+  const int q_row = wave * 8 + (lane >> 3);
+  const int chunk = (lane & 7) ^ ((q_row >> 1) & 7);  // logical chunk whose slot this lane fills
+  uint32_t va[2][NA], vb[2][NB];                      // byte offsets from the tile's first row / channel
 #pragma unroll
-    for (int e = 0; e < NA + NB; ++e) request(0, 0, e);
-    if (nk > 1) {
+  for (int h = 0; h < 2; ++h) {
 #pragma unroll
-      for (int e = 0; e < NA + NB; ++e) request(1, BK, e);
+    for (int e = 0; e < NA; ++e)
+      va[h][e] = (uint32_t)min(h * 64 * MH + e * 32 + q_row, p.m - 1 - m0) * (uint32_t)p.lda + chunk * 16;
+#pragma unroll
+    for (int e = 0; e < NB; ++e) {
+      const int r = e * 32 + q_row;
+      vb[h][e] = (uint32_t)min(DUAL ? h * 64 + (r & 63) : h * 128 + r, p.n - 1 - n0) * (uint32_t)p.ldb + chunk * 16;
     }
   }
-  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-  __syncthreads();
-#pragma unroll
-  for (int i = 0; i < MT; ++i) read_a(0, 0, i);
-#pragma unroll
-  for (int jn = 0; jn < NT; ++jn) read_b(0, 0, jn);
+  const uint8_t* base_a = p.a + (int64_t)m0 * p.lda + k_begin;
+  const uint8_t* base_b0 = p.b0 + (int64_t)n0 * p.ldb + k_begin;
+  const uint8_t* base_b1 = DUAL ? p.b1 + (int64_t)n0 * p.ldb + k_begin : base_b0;
+  const uint32_t lds_w = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)lds0 + wave * 1024);
+  // request e of quarter Q (0 A0, 1 B0, 2 B1, 3 A1) of tile t (past the last one: the last again) into ring slot S
+  auto request = [&](auto s_c, auto q_c, auto e_c, int t) {
+    constexpr int S = decltype(s_c)::value, Q = decltype(q_c)::value, E = decltype(e_c)::value;
+    const int koff = min(t, nk - 1) * BK;
+    if constexpr (Q == 0 || Q == 3) {
+      if constexpr (E < NA) to_lds<S * TILE + (Q ? QA : 0) + E * 4096>(va[Q ? 1 : 0][E], base_a + koff, lds_w);
+    } else {
+      to_lds<S * TILE + 2 * QA + (Q - 1) * QB + E * 4096>(vb[Q - 1][E], (DUAL && E >= 2 ? base_b1 : base_b0) + koff, lds_w);
+    }
+  };
+  auto request_all = [&](auto s_c, auto q_c, int t) {
+    request(s_c, q_c, Const<0>{}, t);
+    request(s_c, q_c, Const<1>{}, t);
+    request(s_c, q_c, Const<2>{}, t);
+    request(s_c, q_c, Const<3>{}, t);
+  };
 
-  for (int kt = 0; kt < nk; ++kt) {
-    const int buf = kt & 1;
-    const int k2 = (kt + 2) * BK;
-    const bool more = kt + 2 < nk;  // requests past the last tile are skipped (the waits are explicit)
-    // first k-step: reloads fetch the second k-step of the same tile
-    k_step(buf, 1, [] {}, [](int) {});
-    // second k-step: barrier after column 0, then reloads from tile kt+1 and the requests of tile kt+2
-    k_step(
-        buf ^ 1, 0,
-        [&] {
-          asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
-          __builtin_amdgcn_s_barrier();
-          __builtin_amdgcn_sched_barrier(0);
-        },
-        [&](int slot) {
-          // the slots of columns 1 .. NT-1 come after the barrier: NA + NB requests spread over them
-          if (slot >= MT) {
-            constexpr int kAfter = MT * (NT - 1);
-            constexpr int per = (NA + NB + kAfter - 1) / kAfter;
+  // ---- fragments: lane l holds row / channel l % 32, logical chunks 4 ks + 2 (l / 32) and the next; every
+  // fragment starts at a row that is a multiple of 32, so the swizzle key is (l / 2) % 8 for all of them.
+  // An LDS instruction reaches 64 KB past its address register: one register per 64 KB. ----
+  constexpr int kReach = (RING * TILE + 65535) / 65536;
+  lds_cchar* fa_base[kReach][4];
+  lds_cchar* fb_base[kReach][4];
+  {
+    const int key = (lane >> 1) & 7;
 #pragma unroll
-            for (int e = (slot - MT) * per; e < (slot - MT + 1) * per; ++e)
-              if (e < NA + NB && more) request(buf, k2, e);
-          }
-        });
+    for (int w = 0; w < kReach; ++w)
+#pragma unroll
+      for (int cc = 0; cc < 4; ++cc) {
+        const int c = 4 * (cc >> 1) + 2 * (lane >> 5) + (cc & 1);
+        const int off = (lane & 31) * BK + ((c ^ key) << 4) + w * 65536;
+        fa_base[w][cc] = lds0 + wm * (32 * MH) * BK + off;
+        fb_base[w][cc] = lds0 + wn * (DUAL ? 32 : 64) * BK + off;
+      }
   }
+  v8i fa[2][MH][2], fb[2][2][2];  // [half or register set][fragment][k-step]
+  // one 16-byte read: number i of quarter Q's 8 (A: 4 MH), into register set `set`
+  auto read_one = [&](auto s_c, auto q_c, auto set_c, auto i_c) {
+    constexpr int S = decltype(s_c)::value, Q = decltype(q_c)::value, SET = decltype(set_c)::value, I = decltype(i_c)::value;
+    constexpr int F = I >> 2, CC = I & 3;
+    if constexpr (Q == 0 || Q == 3) {
+      if constexpr (F < MH) {
+        constexpr int OFF = S * TILE + (Q ? QA : 0) + F * 32 * BK;
+        const u32x4 v = *reinterpret_cast<lds_cu32x4*>(fa_base[OFF >> 16][CC] + (OFF & 65535));
+#pragma unroll
+        for (int w = 0; w < 4; ++w) fa[SET][F][CC >> 1][(CC & 1) * 4 + w] = (int)v[w];
+      }
+    } else {
+      constexpr int OFF = S * TILE + 2 * QA + (Q - 1) * QB + F * (DUAL ? 64 : 32) * BK;
+      const u32x4 v = *reinterpret_cast<lds_cu32x4*>(fb_base[OFF >> 16][CC] + (OFF & 65535));
+#pragma unroll
+      for (int w = 0; w < 4; ++w) fb[SET][F][CC >> 1][(CC & 1) * 4 + w] = (int)v[w];
+    }
+  };
+  auto read_all = [&](auto s_c, auto q_c, auto set_c) {
+    read_one(s_c, q_c, set_c, Const<0>{});
+    read_one(s_c, q_c, set_c, Const<1>{});
+    read_one(s_c, q_c, set_c, Const<2>{});
+    read_one(s_c, q_c, set_c, Const<3>{});
+    read_one(s_c, q_c, set_c, Const<4>{});
+    read_one(s_c, q_c, set_c, Const<5>{});
+    read_one(s_c, q_c, set_c, Const<6>{});
+    read_one(s_c, q_c, set_c, Const<7>{});
+  };
 
-  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // nothing may land in LDS after the workgroup has gone
+  f32x16 acc[2][MH][2][2];  // [row half][row fragment][column half][column fragment]
+#pragma unroll
+  for (int i = 0; i < 8 * MH; ++i)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) (&acc[0][0][0][0])[i][r] = 0.f;
+
+  // Quarters in the order they are requested and read: u = 4 t + {0 A0, 1 B0, 2 B1, 3 A1} of tile t.
+  // Requests of the n quarters after quarter u:
+  constexpr auto in_flight = [](int u, int n) {
+    int c = 0;
+    for (int i = 1; i <= n; ++i) c += ((u + i) % 4 == 0 || (u + i) % 4 == 3) ? NA : NB;
+    return c;
+  };
+  // One phase: quadrant (HA, HB) of the tile whose B halves sit in register sets PAR (B0) and 1 - PAR (B1);
+  // reads quarter RQ from ring slot RS into register set RSET; requests quarter GQ of tile gt into slot GS.
+  auto phase = [&](auto ha_c, auto hb_c, auto bset_c, auto rs_c, auto rq_c, auto rset_c, auto gs_c, auto gq_c, int gt) {
+    constexpr int HA = decltype(ha_c)::value, HB = decltype(hb_c)::value, BS = decltype(bset_c)::value;
+    auto slot = [&](auto q_c) {
+      constexpr int q = decltype(q_c)::value;
+      constexpr int ks = q / (2 * MH), i = (q % (2 * MH)) / 2, j = q % 2;
+      acc[HA][i][HB][j] =
+          __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(fb[BS][j][ks], fa[HA][i][ks], acc[HA][i][HB][j], 0, 0, 0, 0, 0, 0);
+      // the eight reads (four for a short A quarter) go with the first MFMAs, so that they have
+      // landed when the phase ends; the requests one to an MFMA from the first
+      if constexpr (q < 4) {
+        read_one(rs_c, rq_c, rset_c, Const<2 * (q & 3)>{});
+        read_one(rs_c, rq_c, rset_c, Const<2 * (q & 3) + 1>{});
+        request(gs_c, gq_c, Const<(q & 3)>{}, gt);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    };
+    slot(Const<0>{});
+    slot(Const<1>{});
+    slot(Const<2>{});
+    slot(Const<3>{});
+    if constexpr (MH == 2) {
+      slot(Const<4>{});
+      slot(Const<5>{});
+      slot(Const<6>{});
+      slot(Const<7>{});
+    }
+    // the quarter the next phase reads has landed (this wavefront's part), this phase's reads are in registers
+    constexpr int RQ = decltype(rq_c)::value;
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(in_flight(RQ + 1, 4 * RING - 2)) : "memory");
+    __builtin_amdgcn_sched_barrier(0);
+  };
+
+  // Prologue: the first RING tiles requested, A0 and B0 of tile 0 read, A0 of tile RING requested.
+  auto prologue = [&](auto s_c) {
+    constexpr int S = decltype(s_c)::value;
+    if constexpr (S < RING) {
+      request_all(s_c, Const<0>{}, S);
+      request_all(s_c, Const<1>{}, S);
+      request_all(s_c, Const<2>{}, S);
+      request_all(s_c, Const<3>{}, S);
+    }
+  };
+  prologue(Const<0>{});
+  prologue(Const<1>{});
+  prologue(Const<2>{});
+  asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(in_flight(2, 4 * RING - 3)) : "memory");  // quarters 0, 1, 2 have landed
+  __builtin_amdgcn_sched_barrier(0);
+  read_all(Const<0>{}, Const<0>{}, Const<0>{});
+  read_all(Const<0>{}, Const<1>{}, Const<0>{});
+  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+  __builtin_amdgcn_sched_barrier(0);
+  request_all(Const<0>{}, Const<0>{}, RING);
+
+  auto k_tile = [&](auto s_c, auto par_c, int t) {
+    constexpr int S = decltype(s_c)::value, PAR = decltype(par_c)::value, S1 = (S + 1) % RING;
+    typedef Const<0> C0;
+    typedef Const<1> C1;
+    //    quadrant        B regs            reads                                  requests
+    phase(C0{}, C0{}, Const<PAR>{}, s_c, Const<2>{}, Const<1 - PAR>{}, s_c, Const<1>{}, t + RING);
+    phase(C0{}, C1{}, Const<1 - PAR>{}, s_c, Const<3>{}, C1{}, s_c, Const<2>{}, t + RING);
+    phase(C1{}, C1{}, Const<1 - PAR>{}, Const<S1>{}, Const<0>{}, C0{}, s_c, Const<3>{}, t + RING);
+    phase(C1{}, C0{}, Const<PAR>{}, Const<S1>{}, Const<1>{}, Const<1 - PAR>{}, Const<S1>{}, Const<0>{}, t + 1 + RING);
+  };
+  if constexpr (RING == 2) {
+    int t = 0;
+    for (; t + 1 < nk; t += 2) {
+      k_tile(Const<0>{}, Const<0>{}, t);
+      k_tile(Const<1>{}, Const<1>{}, t + 1);
+    }
+    if (t < nk) k_tile(Const<0>{}, Const<0>{}, t);
+  } else {
+    int t = 0;
+    for (; t + 5 < nk; t += 6) {
+      k_tile(Const<0>{}, Const<0>{}, t);
+      k_tile(Const<1>{}, Const<1>{}, t + 1);
+      k_tile(Const<2>{}, Const<0>{}, t + 2);
+      k_tile(Const<0>{}, Const<1>{}, t + 3);
+      k_tile(Const<1>{}, Const<0>{}, t + 4);
+      k_tile(Const<2>{}, Const<1>{}, t + 5);
+    }
+    if (t < nk) k_tile(Const<0>{}, Const<0>{}, t);
+    if (t + 1 < nk) k_tile(Const<1>{}, Const<1>{}, t + 1);
+    if (t + 2 < nk) k_tile(Const<2>{}, Const<0>{}, t + 2);
+    if (t + 3 < nk) k_tile(Const<0>{}, Const<1>{}, t + 3);
+    if (t + 4 < nk) k_tile(Const<1>{}, Const<0>{}, t + 4);
+  }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // nothing may land in LDS after this
+  __syncthreads();
 
   // ---- epilogue ----------------------------------------------------------------------------------
-  // acc[i][jn][r]: row m0 + wm*MT*32 + i*32 + (r/4)*8 + (lane/32)*4 + r%4, column lane % 32 of fragment jn
-  OutT* c = reinterpret_cast<OutT*>(p.c);
-  const int row_base = m0 + wm * MT * 32 + (lane >> 5) * 4;
-  if constexpr (!DUAL) {
-    if (p.splits > 1) {
-      // raw accumulators to this split's slab, four consecutive columns of a row per store (n % 4 == 0)
-      float* mine = p.slabs + (int64_t)split * p.m * p.n;
-      const int my_row = row_base + (lane & 3);
-      const int col_shift = ((lane & 31) & ~3) - (lane & 31);
+  // acc[ha][i][hb][j][r]: row m0 + ha*64*MH + wm*32*MH + i*32 + lane%32, channel (r/4)*8 + (lane/32)*4 + r%4 of its
+  // fragment: a lane owns whole runs of four channels of one row.  The matrix pipes idle meanwhile, so a
+  // lane's first address is computed once, every other one is a wave-uniform distance away, and only tiles at
+  // the right and lower edge check bounds.
+  constexpr int JN = DUAL ? 1 : 2;          // output fragments of a quadrant
+  constexpr int HC = DUAL ? 64 : 128;       // output channels of a column half
+  const int c_row = m0 + wm * 32 * MH + (lane & 31), c_col = n0 + wn * (DUAL ? 32 : 64);
+  const int hi = lane >> 5;
+  if constexpr (SPLIT) {
+    // raw accumulators to this split's slab (n % 4 == 0)
+    float* mine = p.slabs + (int64_t)split * p.m * p.n + (int64_t)c_row * p.n + c_col + hi * 4;
 #pragma unroll
-      for (int i = 0; i < MT; ++i)
+    for (int ha = 0; ha < 2; ++ha)
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          const int row = my_row + i * 32 + q * 8;
+      for (int i = 0; i < MH; ++i) {
+        float* dst = mine + (int64_t)(ha * 64 * MH + i * 32) * p.n;
+        if (c_row + ha * 64 * MH + i * 32 >= p.m) continue;
 #pragma unroll
-          for (int jn = 0; jn < NT; ++jn) {
-            float v[4];
+        for (int hb = 0; hb < 2; ++hb)
 #pragma unroll
-            for (int k = 0; k < 4; ++k) v[k] = acc[i][jn][q * 4 + k];
-            quad_transpose(v, lane);
-            const int c0 = col[jn] + col_shift;
-            if (row < p.m && c0 < p.n) *reinterpret_cast<float4*>(mine + (int64_t)row * p.n + c0) = float4{v[0], v[1], v[2], v[3]};
-          }
-        }
-      return;
-    }
-  }
-  // Row scales from the LDS copy made at the start (visible since the loop's barriers): four
-  // consecutive rows per read.  One global load per row here would put 16 * MT loads per lane
-  // through the CU's address unit while the matrix pipes idle.
-  float sr[MT][16];
+          for (int j = 0; j < 2; ++j)
 #pragma unroll
-  for (int i = 0; i < MT; ++i)
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const float4 v = *reinterpret_cast<const float4*>(s_rows + wm * MT * 32 + (lane >> 5) * 4 + i * 32 + q * 8);
-      sr[i][q * 4 + 0] = v.x;
-      sr[i][q * 4 + 1] = v.y;
-      sr[i][q * 4 + 2] = v.z;
-      sr[i][q * 4 + 3] = v.w;
-    }
-  if (p.n % 4 == 0 && p.ldc % 4 == 0) {
-    // rows of four: quad-transposed so that every lane writes four consecutive columns of one row
-    const int my_row = row_base + (lane & 3);            // + i * 32 + q * 8
-    const int col_shift = ((lane & 31) & ~3) - (lane & 31);  // this lane's first column after the transpose
-#pragma unroll
-    for (int i = 0; i < MT; ++i)
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        const int row = my_row + i * 32 + q * 8;
-        const bool row_ok = row < p.m;
-#pragma unroll
-        for (int jn = 0; jn < (DUAL ? NT / 2 : NT); ++jn) {
-          float v[4];
-#pragma unroll
-          for (int k = 0; k < 4; ++k) {
-            const int r = q * 4 + k;
-            if constexpr (DUAL) {
-              const float g = acc[i][jn][r] * sr[i][r] * sc[jn], u = acc[i][jn + NT / 2][r] * sr[i][r] * sc[jn + NT / 2];
-              v[k] = silu(g) * u;
-            } else {
-              v[k] = acc[i][jn][r] * sr[i][r] * sc[jn];
+            for (int q = 0; q < 4; ++q) {
+              const f32x16& t = acc[ha][i][hb][j];
+              const int cc = hb * HC + j * 32 + q * 8;
+              if (c_col + hi * 4 + cc < p.n)
+                *reinterpret_cast<float4*>(dst + cc) = float4{t[q * 4], t[q * 4 + 1], t[q * 4 + 2], t[q * 4 + 3]};
             }
+      }
+  } else {
+    float sr[2][MH];  // this lane's row scales
+#pragma unroll
+    for (int ha = 0; ha < 2; ++ha)
+#pragma unroll
+      for (int i = 0; i < MH; ++i) sr[ha][i] = s_rows[wm * 32 * MH + ha * 64 * MH + i * 32 + (lane & 31)];
+    OutT* c = reinterpret_cast<OutT*>(p.c);
+    auto finish = [&](auto check_c) {
+      constexpr bool CHECK = decltype(check_c)::value != 0;
+      constexpr int VEC = 16 / (int)sizeof(OutT);  // elements of a lane's store
+      const bool vec = !CHECK || (p.n % VEC == 0 && p.ldc % VEC == 0);
+      OutT* lane_c = c + (int64_t)c_row * p.ldc + c_col + hi * VEC;
+#pragma unroll
+      for (int hb = 0; hb < 2; ++hb)
+#pragma unroll
+        for (int j = 0; j < JN; ++j) {
+          const int cc0 = hb * HC + j * 32;
+          float s0[16], s1[16];  // channel scales of this fragment (gate, up)
+#pragma unroll
+          for (int q = 0; q < 4; ++q) {
+            const float* src = s_cols + hb * 128 + (DUAL ? wn * 32 : wn * 64 + j * 32) + q * 8 + hi * 4;
+            *reinterpret_cast<float4*>(&s0[q * 4]) = *reinterpret_cast<const float4*>(src);
+            if constexpr (DUAL) *reinterpret_cast<float4*>(&s1[q * 4]) = *reinterpret_cast<const float4*>(src + 64);
           }
-          quad_transpose(v, lane);
-          const int c0 = col[jn] + col_shift;
-          if (row_ok && c0 < p.n) store4<OutT>(c + (int64_t)row * p.ldc + c0, v);
+#pragma unroll
+          for (int ha = 0; ha < 2; ++ha)
+#pragma unroll
+            for (int i = 0; i < MH; ++i) {
+              const int rr = ha * 64 * MH + i * 32;
+              OutT* dst = lane_c + (int64_t)rr * p.ldc + cc0;
+              float v[16];
+#pragma unroll
+              for (int r = 0; r < 16; ++r) {
+                if constexpr (DUAL) {
+                  const float g = acc[ha][i][hb][0][r] * sr[ha][i] * s0[r], u = acc[ha][i][hb][1][r] * sr[ha][i] * s1[r];
+                  v[r] = silu(g) * u;
+                } else {
+                  v[r] = acc[ha][i][hb][j][r] * sr[ha][i] * s0[r];
+                }
+              }
+              if (vec) {
+                if (CHECK && c_row + rr >= p.m) continue;
+                if constexpr (sizeof(OutT) == 4) {
+#pragma unroll
+                  for (int q = 0; q < 4; ++q)
+                    if (!CHECK || c_col + hi * 4 + cc0 + q * 8 < p.n)
+                      *reinterpret_cast<float4*>(dst + q * 8) = float4{v[q * 4], v[q * 4 + 1], v[q * 4 + 2], v[q * 4 + 3]};
+                } else {
+                  // the two halves of the wavefront trade runs, so that a lane stores eight channels at once
+#pragma unroll
+                  for (int q = 0; q < 4; q += 2) {
+                    uint32_t w[2][2];
+#pragma unroll
+                    for (int d = 0; d < 2; ++d) {
+                      typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+                      const u32x2 x = __builtin_amdgcn_permlane32_swap(pack2<OutT>(v[q * 4 + 2 * d], v[q * 4 + 2 * d + 1]),
+                                                                       pack2<OutT>(v[q * 4 + 4 + 2 * d], v[q * 4 + 5 + 2 * d]), false, false);
+                      w[0][d] = x[0];
+                      w[1][d] = x[1];
+                    }
+                    if (!CHECK || c_col + hi * 8 + cc0 + q * 8 < p.n)
+                      *reinterpret_cast<u32x4*>(dst + q * 8) = u32x4{w[0][0], w[0][1], w[1][0], w[1][1]};
+                  }
+                }
+              } else {
+#pragma unroll
+                for (int r = 0; r < 16; ++r) {
+                  const int col = c_col + cc0 + (r >> 2) * 8 + hi * 4 + (r & 3);
+                  if (c_row + rr < p.m && col < p.n) c[(int64_t)(c_row + rr) * p.ldc + col] = (OutT)v[r];
+                }
+              }
+            }
         }
-      }
-    return;
+    };
+    if (m0 + BM <= p.m && n0 + (DUAL ? BN / 2 : BN) <= p.n && p.ldc % (16 / (int)sizeof(OutT)) == 0) finish(Const<0>{});
+    else finish(Const<1>{});
   }
-#pragma unroll
-  for (int i = 0; i < MT; ++i)
-#pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      const int row = row_base + i * 32 + (r >> 2) * 8 + (r & 3);
-      const bool row_ok = row < p.m;
-      if constexpr (DUAL) {
-#pragma unroll
-        for (int jn = 0; jn < NT / 2; ++jn) {
-          const float g = acc[i][jn][r] * sr[i][r] * sc[jn], u = acc[i][jn + NT / 2][r] * sr[i][r] * sc[jn + NT / 2];
-          if (row_ok && col[jn] < p.n) c[(int64_t)row * p.ldc + col[jn]] = (OutT)(silu(g) * u);
-        }
-      } else {
-#pragma unroll
-        for (int jn = 0; jn < NT; ++jn)
-          if (row_ok && col[jn] < p.n) c[(int64_t)row * p.ldc + col[jn]] = (OutT)(acc[i][jn][r] * sr[i][r] * sc[jn]);
-      }
-    }
 }
 
-template <int MT, int NT, int WM, int WN, bool DUAL, typename OutT>
+template <int MH, bool DUAL, typename OutT, bool SPLIT = false>
 int launch(Params p, hipStream_t st) {
-  constexpr int BM = 32 * MT * WM;
+  constexpr int BM = 128 * MH;
+  constexpr int RING = MH == 2 ? 2 : 3;  // 128 or 144 KB of LDS
   p.tiles_m = (p.m + BM - 1) / BM;
   const int bn_out = DUAL ? BN / 2 : BN;
   p.tiles_n = (p.n + bn_out - 1) / bn_out;
-  const size_t smem = 2 * (size_t)(BM * BK + BN * BK) + BM * sizeof(float);
-  auto kern = gemm8_kernel<MT, NT, WM, WN, DUAL, OutT>;
+  const size_t smem = (size_t)RING * (BM + BN) * BK + (BM + BN) * sizeof(float);
+  auto kern = gemm8_kernel<MH, RING, DUAL, SPLIT, OutT>;
   static std::atomic<bool> attr_set{false};  // per instantiation; callers hold the dispatch lock
   if (!attr_set.load(std::memory_order_acquire)) {
     PTO_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
                                       (int)smem));
     attr_set.store(true, std::memory_order_release);
   }
-  hipLaunchKernelGGL(kern, dim3(p.tiles_m * p.tiles_n * p.splits), dim3(64 * WM * WN), smem, st, p);
+  hipLaunchKernelGGL(kern, dim3(p.tiles_m * p.tiles_n * p.splits), dim3(256), smem, st, p);
   PTO_CHECK_HIP(hipGetLastError());
   return PTO_HIP_OK;
 }
@@ -430,18 +505,11 @@ __global__ __launch_bounds__(256) void gemm8_finish_kernel(const float* __restri
   }
 }
 
-// Tile height: 256 rows unless that leaves CUs idle and 128 rows do not; eight wavefronts (two per
-// SIMD).  Four wavefronts of 128 x 128 on the tall tile read a third less from LDS per MFMA but
-// leave a SIMD nothing to issue while its one wavefront waits (LLaMA-7B block: 361 us against 334 us
-// when it was measured; rebuilt as the 16-bit GEMM's four-wavefront form is - five rotating stages of
-// 64 codes, requests three iterations ahead, a loop of loop-invariant addresses plus immediates -
-// it gave the same bits in 309 us against 293: with 64-byte rows the tiles cost twice the L2
-// requests and the wavefronts wait on them for 63 % of their cycles.  That form is not built).
+// Tile height: 256 rows unless that leaves CUs idle and 128 rows do not.
 // A single-operand pass whose tall tiles fill less than half the CUs splits k instead of halving the
-// tile: a k-tile takes a workgroup the same ~1.4 us with 128 rows as with 256 (the tile's arrival,
-// not the MFMAs, sets it), so two workgroups per 256 x 256 tile do the same work in half the k-tiles.
+// tile: a k-tile of 128 rows draws three quarters of the bytes for half the products.
 // At exactly half (the LLaMA-7B down pass at 2048 tokens: 128 tall tiles on 256 CUs) the 128-row
-// tiles fill every CU in one round and need neither slabs nor a finish launch: block 293 -> 279 us.
+// tiles fill every CU in one round and need neither slabs nor a finish launch (block 268 us; 272 split in two).
 template <bool DUAL, typename OutT>
 int launch_any(const Params& p0, hipStream_t st) {
   Params p = p0;
@@ -464,7 +532,7 @@ int launch_any(const Params& p0, hipStream_t st) {
       const int rc = pto_hip::gemm_workspace((size_t)p.splits * p.m * p.n * sizeof(float), &ws);
       if (rc) return rc;
       p.slabs = reinterpret_cast<float*>(ws);
-      const int rc2 = launch<4, 2, 2, 4, DUAL, OutT>(p, st);
+      const int rc2 = launch<2, DUAL, float, true>(p, st);
       if (rc2) return rc2;
       const unsigned bx = (unsigned)((p.n / 4 + 255) / 256);
       const unsigned by = (unsigned)std::min<int64_t>(p.m, std::max<int64_t>(1, 4096 / bx));
@@ -474,8 +542,9 @@ int launch_any(const Params& p0, hipStream_t st) {
       return PTO_HIP_OK;
     }
   }
-  if (tall < num_cu && p.m > 128) return launch<2, 2, 2, 4, DUAL, OutT>(p, st);
-  return launch<4, 2, 2, 4, DUAL, OutT>(p, st);
+  const int64_t variant = pto_hip::ctx().gemm_variant;  // 4 and 5 force a tile height
+  if (variant == 5 || (variant != 4 && tall < num_cu && p.m > 128)) return launch<1, DUAL, OutT>(p, st);
+  return launch<2, DUAL, OutT>(p, st);
 }
 
 // ---- row kernels: (RMSNorm +) per-row e4m3 quantisation -----------------------------------------

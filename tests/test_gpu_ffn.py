@@ -648,6 +648,40 @@ def test_ffn_block_fp8_llama7b_shape_rows_and_distance_to_16_bit(worker):
     assert 1e-3 < rel < 0.08, rel
 
 
+@pytest.mark.parametrize("variant", [4, 5])  # 256- and 128-row tiles
+@pytest.mark.parametrize("m,n", [(1, 256), (129, 72), (257, 37), (384, 264)])
+def test_gemm_fp8_tile_edges_and_k_tile_counts(worker, variant, m, n):
+    """Every remainder of the k loop's unroll (1 to 8 and 13 k-tiles of 128), ragged rows and channels, in both tile
+    heights.  Small-integer operands with power-of-two scales make the product exact whatever the order of the
+    sums: equal to the integer product, and its 16-bit rounding; the gate/up pass within one 16-bit ulp."""
+    _lib, lib, code = _fp8_stage_lib()
+    g = torch.Generator().manual_seed(m + n)
+    worker.set_option("gemm_variant", variant)
+    try:
+        for k in [128 * t for t in (1, 2, 3, 4, 5, 6, 7, 8, 13)]:
+            a = torch.randint(-3, 4, (m, k), generator=g).float()
+            w = torch.randint(-3, 4, (n, k), generator=g).float()
+            u = torch.randint(-3, 4, (n, k), generator=g).float()
+            a8, w8, u8 = (t.to(torch.float8_e4m3fn).cuda() for t in (a, w, u))
+            sa, sw = torch.full((m,), 0.0625, device="cuda"), torch.full((n,), 0.25, device="cuda")
+            want = (a @ w.t()) * 0.015625
+            for dt in (torch.float32, torch.bfloat16):
+                out = torch.full((m, n), float("nan"), dtype=dt, device="cuda")
+                _lib.check(lib.pto_hip_projection_fp8(a8.data_ptr(), sa.data_ptr(), w8.data_ptr(), sw.data_ptr(),
+                                                      out.data_ptr(), m, k, n, code(dt), 0))
+                worker.sync()
+                assert torch.equal(out.cpu(), want.to(dt)), (k, dt)
+            h = torch.full((m, n), float("nan"), dtype=torch.bfloat16, device="cuda")
+            _lib.check(lib.pto_hip_gate_up_swiglu_fp8(a8.data_ptr(), sa.data_ptr(), w8.data_ptr(), sw.data_ptr(),
+                                                      u8.data_ptr(), sw.data_ptr(), h.data_ptr(), m, k, n,
+                                                      code(torch.bfloat16), 0))
+            worker.sync()
+            ref = oracle.swiglu(want, (a @ u.t()) * 0.015625)
+            validate_golden({"h": h.cpu().float()}, {"h": ref}, rtol=8e-3, atol=1e-6)  # one bf16 ulp is 2^-7
+    finally:
+        worker.set_option("gemm_variant", 0)
+
+
 @pytest.mark.parametrize("m,k,n,splits", [(2048, 11008, 4096, 2),    # the LLaMA-7B down pass, split in two
                                           (1024, 11008, 4096, 0),    # ... at 1024 tokens: the library's own choice (4)
                                           (300, 4096, 520, 3), (257, 4096, 256, 4), (1000, 2048, 1024, 2)])
