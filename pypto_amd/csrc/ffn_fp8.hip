@@ -44,9 +44,9 @@ struct Params {
   int64_t lda, ldb, ldc;
   int m, n, k;
   int tiles_m, tiles_n;
-  // k split over `splits` workgroups per output tile (single-operand pass only): each writes its raw
-  // fp32 accumulators to its own slab [split][m][n]; gemm8_finish_kernel sums the slabs in split
-  // order and applies the scales.  splits == 1: the epilogue finishes the tile.
+  // k split over `splits` workgroups per output tile: each writes its raw fp32 accumulators to its own slab
+  // ([split][m][n]; in the gate/up pass [split][2][m][n], gate then up); a finish kernel sums the slabs in
+  // split order and applies the scales.  splits == 1: the epilogue finishes the tile.
   int splits, k_per_split;
   float* slabs;
 };
@@ -364,7 +364,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
   const int hi = lane >> 5;
   if constexpr (SPLIT) {
     // raw accumulators to this split's slab (n % 4 == 0)
-    float* mine = p.slabs + (int64_t)split * p.m * p.n + (int64_t)c_row * p.n + c_col + hi * 4;
+    const int64_t mn = (int64_t)p.m * p.n;
+    float* mine = p.slabs + (int64_t)split * (DUAL ? 2 : 1) * mn + (int64_t)c_row * p.n + c_col + hi * 4;
 #pragma unroll
     for (int ha = 0; ha < 2; ++ha)
 #pragma unroll
@@ -378,9 +379,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
               const f32x16& t = acc[ha][i][hb][j];
-              const int cc = hb * HC + j * 32 + q * 8;
+              const int cc = hb * HC + (DUAL ? 0 : j * 32) + q * 8;
               if (c_col + hi * 4 + cc < p.n)
-                *reinterpret_cast<float4*>(dst + cc) = float4{t[q * 4], t[q * 4 + 1], t[q * 4 + 2], t[q * 4 + 3]};
+                *reinterpret_cast<float4*>(dst + (DUAL && j ? mn : 0) + cc) = float4{t[q * 4], t[q * 4 + 1], t[q * 4 + 2], t[q * 4 + 3]};
             }
       }
   } else {
@@ -482,69 +483,111 @@ int launch(Params p, hipStream_t st) {
   return PTO_HIP_OK;
 }
 
-// Sum of the k splits' slabs in split order, times the row and column scales, cast and store.
-template <typename OutT>
+// Four outputs of one row from the k splits' slabs: the sums in split order, times the row and channel
+// scales (and SwiGLU for the gate/up pass, whose slabs are [split][2][m][n]).
+template <bool DUAL>
+__device__ __forceinline__ void sum_slabs(const float* src, int64_t mn, int splits, float row_scale, const float4& w0,
+                                          const float4& w1, float (&out)[4]) {
+  constexpr int kMats = DUAL ? 2 : 1;
+  float4 t[kMats];
+#pragma unroll
+  for (int mat = 0; mat < kMats; ++mat) t[mat] = *reinterpret_cast<const float4*>(src + mat * mn);
+  for (int s = 1; s < splits; ++s) {
+#pragma unroll
+    for (int mat = 0; mat < kMats; ++mat) {
+      const float4 v = *reinterpret_cast<const float4*>(src + ((int64_t)s * kMats + mat) * mn);
+      t[mat] = float4{t[mat].x + v.x, t[mat].y + v.y, t[mat].z + v.z, t[mat].w + v.w};
+    }
+  }
+  const float r = row_scale;
+  const float g[4] = {t[0].x * r * w0.x, t[0].y * r * w0.y, t[0].z * r * w0.z, t[0].w * r * w0.w};
+  if constexpr (DUAL) {
+    const float u[4] = {t[1].x * r * w1.x, t[1].y * r * w1.y, t[1].z * r * w1.z, t[1].w * r * w1.w};
+#pragma unroll
+    for (int k = 0; k < 4; ++k) out[k] = silu(g[k]) * u[k];
+  } else {
+#pragma unroll
+    for (int k = 0; k < 4; ++k) out[k] = g[k];
+  }
+}
+
+template <bool DUAL, typename OutT>
 __global__ __launch_bounds__(256) void gemm8_finish_kernel(const float* __restrict__ slabs, int splits,
-                                                           const float* __restrict__ sa, const float* __restrict__ sb,
-                                                           OutT* __restrict__ c, int64_t ldc, int m, int n) {
+                                                           const float* __restrict__ sa, const float* __restrict__ sb0,
+                                                           const float* __restrict__ sb1, OutT* __restrict__ c, int64_t ldc,
+                                                           int m, int n) {
   // blockIdx.x, threadIdx.x: four columns; blockIdx.y: rows, strided (no division per element)
   const int col = (blockIdx.x * 256 + threadIdx.x) * 4;
   if (col >= n) return;
   const int64_t mn = (int64_t)m * n;
-  const float4 w = *reinterpret_cast<const float4*>(sb + col);
+  const float4 w0 = *reinterpret_cast<const float4*>(sb0 + col);
+  const float4 w1 = DUAL ? *reinterpret_cast<const float4*>(sb1 + col) : w0;
   for (int64_t row = blockIdx.y; row < m; row += gridDim.y) {
-    const float* src = slabs + row * n + col;
-    float4 t = *reinterpret_cast<const float4*>(src);
-    for (int s = 1; s < splits; ++s) {
-      const float4 v = *reinterpret_cast<const float4*>(src + s * mn);
-      t = float4{t.x + v.x, t.y + v.y, t.z + v.z, t.w + v.w};
-    }
-    const float r = sa[row];
-    const float out[4] = {t.x * r * w.x, t.y * r * w.y, t.z * r * w.z, t.w * r * w.w};
+    float out[4];
+    sum_slabs<DUAL>(slabs + row * n + col, mn, splits, sa[row], w0, w1, out);
     store4<OutT>(c + row * ldc + col, out);
   }
 }
 
-// Tile height: 256 rows unless that leaves CUs idle and 128 rows do not.
-// A single-operand pass whose tall tiles fill less than half the CUs splits k instead of halving the
-// tile: a k-tile of 128 rows draws three quarters of the bytes for half the products.
-// At exactly half (the LLaMA-7B down pass at 2048 tokens: 128 tall tiles on 256 CUs) the 128-row
-// tiles fill every CU in one round and need neither slabs nor a finish launch (block 268 us; 272 split in two).
+// Picks the tile height and the k splits and launches the tiles.  With p.splits > 1 afterwards the slabs
+// hold the raw sums and the caller finishes them.
 template <bool DUAL, typename OutT>
-int launch_any(const Params& p0, hipStream_t st) {
-  Params p = p0;
-  p.splits = 1;
-  p.k_per_split = p.k;
-  p.slabs = nullptr;
-  const int64_t num_cu = pto_hip::ctx().num_cu;
+int launch_tiles(Params& p, hipStream_t st) {
+  const int64_t num_cu = pto_hip::ctx().num_cu, variant = pto_hip::ctx().gemm_variant, forced = pto_hip::ctx().gemm_splits;
   const int64_t tiles_n = (p.n + (DUAL ? 127 : 255)) / (DUAL ? 128 : 256);
-  const int64_t tall = (int64_t)((p.m + 255) / 256) * tiles_n;
-  if constexpr (!DUAL) {
-    const int nk = p.k / BK;
-    // by default only where even 128-row tiles would leave CUs idle (see above)
-    const int64_t forced = pto_hip::ctx().gemm_splits;
-    const int64_t want = forced > 0 ? forced : (2 * tall < num_cu ? std::min<int64_t>(num_cu / tall, 4) : 1);
-    if (pto_hip::ctx().gemm_variant == 0 && p.m > 128 && want >= 2 && nk >= 8 * want && p.n % 4 == 0 && p.ldc % 4 == 0) {
-      const int per = (int)((nk + want - 1) / want);
-      p.k_per_split = per * BK;
-      p.splits = (nk + per - 1) / per;
-      void* ws = nullptr;
-      const int rc = pto_hip::gemm_workspace((size_t)p.splits * p.m * p.n * sizeof(float), &ws);
-      if (rc) return rc;
-      p.slabs = reinterpret_cast<float*>(ws);
-      const int rc2 = launch<2, DUAL, float, true>(p, st);
-      if (rc2) return rc2;
-      const unsigned bx = (unsigned)((p.n / 4 + 255) / 256);
-      const unsigned by = (unsigned)std::min<int64_t>(p.m, std::max<int64_t>(1, 4096 / bx));
-      hipLaunchKernelGGL((gemm8_finish_kernel<OutT>), dim3(bx, by), dim3(256), 0, st, p.slabs, p.splits, p.sa, p.sb0,
-                         reinterpret_cast<OutT*>(p.c), p.ldc, p.m, p.n);
-      PTO_CHECK_HIP(hipGetLastError());
-      return PTO_HIP_OK;
+  const int nk = p.k / BK;
+  const bool can_split = p.n % 4 == 0 && p.ldc % 4 == 0;
+  bool tall = variant != 5;
+  int splits = can_split && nk >= 2 ? (int)std::min<int64_t>(std::max<int64_t>(forced, 1), nk) : 1;
+  if (variant == 0) {
+    // The pair of tile height and k splits with the least estimated time in microseconds: rounds of
+    // workgroups over the CUs x (k-tiles x the time of one, growing with the share of CUs that are busy, plus a
+    // tile's start and epilogue), not less than the weights take to arrive; with k split, plus the finish launch
+    // and the slabs' way out and back.  Fitted to timings of every pair at 8 to 4096 rows of four weight
+    // shapes (hidden 1024 to 5120): the pair it picks is 0.9 % from the best one on average, 15 % at worst.
+    const int from = forced > 0 ? splits : 1, to = forced > 0 ? splits : can_split ? std::max(1, std::min(16, nk / 2)) : 1;
+    double best = 1e30;
+    for (int th = 1; th >= 0; --th) {
+      const int64_t tiles = (p.m + (th ? 255 : 127)) / (th ? 256 : 128) * tiles_n;
+      for (int sp = from; sp <= to; ++sp) {
+        const int64_t per = (nk + sp - 1) / sp, real = (nk + per - 1) / per, wgs = tiles * real;
+        const double load = std::min(1.0, (double)wgs / (double)num_cu);
+        const double tile_us = th ? 1.13 + 0.19 * load : 0.64 + 0.26 * load;
+        double t = std::max((double)((wgs + num_cu - 1) / num_cu) * ((double)per * tile_us + (th ? 6.8 : 3.7)),
+                            7.2 + (double)p.k * p.n * (DUAL ? 2 : 1) / 9.2e6);
+        if (real > 1) t += 3.0 + 2.0 * (double)real * p.m * p.n * (DUAL ? 8 : 4) / 4.9e6;
+        if (t < best) {
+          best = t;
+          tall = th != 0;
+          splits = sp;
+        }
+      }
     }
   }
-  const int64_t variant = pto_hip::ctx().gemm_variant;  // 4 and 5 force a tile height
-  if (variant == 5 || (variant != 4 && tall < num_cu && p.m > 128)) return launch<1, DUAL, OutT>(p, st);
-  return launch<2, DUAL, OutT>(p, st);
+  const int per = (nk + splits - 1) / splits;
+  p.k_per_split = per * BK;
+  p.splits = (nk + per - 1) / per;
+  p.slabs = nullptr;
+  if (p.splits > 1) {
+    void* ws = nullptr;
+    const int rc = pto_hip::gemm_workspace((size_t)p.splits * (DUAL ? 2 : 1) * p.m * p.n * sizeof(float), &ws);
+    if (rc) return rc;
+    p.slabs = reinterpret_cast<float*>(ws);
+    return tall ? launch<2, DUAL, float, true>(p, st) : launch<1, DUAL, float, true>(p, st);
+  }
+  return tall ? launch<2, DUAL, OutT>(p, st) : launch<1, DUAL, OutT>(p, st);
+}
+
+template <bool DUAL, typename OutT>
+int launch_any(Params p, hipStream_t st) {
+  const int rc = launch_tiles<DUAL, OutT>(p, st);
+  if (rc || p.splits == 1) return rc;
+  const unsigned bx = (unsigned)((p.n / 4 + 255) / 256);
+  const unsigned by = (unsigned)std::min<int64_t>(p.m, std::max<int64_t>(1, 4096 / bx));
+  hipLaunchKernelGGL((gemm8_finish_kernel<DUAL, OutT>), dim3(bx, by), dim3(256), 0, st, p.slabs, p.splits, p.sa, p.sb0,
+                     p.sb1, reinterpret_cast<OutT*>(p.c), p.ldc, p.m, p.n);
+  PTO_CHECK_HIP(hipGetLastError());
+  return PTO_HIP_OK;
 }
 
 // ---- row kernels: (RMSNorm +) per-row e4m3 quantisation -----------------------------------------
@@ -571,10 +614,16 @@ __device__ __forceinline__ float block_reduce(float v, bool take_max, float* sha
 // One workgroup per row, the row held in registers.  NORM: y = T(x * rsqrt(mean x^2 + eps) * gamma)
 // first (rounded to the 16-bit activation type, as the 16-bit block's RMSNorm output is); then
 // scale = amax|y| / 448 (1 for an all-zero row) and codes = e4m3(clamp(y / scale)).
-template <typename TI, bool NORM>
+// SLABS: y = T(SwiGLU of the gate/up pass's k-split slabs), the row that gemm8_finish_kernel would write.
+struct SlabRows {
+  const float *slabs, *sa, *sb0, *sb1;  // [splits][2][rows][cols], row scales, channel scales of gate and up
+  int64_t mn;                           // rows * cols
+  int splits;
+};
+template <typename TI, bool NORM, bool SLABS = false>
 __global__ __launch_bounds__(kRowThreads) void row_quant_kernel(const TI* __restrict__ x, const float* __restrict__ gamma,
                                                                 uint8_t* __restrict__ codes, float* __restrict__ scale,
-                                                                int64_t cols, float eps) {
+                                                                int64_t cols, float eps, SlabRows sl) {
   typedef __attribute__((__vector_size__(8 * sizeof(TI)))) TI vec8;
   __shared__ float red[kRowThreads / 64];
   const int64_t row = blockIdx.x;
@@ -588,7 +637,19 @@ __global__ __launch_bounds__(kRowThreads) void row_quant_kernel(const TI* __rest
   for (int u = 0; u < kRowVecs; ++u) {
     const int i = threadIdx.x + u * kRowThreads;
     if (i < nvec) {
-      y[u] = xr[i];
+      if constexpr (SLABS) {
+#pragma unroll
+        for (int half = 0; half < 2; ++half) {
+          const int col = 8 * i + 4 * half;
+          float v[4];
+          sum_slabs<true>(sl.slabs + row * cols + col, sl.mn, sl.splits, sl.sa[row], *reinterpret_cast<const float4*>(sl.sb0 + col),
+                          *reinterpret_cast<const float4*>(sl.sb1 + col), v);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) y[u][4 * half + e] = (TI)v[e];
+        }
+      } else {
+        y[u] = xr[i];
+      }
       if constexpr (NORM) {
 #pragma unroll
         for (int e = 0; e < 8; ++e) ss += (float)y[u][e] * (float)y[u][e];
@@ -661,7 +722,7 @@ int row_quant(const void* x, const float* gamma, bool norm, void* codes, float* 
   if (rows == 0) return PTO_HIP_OK;
   dim3 grid((unsigned)rows), block(kRowThreads);
   auto go = [&](auto kern, auto* typed) {
-    hipLaunchKernelGGL(kern, grid, block, 0, st, typed, gamma, reinterpret_cast<uint8_t*>(codes), scale, cols, eps);
+    hipLaunchKernelGGL(kern, grid, block, 0, st, typed, gamma, reinterpret_cast<uint8_t*>(codes), scale, cols, eps, SlabRows{});
   };
   if (x_dtype == PTO_HIP_BF16) {
     if (norm) go(row_quant_kernel<__bf16, true>, reinterpret_cast<const __bf16*>(x));
@@ -845,11 +906,22 @@ extern "C" int pto_hip_ffn_swiglu_fp8(const void* x, const float* gamma, const v
   p1.m = (int)tokens;
   p1.n = (int)intermediate;
   p1.k = (int)hidden;
-  rc = x_dtype == PTO_HIP_BF16 ? gemm8::launch_any<true, __bf16>(p1, st) : gemm8::launch_any<true, _Float16>(p1, st);
+  const bool bf16 = x_dtype == PTO_HIP_BF16;
+  rc = bf16 ? gemm8::launch_tiles<true, __bf16>(p1, st) : gemm8::launch_tiles<true, _Float16>(p1, st);
   if (rc) return rc;
-
-  rc = gemm8::row_quant(h, nullptr, false, h8, sh, tokens, intermediate, 0.f, x_dtype, st);
-  if (rc) return rc;
+  if (p1.splits > 1) {
+    // k split: the quantiser sums the slabs itself, h is not written
+    const gemm8::SlabRows sl{p1.slabs, p1.sa, p1.sb0, p1.sb1, tokens * intermediate, p1.splits};
+    const dim3 grid((unsigned)tokens), block(gemm8::kRowThreads);
+    if (bf16)
+      hipLaunchKernelGGL((gemm8::row_quant_kernel<__bf16, false, true>), grid, block, 0, st, nullptr, nullptr, h8, sh, intermediate, 0.f, sl);
+    else
+      hipLaunchKernelGGL((gemm8::row_quant_kernel<_Float16, false, true>), grid, block, 0, st, nullptr, nullptr, h8, sh, intermediate, 0.f, sl);
+    PTO_CHECK_HIP(hipGetLastError());
+  } else {
+    rc = gemm8::row_quant(h, nullptr, false, h8, sh, tokens, intermediate, 0.f, x_dtype, st);
+    if (rc) return rc;
+  }
 
   gemm8::Params p2{};
   p2.a = h8;

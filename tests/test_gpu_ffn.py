@@ -682,6 +682,50 @@ def test_gemm_fp8_tile_edges_and_k_tile_counts(worker, variant, m, n):
         worker.set_option("gemm_variant", 0)
 
 
+@pytest.mark.parametrize("variant", [4, 5])
+@pytest.mark.parametrize("m,k,n,splits", [(1, 512, 128, 2), (33, 640, 200, 3), (129, 2048, 384, 16), (300, 896, 260, 4)])
+def test_gate_up_fp8_k_split_and_fused_quantiser(worker, variant, m, k, n, splits):
+    """The gate/up pass with k split (uneven shares included): the same h as the unsplit pass up to the order of
+    the fp32 sums - exact here, small integers - and the block, whose quantiser sums the slabs itself, is
+    bit-identical to the chain of stages under the same split."""
+    from pypto_amd.runtime import ffn_block_fp8
+
+    _lib, lib, code = _fp8_stage_lib()
+    g = torch.Generator().manual_seed(m + k)
+    a, wg, wu = (torch.randint(-3, 4, s, generator=g).float().to(torch.float8_e4m3fn).cuda() for s in ((m, k), (n, k), (n, k)))
+    sa, sw = torch.full((m,), 0.0625, device="cuda"), torch.full((n,), 0.25, device="cuda")
+    hs = []
+    try:
+        worker.set_option("gemm_variant", variant)
+        for sp in (1, splits):
+            worker.set_option("gemm_splits", sp)
+            h = torch.full((m, n), float("nan"), dtype=torch.bfloat16, device="cuda")
+            _lib.check(lib.pto_hip_gate_up_swiglu_fp8(a.data_ptr(), sa.data_ptr(), wg.data_ptr(), sw.data_ptr(), wu.data_ptr(),
+                                                      sw.data_ptr(), h.data_ptr(), m, k, n, code(torch.bfloat16), 0))
+            worker.sync()
+            hs.append(h.cpu())
+        assert torch.equal(hs[0], hs[1])
+        if n % 128 == 0:
+            q, _ = workloads.ffn_fp8_inputs(tokens=m, hidden=k, intermediate=n, seed=3, device="cuda")
+            with worker.register(ffn_block_fp8) as hd:
+                hd(*q.args())
+            x8, hb = torch.zeros((m, k), dtype=torch.uint8, device="cuda"), torch.zeros((m, n), dtype=torch.bfloat16, device="cuda")
+            h8, sx, sh = torch.zeros((m, n), dtype=torch.uint8, device="cuda"), torch.zeros(m, device="cuda"), torch.zeros(m, device="cuda")
+            out = torch.zeros_like(q.out)
+            b16 = code(torch.bfloat16)
+            _lib.check(lib.pto_hip_rms_norm_quantize_fp8(q.x.data_ptr(), q.gamma.data_ptr(), x8.data_ptr(), sx.data_ptr(), m, k, q.eps, b16, 0))
+            _lib.check(lib.pto_hip_gate_up_swiglu_fp8(x8.data_ptr(), sx.data_ptr(), q.w_gate8.data_ptr(), q.w_gate_scale.data_ptr(),
+                                                      q.w_up8.data_ptr(), q.w_up_scale.data_ptr(), hb.data_ptr(), m, k, n, b16, 0))
+            _lib.check(lib.pto_hip_quantize_rows_fp8(hb.data_ptr(), h8.data_ptr(), sh.data_ptr(), m, n, b16, 0))
+            _lib.check(lib.pto_hip_projection_fp8(h8.data_ptr(), sh.data_ptr(), q.w_down8.data_ptr(), q.w_down_scale.data_ptr(),
+                                                  out.data_ptr(), m, n, k, code(torch.float32), 0))
+            worker.sync()
+            assert torch.equal(q.out, out)
+    finally:
+        worker.set_option("gemm_variant", 0)
+        worker.set_option("gemm_splits", 0)
+
+
 @pytest.mark.parametrize("m,k,n,splits", [(2048, 11008, 4096, 2),    # the LLaMA-7B down pass, split in two
                                           (1024, 11008, 4096, 0),    # ... at 1024 tokens: the library's own choice (4)
                                           (300, 4096, 520, 3), (257, 4096, 256, 4), (1000, 2048, 1024, 2)])
