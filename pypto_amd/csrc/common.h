@@ -69,9 +69,9 @@ struct Context {
   int64_t w8a16_nt = 1;            // skinny projections: weight rows read with non-temporal loads
   int64_t gemm_variant = 0;
   int64_t gemm_splits = 0;       // k splits of the tiled GEMM: 0 = by shape, 1..16 = as given (when k allows)
-  int64_t w8a16_wgs_per_cu = 1;  // workgroups of the W8A16 partial kernel aimed at per compute unit
+  int64_t w8a16_wgs_per_cu = 1;  // most workgroups of the skinny projection kernel per compute unit
   int64_t w8a16_wide = 1;        // int8 codes read 16 per lane: 0 never, 1 for large matrices, 2 whenever shapes allow
-  int64_t w8a16_min_steps = 8;   // fewest 32-row steps per wavefront before k is split further
+  int64_t w8a16_min_steps = 2;   // fewest 32-row steps per wavefront before k is split further
   int64_t w8a16_gemm_rows = 33;  // rows from which int8 projections run as a tiled GEMM (0 = never)
 };
 
@@ -90,18 +90,39 @@ std::recursive_mutex& dispatch_mutex();
 int workspace(size_t bytes, void** ptr);
 
 // ---- W8A16 decode projections, shared with the composed decoder layer -------------------
-constexpr int kW8Slab = 128;  // output channels per workgroup of the partial kernel
-constexpr int kW8MaxM = 32;   // rows of a partial slab (activation rows are at most this many)
-// fp32 partial sums of a projection, one slab per k split: element (s, m, n) of projection i is
-// part[i][s * slab_stride + m * N + n].  The skinny kernels write [32, N] slabs into the shared
-// workspace; the tiled GEMM writes [M, N] slabs into its own scratch area (or, with one split, the
-// finished product into the caller's buffer: `scaled` then says the channel scales are in).
+constexpr int kW8MaxM = 32;   // activation rows of the skinny kernels are at most this many
+// Which workgroups of the skinny projection kernel share an output slab.  The (slab, 32-row k step) units of a
+// launch form one list, slab by slab, and workgroup w of `wgs` takes the units [w * units / wgs,
+// (w + 1) * units / wgs): a slab (2^shift channels, ks units) is the work of as many consecutive workgroups as
+// its units fall to, and the j-th of them writes partial slab j.  units 0: every channel has `splits` slabs.
+struct SlabMap {
+  unsigned units, wgs, ks;
+  int shift, slabs;  // slabs of one matrix (those of a pair's second matrix follow)
+};
+// Partial slabs of channel `ch` of matrix `mat`.
+__device__ __forceinline__ int slab_count(const SlabMap& s, int splits, int mat, int ch) {
+  if (s.units == 0) return splits;
+  const unsigned first = (unsigned)(mat * s.slabs + (ch >> s.shift)) * s.ks;
+  return (int)(((first + s.ks) * s.wgs - 1) / s.units - ((first + 1) * s.wgs - 1) / s.units) + 1;
+}
+// fp32 partial sums of a projection: element (s, m, n) of projection i is part[i][s * slab_stride + m * N + n] for
+// s below slab_count(map, splits, i, n).  The skinny kernels write [M, N] slabs into the shared workspace; the
+// tiled GEMM writes [M, N] slabs into its own scratch area (or, with one split, the finished product into the
+// caller's buffer: `scaled` then says the channel scales are in).
 struct W8Partials {
   float* part[2];
   int splits;
   int64_t slab_stride;
   bool scaled;
+  SlabMap map;
 };
+// A finished fp32 product as a single slab.
+inline W8Partials finished_slab(const float* product) {
+  W8Partials p{};
+  p.part[0] = const_cast<float*>(product);
+  p.splits = 1;
+  return p;
+}
 // Launches the partial kernel for x[M, K] @ wq0[K, N] (and wq1 when non-null).  x_blocked: x is
 // stored [K/8][32][8] - element (m, k) at ((k/8)*32 + m)*8 + k%8 - the layout the layer's own
 // producers write so that a wavefront's activation reads are whole consecutive cache lines.
@@ -139,13 +160,13 @@ int gemm_partials(const void* x, const void* w, const float* scale, int64_t m, i
 // RoPE + K/V append reading either final fp32 projections (qkv_scale null, splits 1) or the
 // partial sums of the q/k/v projection (summed in split order and scaled per channel).
 // rope_width: columns of the cos/sin tables, head_dim / 2 or head_dim.
-int rope_kv_cache_update(const float* qkv, const float* qkv_scale, int splits, int64_t split_stride,
+int rope_kv_cache_update(const W8Partials& qkv, const float* qkv_scale,
                          const int32_t* seq_lens, const float* rope_cos, const float* rope_sin,
                          const int32_t* block_table, void* key_cache, void* value_cache, void* q_out,
                          int64_t batch, int64_t num_heads, int64_t kv_head_num, int64_t head_dim,
                          int64_t block_size, int64_t max_num_blocks_per_req, int64_t max_pos, int rope_width,
                          int64_t pool_rows, int dtype, void* stream);
-int rope_kv_cache_update_fp8(const float* qkv, const float* qkv_scale, int splits, int64_t split_stride,
+int rope_kv_cache_update_fp8(const W8Partials& qkv, const float* qkv_scale,
                              const int32_t* seq_lens, const float* rope_cos, const float* rope_sin,
                              const int32_t* block_table, void* key_cache, void* value_cache, float* k_scale,
                              float* v_scale, void* q_out, int64_t batch, int64_t num_heads, int64_t kv_head_num,

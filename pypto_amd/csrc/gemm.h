@@ -941,6 +941,7 @@ int launch_variant(GemmParams p, hipStream_t st) {
     o.splits = p.splits;
     o.slab_stride = (int64_t)p.m * p.n;
     o.scaled = p.splits == 1;
+    o.map = pto_hip::SlabMap{};
     return PTO_HIP_OK;
   }
   if (p.splits == 1) return rc;

@@ -60,12 +60,12 @@ int layer_large_batch(const PtoHipDecoderLayerArgs* a, int rope_w, void* stream)
   const float* qkv_scale = parts.scaled ? nullptr : a->wqkv_s;
   const int64_t pool_blocks = a->pool_rows / (hkv * a->block_size);
   if (fp8kv)
-    rc = rope_kv_cache_update_fp8(parts.part[0], qkv_scale, parts.splits, parts.slab_stride, a->seq_lens, a->rope_cos,
+    rc = rope_kv_cache_update_fp8(parts, qkv_scale, a->seq_lens, a->rope_cos,
                                   a->rope_sin, a->block_table, a->key_cache, a->value_cache, a->k_scale, a->v_scale,
                                   q16, b, hq, hkv, d, a->block_size, a->max_num_blocks_per_req, a->max_pos, rope_w,
                                   pool_blocks, dt, stream);
   else
-    rc = rope_kv_cache_update(parts.part[0], qkv_scale, parts.splits, parts.slab_stride, a->seq_lens, a->rope_cos,
+    rc = rope_kv_cache_update(parts, qkv_scale, a->seq_lens, a->rope_cos,
                               a->rope_sin, a->block_table, a->key_cache, a->value_cache, q16, b, hq, hkv, d,
                               a->block_size, a->max_num_blocks_per_req, a->max_pos, rope_w, a->pool_rows, dt, stream);
   if (rc) return rc;
@@ -201,12 +201,12 @@ extern "C" int pto_hip_decoder_layer_decode(const PtoHipDecoderLayerArgs* a, voi
   // 3. finish of the projection + RoPE at pos = seq_len - 1, append K/V, rotated Q
   if (fp8kv) {
     const int64_t pool_blocks = a->pool_rows / (hkv * a->block_size);
-    rc = rope_kv_cache_update_fp8(parts.part[0], a->wqkv_s, parts.splits, (int64_t)kW8MaxM * qkv_n, a->seq_lens,
+    rc = rope_kv_cache_update_fp8(parts, a->wqkv_s, a->seq_lens,
                                   a->rope_cos, a->rope_sin, a->block_table, a->key_cache, a->value_cache, a->k_scale,
                                   a->v_scale, q16, b, hq, hkv, d, a->block_size, a->max_num_blocks_per_req,
                                   a->max_pos, rope_w, pool_blocks, dt, stream);
   } else {
-    rc = rope_kv_cache_update(parts.part[0], a->wqkv_s, parts.splits, (int64_t)kW8MaxM * qkv_n, a->seq_lens,
+    rc = rope_kv_cache_update(parts, a->wqkv_s, a->seq_lens,
                               a->rope_cos, a->rope_sin, a->block_table, a->key_cache, a->value_cache, q16, b, hq,
                               hkv, d, a->block_size, a->max_num_blocks_per_req, a->max_pos, rope_w, a->pool_rows, dt,
                               stream);

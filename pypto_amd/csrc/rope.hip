@@ -15,7 +15,8 @@ namespace {
 struct RopeParams {
   const float* qkv;        // [B, (Hq + 2*Hkv) * D] fp32 projections, or their k-split partial sums
   const float* scale;      // per-channel scales of the partial sums; null when qkv is final
-  int splits;              // partial slabs to sum (1 when qkv is final)
+  int splits;              // partial slabs to sum (1 when qkv is final), see slab_count
+  pto_hip::SlabMap map;
   int64_t split_stride;    // elements between consecutive partial slabs
   const int32_t* seq_lens; // [B]
   const float* cos;        // [max_pos, rope_w]: rope_w = D/2 (one angle per pair) or D (the
@@ -41,15 +42,16 @@ __global__ __launch_bounds__(128) void rope_kv_kernel(RopeParams p) {
   auto fetch = [&](int i) {
     float v = 0.f;
     const float* q = p.qkv + src + i;
+    const int splits = pto_hip::slab_count(p.map, p.splits, 0, head * p.d + i);
     int s = 0;
-    for (; s + 4 <= p.splits; s += 4) {
+    for (; s + 4 <= splits; s += 4) {
       float t[4];
 #pragma unroll
       for (int u = 0; u < 4; ++u) t[u] = q[(size_t)(s + u) * p.split_stride];
 #pragma unroll
       for (int u = 0; u < 4; ++u) v += t[u];
     }
-    for (; s < p.splits; ++s) v += q[(size_t)s * p.split_stride];
+    for (; s < splits; ++s) v += q[(size_t)s * p.split_stride];
     return p.scale ? v * p.scale[(size_t)head * p.d + i] : v;
   };
   const bool is_q = head < p.hq, is_k = !is_q && head < p.hq + p.hkv;
@@ -128,15 +130,16 @@ __global__ __launch_bounds__(64) void rope_kv_fp8_kernel(RopeFp8Params pp) {
   auto fetch = [&](int i) {
     float v = 0.f;
     const float* q = p.qkv + src + i;
+    const int splits = pto_hip::slab_count(p.map, p.splits, 0, head * p.d + i);
     int s = 0;
-    for (; s + 4 <= p.splits; s += 4) {
+    for (; s + 4 <= splits; s += 4) {
       float t[4];
 #pragma unroll
       for (int u = 0; u < 4; ++u) t[u] = q[(size_t)(s + u) * p.split_stride];
 #pragma unroll
       for (int u = 0; u < 4; ++u) v += t[u];
     }
-    for (; s < p.splits; ++s) v += q[(size_t)s * p.split_stride];
+    for (; s < splits; ++s) v += q[(size_t)s * p.split_stride];
     return p.scale ? v * p.scale[(size_t)head * p.d + i] : v;
   };
   const bool is_q = head < p.hq, is_k = !is_q && head < p.hq + p.hkv;
@@ -247,7 +250,7 @@ int cast_from_f32(const float* in, void* out, size_t n, int out_dtype, hipStream
 }  // namespace pto_hip
 
 namespace pto_hip {
-int rope_kv_cache_update(const float* qkv, const float* qkv_scale, int splits, int64_t split_stride,
+int rope_kv_cache_update(const W8Partials& qkv, const float* qkv_scale,
                          const int32_t* seq_lens, const float* rope_cos, const float* rope_sin,
                          const int32_t* block_table, void* key_cache, void* value_cache, void* q_out,
                          int64_t batch, int64_t num_heads, int64_t kv_head_num, int64_t head_dim,
@@ -264,13 +267,14 @@ int rope_kv_cache_update(const float* qkv, const float* qkv_scale, int splits, i
                 "rope_kv_cache_update: non-positive extent");
   PTO_CHECK_ARG(dtype == PTO_HIP_BF16 || dtype == PTO_HIP_FP16,
                 "rope_kv_cache_update: cache/query dtype %s not in {BF16, FP16}", dtype_name(dtype));
-  PTO_CHECK_ARG(qkv && seq_lens && rope_cos && rope_sin && block_table && key_cache && value_cache && q_out,
+  PTO_CHECK_ARG(qkv.part[0] && seq_lens && rope_cos && rope_sin && block_table && key_cache && value_cache && q_out,
                 "rope_kv_cache_update: null tensor pointer");
   RopeParams p{};
-  p.qkv = qkv;
+  p.qkv = qkv.part[0];
   p.scale = qkv_scale;
-  p.splits = splits;
-  p.split_stride = split_stride;
+  p.splits = qkv.splits;
+  p.split_stride = qkv.slab_stride;
+  p.map = qkv.map;
   p.seq_lens = seq_lens;
   p.cos = rope_cos;
   p.sin = rope_sin;
@@ -301,7 +305,7 @@ int rope_kv_cache_update(const float* qkv, const float* qkv_scale, int splits, i
 }  // namespace pto_hip
 
 namespace pto_hip {
-int rope_kv_cache_update_fp8(const float* qkv, const float* qkv_scale, int splits, int64_t split_stride,
+int rope_kv_cache_update_fp8(const W8Partials& qkv, const float* qkv_scale,
                              const int32_t* seq_lens, const float* rope_cos, const float* rope_sin,
                              const int32_t* block_table, void* key_cache, void* value_cache, float* k_scale,
                              float* v_scale, void* q_out, int64_t batch, int64_t num_heads, int64_t kv_head_num,
@@ -319,16 +323,17 @@ int rope_kv_cache_update_fp8(const float* qkv, const float* qkv_scale, int split
                 "rope_kv_cache_update_fp8: non-positive extent");
   PTO_CHECK_ARG(q_dtype == PTO_HIP_BF16 || q_dtype == PTO_HIP_FP16,
                 "rope_kv_cache_update_fp8: query dtype %s not in {BF16, FP16}", dtype_name(q_dtype));
-  PTO_CHECK_ARG(qkv && seq_lens && rope_cos && rope_sin && block_table && key_cache && value_cache && k_scale &&
+  PTO_CHECK_ARG(qkv.part[0] && seq_lens && rope_cos && rope_sin && block_table && key_cache && value_cache && k_scale &&
                     v_scale && q_out,
                 "rope_kv_cache_update_fp8: null tensor pointer");
   PTO_CHECK_ARG(((uintptr_t)key_cache | (uintptr_t)value_cache) % 4 == 0, "rope_kv_cache_update_fp8: misaligned cache");
   RopeFp8Params pp{};
   RopeParams& p = pp.r;
-  p.qkv = qkv;
+  p.qkv = qkv.part[0];
   p.scale = qkv_scale;
-  p.splits = splits;
-  p.split_stride = split_stride;
+  p.splits = qkv.splits;
+  p.split_stride = qkv.slab_stride;
+  p.map = qkv.map;
   p.seq_lens = seq_lens;
   p.cos = rope_cos;
   p.sin = rope_sin;
@@ -369,7 +374,7 @@ extern "C" int pto_hip_rope_kv_cache_update_fp8(const float* qkv, const int32_t*
                                                 int64_t max_num_blocks_per_req, int64_t max_pos,
                                                 int64_t pool_blocks, int q_dtype, void* stream) {
   PTO_DISPATCH_LOCK();
-  return pto_hip::rope_kv_cache_update_fp8(qkv, nullptr, 1, 0, seq_lens, rope_cos, rope_sin, block_table, key_cache,
+  return pto_hip::rope_kv_cache_update_fp8(pto_hip::finished_slab(qkv), nullptr, seq_lens, rope_cos, rope_sin, block_table, key_cache,
                                            value_cache, k_scale, v_scale, q_out, batch, num_heads, kv_head_num,
                                            head_dim, block_size, max_num_blocks_per_req, max_pos, (int)(head_dim / 2),
                                            pool_blocks, q_dtype, stream);
@@ -382,7 +387,7 @@ extern "C" int pto_hip_rope_kv_cache_update(const float* qkv, const int32_t* seq
                                             int64_t block_size, int64_t max_num_blocks_per_req,
                                             int64_t max_pos, int64_t pool_rows, int dtype, void* stream) {
   PTO_DISPATCH_LOCK();
-  return pto_hip::rope_kv_cache_update(qkv, nullptr, 1, 0, seq_lens, rope_cos, rope_sin, block_table, key_cache,
+  return pto_hip::rope_kv_cache_update(pto_hip::finished_slab(qkv), nullptr, seq_lens, rope_cos, rope_sin, block_table, key_cache,
                                        value_cache, q_out, batch, num_heads, kv_head_num, head_dim, block_size,
                                        max_num_blocks_per_req, max_pos, (int)(head_dim / 2), pool_rows, dtype, stream);
 }

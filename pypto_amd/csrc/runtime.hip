@@ -621,7 +621,7 @@ int run_rope_kv_fp8(const PtoHipChipTensor* t, int nt, const uint64_t* s, int ns
   PTO_CHECK_ARG((t[9].dtype == PTO_HIP_BF16 || t[9].dtype == PTO_HIP_FP16) && numel(t[9]) == batch * hq * d,
                 "rope_kv_cache_update_fp8: q_out must be BF16 or FP16 [B*Hq, D]");
   return rope_kv_cache_update_fp8(
-      reinterpret_cast<const float*>(tptr(t[0])), nullptr, 1, 0, reinterpret_cast<const int32_t*>(tptr(t[1])),
+      finished_slab(reinterpret_cast<const float*>(tptr(t[0]))), nullptr, reinterpret_cast<const int32_t*>(tptr(t[1])),
       reinterpret_cast<const float*>(tptr(t[2])), reinterpret_cast<const float*>(tptr(t[3])),
       reinterpret_cast<const int32_t*>(tptr(t[4])), tptr_mut(t[5]), tptr_mut(t[6]),
       reinterpret_cast<float*>(tptr_mut(t[7])), reinterpret_cast<float*>(tptr_mut(t[8])), tptr_mut(t[9]), batch, hq,
@@ -652,7 +652,7 @@ int run_rope_kv(const PtoHipChipTensor* t, int nt, const uint64_t* s, int ns, hi
   PTO_CHECK_ARG(t[5].dtype == t[6].dtype && t[5].dtype == t[7].dtype && numel(t[5]) == numel(t[6]) &&
                     numel(t[5]) % d == 0 && numel(t[7]) == batch * hq * d,
                 "rope_kv_cache_update: caches and q_out must share a dtype; caches [rows, D], q_out [B*Hq, D]");
-  return rope_kv_cache_update(reinterpret_cast<const float*>(tptr(t[0])), nullptr, 1, 0,
+  return rope_kv_cache_update(finished_slab(reinterpret_cast<const float*>(tptr(t[0]))), nullptr,
                                       reinterpret_cast<const int32_t*>(tptr(t[1])),
                                       reinterpret_cast<const float*>(tptr(t[2])),
                                       reinterpret_cast<const float*>(tptr(t[3])),

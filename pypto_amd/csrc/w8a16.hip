@@ -5,20 +5,26 @@
 // projection.py:145-177) with int8 weights and one fp32 scale per output channel.  Decode
 // batches are small (M <= 32), so the work is reading the weights once: HBM-bound.
 //
-//   * a workgroup of four wavefronts owns 128 output channels over a k range; the wavefronts
-//     take the range's 32-row steps in turn.  Per step a lane reads 8 bytes (8 channels) of 8
-//     k-rows - whole 128-byte row segments per 16 lanes - keeps the next step's loads in flight,
+//   * the (128- or 256-channel slab, 32-row step) units of a launch are shared out evenly over one
+//     workgroup of four wavefronts per CU, whole numbers of workgroups to a slab where that covers the CUs; the
+//     wavefronts take a share's steps in turn.  Per step a lane reads 8 or 16 bytes of 8
+//     k-rows - whole row segments per 16 lanes - keeps the next step's loads in flight,
 //     widens the int8 codes to fp32 and packs them, transposed, straight into MFMA B operands
-//     (the high halves of the fp32 values are exact bf16), then issues 16 v_mfma_f32_16x16x32;
-//   * the four accumulators are summed through LDS in a fixed order, so one workgroup writes
-//     one fp32 partial slab; k is split across workgroups only as far as filling the machine
-//     needs;
-//   * the partial slabs are summed in split order, scaled per channel and finished by a small
+//     (the high halves of the fp32 values are exact bf16), then issues its v_mfma_f32_16x16x32;
+//   * at the end of a slab's share the four accumulators are summed through LDS in a fixed order and
+//     written as one fp32 partial slab;
+//   * the partial slabs are summed in order, scaled per channel and finished by a small
 //     second kernel: residual add / SwiGLU / cast, or residual add + RMSNorm of the whole row.
 //     The RoPE kernel reads the q/k/v partials directly.
+// Launch and finish, cold weights, 16 rows: 16 MB of 16-bit weights 11.3 us, 356 MB 63 us (5.7 TB/s); int8 117 MB 26 us.
+// In the decoder layer (trace, equal k ranges on the CUs and 32 rows always before -> now): one sequence, int8
+// q/k/v 11.0 -> 8.5 us, o 10.1 -> 8.0, gate/up 25.7 -> 22.9, down 13.6 -> 12.4; sixteen sequences, 16-bit weights of a 5120-wide
+// model: q/k/v 16.5 -> 14.6, o 13.2 -> 12.2, gate/up 76.0 -> 59.8, down 34.2 -> 32.4; steps 84 -> 75 and 188 -> 169 us,
+// 32 sequences int8 (two row groups) 163.6 -> 161.0.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <atomic>
 #include <type_traits>
 
 #include "common.h"
@@ -30,17 +36,18 @@ typedef __attribute__((__vector_size__(4 * sizeof(uint32_t)))) uint32_t u32x4;
 typedef __attribute__((__vector_size__(8 * sizeof(__bf16)))) __bf16 bf16x8;
 typedef __attribute__((__vector_size__(8 * sizeof(_Float16)))) _Float16 f16x8;
 
-constexpr int kSlab = pto_hip::kW8Slab;  // output channels per workgroup (8 per lane); twice that with 16 per lane
 constexpr int kStep = 32;                // k rows per step
 constexpr int kMaxM = pto_hip::kW8MaxM;
-constexpr int kWavesPerWg = 4;           // wavefronts per workgroup of the partial kernel
+constexpr int kWaves = 4;                // wavefronts per workgroup of the partial kernel
 
 struct GemvParams {
   const uint16_t* x;    // [M, K] 16-bit activations
   const void* wq[2];    // [K, N] each (int8 codes or 16-bit weights); the second is the up projection of a pair
-  float* part[2];       // [splits, 32, N] each
-  int m, k, n, slabs, n_mats, splits, k_per_split;
-  int x_blocked;  // activations stored [K/8][32][8] (see w8a16_partials) instead of row-major
+  float* part[2];       // [partial slabs, M, N] each
+  int m, k, n, x_blocked;  // x_blocked: activations stored [K/8][32][8] (see w8a16_partials) instead of row-major
+  int slabs, ks;        // output slabs of one matrix, 32-row steps of one slab
+  int per_wg, extra;    // units / workgroups and its remainder (see SlabMap)
+  int mapped;           // 0: a workgroup per slab
 };
 
 template <bool BF16>
@@ -70,80 +77,100 @@ typedef uint32_t u32x2 __attribute__((__vector_size__(2 * sizeof(uint32_t))));
 
 // One register stage of a lane: kCols channels of the k rows kg*8 .. kg*8+7, and the activations.
 // W8: int8 weight codes, 8 bytes (kCols 8) or 16 bytes (kCols 16) per row and lane; otherwise
-// 16-bit weights of the activation type (16 bytes = 8 channels).  A lane load of 16 bytes moves
-// twice the weights per request; the int8 form with 8-byte loads is kept for channel counts that
-// are not a multiple of 16.
-template <bool W8, int kCols>
+// 16-bit weights of the activation type (16 bytes = 8 channels).
+template <bool W8, int kCols, int MT>
 struct Stage {
   typename std::conditional<(W8 && kCols == 8), u32x2, u32x4>::type w[8];
-  u32x4 xa[2];  // activations of rows c and c+16, k = kg*8 .. +8
+  u32x4 xa[MT];  // activations of rows c (and c+16), k = kg*8 .. +8
 };
 
-// kWaves wavefronts per workgroup, kStages register stages per wavefront (kStages - 1 in flight),
-// kOcc wavefronts per SIMD the register budget is cut for.
-template <bool BF16, bool W8, int kCols, int kWaves, int kStages, int kOcc, bool NT = false>
-__global__ __launch_bounds__(kWaves * 64) __attribute__((amdgpu_waves_per_eu(kOcc, kOcc))) void w8a16_partial_kernel(
-    GemvParams p) {
+// Workgroup w of G takes the units (slab, 32-row step) [w U / G, (w + 1) U / G) of the list that walks the
+// slabs one after the other (SlabMap): every CU streams the same number of bytes, whatever the
+// shape.  A launch lasts as long as the CU with the most bytes: cut into equal k ranges instead, 272
+// workgroups of a 356 MB pair of 16-bit matrices on 256 CUs read at 4.5 TB/s and 544 at 5.3, where 256 even
+// shares reach 6.5 (load-only twins of this kernel).  The four wavefronts take a run's steps in turn; when
+// a run ends (the slab's last step or the workgroup's) their accumulators are summed through LDS, one after
+// the other, and written as the next partial slab of those channels; the next run's first rows
+// are in flight meanwhile.  MT: 16-row groups of activations (M <= 16 needs one: half the MFMAs,
+// activations and partial sums).  Rows past M are computed on row M - 1 and not written.
+template <bool BF16, bool W8, int kCols, int MT, bool NT>
+__global__ __launch_bounds__(kWaves * 64) __attribute__((amdgpu_waves_per_eu(1, 2))) void w8a16_partial_kernel(GemvParams p) {
   static_assert(kCols == 8 || (W8 && kCols == 16), "16 channels per lane only with int8 codes");
-  constexpr int kHalf = kWaves / 2;
-  constexpr int kSlab = 16 * kCols;  // output channels per workgroup: 16 lanes of kCols channels
-  __shared__ float red[kHalf * kMaxM * kSlab];  // 16 or 32 KiB per wavefront of the lower half
+  constexpr int kSlab = 16 * kCols;  // output channels of a slab: 16 lanes of kCols channels
+  constexpr int kRows = 16 * MT;
+  extern __shared__ __attribute__((aligned(16))) float red[];  // [kWaves][kRows][kSlab]
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // uniform: row addresses stay scalar
   const int c = lane & 15, kg = lane >> 4;
 
-  const int per_split = p.slabs * p.n_mats;
-  const int split = blockIdx.x / per_split, rem = blockIdx.x % per_split;
-  const int mat = rem / p.slabs, slab = rem % p.slabs;
-  const int k_begin = split * p.k_per_split;
-  const int k_end = min(p.k, k_begin + p.k_per_split);
-  const int n_steps = (k_end - k_begin + kStep - 1) / kStep;
-
-  const int n0 = slab * kSlab + c * kCols;
-  // Row-major x: lane (c, kg) reads 16 bytes of rows c and c+16 at k = kstep + 8*kg.  Blocked x
-  // keeps the 32 rows of each 8-k group together, so the same two reads of a wavefront cover 2 KB
-  // of consecutive bytes instead of 32 half cache lines.
-  const int x_step = p.x_blocked ? kMaxM : 1;  // elements per unit of k
-  const uint16_t* xp0 = p.x_blocked ? p.x + (size_t)(kg * kMaxM + min(c, p.m - 1)) * 8
-                                    : p.x + (size_t)min(c, p.m - 1) * p.k + kg * 8;
-  const uint16_t* xp1 = p.x_blocked ? p.x + (size_t)(kg * kMaxM + min(c + 16, p.m - 1)) * 8
-                                    : p.x + (size_t)min(c + 16, p.m - 1) * p.k + kg * 8;
-  const bool m0_ok = c < p.m, m1_ok = c + 16 < p.m;
-
-  f32x4 acc[kCols][2];
-#pragma unroll
-  for (int i = 0; i < kCols; ++i)
-#pragma unroll
-    for (int h = 0; h < 2; ++h) acc[i][h] = f32x4{0.f, 0.f, 0.f, 0.f};
-
-  // Loads never depend on a condition, so the number of requests in flight is known at compile
-  // time: steps past the end re-read the wavefront's last one (a cache hit), and a last step
-  // that would reach past row k is moved back to end at row k - the rows it then repeats are
-  // multiplied by zeroed activations.  A row address is a wavefront-uniform row base plus a
-  // per-lane offset that never changes.
-  const int last_step = wave < n_steps ? wave + (n_steps - 1 - wave) / kWaves * kWaves : n_steps - 1;
-  constexpr int kWBytes = W8 ? 1 : 2;  // bytes per weight
-  typedef typename std::conditional<(W8 && kCols == 8), u32x2, u32x4>::type wvec_t;
-  const char* wbase = reinterpret_cast<const char*>(p.wq[mat]);
-  const uint32_t lane_off = (uint32_t)min(n0, p.n - kCols) + (uint32_t)(kg * 8) * (uint32_t)p.n;
-  auto step_row = [&](int step) { return min(k_begin + step * kStep, p.k - kStep); };
-  auto load = [&](Stage<W8, kCols>& s, int step) {
-    const int kstep = step_row(min(step, last_step));
-    s.xa[0] = *reinterpret_cast<const u32x4*>(xp0 + (size_t)kstep * x_step);
-    s.xa[1] = *reinterpret_cast<const u32x4*>(xp1 + (size_t)kstep * x_step);
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      const char* row = wbase + (size_t)(kstep + e) * p.n * kWBytes;  // uniform
-      if constexpr (NT) s.w[e] = __builtin_nontemporal_load(reinterpret_cast<const wvec_t*>(row + (size_t)lane_off * kWBytes));
-      else s.w[e] = *reinterpret_cast<const wvec_t*>(row + (size_t)lane_off * kWBytes);
+  // this workgroup's units, and a cursor over them in rounds of kWaves steps of one slab
+  const int wg = blockIdx.x, wgs = gridDim.x;
+  const int u_begin = wg * p.per_wg + wg * p.extra / wgs, u_end = (wg + 1) * p.per_wg + (wg + 1) * p.extra / wgs;
+  struct Cursor {
+    int slab, step, end;  // the round's first step and the end of its run
+  };
+  auto run_end = [&](int slab) { return min(p.ks, u_end - slab * p.ks); };
+  auto last_of_run = [&](const Cursor& cur) { return cur.step + kWaves >= cur.end; };
+  auto last = [&](const Cursor& cur) { return last_of_run(cur) && cur.slab * p.ks + cur.end >= u_end; };
+  auto advance = [&](Cursor& cur) {
+    if (!last_of_run(cur)) {
+      cur.step += kWaves;
+    } else {
+      cur.slab += 1;
+      cur.step = 0;
+      cur.end = run_end(cur.slab);
     }
   };
-  auto compute = [&](const Stage<W8, kCols>& s, int step) {
-    const int row0 = step_row(step) + kg * 8;  // first of this lane's 8 rows
-    const bool k_ok = row0 >= k_begin + step * kStep && row0 < k_end;
-    const u32x4 z = {0u, 0u, 0u, 0u};
-    const u32x4 a0 = (k_ok && m0_ok) ? s.xa[0] : z;
-    const u32x4 a1 = (k_ok && m1_ok) ? s.xa[1] : z;
+
+  // Row-major x: lane (c, kg) reads 16 bytes of rows c and c+16 at k = kstep + 8*kg.  Blocked x
+  // keeps the 32 rows of each 8-k group together, so the same reads of a wavefront cover
+  // consecutive bytes instead of half cache lines.
+  const int x_step = p.x_blocked ? kMaxM : 1;  // elements per unit of k
+  const uint16_t* xp[MT];
+#pragma unroll
+  for (int h = 0; h < MT; ++h) {
+    const int row = min(c + 16 * h, p.m - 1);
+    xp[h] = p.x_blocked ? p.x + (size_t)(kg * kMaxM + row) * 8 : p.x + (size_t)row * p.k + kg * 8;
+  }
+
+  f32x4 acc[kCols][MT];
+  auto clear = [&] {
+#pragma unroll
+    for (int i = 0; i < kCols; ++i)
+#pragma unroll
+      for (int h = 0; h < MT; ++h) acc[i][h] = f32x4{0.f, 0.f, 0.f, 0.f};
+  };
+  clear();
+
+  // Loads never depend on a condition, so the number of requests in flight is known at compile
+  // time: a wavefront without a step of its own in a round reads the run's last one again, and a last step
+  // that would reach past row k is moved back to end at row k - the rows it then repeats are
+  // multiplied by zeroed activations.  A row address is a wavefront-uniform row base plus a
+  // per-lane offset.
+  constexpr int kWBytes = W8 ? 1 : 2;  // bytes per weight
+  typedef typename std::conditional<(W8 && kCols == 8), u32x2, u32x4>::type wvec_t;
+  auto load = [&](Stage<W8, kCols, MT>& s, const Cursor& cur) {
+    const int row0 = min(min(cur.step + wave, cur.end - 1) * kStep, p.k - kStep);
+    const int mat = cur.slab >= p.slabs ? 1 : 0;
+    const int n0 = min((cur.slab - mat * p.slabs) * kSlab + c * kCols, p.n - kCols);
+    const uint32_t lane_off = ((uint32_t)n0 + (uint32_t)(kg * 8) * (uint32_t)p.n) * kWBytes;
+    const char* wbase = reinterpret_cast<const char*>(p.wq[mat]) + (size_t)row0 * p.n * kWBytes;
+#pragma unroll
+    for (int h = 0; h < MT; ++h) s.xa[h] = *reinterpret_cast<const u32x4*>(xp[h] + (size_t)row0 * x_step);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const char* row = wbase + (size_t)e * p.n * kWBytes;  // uniform
+      if constexpr (NT) s.w[e] = __builtin_nontemporal_load(reinterpret_cast<const wvec_t*>(row + lane_off));
+      else s.w[e] = *reinterpret_cast<const wvec_t*>(row + lane_off);
+    }
+  };
+  auto compute = [&](const Stage<W8, kCols, MT>& s, const Cursor& cur) {
+    const int step = cur.step + wave;
+    if (step >= cur.end) return;  // uniform: no step for this wavefront in this round
+    const bool k_ok = min(step * kStep, p.k - kStep) + kg * 8 >= step * kStep;
+    u32x4 a[MT];
+#pragma unroll
+    for (int h = 0; h < MT; ++h) a[h] = k_ok ? s.xa[h] : u32x4{0u, 0u, 0u, 0u};
 #pragma unroll
     for (int i = 0; i < kCols; ++i) {
       // channel n0 + i: its 8 k-values, as packed pairs (k, k+1)
@@ -163,77 +190,82 @@ __global__ __launch_bounds__(kWaves * 64) __attribute__((amdgpu_waves_per_eu(kOc
 #pragma unroll
         for (int q = 0; q < 4; ++q) b[q] = __builtin_amdgcn_perm(s.w[2 * q + 1][i >> 1], s.w[2 * q][i >> 1], sel);
       }
-      acc[i][0] = mfma16<BF16>(a0, b, acc[i][0]);
-      acc[i][1] = mfma16<BF16>(a1, b, acc[i][1]);
+#pragma unroll
+      for (int h = 0; h < MT; ++h) acc[i][h] = mfma16<BF16>(a[h], b, acc[i][h]);
       __builtin_amdgcn_sched_barrier(0);  // keep the conversions next to their MFMAs
     }
   };
 
-  // Wavefront w takes steps w, w + kWaves, ...; kStages register stages, all but the one being
-  // consumed in flight.  The trip count is rounded up to whole rounds of kStages: surplus steps
-  // multiply by zero.
-  Stage<W8, kCols> st[kStages];
+  // End of a run: the wavefronts' accumulators through LDS into one partial slab.  acc[i][h][r] is row
+  // h*16 + 4*kg + r, channel c*kCols + i; the float4s of a row are kept in the order (v, c) - channels c*kCols + 4v .. -
+  // so that neither the writes nor the reads of 16 lanes collide in a bank.
+  constexpr int kQuads = kSlab / 4;
+  auto finish_run = [&](const Cursor& cur) {
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");  // the last run's sums have been read
+    float4* mine = reinterpret_cast<float4*>(red) + wave * (kRows * kQuads) + c;
 #pragma unroll
-  for (int u = 0; u < kStages - 1; ++u) load(st[u], wave + u * kWaves);
-  for (int s = wave; s < n_steps; s += kStages * kWaves) {
+    for (int h = 0; h < MT; ++h)
 #pragma unroll
-    for (int u = 0; u < kStages; ++u) {
-      load(st[(u + kStages - 1) % kStages], s + (u + kStages - 1) * kWaves);
-      compute(st[u], s + u * kWaves);
-    }
-  }
-
-  // ---- sum the accumulators: upper half -> LDS -> lower half -> LDS -> all threads ----------
-  // acc[i][h][r]: row m = h*16 + 4*kg + r, channel c*8 + i of the slab.
-  if (wave >= kHalf) {
-    float* dst = red + (wave - kHalf) * (kMaxM * kSlab) + lane;
-#pragma unroll
-    for (int i = 0; i < kCols; ++i)
-#pragma unroll
-      for (int h = 0; h < 2; ++h)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) dst[((i * 2 + h) * 4 + r) * 64] = acc[i][h][r];
-  }
-  __syncthreads();
-  if (wave < kHalf) {
-    const float* src = red + wave * (kMaxM * kSlab) + lane;
-#pragma unroll
-    for (int i = 0; i < kCols; ++i)
-#pragma unroll
-      for (int h = 0; h < 2; ++h)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) acc[i][h][r] += src[((i * 2 + h) * 4 + r) * 64];
-  }
-  __syncthreads();
-  if (wave < kHalf) {
-    float* dst = red + wave * (kMaxM * kSlab);
-#pragma unroll
-    for (int h = 0; h < 2; ++h)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int m = h * 16 + 4 * kg + r;
-        float4* d4 = reinterpret_cast<float4*>(dst + m * kSlab + c * kCols);
+      for (int r = 0; r < 4; ++r)
 #pragma unroll
         for (int v = 0; v < kCols / 4; ++v)
-          d4[v] = float4{acc[4 * v][h][r], acc[4 * v + 1][h][r], acc[4 * v + 2][h][r], acc[4 * v + 3][h][r]};
+          mine[(h * 16 + 4 * kg + r) * kQuads + v * 16] =
+              float4{acc[4 * v][h][r], acc[4 * v + 1][h][r], acc[4 * v + 2][h][r], acc[4 * v + 3][h][r]};
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    const int mat = cur.slab >= p.slabs ? 1 : 0;
+    // partial slab number: how many workgroups before this one hold steps of the slab (the one
+    // that holds its first unit has number 0)
+    const int first = cur.slab * p.ks;
+    const int owner = p.mapped ? (int)(((unsigned)(first + 1) * (unsigned)wgs - 1) / (unsigned)(p.per_wg * wgs + p.extra)) : wg;
+    const int q = tid % kQuads, n = (cur.slab - mat * p.slabs) * kSlab + (q & 15) * kCols + (q >> 4) * 4;
+    float* out = p.part[mat] + (size_t)(wg - owner) * p.m * p.n + n;
+    if (n < p.n) {
+      for (int row = tid / kQuads; row < p.m; row += kWaves * 64 / kQuads) {
+        const float4* src = reinterpret_cast<const float4*>(red) + row * kQuads + q;
+        float4 a = src[0];
+#pragma unroll
+        for (int w = 1; w < kWaves; ++w) {
+          const float4 v = src[w * (kRows * kQuads)];
+          a.x += v.x; a.y += v.y; a.z += v.z; a.w += v.w;
+        }
+        *reinterpret_cast<float4*>(out + (size_t)row * p.n) = a;
       }
-  }
-  __syncthreads();
-  // thread t sums one float4 chunk of rows t / chunks, t / chunks + rows per pass, ... over the
-  // remaining slices (chunks = float4s per slab row)
-  constexpr int kChunks = kSlab / 4;
-  constexpr int kRowsPerPass = kWaves * 64 / kChunks;
-#pragma unroll
-  for (int m = tid / kChunks; m < kMaxM; m += kRowsPerPass) {
-    const int ch = (tid % kChunks) * 4;
-    float4 a = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int w = 0; w < kHalf; ++w) {
-      const float4 v = *reinterpret_cast<const float4*>(red + w * (kMaxM * kSlab) + m * kSlab + ch);
-      a.x += v.x; a.y += v.y; a.z += v.z; a.w += v.w;
     }
-    const int n = slab * kSlab + ch;
-    if (n < p.n) *reinterpret_cast<float4*>(p.part[mat] + ((size_t)split * kMaxM + m) * p.n + n) = a;
+    clear();
+  };
+
+  Cursor use, ahead;
+  use.slab = u_begin / p.ks;
+  use.step = u_begin - use.slab * p.ks;
+  use.end = run_end(use.slab);
+  ahead = use;
+  // Two register stages, one of them in flight while the other is multiplied (three and four measured slower: one
+  // sequence's layer 75.2 -> 77.8 / 79.2 us).  The last round is a copy of its own that requests nothing:
+  // behind a branch around the loads the compiler would wait for all of them in every round, and reading
+  // the last rows again costs as much as a new round.
+  Stage<W8, kCols, MT> st[2];
+  load(st[0], ahead);
+  auto round = [&](const Stage<W8, kCols, MT>& cur) {
+    compute(cur, use);
+    if (last_of_run(use)) finish_run(use);
+  };
+  for (;;) {
+    if (last(use)) {
+      round(st[0]);
+      break;
+    }
+    advance(ahead);
+    load(st[1], ahead);
+    round(st[0]);
+    advance(use);
+    if (last(use)) {
+      round(st[1]);
+      break;
+    }
+    advance(ahead);
+    load(st[0], ahead);
+    round(st[1]);
+    advance(use);
   }
 }
 
@@ -247,6 +279,7 @@ struct FinishParams {
   int m, n, splits, res_dtype, out_dtype;
   int out_blocked;  // write out as [N/8][32][8] for the next projection
   int64_t stride;
+  pto_hip::SlabMap map;
 };
 
 // Element index of (row m, channel n) in the blocked activation layout [N/8][32][8].
@@ -306,9 +339,9 @@ __global__ __launch_bounds__(256) void w8a16_finish_kernel(FinishParams p) {
   const int n = (blockIdx.x * 256 + threadIdx.x) * 4;
   const int m = blockIdx.y;
   if (n >= p.n) return;
-  float4 a = sum_splits(p.part0, p.scale0, p.splits, (size_t)p.stride, m, n, p.n);
+  float4 a = sum_splits(p.part0, p.scale0, pto_hip::slab_count(p.map, p.splits, 0, n), (size_t)p.stride, m, n, p.n);
   if (p.part1) {
-    const float4 u = sum_splits(p.part1, p.scale1, p.splits, (size_t)p.stride, m, n, p.n);
+    const float4 u = sum_splits(p.part1, p.scale1, pto_hip::slab_count(p.map, p.splits, 1, n), (size_t)p.stride, m, n, p.n);
     a = float4{silu_mul(a.x, u.x), silu_mul(a.y, u.y), silu_mul(a.z, u.z), silu_mul(a.w, u.w)};
   }
   const size_t idx = (size_t)m * p.n + n;
@@ -335,6 +368,7 @@ struct FinishNormParams {
   int out_blocked;
   float eps;
   int64_t stride;  // elements between splits
+  pto_hip::SlabMap map;
 };
 
 __global__ __launch_bounds__(kNormThreads) void w8a16_finish_norm_kernel(FinishNormParams p) {
@@ -347,7 +381,7 @@ __global__ __launch_bounds__(kNormThreads) void w8a16_finish_norm_kernel(FinishN
     const int n = (threadIdx.x + u * kNormThreads) * 4;
     if (n < p.n) {
       g[u] = *reinterpret_cast<const float4*>(p.gamma + n);
-      float4 a = sum_splits(p.part, p.scale, p.splits, (size_t)p.stride, m, n, p.n);
+      float4 a = sum_splits(p.part, p.scale, pto_hip::slab_count(p.map, p.splits, 0, n), (size_t)p.stride, m, n, p.n);
       const float4 r = load4_as_f32(p.residual, (size_t)m * p.n + n, p.res_dtype);
       a.x += r.x; a.y += r.y; a.z += r.z; a.w += r.w;
       v[u] = a;
@@ -393,35 +427,18 @@ int check_common(const char* what, int64_t m, int64_t k, int64_t n, int x_dtype,
   return PTO_HIP_OK;
 }
 
-// k splits.  A CU pulls its weight bytes at a bounded rate (about its 1/num_cu share of the HBM
-// rate), so a launch lasts as long as the CU with the most bytes: 272 workgroups on 256 CUs leave
-// 16 CUs with twice the work and ran 1.5x longer than 256 would.  The split count is the one
-// that minimises   rounds x (steps per wavefront + ramp) + splits x partial-sum cost,
-// rounds = ceil(workgroups / (wgs_per_cu x num_cu)); the constants are fitted to measured
-// launches (ramp 2.5 steps; one split's partial sums cost about n_total / 10000 steps).
-// Split boundaries fall on multiples of the rows one round of the wavefronts covers, and a
-// wavefront keeps at least min_steps steps when k allows.
-void choose_splits(int64_t k, int64_t slabs_total, int64_t n_total, int waves, int* splits, int* k_per_split) {
-  const int kUnit = kStep * waves;  // k rows one round of the wavefronts covers
-  const pto_hip::Context& cx = pto_hip::ctx();
-  const int64_t units = (k + kUnit - 1) / kUnit;
-  const int64_t capacity = std::max<int64_t>(1, cx.w8a16_wgs_per_cu * cx.num_cu);
-  const double ramp = 2.5, partial_cost = (double)n_total / 10000.0;
-  int64_t best_per = units;
-  double best_cost = 1e30;
-  for (int64_t want = 1; want <= std::min<int64_t>(units, 16); ++want) {
-    const int64_t per = (units + want - 1) / want;
-    if (want > 1 && per < cx.w8a16_min_steps) break;
-    const int64_t real = (units + per - 1) / per;
-    const int64_t rounds = (slabs_total * real + capacity - 1) / capacity;
-    const double cost = (double)rounds * ((double)per + ramp) + (real > 1 ? (double)real * partial_cost : 0.0);
-    if (cost < best_cost) {
-      best_cost = cost;
-      best_per = per;
-    }
+template <bool BF16, bool W8, int kCols, int MT>
+int launch_partial(const GemvParams& p, int wgs, bool nt, hipStream_t st) {
+  const size_t smem = (size_t)kWaves * 16 * MT * 16 * kCols * sizeof(float);
+  auto kern = nt ? w8a16_partial_kernel<BF16, W8, kCols, MT, true> : w8a16_partial_kernel<BF16, W8, kCols, MT, false>;
+  static std::atomic<bool> attr_set[2];  // per instantiation; callers hold the dispatch lock
+  if (!attr_set[nt].load(std::memory_order_acquire)) {
+    PTO_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem));
+    attr_set[nt].store(true, std::memory_order_release);
   }
-  *splits = (int)((units + best_per - 1) / best_per);
-  *k_per_split = (int)(best_per * kUnit);
+  hipLaunchKernelGGL(kern, dim3((unsigned)wgs), dim3(kWaves * 64), smem, st, p);
+  PTO_CHECK_HIP(hipGetLastError());
+  return PTO_HIP_OK;
 }
 
 }  // namespace
@@ -437,52 +454,61 @@ int w8a16_partials(const void* x, bool x_blocked, const void* wq0, const void* w
   p.m = (int)m;
   p.k = (int)k;
   p.n = (int)n;
-  // int8 codes are read 16 per lane (a 256-channel slab per workgroup, half the requests per byte)
-  // for large matrices when rows and base addresses allow 16-byte loads, else 8 per lane like the
-  // 16-bit weights.  Every workgroup also reads the activations of its k range - 64 bytes per k row
-  // next to 128 bytes of codes with a 128-channel slab - and a CU takes in a bounded number of bytes
-  // per second whatever they are (counters: the decoder layer's gate/up launch requests 177 MB from
-  // L2 for 117 MB of codes, 6.2 TB/s over the chip), so the wider slab moves a sixth less per code.
-  // Measured: 117 MB of codes (two 4096 x 14336 matrices) 28.2 -> 25.6 us, 235 MB 3.6 -> 4.5 TB/s,
-  // 525 MB 4.2 -> 4.8 TB/s; but 59 MB 16.1 -> 17.2 us, 25 MB 10.2 -> 13.0 us (half the slabs, so twice
-  // the k splits or fewer workgroups), hence the size bound.
-  const bool wide = !w16 && ctx().w8a16_wide != 0 && n % 16 == 0 && ((uintptr_t)wq0 | (uintptr_t)wq1) % 16 == 0 &&
-                    (ctx().w8a16_wide == 2 || k * n * (wq1 ? 2 : 1) >= (int64_t)100 * 1000 * 1000);
-  const int slab_cols = wide ? 2 * kSlab : kSlab;
-  p.slabs = (int)((n + slab_cols - 1) / slab_cols);
-  p.n_mats = wq1 ? 2 : 1;
   p.x_blocked = x_blocked ? 1 : 0;
-  choose_splits(k, (int64_t)p.slabs * p.n_mats, n * p.n_mats, kWavesPerWg, &p.splits, &p.k_per_split);
-  const size_t one = (size_t)p.splits * kMaxM * n * sizeof(float);
+  const Context& cx = ctx();
+  const int n_mats = wq1 ? 2 : 1;
+  // int8 codes are read 16 per lane (256-channel slabs, 256-byte row pieces instead of 128) when rows and base
+  // addresses allow 16-byte loads and the matrices are large.  Twice the channels in a slab are twice the partial
+  // sums at the same number of workgroups, and 32 instead of 16 KB per wavefront through LDS at the end of a run.
+  // Measured with their finish at 1 / 16 / 32 rows: 178 MB 36.0 / 38.8 / 44.6 us (8 per lane: 36.4 / 42.0 / 50.2), 117 MB
+  // 24.1 / 26.0 / 29.6 (25.6 / 29.2 / 34.0), 89 MB 20.4 / 22.1 / 25.7 (21.9 / 24.9 / 28.6); but 67 MB 16.5 / 18.2 / 21.7
+  // (15.6 / 17.7 / 20.7), 59 MB 15.8 / 17.5 / 20.7 (14.7 / 16.5 / 19.2), 17 MB 9.0 / 10.5 / 12.7 (8.2 / 9.3 / 10.8).
+  const bool wide = !w16 && cx.w8a16_wide != 0 && n % 16 == 0 && ((uintptr_t)wq0 | (uintptr_t)wq1) % 16 == 0 &&
+                    (cx.w8a16_wide == 2 || k * n * n_mats >= (int64_t)80 * 1000 * 1000);
+  const int cols = wide ? 16 : 8, slab = 16 * cols;
+  p.slabs = (int)((n + slab - 1) / slab);
+  p.ks = (int)((k + kStep - 1) / kStep);
+  // Workgroups: one per CU at most (a second one on some CUs is what the slowest CU waits for: 17 MB of codes take
+  // 8.2 us on 256 and 9.9 on 288), and where the slabs allow it a whole number of them per slab, so that
+  // a workgroup has one run and its partial sums one slab (117 MB pair at 32 rows: 224 workgroups 29.6 us, 256 33.0).
+  // Of those the smallest number with the same count of rounds per wavefront, at least min_steps of them.
+  const int64_t slabs_total = (int64_t)p.slabs * n_mats, units = slabs_total * p.ks;
+  const int64_t most = std::max<int64_t>(1, cx.w8a16_wgs_per_cu * cx.num_cu);
+  int64_t wgs = most;
+  if (slabs_total <= most) {
+    auto rounds = [&](int64_t per_slab) { return ((p.ks + per_slab - 1) / per_slab + kWaves - 1) / kWaves; };
+    int64_t per_slab = std::max<int64_t>(1, std::min<int64_t>(most / slabs_total, p.ks / (kWaves * cx.w8a16_min_steps)));
+    while (per_slab > 1 && rounds(per_slab - 1) == rounds(per_slab)) --per_slab;
+    wgs = slabs_total * per_slab;
+  }
+  // (units * wgs is computed in 32 bits by the kernels; shapes beyond that get a workgroup per slab)
+  const bool mapped = units * wgs < (1ll << 31);
+  if (!mapped) wgs = (int64_t)p.slabs * n_mats;
+  p.per_wg = (int)(units / wgs);
+  p.extra = (int)(units % wgs);
+  p.mapped = mapped ? 1 : 0;
+  out->map = mapped ? SlabMap{(unsigned)units, (unsigned)wgs, (unsigned)p.ks, wide ? 8 : 7, p.slabs} : SlabMap{};
+  out->splits = mapped ? (int)((p.ks * wgs + units - 1) / units) + 1 : 1;  // at most
+  const size_t one = (size_t)out->splits * m * n * sizeof(float);
   void* ws = nullptr;
-  int rc = workspace(one * p.n_mats, &ws);
+  int rc = workspace(one * n_mats, &ws);
   if (rc) return rc;
   p.part[0] = reinterpret_cast<float*>(ws);
   p.part[1] = reinterpret_cast<float*>(reinterpret_cast<char*>(ws) + one);
-  const dim3 grid((unsigned)(p.slabs * p.n_mats * p.splits));
-  // Four wavefronts x two stages: measured best in the decoder layer against 2, 4 and 8 wavefronts
-  // with 2-4 stages (more requests in flight per CU only lengthened the memory queueing delay).
-  const dim3 block((unsigned)kWavesPerWg * 64);
-  const bool bf = x_dtype == PTO_HIP_BF16;
-  const bool nt = ctx().w8a16_nt != 0;
-  auto go = [&](auto plain, auto streamed) { hipLaunchKernelGGL(nt ? streamed : plain, grid, block, 0, st, p); };
-  if (w16) {  // twice the bytes per stage: three wavefronts per SIMD
-    if (bf) go(w8a16_partial_kernel<true, false, 8, kWavesPerWg, 2, 3>, w8a16_partial_kernel<true, false, 8, kWavesPerWg, 2, 3, true>);
-    else go(w8a16_partial_kernel<false, false, 8, kWavesPerWg, 2, 3>, w8a16_partial_kernel<false, false, 8, kWavesPerWg, 2, 3, true>);
-  } else if (wide) {  // 32 accumulators per lane: two wavefronts per SIMD
-    if (bf) go(w8a16_partial_kernel<true, true, 16, kWavesPerWg, 2, 2>, w8a16_partial_kernel<true, true, 16, kWavesPerWg, 2, 2, true>);
-    else go(w8a16_partial_kernel<false, true, 16, kWavesPerWg, 2, 2>, w8a16_partial_kernel<false, true, 16, kWavesPerWg, 2, 2, true>);
-  } else {
-    // register budget of three wavefronts per SIMD: with four (128 registers) one value spilled to
-    // scratch memory (decoder layer 183.0 -> 181.3 us a step)
-    if (bf) go(w8a16_partial_kernel<true, true, 8, kWavesPerWg, 2, 3>, w8a16_partial_kernel<true, true, 8, kWavesPerWg, 2, 3, true>);
-    else go(w8a16_partial_kernel<false, true, 8, kWavesPerWg, 2, 3>, w8a16_partial_kernel<false, true, 8, kWavesPerWg, 2, 3, true>);
-  }
-  PTO_CHECK_HIP(hipGetLastError());
+  const bool bf = x_dtype == PTO_HIP_BF16, nt = cx.w8a16_nt != 0, two = m > 16;
+  auto go = [&](auto w8, auto kcols) {
+    constexpr bool W8 = decltype(w8)::value;
+    constexpr int C = decltype(kcols)::value;
+    if (bf) return two ? launch_partial<true, W8, C, 2>(p, (int)wgs, nt, st) : launch_partial<true, W8, C, 1>(p, (int)wgs, nt, st);
+    return two ? launch_partial<false, W8, C, 2>(p, (int)wgs, nt, st) : launch_partial<false, W8, C, 1>(p, (int)wgs, nt, st);
+  };
+  typedef std::integral_constant<int, 8> C8;
+  typedef std::integral_constant<int, 16> C16;
+  rc = w16 ? go(std::false_type{}, C8{}) : wide ? go(std::true_type{}, C16{}) : go(std::true_type{}, C8{});
+  if (rc) return rc;
   out->part[0] = p.part[0];
   out->part[1] = wq1 ? p.part[1] : nullptr;
-  out->splits = p.splits;
-  out->slab_stride = (int64_t)kMaxM * n;
+  out->slab_stride = m * n;
   out->scaled = false;
   return PTO_HIP_OK;
 }
@@ -503,6 +529,7 @@ int w8a16_finish(const W8Partials& parts, const float* scale0, const float* scal
   f.out_dtype = out_dtype;
   f.out_blocked = out_blocked ? 1 : 0;
   f.stride = parts.slab_stride;
+  f.map = parts.map;
   hipLaunchKernelGGL(w8a16_finish_kernel, dim3((unsigned)((n / 4 + 255) / 256), (unsigned)m), dim3(256), 0, st, f);
   PTO_CHECK_HIP(hipGetLastError());
   return PTO_HIP_OK;
@@ -527,6 +554,7 @@ int w8a16_finish_norm(const W8Partials& parts, const float* scale, const void* r
   f.out_blocked = out_blocked ? 1 : 0;
   f.eps = eps;
   f.stride = parts.slab_stride;
+  f.map = parts.map;
   hipLaunchKernelGGL(w8a16_finish_norm_kernel, dim3((unsigned)m), dim3(kNormThreads), 0, st, f);
   PTO_CHECK_HIP(hipGetLastError());
   return PTO_HIP_OK;

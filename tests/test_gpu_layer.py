@@ -5,7 +5,8 @@ import torch
 
 import oracle
 from pypto_amd import workloads
-from pypto_amd.runtime import (decoder_layer_decode, decoder_layer_decode_fp8kv, decoder_layer_decode_w16, rope_kv_cache_update, rope_kv_cache_update_fp8,
+from pypto_amd.runtime import (decoder_layer_decode, decoder_layer_decode_fp8kv, decoder_layer_decode_w16, gate_up_swiglu,
+                               projection, rope_kv_cache_update, rope_kv_cache_update_fp8,
                                validate_golden, w8a16_matmul,
                                w8a16_matmul_residual, w8a16_swiglu)
 
@@ -639,3 +640,40 @@ def test_llama_mini_argument_rules(worker):
         bad[2] = torch.zeros(8, 32)
         with pytest.raises(ValueError, match="cos_emb"):
             h(*bad)
+
+
+@pytest.mark.parametrize("kind", ["int8", "int8_wide", "w16"])
+@pytest.mark.parametrize("m,k,n,pair", [(1, 48, 33040, False),   # more slabs than CUs: shares of the list cross slabs, k ends in half a step
+                                        (17, 112, 20800, True),  # ... of a pair of matrices, two row groups
+                                        (16, 1040, 304, False),  # a few slabs, several workgroups on each, a ragged last slab
+                                        (32, 4096, 128, True), (5, 32, 16, False)])
+def test_skinny_projection_shares_are_exact(worker, kind, m, k, n, pair):
+    """Every share of the (slab, step) list against the integer product: small-integer operands make every sum exact
+    whatever its order, so a row, channel or step counted twice or left out shows."""
+    g = torch.Generator().manual_seed(m + k + n)
+    x = torch.randint(-2, 3, (m, k), generator=g).to(torch.bfloat16)
+    w = [torch.randint(-3, 4, (k, n), generator=g) for _ in range(2)]
+    one = torch.ones(n)
+    out = torch.full((m, n), float("nan"), dtype=torch.float32 if not pair else torch.bfloat16)
+    worker.set_option("w8a16_wide", {"int8": 0, "int8_wide": 2, "w16": 1}[kind])
+    try:
+        if kind == "w16":
+            ws = [t.to(torch.bfloat16) for t in w]
+            if pair:
+                worker.run(gate_up_swiglu, x, ws[0], ws[1], out)
+            else:
+                worker.run(projection, x, ws[0], out)
+        else:
+            ws = [t.to(torch.int8) for t in w]
+            if pair:
+                worker.run(w8a16_swiglu, x, ws[0], one, ws[1], one, out)
+            else:
+                worker.run(w8a16_matmul, x, ws[0], one, out)
+    finally:
+        worker.set_option("w8a16_wide", 1)
+    gate, up = (x.double() @ t.double() for t in w)
+    if pair:
+        # one bf16 ulp (2^-7) of SwiGLU's value; exact zeros stay zeros
+        torch.testing.assert_close(out.double(), oracle.swiglu(gate, up), rtol=2 ** -7, atol=1e-30)
+    else:
+        assert torch.equal(out.double(), gate)
