@@ -504,15 +504,31 @@ int launch_gemm(GemmParams p, hipStream_t st) {
 // A row the swizzle key is (row / 4) % 4 (16 consecutive rows of a fragment read then cover all 16
 // slots of four rows' worth of banks), B keeps 64-byte group g ^ (k-row % 8).  Built for 16-bit
 // weights with n and every k range multiples of the tile (EDGE_M: any number of rows).
+//
+// MT: the tile is 64 * MT rows high, a wavefront's part 32 * MT.  The loop's time is the MFMAs of the rows the tile has,
+// padding included: 333 rows are 512 rows' work on 256-row tiles, 384 on 192-row ones.  A stage is 4 KB smaller
+// per 64 rows, and what that leaves of the LDS goes into more stages in flight.  The low tiles replace eight-wavefront
+// ones wherever n and k allow; passes with their finish, best split count of each: 4096 x 14336 gate/up at 128 / 333 /
+// 700 rows 67 / 97 / 193 -> 60 / 88 / 167 us, 14336 x 4096 at 96 / 333 / 2500 rows 37 / 65 / 282 -> 33 / 56 / 245,
+// 1024 x 3072 gate/up at 96 / 512 rows 14.5 / 16.5 -> 12.3 / 12.8.
 constexpr int QK = 32;   // k extent of a stage
-constexpr int QST = 5;   // stages
-constexpr int kQuadStageBytes = (256 * QK + QK * BN) * 2;  // A rows, then B rows
+constexpr int quad_stages(int mt) { return mt >= 3 ? 5 : mt == 2 ? 6 : 8; }
+constexpr int quad_stage_bytes(int mt) { return (64 * mt * QK + QK * BN) * 2; }  // A rows, then B rows
 typedef __attribute__((address_space(3))) const char lds_cchar;
 typedef __attribute__((address_space(3))) const u32x4 lds_cu32x4;
 template <int N>
 struct QuadConst {
   static constexpr int value = N;
 };
+
+// f(QuadConst<0>) .. f(QuadConst<N - 1>)
+template <int I, int N, typename F>
+__device__ __forceinline__ void quad_for(F&& f) {
+  if constexpr (I < N) {
+    f(QuadConst<I>{});
+    quad_for<I + 1, N>(f);
+  }
+}
 
 // One direct request: 16 bytes per lane from `src` to the KB of LDS at lds_w + OFF (wave-uniform).
 template <int OFF>
@@ -523,10 +539,12 @@ __device__ __forceinline__ void quad_to_lds(const char* src, uint32_t lds_w) {
 #pragma clang diagnostic pop
 }
 
-template <bool DUAL, bool BF16, typename OutT, bool EDGE_M>
+template <int MT, bool DUAL, bool BF16, typename OutT, bool EDGE_M>
 __global__ __launch_bounds__(256) void gemm_quad_kernel(GemmParams p) {
-  constexpr int MT = 4, NT = 4;
-  constexpr int A_BYTES = 256 * QK * 2;
+  constexpr int NT = 4;
+  constexpr int BM = 64 * MT;
+  constexpr int QST = quad_stages(MT), kStageBytes = quad_stage_bytes(MT);
+  constexpr int A_BYTES = BM * QK * 2;
   extern __shared__ __attribute__((aligned(16))) uint16_t smem[];
   lds_cchar* lds0 = (lds_cchar*)smem;
   const int tid = threadIdx.x;
@@ -540,14 +558,14 @@ __global__ __launch_bounds__(256) void gemm_quad_kernel(GemmParams p) {
   tile_coords(tile, p.tiles_m, p.tiles_n, tm, tn);
   const int k_begin = split * p.k_per_split;
   const int klen = min(p.k, k_begin + p.k_per_split) - k_begin;
-  const int m0 = tm * 256;
+  const int m0 = tm * BM;
   const int n0 = tn * (DUAL ? BN / 2 : BN);
   const int nk = klen / QK;
 
   // Requests.  A: instruction e brings rows 64 e + 16 wave + lane / 4, the lane's bytes land in slot
   // lane % 4 of its row.  B: instruction e brings k-rows 8 e + 2 wave + lane / 32, slot lane % 32.
   // Either way a wavefront's instruction e fills the KB at e * 4 KB + wave * 1 KB of its operand's
-  // half of the stage.
+  // part of the stage.
   const int a_chunk = (lane & 3) ^ ((lane >> 4) & 3);
   const int b_krow = 2 * wave + (lane >> 5);
   const int b_chunk = ((((lane & 31) >> 2) ^ (b_krow & 7)) << 2) | (lane & 3);
@@ -557,13 +575,16 @@ __global__ __launch_bounds__(256) void gemm_quad_kernel(GemmParams p) {
     bsrc = b_chunk < 16 ? p.b0 : p.b1;
     b_col = n0 + (b_chunk & 15) * 8;
   }
-  const char* ga[4];  // this lane's source of request e, for the stage requested next
+  const char* ga[MT];  // this lane's source of request e, for the stage requested next
   const char* gb[4];
 #pragma unroll
-  for (int e = 0; e < 4; ++e) {
+  for (int e = 0; e < MT; ++e) {
     int a_row = m0 + 64 * e + 16 * wave + (lane >> 2);
     if (EDGE_M) a_row = min(a_row, p.m - 1);  // rows past the end read the last row; their products are not stored
     ga[e] = reinterpret_cast<const char*>(p.a + (int64_t)a_row * p.lda + k_begin + a_chunk * 8);
+  }
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
     gb[e] = reinterpret_cast<const char*>(bsrc + (int64_t)(k_begin + 8 * e + b_krow) * p.ldb + b_col);
   }
   const int64_t a_adv = QK * 2, b_adv = (int64_t)QK * p.ldb * 2;  // bytes from one stage to the next
@@ -581,19 +602,20 @@ __global__ __launch_bounds__(256) void gemm_quad_kernel(GemmParams p) {
   // 64 KB past its address register, two stages: one register per pair of stages.
   const int a_key = ((lane & 31) >> 2) & 3;
   const int grp = lane >> 4, sub = lane & 15;
-  lds_cchar* a_base[3][2];
-  lds_cchar* b_base[3][NT][2];
+  constexpr int kPairs = (QST + 1) / 2;
+  lds_cchar* a_base[kPairs][2];
+  lds_cchar* b_base[kPairs][NT][2];
 #pragma unroll
-  for (int h = 0; h < 3; ++h) {
+  for (int h = 0; h < kPairs; ++h) {
 #pragma unroll
     for (int ks = 0; ks < 2; ++ks)
-      a_base[h][ks] = lds0 + h * 2 * kQuadStageBytes + ((wm * 128 + (lane & 31)) * QK + (((2 * ks) | (lane >> 5)) ^ a_key) * 8) * 2;
+      a_base[h][ks] = lds0 + h * 2 * kStageBytes + ((wm * 32 * MT + (lane & 31)) * QK + (((2 * ks) | (lane >> 5)) ^ a_key) * 8) * 2;
 #pragma unroll
     for (int jn = 0; jn < NT; ++jn) {
       const int col = DUAL ? ((jn / 2) * (BN / 2) + wn * 64 + (jn % 2) * 32) : (wn * 128 + jn * 32);
 #pragma unroll
       for (int half = 0; half < 2; ++half)
-        b_base[h][jn][half] = lds0 + h * 2 * kQuadStageBytes + A_BYTES +
+        b_base[h][jn][half] = lds0 + h * 2 * kStageBytes + A_BYTES +
                               (((grp >> 1) * 8 + half * 4 + (sub >> 2)) * BN + (((col >> 5) ^ (half * 4 + (sub >> 2))) << 5) +
                                (grp & 1) * 16 + (sub & 3) * 4) * 2;
     }
@@ -601,7 +623,7 @@ __global__ __launch_bounds__(256) void gemm_quad_kernel(GemmParams p) {
   u32x4 fa[2][MT], fb[2][NT];
   auto read_one = [&](auto st_c, int ks, int set, int r) {
     constexpr int ST = decltype(st_c)::value;
-    constexpr int kOff = (ST % 2) * kQuadStageBytes;
+    constexpr int kOff = (ST % 2) * kStageBytes;
     if (r < MT) {
       fa[set][r] = *reinterpret_cast<lds_cu32x4*>(a_base[ST / 2][ks] + kOff + r * 32 * QK * 2);
     } else {
@@ -612,41 +634,30 @@ __global__ __launch_bounds__(256) void gemm_quad_kernel(GemmParams p) {
       fb[set][jn][half * 2 + 1] = v.y;
     }
   };
-  constexpr int kReads = MT + 2 * NT;  // 12 LDS reads per k-step
-  constexpr int kSlots = MT * NT;      // 16 MFMAs per k-step
-  constexpr int kInFlight = 8 * (QST - 3);  // every wait leaves the requests of the newest QST - 3 stages outstanding
+  constexpr int kReads = MT + 2 * NT;  // LDS reads per k-step
+  constexpr int kSlots = MT * NT;      // MFMAs per k-step
+  constexpr int kReadsPerSlot = (kReads + kSlots - 1) / kSlots;
+  constexpr int kRequests = MT + 4;    // per stage: A, then B
+  constexpr int kInFlight = kRequests * (QST - 3);  // every wait leaves the requests of the newest QST - 3 stages outstanding
 
-  // request e (0-3: A, 4-7: B) of the stage the pointers stand at, into buffer ST
-  auto request = [&](auto st_c, int e) {
-    constexpr int ST = decltype(st_c)::value;
-    if (e == 0) quad_to_lds<ST * kQuadStageBytes + 0 * 4096>(ga[0], lds_w);
-    if (e == 1) quad_to_lds<ST * kQuadStageBytes + 1 * 4096>(ga[1], lds_w);
-    if (e == 2) quad_to_lds<ST * kQuadStageBytes + 2 * 4096>(ga[2], lds_w);
-    if (e == 3) quad_to_lds<ST * kQuadStageBytes + 3 * 4096>(ga[3], lds_w);
-    if (e == 4) quad_to_lds<ST * kQuadStageBytes + 4 * 4096>(gb[0], lds_w);
-    if (e == 5) quad_to_lds<ST * kQuadStageBytes + 5 * 4096>(gb[1], lds_w);
-    if (e == 6) quad_to_lds<ST * kQuadStageBytes + 6 * 4096>(gb[2], lds_w);
-    if (e == 7) quad_to_lds<ST * kQuadStageBytes + 7 * 4096>(gb[3], lds_w);
+  // request e of the stage the pointers stand at, into buffer ST
+  auto request = [&](auto st_c, auto e_c) {
+    constexpr int ST = decltype(st_c)::value, E = decltype(e_c)::value;
+    if constexpr (E < MT) quad_to_lds<ST * kStageBytes + E * 4096>(ga[E], lds_w);
+    else quad_to_lds<ST * kStageBytes + E * 4096>(gb[E - MT], lds_w);
   };
   // moves the pointers on to stage `next` unless that is past the end (then the last stage is requested again)
   auto advance = [&](int next) {
     const int64_t da = next < nk ? a_adv : 0, db = next < nk ? b_adv : 0;
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      ga[e] += da;
-      gb[e] += db;
-    }
-  };
-  auto prologue_stage = [&](auto st_c) {
-    constexpr int ST = decltype(st_c)::value;
+    for (int e = 0; e < MT; ++e) ga[e] += da;
 #pragma unroll
-    for (int e = 0; e < 8; ++e) request(st_c, e);
-    advance(ST + 1);
+    for (int e = 0; e < 4; ++e) gb[e] += db;
   };
-  prologue_stage(QuadConst<0>{});
-  prologue_stage(QuadConst<1>{});
-  prologue_stage(QuadConst<2>{});
-  prologue_stage(QuadConst<3>{});
+  quad_for<0, QST - 1>([&](auto st_c) {
+    quad_for<0, kRequests>([&](auto e_c) { request(st_c, e_c); });
+    advance(decltype(st_c)::value + 1);
+  });
   asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kInFlight) : "memory");  // stages 0 and 1 have landed
   __syncthreads();
 #pragma unroll
@@ -656,19 +667,25 @@ __global__ __launch_bounds__(256) void gemm_quad_kernel(GemmParams p) {
   auto iteration = [&](auto st_c, int t) {
     constexpr int ST = decltype(st_c)::value;
     // k-step 0: fragments of k-step 1 and the requests of stage t + QST - 1 (its buffer was last read in iteration t - 1)
-#pragma unroll
-    for (int q = 0; q < kSlots; ++q) {
+    quad_for<0, kSlots>([&](auto q_c) {
+      constexpr int q = decltype(q_c)::value;
       acc[q / NT][q % NT] = mfma32<BF16>(fa[0][q / NT], fb[0][q % NT], acc[q / NT][q % NT]);
-      if (q < kReads) read_one(st_c, 1, 1, q);
-      if ((q & 1) == 0) request(QuadConst<(ST + QST - 1) % QST>{}, q >> 1);
+#pragma unroll
+      for (int r = q * kReadsPerSlot; r < (q + 1) * kReadsPerSlot; ++r)
+        if (r < kReads) read_one(st_c, 1, 1, r);
+      quad_for<0, kRequests>([&](auto e_c) {
+        if constexpr (decltype(e_c)::value * kSlots / kRequests == q) request(QuadConst<(ST + QST - 1) % QST>{}, e_c);
+      });
       __builtin_amdgcn_sched_barrier(0);
-    }
+    });
     advance(t + QST);
     // k-step 1: first fragments of stage t + 1, complete since the last barrier
 #pragma unroll
     for (int q = 0; q < kSlots; ++q) {
       acc[q / NT][q % NT] = mfma32<BF16>(fa[1][q / NT], fb[1][q % NT], acc[q / NT][q % NT]);
-      if (q < kReads) read_one(QuadConst<(ST + 1) % QST>{}, 0, 0, q);
+#pragma unroll
+      for (int r = q * kReadsPerSlot; r < (q + 1) * kReadsPerSlot; ++r)
+        if (r < kReads) read_one(QuadConst<(ST + 1) % QST>{}, 0, 0, r);
       __builtin_amdgcn_sched_barrier(0);
     }
     asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kInFlight) : "memory");  // this wavefront's part of stage t + 2 has landed
@@ -677,23 +694,18 @@ __global__ __launch_bounds__(256) void gemm_quad_kernel(GemmParams p) {
   const int rounds = nk / QST;
   int t = 0;
   for (int round = 0; round < rounds; ++round, t += QST) {
-    iteration(QuadConst<0>{}, t);
-    iteration(QuadConst<1>{}, t + 1);
-    iteration(QuadConst<2>{}, t + 2);
-    iteration(QuadConst<3>{}, t + 3);
-    iteration(QuadConst<4>{}, t + 4);
+    quad_for<0, QST>([&](auto st_c) { iteration(st_c, t + decltype(st_c)::value); });
   }
-  if (t < nk) iteration(QuadConst<0>{}, t);
-  if (t + 1 < nk) iteration(QuadConst<1>{}, t + 1);
-  if (t + 2 < nk) iteration(QuadConst<2>{}, t + 2);
-  if (t + 3 < nk) iteration(QuadConst<3>{}, t + 3);
+  quad_for<0, QST - 1>([&](auto st_c) {
+    if (t + decltype(st_c)::value < nk) iteration(st_c, t + decltype(st_c)::value);
+  });
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // nothing may land in LDS after the workgroup has gone
 
-  // ---- epilogue (row = m0 + wm*128 + i*32 + (r/4)*8 + (lane/32)*4 + r%4, column lane%32 + ...) ----
+  // ---- epilogue (row = m0 + wm*32*MT + i*32 + (r/4)*8 + (lane/32)*4 + r%4, column lane%32 + ...) ----
   // Only the last row tile of a ragged problem checks its rows: the checks keep the stores of a tile
   // from being issued as one batch, which every other tile should not pay for.
   OutT* c = reinterpret_cast<OutT*>(p.c);
-  const int row_base = m0 + wm * 128 + (lane >> 5) * 4;
+  const int row_base = m0 + wm * 32 * MT + (lane >> 5) * 4;
   const int col0 = (DUAL ? n0 + wn * 64 : n0 + wn * 128) + (lane & 31);
   const int64_t mn = (int64_t)p.m * p.n;
   constexpr int JN = DUAL ? NT / 2 : NT;
@@ -739,16 +751,16 @@ __global__ __launch_bounds__(256) void gemm_quad_kernel(GemmParams p) {
       }
     }
   };
-  if (EDGE_M && m0 + 256 > p.m) epilogue(QuadConst<1>{});
+  if (EDGE_M && m0 + BM > p.m) epilogue(QuadConst<1>{});
   else epilogue(QuadConst<0>{});
 }
 
-template <bool DUAL, bool BF16, typename OutT, bool EDGE_M>
+template <int MT, bool DUAL, bool BF16, typename OutT, bool EDGE_M>
 int launch_quad_e(GemmParams p, hipStream_t st) {
-  p.tiles_m = (p.m + 255) / 256;
+  p.tiles_m = (p.m + 64 * MT - 1) / (64 * MT);
   p.tiles_n = p.n / (DUAL ? BN / 2 : BN);
-  const size_t smem = (size_t)QST * kQuadStageBytes;
-  auto kern = gemm_quad_kernel<DUAL, BF16, OutT, EDGE_M>;
+  const size_t smem = (size_t)quad_stages(MT) * quad_stage_bytes(MT);
+  auto kern = gemm_quad_kernel<MT, DUAL, BF16, OutT, EDGE_M>;
   static std::atomic<bool> attr_set{false};  // per instantiation; callers hold the dispatch lock
   if (!attr_set.load(std::memory_order_acquire)) {
     PTO_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
@@ -762,8 +774,14 @@ int launch_quad_e(GemmParams p, hipStream_t st) {
 
 // m ragged: the same loop with the A row pointers clamped once and the stores of the missing rows skipped
 template <bool DUAL, bool BF16, typename OutT>
-int launch_quad(const GemmParams& p, hipStream_t st) {
-  return p.m % 256 == 0 ? launch_quad_e<DUAL, BF16, OutT, false>(p, st) : launch_quad_e<DUAL, BF16, OutT, true>(p, st);
+int launch_quad(const GemmParams& p, int height, hipStream_t st) {
+  switch (height) {
+    case 1: return launch_quad_e<1, DUAL, BF16, OutT, true>(p, st);
+    case 2: return launch_quad_e<2, DUAL, BF16, OutT, true>(p, st);
+    case 3: return launch_quad_e<3, DUAL, BF16, OutT, true>(p, st);
+    default:
+      return p.m % 256 == 0 ? launch_quad_e<4, DUAL, BF16, OutT, false>(p, st) : launch_quad_e<4, DUAL, BF16, OutT, true>(p, st);
+  }
 }
 
 // Sum of the split-K slabs in split order (so the result does not depend on which workgroup
@@ -839,6 +857,49 @@ int launch_finish(const GemmParams& p, hipStream_t st) {
   return PTO_HIP_OK;
 }
 
+// Tile height (64 * *height rows, 0: the 256-row tile with eight wavefronts) and k split count of a product with 16-bit
+// weights: the pair with the least estimated time in microseconds, fitted to every pair (with its finish launch) at 33 to
+// 4000 rows of eleven weight shapes; 0.9 % from the best pair on average, 11 % at most.  Whole rounds of
+// workgroups over the CUs cost (a + b) ns per k row a workgroup walks, a last partial one a + b * its share of the CUs -
+// L2 and the clock are shared -, each round c more for its start and its stores; not less than the weights take to
+// stream; a split the finish launch and the slabs' way out and back, dearer once they outgrow the last-level cache.
+// The 256-row form with a ragged last row tile keeps 80 registers in scratch in the single-operand
+// pass, which slows its slab stores (4096 x 4096 at 400 rows 50 us, 34 with eight wavefronts): there the eight-wavefront
+// form is a candidate too.  `forced`: height given, only the split count is chosen.
+template <bool DUAL>
+void choose_quad(const GemmParams& p, int64_t num_cu, int forced, int* height, int* want) {
+  struct Cost {
+    double a, b, c;
+  };
+  static constexpr Cost kCost[5] = {{16.84, 7.88, 2.31}, {5.8, 6.58, 2.03}, {10.02, 5.93, 2.83}, {12.72, 5.69, 4.69}, {16.16, 8.28, 3.52}};  // [0]: eight wavefronts
+  const double weights_mb = (double)p.k * p.n * (DUAL ? 2 : 1) * 2e-6;
+  double best = 1e30;
+  for (int h = 0; h <= 4; ++h) {
+    if (forced ? h != forced : (h == 0 && (DUAL || p.m % 256 == 0))) continue;
+    const int bm = h ? 64 * h : 256;
+    const int64_t tiles = (int64_t)((p.m + bm - 1) / bm) * (p.n / (DUAL ? BN / 2 : BN));
+    for (int s = 1; s <= kMaxSplits; ++s) {
+      if (s > 1 && p.k < 4 * BK * s) break;
+      const int64_t kps = ((p.k + s * BK - 1) / (s * BK)) * BK;
+      if ((p.k + kps - 1) / kps != s) continue;
+      const int64_t full = tiles * s / num_cu, left = tiles * s % num_cu;
+      const Cost& q = kCost[h];
+      double t = (double)kps * 1e-3 * ((double)full * (q.a + q.b) + (left ? q.a + q.b * (double)left / (double)num_cu : 0.0)) +
+                 q.c * (double)(full + (left ? 1 : 0));
+      t = std::max(t, weights_mb / 10.2);
+      if (s > 1) {
+        const double slab_mb = (double)s * p.m * p.n * (DUAL ? 2 : 1) * 4e-6;
+        t += 2.95 + slab_mb * (DUAL ? 0.177 : 0.374) + std::max(slab_mb - 128.0, 0.0) * 0.29;
+      }
+      if (t < best) {
+        best = t;
+        *height = h;
+        *want = s;
+      }
+    }
+  }
+}
+
 template <bool DUAL, bool BF16, typename OutT, bool W8 = false>
 int launch_variant(GemmParams p, hipStream_t st) {
   const int64_t variant = pto_hip::ctx().gemm_variant;
@@ -846,7 +907,8 @@ int launch_variant(GemmParams p, hipStream_t st) {
   p.splits = 1;
   p.k_per_split = p.k;
   p.slabs = nullptr;
-  // variant 0 (default): eight wavefronts (two per SIMD); up to 64 rows a 64x256 tile with k split
+  // variant 0 (default): with 16-bit weights and whole tiles in n and k see choose_quad.  Otherwise
+  // eight wavefronts (two per SIMD); up to 64 rows a 64x256 tile with k split
   // over up to 16 workgroups per tile while CUs would idle, beyond that the 256x256 or the 128x256
   // tile and the k split count with the least estimated time (below).  Splits write fp32 slabs
   // that a second kernel sums in split order.
@@ -858,9 +920,23 @@ int launch_variant(GemmParams p, hipStream_t st) {
   const int64_t small_tiles = (int64_t)((p.m + 127) / 128) * tiles_n;
   const bool few = big_tiles < num_cu;
   int want = 1;
+  // 16-bit weights, whole tiles in n and k: the four-wavefront form, its tile height and the k split count by
+  // estimated time (choose_quad); `quad_height` 0 is the eight-wavefront form, also where those are not met.
+  int quad_height = 0;
+  bool quad_chosen = false;
+  if constexpr (!W8) {
+    if (p.n % (DUAL ? BN / 2 : BN) == 0 && p.k % QK == 0) {
+      const int64_t rows = pto_hip::ctx().gemm_quad_rows;
+      if (variant == 7) quad_height = rows ? (int)rows / 64 : 4;
+      if (variant == 0) {
+        quad_chosen = true;
+        choose_quad<DUAL>(p, num_cu, (int)rows / 64, &quad_height, &want);
+      }
+    }
+  }
   bool small_tile = variant == 5;
   if ((variant == 4 || variant == 7) && few) want = 2;
-  if (variant == 0 && p.m > 64) {
+  if (variant == 0 && !quad_chosen && p.m > 64) {
     // Estimated time of each (tile height, k splits) pair, in microseconds, fitted to measured
     // launches: rounds of workgroups over the CUs x the k rows one workgroup walks x the time per
     // k row (a 256-row tile 18 ns when few CUs are busy up to 27.5 ns when all are, a 128-row
@@ -884,9 +960,7 @@ int launch_variant(GemmParams p, hipStream_t st) {
         const double ns_row =
             (tall ? 18.1 + 9.4 * load : 11.0 + 6.5 * load) + (W8 && rounds > 1 ? (tall ? 2.5 : 4.5) : 0.0);
         const double slab_mb = (double)real * p.m * p.n * mats * 4.0 / 1e6;  // written, then read back
-        // where the tall tile runs as four wavefronts (see below) it measured about 5 % faster
-        const bool as_quad = !W8 && tall && p.n % (DUAL ? BN / 2 : BN) == 0 && p.k % QK == 0;
-        const double t = std::max((double)rounds * (double)kps * ns_row * (as_quad ? 0.95 : 1.0) * 1e-3, stream_us) +
+        const double t = std::max((double)rounds * (double)kps * ns_row * 1e-3, stream_us) +
                          (real > 1 ? 7.0 + 2.0 * slab_mb / (slab_mb <= 128.0 ? 8.0 : 4.0) : 0.0);
         if (t < best) {
           best = t;
@@ -899,7 +973,7 @@ int launch_variant(GemmParams p, hipStream_t st) {
   // Up to 64 rows: a 64-row tile.  With the 128-row tile the MFMA work on its padding rows, not
   // the weight stream, set the time for int8 codes (half the bytes of 16-bit weights: decoder
   // layer at batch 64 205 -> 177 us) and still cost 2-5 % with 16-bit weights.
-  const bool tiny_tile = variant == 6 || (variant == 0 && p.m <= 64);
+  const bool tiny_tile = variant == 6 || (variant == 0 && !quad_chosen && p.m <= 64);
   if (tiny_tile) {
     const int64_t tiny_tiles = (int64_t)((p.m + 63) / 64) * tiles_n;
     small_tile = false;
@@ -917,16 +991,11 @@ int launch_variant(GemmParams p, hipStream_t st) {
     }
   }
   int rc = PTO_HIP_OK;
-  // The four-wavefront form of the tall tile (bit-identical to the eight-wavefront one) wherever it
-  // is built: measured ahead by 1-6 % on every shape tried (LLaMA-7B block at 1024 / 2048 / 4096 / 8192
-  // tokens 346 -> 335, 510 -> 490, 956 -> 936, 1831 -> 1795 us on one box; hidden 8192 at 1024 tokens
-  // 1280 -> 1200; hidden 2048 at 4096 tokens 383 -> 380).  "gemm_variant" 4 keeps eight wavefronts.
+  // "gemm_variant" 4 keeps eight wavefronts; both forms give identical bits.
   bool quad = false;
   if constexpr (!W8) {
-    const bool fits = !tiny_tile && !small_tile && p.n % (DUAL ? BN / 2 : BN) == 0 && p.k % QK == 0 &&
-                      p.k_per_split % QK == 0;
-    quad = fits && (variant == 7 || variant == 0);
-    if (quad) rc = launch_quad<DUAL, BF16, OutT>(p, st);
+    quad = quad_height > 0 && p.k_per_split % QK == 0;
+    if (quad) rc = launch_quad<DUAL, BF16, OutT>(p, quad_height, st);
   }
   if (!quad) {
     if (tiny_tile) rc = launch_gemm<1, 2, 4, DUAL, BF16, OutT, W8>(p, st);

@@ -790,3 +790,39 @@ def test_ffn_block_fp8_argument_rules(worker):
         bad[6] = q.w_down8.view(torch.uint8).to(torch.int8)
         with pytest.raises(ValueError, match="FP8E4M3FN"):
             hd(*bad)
+
+
+@pytest.mark.parametrize("m", [33, 64, 65, 128, 191, 193, 257])
+@pytest.mark.parametrize("dual,k,n", [(True, 512, 384), (False, 32 * 13, 256), (True, 2080, 128), (False, 1536, 512)])
+def test_gemm_four_wavefront_tile_heights(worker, dual, k, n, m):
+    """Every tile height of the four-wavefront form, at the edges of its row tiles and at k lengths of fewer, as
+    many and more stages than it keeps in flight: the same 16-wide k steps into the same accumulators as
+    the eight-wavefront form, so the same bits at the same split count, for both 16-bit types."""
+    _lib, lib, dtype_code = _fp8_stage_lib()
+    g = torch.Generator().manual_seed(m + k)
+    try:
+        for dt in (torch.bfloat16, torch.float16):
+            x = torch.randn((m, k), generator=g).to(dt).cuda()
+            w = [(torch.randn((k, n), generator=g) * k**-0.5).to(dt).cuda() for _ in range(2)]
+            for kk, splits in ((k, 1), (k, 2), (k, 3), (32, 1), (160, 1)):
+                got = []
+                for variant, rows in ((4, 0), (7, 64), (7, 128), (7, 192), (7, 256), (0, 0)):
+                    worker.set_option("gemm_splits", splits)
+                    worker.set_option("gemm_variant", variant)
+                    worker.set_option("gemm_quad_rows", rows)
+                    out = torch.full((m, n), float("nan"), dtype=dt if dual else torch.float32, device="cuda")
+                    xk = x[:, :kk].contiguous()
+                    if dual:
+                        _lib.check(lib.pto_hip_gate_up_swiglu(xk.data_ptr(), w[0].data_ptr(), w[1].data_ptr(), out.data_ptr(),
+                                                              m, kk, n, dtype_code(dt), 0))
+                    else:
+                        _lib.check(lib.pto_hip_projection(xk.data_ptr(), w[0].data_ptr(), None, out.data_ptr(), m, kk, n,
+                                                          dtype_code(dt), 0, dtype_code(torch.float32), 0))
+                    worker.sync()
+                    got.append(out.cpu())
+                assert not got[0].isnan().any()
+                for o in got[1:]:
+                    assert torch.equal(o, got[0]), (kk, splits)
+    finally:
+        for name in ("gemm_splits", "gemm_variant", "gemm_quad_rows"):
+            worker.set_option(name, 0)
