@@ -9,6 +9,7 @@
 #include <hip/hip_runtime.h>
 
 #include "common.h"
+#include "slab_sum.h"
 
 namespace {
 
@@ -37,22 +38,28 @@ __global__ __launch_bounds__(128) void rope_kv_kernel(RopeParams p) {
   const int half = p.d / 2;
   const int pos = p.seq_lens[b] - 1;
   const size_t src = ((size_t)b * (p.hq + 2 * p.hkv) + head) * p.d;
-  // channel value: sum of the partial slabs in split order, times the channel scale
-  // (loads go out four at a time; the additions keep the order)
+  // channel values: sum of the partial slabs in split order, times the channel scale
   auto fetch = [&](int i) {
-    float v = 0.f;
-    const float* q = p.qkv + src + i;
-    const int splits = pto_hip::slab_count(p.map, p.splits, 0, head * p.d + i);
-    int s = 0;
-    for (; s + 4 <= splits; s += 4) {
-      float t[4];
-#pragma unroll
-      for (int u = 0; u < 4; ++u) t[u] = q[(size_t)(s + u) * p.split_stride];
-#pragma unroll
-      for (int u = 0; u < 4; ++u) v += t[u];
+    const float* src1[1] = {p.qkv + src + i};
+    float v[1] = {0.f};
+    pto_hip::add_slabs(src1, pto_hip::slab_count(p.map, p.splits, 0, head * p.d + i), (size_t)p.split_stride, v);
+    return p.scale ? v[0] * p.scale[(size_t)head * p.d + i] : v[0];
+  };
+  // the two channels of a rotated pair, requested together
+  auto fetch_pair = [&](int i, float& lo, float& hi) {
+    const int ch = head * p.d + i;
+    const int n_lo = pto_hip::slab_count(p.map, p.splits, 0, ch), n_hi = pto_hip::slab_count(p.map, p.splits, 0, ch + half);
+    if (n_lo == n_hi) {
+      const float s_lo = p.scale ? p.scale[ch] : 1.f, s_hi = p.scale ? p.scale[ch + half] : 1.f;
+      const float* src2[2] = {p.qkv + src + i, p.qkv + src + i + half};
+      float v[2] = {0.f, 0.f};
+      pto_hip::add_slabs(src2, n_lo, (size_t)p.split_stride, v);
+      lo = v[0] * s_lo;
+      hi = v[1] * s_hi;
+    } else {
+      lo = fetch(i);
+      hi = fetch(i + half);
     }
-    for (; s < splits; ++s) v += q[(size_t)s * p.split_stride];
-    return p.scale ? v * p.scale[(size_t)head * p.d + i] : v;
   };
   const bool is_q = head < p.hq, is_k = !is_q && head < p.hq + p.hkv;
   T* dst;
@@ -74,7 +81,8 @@ __global__ __launch_bounds__(128) void rope_kv_kernel(RopeParams p) {
   }
   const int cpos = pos < 0 ? 0 : (pos >= p.max_pos ? p.max_pos - 1 : pos);
   for (int i = threadIdx.x; i < half; i += blockDim.x) {
-    const float lo = fetch(i), hi = fetch(i + half);
+    float lo, hi;
+    fetch_pair(i, lo, hi);
     if (is_q || is_k) {
       const size_t t_lo = (size_t)cpos * p.rope_w + i, t_hi = p.rope_w == p.d ? t_lo + half : t_lo;
       dst[i] = (T)(lo * p.cos[t_lo] - hi * p.sin[t_lo]);
@@ -127,20 +135,28 @@ __global__ __launch_bounds__(64) void rope_kv_fp8_kernel(RopeFp8Params pp) {
   const int half = p.d / 2;
   const int pos = p.seq_lens[b] - 1;
   const size_t src = ((size_t)b * (p.hq + 2 * p.hkv) + head) * p.d;
+  // channel values: sum of the partial slabs in split order, times the channel scale
   auto fetch = [&](int i) {
-    float v = 0.f;
-    const float* q = p.qkv + src + i;
-    const int splits = pto_hip::slab_count(p.map, p.splits, 0, head * p.d + i);
-    int s = 0;
-    for (; s + 4 <= splits; s += 4) {
-      float t[4];
-#pragma unroll
-      for (int u = 0; u < 4; ++u) t[u] = q[(size_t)(s + u) * p.split_stride];
-#pragma unroll
-      for (int u = 0; u < 4; ++u) v += t[u];
+    const float* src1[1] = {p.qkv + src + i};
+    float v[1] = {0.f};
+    pto_hip::add_slabs(src1, pto_hip::slab_count(p.map, p.splits, 0, head * p.d + i), (size_t)p.split_stride, v);
+    return p.scale ? v[0] * p.scale[(size_t)head * p.d + i] : v[0];
+  };
+  // the two channels of a rotated pair, requested together
+  auto fetch_pair = [&](int i, float& lo, float& hi) {
+    const int ch = head * p.d + i;
+    const int n_lo = pto_hip::slab_count(p.map, p.splits, 0, ch), n_hi = pto_hip::slab_count(p.map, p.splits, 0, ch + half);
+    if (n_lo == n_hi) {
+      const float s_lo = p.scale ? p.scale[ch] : 1.f, s_hi = p.scale ? p.scale[ch + half] : 1.f;
+      const float* src2[2] = {p.qkv + src + i, p.qkv + src + i + half};
+      float v[2] = {0.f, 0.f};
+      pto_hip::add_slabs(src2, n_lo, (size_t)p.split_stride, v);
+      lo = v[0] * s_lo;
+      hi = v[1] * s_hi;
+    } else {
+      lo = fetch(i);
+      hi = fetch(i + half);
     }
-    for (; s < splits; ++s) v += q[(size_t)s * p.split_stride];
-    return p.scale ? v * p.scale[(size_t)head * p.d + i] : v;
   };
   const bool is_q = head < p.hq, is_k = !is_q && head < p.hq + p.hkv;
   const int cpos = pos < 0 ? 0 : (pos >= p.max_pos ? p.max_pos - 1 : pos);
@@ -148,7 +164,8 @@ __global__ __launch_bounds__(64) void rope_kv_fp8_kernel(RopeFp8Params pp) {
   if (is_q) {
     TQ* dst = reinterpret_cast<TQ*>(p.q_out) + ((size_t)b * p.hq + head) * p.d;
     for (int i = lane; i < half; i += 64) {
-      const float lo = fetch(i), hi = fetch(i + half);
+      float lo, hi;
+      fetch_pair(i, lo, hi);
       const size_t t_lo = (size_t)cpos * p.rope_w + i, t_hi = p.rope_w == p.d ? t_lo + half : t_lo;
       dst[i] = (TQ)(lo * p.cos[t_lo] - hi * p.sin[t_lo]);
       dst[i + half] = (TQ)(hi * p.cos[t_hi] + lo * p.sin[t_hi]);
@@ -185,7 +202,8 @@ __global__ __launch_bounds__(64) void rope_kv_fp8_kernel(RopeFp8Params pp) {
         float v;
         if (is_k) {
           const int i = e < half ? e : e - half;
-          const float lo = fetch(i), hi = fetch(i + half);
+          float lo, hi;
+          fetch_pair(i, lo, hi);
           const size_t t_lo = (size_t)cpos * p.rope_w + i, t_hi = p.rope_w == p.d ? t_lo + half : t_lo;
           v = e < half ? lo * p.cos[t_lo] - hi * p.sin[t_lo] : hi * p.cos[t_hi] + lo * p.sin[t_hi];
         } else {

@@ -28,6 +28,7 @@
 #include <type_traits>
 
 #include "common.h"
+#include "slab_sum.h"
 
 namespace {
 
@@ -308,27 +309,29 @@ __device__ __forceinline__ void store4_from_f32(void* p, size_t i, int dt, float
   }
 }
 
-// Sum of the k splits of four channels, in split order, times the channel scales.  Loads go out
-// four at a time; the additions keep the order.
+// Sums of the k splits of four channels of K matrices with `splits` slabs each, in split order, times the channel scales.
+template <int K>
+__device__ __forceinline__ void sum_splits(const float* const (&part)[K], const float* const (&scale)[K], int splits,
+                                           size_t stride, int m, int n, int nn, f32x4 (&sum)[K]) {
+  const f32x4* src[K];
+  f32x4 sc[K];
+#pragma unroll
+  for (int k = 0; k < K; ++k) {
+    src[k] = reinterpret_cast<const f32x4*>(part[k] + (size_t)m * nn + n);
+    sum[k] = f32x4{0.f, 0.f, 0.f, 0.f};
+    sc[k] = scale[k] ? *reinterpret_cast<const f32x4*>(scale[k] + n) : f32x4{1.f, 1.f, 1.f, 1.f};  // none: unquantised weights
+  }
+  pto_hip::add_slabs(src, splits, stride / 4, sum);
+#pragma unroll
+  for (int k = 0; k < K; ++k) sum[k] *= sc[k];
+}
 __device__ __forceinline__ float4 sum_splits(const float* part, const float* scale, int splits, size_t stride, int m,
                                              int n, int nn) {
-  float4 a = {0.f, 0.f, 0.f, 0.f};
-  const float* src = part + (size_t)m * nn + n;
-  int s = 0;
-  for (; s + 4 <= splits; s += 4) {
-    float4 v[4];
-#pragma unroll
-    for (int j = 0; j < 4; ++j) v[j] = *reinterpret_cast<const float4*>(src + (size_t)(s + j) * stride);
-#pragma unroll
-    for (int j = 0; j < 4; ++j) { a.x += v[j].x; a.y += v[j].y; a.z += v[j].z; a.w += v[j].w; }
-  }
-  for (; s < splits; ++s) {
-    const float4 v = *reinterpret_cast<const float4*>(src + (size_t)s * stride);
-    a.x += v.x; a.y += v.y; a.z += v.z; a.w += v.w;
-  }
-  if (!scale) return a;  // unquantised weights
-  const float4 sc = *reinterpret_cast<const float4*>(scale + n);
-  return float4{a.x * sc.x, a.y * sc.y, a.z * sc.z, a.w * sc.w};
+  const float* parts[1] = {part};
+  const float* scales[1] = {scale};
+  f32x4 sum[1];
+  sum_splits<1>(parts, scales, splits, stride, m, n, nn, sum);
+  return float4{sum[0][0], sum[0][1], sum[0][2], sum[0][3]};
 }
 
 __device__ __forceinline__ float silu_mul(float g, float u) {
@@ -339,14 +342,30 @@ __global__ __launch_bounds__(256) void w8a16_finish_kernel(FinishParams p) {
   const int n = (blockIdx.x * 256 + threadIdx.x) * 4;
   const int m = blockIdx.y;
   if (n >= p.n) return;
-  float4 a = sum_splits(p.part0, p.scale0, pto_hip::slab_count(p.map, p.splits, 0, n), (size_t)p.stride, m, n, p.n);
-  if (p.part1) {
-    const float4 u = sum_splits(p.part1, p.scale1, pto_hip::slab_count(p.map, p.splits, 1, n), (size_t)p.stride, m, n, p.n);
-    a = float4{silu_mul(a.x, u.x), silu_mul(a.y, u.y), silu_mul(a.z, u.z), silu_mul(a.w, u.w)};
-  }
   const size_t idx = (size_t)m * p.n + n;
+  float4 r = {0.f, 0.f, 0.f, 0.f};  // requested with the slabs
+  if (p.residual) r = load4_as_f32(p.residual, idx, p.res_dtype);
+  const int splits0 = pto_hip::slab_count(p.map, p.splits, 0, n);
+  float4 a;
+  if (p.part1) {
+    const int splits1 = pto_hip::slab_count(p.map, p.splits, 1, n);
+    float4 u;
+    if (splits0 == splits1) {
+      const float* parts[2] = {p.part0, p.part1};
+      const float* scales[2] = {p.scale0, p.scale1};
+      f32x4 sum[2];
+      sum_splits<2>(parts, scales, splits0, (size_t)p.stride, m, n, p.n, sum);
+      a = float4{sum[0][0], sum[0][1], sum[0][2], sum[0][3]};
+      u = float4{sum[1][0], sum[1][1], sum[1][2], sum[1][3]};
+    } else {
+      a = sum_splits(p.part0, p.scale0, splits0, (size_t)p.stride, m, n, p.n);
+      u = sum_splits(p.part1, p.scale1, splits1, (size_t)p.stride, m, n, p.n);
+    }
+    a = float4{silu_mul(a.x, u.x), silu_mul(a.y, u.y), silu_mul(a.z, u.z), silu_mul(a.w, u.w)};
+  } else {
+    a = sum_splits(p.part0, p.scale0, splits0, (size_t)p.stride, m, n, p.n);
+  }
   if (p.residual) {
-    const float4 r = load4_as_f32(p.residual, idx, p.res_dtype);
     a.x += r.x; a.y += r.y; a.z += r.z; a.w += r.w;
   }
   store4_from_f32(p.out, p.out_blocked ? blocked_index(m, n) : idx, p.out_dtype, a);
@@ -381,8 +400,8 @@ __global__ __launch_bounds__(kNormThreads) void w8a16_finish_norm_kernel(FinishN
     const int n = (threadIdx.x + u * kNormThreads) * 4;
     if (n < p.n) {
       g[u] = *reinterpret_cast<const float4*>(p.gamma + n);
-      float4 a = sum_splits(p.part, p.scale, pto_hip::slab_count(p.map, p.splits, 0, n), (size_t)p.stride, m, n, p.n);
       const float4 r = load4_as_f32(p.residual, (size_t)m * p.n + n, p.res_dtype);
+      float4 a = sum_splits(p.part, p.scale, pto_hip::slab_count(p.map, p.splits, 0, n), (size_t)p.stride, m, n, p.n);
       a.x += r.x; a.y += r.y; a.z += r.z; a.w += r.w;
       v[u] = a;
       *reinterpret_cast<float4*>(p.sum_out + (size_t)m * p.n + n) = a;

@@ -677,3 +677,25 @@ def test_skinny_projection_shares_are_exact(worker, kind, m, k, n, pair):
         torch.testing.assert_close(out.double(), oracle.swiglu(gate, up), rtol=2 ** -7, atol=1e-30)
     else:
         assert torch.equal(out.double(), gate)
+
+
+@pytest.mark.parametrize("slabs", [1, 2, 3, 4, 5, 6, 7, 8, 9, 16, 19])
+def test_partial_slab_counts_are_exact(worker, slabs):
+    """One 128-channel slab of 8 * slabs steps is the work of `slabs` workgroups: every size of the consumers' load
+    batches and the step past eight, on integer operands whose sums are exact in any order."""
+    g = torch.Generator().manual_seed(slabs)
+    k, n = 256 * slabs, 128
+    x = torch.randint(-2, 3, (3, k), generator=g).to(torch.bfloat16)
+    w = [torch.randint(-3, 4, (k, n), generator=g).to(torch.int8) for _ in range(2)]
+    scale = [torch.rand(n, generator=g).exp2() for _ in range(2)]
+    residual = torch.randint(-8, 9, (3, n), generator=g).float()
+    out, summed, pair = torch.empty(3, n), torch.empty(3, n), torch.empty(3, n, dtype=torch.bfloat16)
+    worker.run(w8a16_matmul, x, w[0], scale[0], out)
+    worker.run(w8a16_matmul_residual, x, w[0], scale[0], residual, summed)
+    worker.run(w8a16_swiglu, x, w[0], scale[0], w[1], scale[1], pair)
+    gate, up = ((x.double() @ t.double()).float() * s for t, s in zip(w, scale))
+    assert torch.equal(out, gate)
+    # product and sum rounded once each, or once together
+    torch.testing.assert_close(summed, gate + residual, rtol=2 ** -22, atol=8 * 2 ** -23 * float(gate.abs().max()))
+    # one bf16 ulp (2^-7) of SwiGLU's value, SiLU's exponential overflowing to zero below
+    torch.testing.assert_close(pair.double(), oracle.swiglu(gate.double(), up.double()), rtol=2 ** -7, atol=1e-30)
