@@ -21,7 +21,8 @@ __device__ __forceinline__ void add_slab_batch(const V* const (&src)[K], size_t 
 // sum[k] += src[k][0] + src[k][stride] + ... (count of them), added in order; stride in elements of V.
 // These kernels are a chain of memory round trips (the slabs come from other XCDs' workgroups): up to
 // eight slabs of every source are requested at once, whatever the count, where a remainder loop makes one trip
-// per slab.
+// per slab.  Decoder layer of one sequence, int8 weights (2 to 8 slabs a channel): batches of four and a serial
+// remainder, the two channels of a rotated pair and the gate and up sums one after the other 74.5 us, so 73.1.
 template <int K, typename V>
 __device__ __forceinline__ void add_slabs(const V* const (&first)[K], int count, size_t stride, V (&sum)[K]) {
   const V* src[K];
