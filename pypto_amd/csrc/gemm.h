@@ -865,7 +865,11 @@ int launch_finish(const GemmParams& p, hipStream_t st) {
 // stream; a split the finish launch and the slabs' way out and back, dearer once they outgrow the last-level cache.
 // The 256-row form with a ragged last row tile keeps 80 registers in scratch in the single-operand
 // pass, which slows its slab stores (4096 x 4096 at 400 rows 50 us, 34 with eight wavefronts): there the eight-wavefront
-// form is a candidate too.  `forced`: height given, only the split count is chosen.
+// form is a candidate too.  Over several rounds the board's power limit sets the clock and the 256-row tile, with the
+// fewest operand bytes per MFMA, gains what launches timed alone do not show: it wins unless another is 3 % ahead (gate/up
+// 4096 x 10752 at 2709 rows, estimates 0.7 % apart: against eight-wavefront tiles chosen as for other shapes the whole block
+// took 665 us for 652 on 192-row tiles and takes 600 for 625 on 256-row ones).
+// `forced`: height given, only the split count is chosen.
 template <bool DUAL>
 void choose_quad(const GemmParams& p, int64_t num_cu, int forced, int* height, int* want) {
   struct Cost {
@@ -891,6 +895,7 @@ void choose_quad(const GemmParams& p, int64_t num_cu, int forced, int* height, i
         const double slab_mb = (double)s * p.m * p.n * (DUAL ? 2 : 1) * 4e-6;
         t += 2.95 + slab_mb * (DUAL ? 0.177 : 0.374) + std::max(slab_mb - 128.0, 0.0) * 0.29;
       }
+      if (h == 4 && full >= 2) t *= 0.97;
       if (t < best) {
         best = t;
         *height = h;
