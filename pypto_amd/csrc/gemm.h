@@ -8,6 +8,7 @@
 #include <atomic>
 
 #include "common.h"
+#include "lds_load.h"
 
 namespace pto_hip {
 namespace gemm {
@@ -235,20 +236,13 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_kernel(GemmParams p) {
   };
   // DIRECT: chunk i of this thread for the tile at k0, written by the hardware to slot tid of the
   // i-th 16 B x T run of the LDS tile (wave-uniform base + lane * 16).
-  // The instruction is written out instead of going through the compiler's builtin: told that a
-  // load writes LDS, the compiler waits for every such load in flight (vmcnt(0)) before each
-  // transposing fragment read, whatever buffer that read addresses, which puts the memory latency
-  // back into the loop.  Here the only waits are the explicit ones before the barriers.
-  auto to_lds = [&](const void* src, const uint16_t* dst) {
-    const uint32_t lds_base = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(const lds_u16*)dst);
-#pragma clang diagnostic push
-#pragma clang diagnostic ignored "-Winline-asm"  // m0 is named as clobbered on purpose
-    asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(src), "s"(lds_base) : "memory", "m0");
-#pragma clang diagnostic pop
+  // The only waits are the explicit ones before the barriers.
+  auto request = [&](const void* src, const uint16_t* dst) {
+    pto_hip::to_lds<0>(src, __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(const lds_u16*)dst));
   };
-  auto direct_a = [&](uint16_t* da, int k0, int i) { to_lds(a_ptr[i] + k0, da + (i * (T / 8) + wave * 8) * LDK); };
+  auto direct_a = [&](uint16_t* da, int k0, int i) { request(a_ptr[i] + k0, da + (i * (T / 8) + wave * 8) * LDK); };
   auto direct_b = [&](uint16_t* db, int k0, int i) {
-    to_lds(b_ptr + (int64_t)(k0 + (T / BCH) * i) * p.ldb * BESZ, db + (i * (T / BCH) + wave * (64 / BCH)) * LDN);
+    request(b_ptr + (int64_t)(k0 + (T / BCH) * i) * p.ldb * BESZ, db + (i * (T / BCH) + wave * (64 / BCH)) * LDN);
   };
   auto load_tile = [&](int k0) {
 #pragma unroll
@@ -530,15 +524,6 @@ __device__ __forceinline__ void quad_for(F&& f) {
   }
 }
 
-// One direct request: 16 bytes per lane from `src` to the KB of LDS at lds_w + OFF (wave-uniform).
-template <int OFF>
-__device__ __forceinline__ void quad_to_lds(const char* src, uint32_t lds_w) {
-#pragma clang diagnostic push
-#pragma clang diagnostic ignored "-Winline-asm"  // m0 is named as clobbered on purpose
-  asm volatile("s_add_u32 m0, %1, %2\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(src), "s"(lds_w), "n"(OFF) : "memory", "m0", "scc");
-#pragma clang diagnostic pop
-}
-
 template <int MT, bool DUAL, bool BF16, typename OutT, bool EDGE_M>
 __global__ __launch_bounds__(256) void gemm_quad_kernel(GemmParams p) {
   constexpr int NT = 4;
@@ -643,8 +628,8 @@ __global__ __launch_bounds__(256) void gemm_quad_kernel(GemmParams p) {
   // request e of the stage the pointers stand at, into buffer ST
   auto request = [&](auto st_c, auto e_c) {
     constexpr int ST = decltype(st_c)::value, E = decltype(e_c)::value;
-    if constexpr (E < MT) quad_to_lds<ST * kStageBytes + E * 4096>(ga[E], lds_w);
-    else quad_to_lds<ST * kStageBytes + E * 4096>(gb[E - MT], lds_w);
+    if constexpr (E < MT) pto_hip::to_lds<ST * kStageBytes + E * 4096>(ga[E], lds_w);
+    else pto_hip::to_lds<ST * kStageBytes + E * 4096>(gb[E - MT], lds_w);
   };
   // moves the pointers on to stage `next` unless that is past the end (then the last stage is requested again)
   auto advance = [&](int next) {

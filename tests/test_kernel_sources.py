@@ -1,0 +1,29 @@
+"""Rules of the hand-written instructions in the kernel sources (CPU: the sources are read, nothing runs)."""
+
+import re
+from pathlib import Path
+
+CSRC = Path(__file__).resolve().parent.parent / "pypto_amd" / "csrc"
+_ASM = re.compile(r"asm volatile\(((?:\s*\"(?:[^\"\\]|\\.)*\")+)")
+
+
+def _instructions(source: str):
+    """The instruction lists of a source's asm statements."""
+    for m in _ASM.finditer(source):
+        text = "".join(re.findall(r"\"((?:[^\"\\]|\\.)*)\"", m.group(1)))
+        yield [i.strip() for i in re.split(r"\\n(?:\\t)?", text) if i.strip()]
+
+
+def test_a_load_into_lds_never_follows_its_m0_write_directly():
+    """A load with its LDS address in m0 needs one wait state after the scalar instruction that writes m0; the compiler
+    adds it to its own code and not inside an asm string, so the string has to hold it."""
+    seen = 0
+    for path in sorted(CSRC.iterdir()):
+        if path.suffix not in (".hip", ".h"):
+            continue
+        for ins in _instructions(path.read_text()):
+            for before, after in zip(ins, ins[1:]):
+                if re.match(r"s_\w+ m0,", before):
+                    seen += 1
+                    assert "lds" not in after, f"{path.name}: '{before}' is followed by '{after}'"
+    assert seen >= 1
