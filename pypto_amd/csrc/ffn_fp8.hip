@@ -16,8 +16,10 @@
 
 #include <algorithm>
 #include <atomic>
+#include <type_traits>
 
 #include "common.h"
+#include "lds_load.h"
 
 namespace pto_hip {
 namespace gemm8 {
@@ -80,19 +82,6 @@ __device__ __forceinline__ int xcd_remap(int pid, int nwg) {
   return base + local;
 }
 
-// One direct request: 16 bytes per lane from sbase + voff to the KB of LDS at lds_w + OFF (wave-uniform).
-// The instruction is written out: told that a load writes LDS, the compiler waits for every such
-// load in flight before each later LDS read, whatever buffer that read addresses.  (s_nop: a write
-// of m0 needs one wait state before a load that reads it.)
-template <int OFF>
-__device__ __forceinline__ void to_lds(uint32_t voff, const uint8_t* sbase, uint32_t lds_w) {
-#pragma clang diagnostic push
-#pragma clang diagnostic ignored "-Winline-asm"  // m0 is named as clobbered on purpose
-  asm volatile("s_add_u32 m0, %2, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(voff), "s"(sbase), "s"(lds_w), "n"(OFF)
-               : "memory", "m0", "scc");
-#pragma clang diagnostic pop
-}
-
 template <int N>
 struct Const {
   static constexpr int value = N;
@@ -127,7 +116,9 @@ struct Const {
 // fetches logical chunk s ^ ((r / 2) % 8) and the fragment reads apply the same XOR: the 16 lanes the
 // LDS checks together for bank conflicts (16 consecutive rows, one logical chunk, 256 bytes = all 64
 // banks) then hit 16 different slots of 8 row pairs.
-template <int MH, int RING, bool DUAL, bool SPLIT, typename OutT>
+// LONG: rows so long that a tile's last one starts 2^32 bytes or more after its first (kLongRow): an address per lane
+// and request instead of 32-bit offsets from the tile's base, which costs every other shape up to 0.9 %.
+template <int MH, int RING, bool DUAL, bool SPLIT, bool LONG, typename OutT>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) void gemm8_kernel(Params p) {
   constexpr int BM = 128 * MH;
   constexpr int QA = 64 * MH * BK, QB = 128 * BK;  // bytes of an A and of a B quarter
@@ -168,30 +159,36 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
   // past the end are clamped (their products are not stored) ----
   const int q_row = wave * 8 + (lane >> 3);
   const int chunk = (lane & 7) ^ ((q_row >> 1) & 7);  // logical chunk whose slot this lane fills
-  uint32_t va[2][NA], vb[2][NB];                      // byte offsets from the tile's first row / channel
+  const uint8_t* base_a = p.a + (int64_t)m0 * p.lda + k_begin;
+  const uint8_t* base_b0 = p.b0 + (int64_t)n0 * p.ldb + k_begin;
+  const uint8_t* base_b1 = DUAL ? p.b1 + (int64_t)n0 * p.ldb + k_begin : base_b0;
+  typedef typename std::conditional<LONG, int64_t, uint32_t>::type Offset;
+  Offset va[2][NA], vb[2][NB];  // byte offsets from the tile's first row / channel
 #pragma unroll
   for (int h = 0; h < 2; ++h) {
 #pragma unroll
     for (int e = 0; e < NA; ++e)
-      va[h][e] = (uint32_t)min(h * 64 * MH + e * 32 + q_row, p.m - 1 - m0) * (uint32_t)p.lda + chunk * 16;
+      va[h][e] = (Offset)min(h * 64 * MH + e * 32 + q_row, p.m - 1 - m0) * (Offset)p.lda + chunk * 16;
 #pragma unroll
     for (int e = 0; e < NB; ++e) {
       const int r = e * 32 + q_row;
-      vb[h][e] = (uint32_t)min(DUAL ? h * 64 + (r & 63) : h * 128 + r, p.n - 1 - n0) * (uint32_t)p.ldb + chunk * 16;
+      vb[h][e] = (Offset)min(DUAL ? h * 64 + (r & 63) : h * 128 + r, p.n - 1 - n0) * (Offset)p.ldb + chunk * 16;
     }
   }
-  const uint8_t* base_a = p.a + (int64_t)m0 * p.lda + k_begin;
-  const uint8_t* base_b0 = p.b0 + (int64_t)n0 * p.ldb + k_begin;
-  const uint8_t* base_b1 = DUAL ? p.b1 + (int64_t)n0 * p.ldb + k_begin : base_b0;
   const uint32_t lds_w = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)lds0 + wave * 1024);
+  auto bring = [&](auto off_c, Offset off, const uint8_t* base) {
+    constexpr int OFF = decltype(off_c)::value;
+    if constexpr (LONG) to_lds<OFF>(base + off, lds_w);
+    else to_lds<OFF>(off, base, lds_w);
+  };
   // request e of quarter Q (0 A0, 1 B0, 2 B1, 3 A1) of tile t (past the last one: the last again) into ring slot S
   auto request = [&](auto s_c, auto q_c, auto e_c, int t) {
     constexpr int S = decltype(s_c)::value, Q = decltype(q_c)::value, E = decltype(e_c)::value;
     const int koff = min(t, nk - 1) * BK;
     if constexpr (Q == 0 || Q == 3) {
-      if constexpr (E < NA) to_lds<S * TILE + (Q ? QA : 0) + E * 4096>(va[Q ? 1 : 0][E], base_a + koff, lds_w);
+      if constexpr (E < NA) bring(Const<S * TILE + (Q ? QA : 0) + E * 4096>{}, va[Q ? 1 : 0][E], base_a + koff);
     } else {
-      to_lds<S * TILE + 2 * QA + (Q - 1) * QB + E * 4096>(vb[Q - 1][E], (DUAL && E >= 2 ? base_b1 : base_b0) + koff, lds_w);
+      bring(Const<S * TILE + 2 * QA + (Q - 1) * QB + E * 4096>{}, vb[Q - 1][E], (DUAL && E >= 2 ? base_b1 : base_b0) + koff);
     }
   };
   auto request_all = [&](auto s_c, auto q_c, int t) {
@@ -463,7 +460,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
   }
 }
 
-template <int MH, bool DUAL, typename OutT, bool SPLIT = false>
+constexpr int64_t kLongRow = (1ll << 32) / 256;  // rows of this many bytes and more: see LONG
+
+template <int MH, bool DUAL, typename OutT, bool SPLIT = false, bool LONG = false>
 int launch(Params p, hipStream_t st) {
   constexpr int BM = 128 * MH;
   constexpr int RING = MH == 2 ? 2 : 3;  // 128 or 144 KB of LDS
@@ -471,7 +470,7 @@ int launch(Params p, hipStream_t st) {
   const int bn_out = DUAL ? BN / 2 : BN;
   p.tiles_n = (p.n + bn_out - 1) / bn_out;
   const size_t smem = (size_t)RING * (BM + BN) * BK + (BM + BN) * sizeof(float);
-  auto kern = gemm8_kernel<MH, RING, DUAL, SPLIT, OutT>;
+  auto kern = gemm8_kernel<MH, RING, DUAL, SPLIT, LONG, OutT>;
   static std::atomic<bool> attr_set{false};  // per instantiation; callers hold the dispatch lock
   if (!attr_set.load(std::memory_order_acquire)) {
     PTO_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
@@ -564,6 +563,7 @@ int launch_tiles(Params& p, hipStream_t st) {
       }
     }
   }
+  const bool long_rows = std::max(p.lda, p.ldb) >= kLongRow;  // built on 128-row tiles
   const int per = (nk + splits - 1) / splits;
   p.k_per_split = per * BK;
   p.splits = (nk + per - 1) / per;
@@ -573,8 +573,10 @@ int launch_tiles(Params& p, hipStream_t st) {
     const int rc = pto_hip::gemm_workspace((size_t)p.splits * (DUAL ? 2 : 1) * p.m * p.n * sizeof(float), &ws);
     if (rc) return rc;
     p.slabs = reinterpret_cast<float*>(ws);
+    if (long_rows) return launch<1, DUAL, float, true, true>(p, st);
     return tall ? launch<2, DUAL, float, true>(p, st) : launch<1, DUAL, float, true>(p, st);
   }
+  if (long_rows) return launch<1, DUAL, OutT, false, true>(p, st);
   return tall ? launch<2, DUAL, OutT>(p, st) : launch<1, DUAL, OutT>(p, st);
 }
 

@@ -19,4 +19,14 @@ __device__ __forceinline__ void to_lds(const void* src, uint32_t lds_w) {
 #pragma clang diagnostic pop
 }
 
+// ... from sbase + voff, the base wave-uniform: no 64-bit address per lane and request.
+template <int OFF>
+__device__ __forceinline__ void to_lds(uint32_t voff, const void* sbase, uint32_t lds_w) {
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"
+  asm volatile("s_add_u32 m0, %2, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(voff), "s"(sbase), "s"(lds_w), "n"(OFF)
+               : "memory", "m0", "scc");
+#pragma clang diagnostic pop
+}
+
 }  // namespace pto_hip

@@ -682,6 +682,41 @@ def test_gemm_fp8_tile_edges_and_k_tile_counts(worker, variant, m, n):
         worker.set_option("gemm_variant", 0)
 
 
+@pytest.mark.parametrize("variant", [0, 4, 5])  # chosen by estimate, 256- and 128-row tiles
+def test_gemm_fp8_rows_beyond_32_bit_offsets(worker, variant):
+    """Rows so long that the last ones of a tile start more than 2^32 bytes after its first: codes in a few columns
+    whose wrapped offsets would land on one another, small integers, so every sum is exact."""
+    _lib, lib, code = _fp8_stage_lib()
+    g = torch.Generator().manual_seed(variant)
+    k = 128 * 132105  # 254 k and 127 * 2 k exceed 2^32 by 30464
+    cols = [5, 30469]
+    small = [torch.randint(1, 8, s, generator=g).float() for s in ((256, 2), (16, 2))]
+    tall, few = (torch.zeros((v.shape[0], k), dtype=torch.uint8, device="cuda") for v in small)
+    for t, v in zip((tall, few), small):
+        t[:, cols] = v.to(torch.float8_e4m3fn).view(torch.uint8).cuda()
+    one = torch.ones(256, device="cuda")
+    worker.set_option("gemm_variant", variant)
+    try:
+        # long rows of a, then of b
+        for a, b, m, n, want in ((tall, few, 256, 16, small[0] @ small[1].t()), (few, tall, 16, 256, small[1] @ small[0].t())):
+            out = torch.full((m, n), float("nan"), device="cuda")
+            _lib.check(lib.pto_hip_projection_fp8(a.data_ptr(), one.data_ptr(), b.data_ptr(), one.data_ptr(), out.data_ptr(),
+                                                  m, k, n, code(torch.float32), 0))
+            worker.sync()
+            assert torch.equal(out.cpu(), want)
+        # the gate/up pass's tile holds 128 channels: the same codes as 128 rows of twice the length
+        for a, b, m, n, kk, va, vb in ((tall, few, 256, 16, k, small[0], small[1]),
+                                       (few, tall, 8, 128, 2 * k, small[1].reshape(8, 4), small[0].reshape(128, 4))):
+            h = torch.full((m, n), float("nan"), dtype=torch.bfloat16, device="cuda")
+            _lib.check(lib.pto_hip_gate_up_swiglu_fp8(a.data_ptr(), one.data_ptr(), b.data_ptr(), one.data_ptr(), b.data_ptr(),
+                                                      one.data_ptr(), h.data_ptr(), m, kk, n, code(torch.bfloat16), 0))
+            worker.sync()
+            p = va @ vb.t()
+            validate_golden({"h": h.cpu().float()}, {"h": oracle.swiglu(p, p)}, rtol=8e-3, atol=0.0)  # one bf16 ulp is 2^-7
+    finally:
+        worker.set_option("gemm_variant", 0)
+
+
 @pytest.mark.parametrize("variant", [4, 5])
 @pytest.mark.parametrize("m,k,n,splits", [(1, 512, 128, 2), (33, 640, 200, 3), (129, 2048, 384, 16), (300, 896, 260, 4)])
 def test_gate_up_fp8_k_split_and_fused_quantiser(worker, variant, m, k, n, splits):
