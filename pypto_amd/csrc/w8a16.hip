@@ -154,7 +154,7 @@ __global__ __launch_bounds__(kWaves * 64) __attribute__((amdgpu_waves_per_eu(1, 
     const int row0 = min(min(cur.step + wave, cur.end - 1) * kStep, p.k - kStep);
     const int mat = cur.slab >= p.slabs ? 1 : 0;
     const int n0 = min((cur.slab - mat * p.slabs) * kSlab + c * kCols, p.n - kCols);
-    const uint32_t lane_off = ((uint32_t)n0 + (uint32_t)(kg * 8) * (uint32_t)p.n) * kWBytes;
+    const size_t lane_off = ((size_t)n0 + (size_t)(kg * 8) * p.n) * kWBytes;
     const char* wbase = reinterpret_cast<const char*>(p.wq[mat]) + (size_t)row0 * p.n * kWBytes;
 #pragma unroll
     for (int h = 0; h < MT; ++h) s.xa[h] = *reinterpret_cast<const u32x4*>(xp[h] + (size_t)row0 * x_step);

@@ -679,6 +679,33 @@ def test_skinny_projection_shares_are_exact(worker, kind, m, k, n, pair):
         assert torch.equal(out.double(), gate)
 
 
+@pytest.mark.parametrize("n", [86_000_128, 172_000_256])  # 16-bit weights, int8 codes
+def test_skinny_projection_rows_beyond_32_bit_offsets(worker, n):
+    """Matrices so wide that a lane's rows start more than 2^32 bytes after its step's first: integers in the last
+    eight rows and channels only, whose wrapped offsets would land on zeros."""
+    from pypto_amd import _lib
+    from pypto_amd.runtime import _dtype_code
+
+    g = torch.Generator().manual_seed(n)
+    k, last, int8 = 32, 4096, n > 100_000_000
+    x = torch.randint(1, 3, (1, k), generator=g).to(torch.bfloat16)
+    vals = torch.randint(1, 4, (8, last), generator=g)
+    w = torch.zeros((k, n), dtype=torch.int8 if int8 else torch.bfloat16, device="cuda")
+    w[24:, n - last:] = vals.to(w.dtype).cuda()
+    out = torch.full((1, n), float("nan"), device="cuda")
+    xd, lib = x.cuda(), _lib.load()
+    if int8:
+        scale = torch.ones(n, device="cuda")
+        _lib.check(lib.pto_hip_w8a16_matmul(xd.data_ptr(), w.data_ptr(), scale.data_ptr(), None, out.data_ptr(), 1, k, n,
+                                            _dtype_code(torch.bfloat16), 0, _dtype_code(torch.float32), 0))
+    else:
+        _lib.check(lib.pto_hip_projection(xd.data_ptr(), w.data_ptr(), None, out.data_ptr(), 1, k, n,
+                                          _dtype_code(torch.bfloat16), 0, _dtype_code(torch.float32), 0))
+    worker.sync()
+    assert not out[:, :n - last].any()
+    assert torch.equal(out[:, n - last:].cpu(), x[:, 24:].float() @ vals.float())
+
+
 @pytest.mark.parametrize("slabs", [1, 2, 3, 4, 5, 6, 7, 8, 9, 16, 19])
 def test_partial_slab_counts_are_exact(worker, slabs):
     """One 128-channel slab of 8 * slabs steps is the work of `slabs` workgroups: every size of the consumers' load
