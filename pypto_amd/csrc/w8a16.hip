@@ -508,7 +508,8 @@ int w8a16_partials(const void* x, bool x_blocked, const void* wq0, const void* w
   p.mapped = mapped ? 1 : 0;
   out->map = mapped ? SlabMap{(unsigned)units, (unsigned)wgs, (unsigned)p.ks, wide ? 8 : 7, p.slabs} : SlabMap{};
   out->splits = mapped ? (int)((p.ks * wgs + units - 1) / units) + 1 : 1;  // at most
-  const size_t one = (size_t)out->splits * m * n * sizeof(float);
+  // scratch for 32 rows whatever m: a call sized once fits every smaller and larger batch of the shape, also under capture
+  const size_t one = (size_t)out->splits * kMaxM * n * sizeof(float);
   void* ws = nullptr;
   int rc = workspace(one * n_mats, &ws);
   if (rc) return rc;

@@ -10,7 +10,7 @@ import pytest
 import torch
 
 from pypto_amd import workloads
-from pypto_amd.runtime import decoder_layer_decode, ffn_block, paged_attention
+from pypto_amd.runtime import decoder_layer_decode, ffn_block, paged_attention, projection
 
 pytestmark = pytest.mark.gpu
 
@@ -102,3 +102,20 @@ def test_attention_and_ffn_replays(worker):
         worker.sync()
         assert torch.equal(got_a, a_args[5]), f"attention replay {step}"
         assert torch.equal(got_f, f_args[5]), f"ffn replay {step}"
+
+
+def test_a_skinny_projection_sizes_its_scratch_for_every_batch(worker):
+    """One eager call is what a caller owes before it captures: the scratch it leaves must do for the other
+    batch sizes of the shape, since it cannot grow under capture."""
+    held = worker.get_option("workspace_bytes")
+    k, n = 32, (held // (4 * 32) // 128 + 512) * 128  # partial sums of 32 rows beyond everything held so far
+    x = torch.randn((32, k), device="cuda").to(torch.bfloat16)
+    w = torch.randn((k, n), device="cuda", dtype=torch.bfloat16)
+    out = torch.empty((32, n), device="cuda")
+    with worker.register(projection) as h:
+        h(x[:1], w, out[:1])
+        sized = worker.get_option("workspace_bytes")
+        assert sized > held
+        h(x, w, out)
+    worker.sync()
+    assert worker.get_option("workspace_bytes") == sized
