@@ -133,8 +133,9 @@ int w8a16_partials(const void* x, bool x_blocked, const void* wq0, const void* w
                    int64_t n, int x_dtype, hipStream_t st, W8Partials* out, bool w16 = false);
 // Grow-only device scratch for intermediates that must survive calls which use workspace().
 int layer_workspace(size_t bytes, void** ptr);
-// Grow-only device scratch for the split-K slabs of the tiled GEMM.
-int gemm_workspace(size_t bytes, void** ptr);
+// Grow-only device scratch for the split-K slabs of the tiled GEMMs.  Null when `st` is being captured and the area
+// would have to grow: the product then runs unsplit.
+int gemm_slabs(size_t bytes, hipStream_t st, void** ptr);
 // out = cast(sum_s(part0) * scale0 [-> SiLU(.) * (sum_s(part1) * scale1)] [+ residual]).
 int w8a16_finish(const W8Partials& parts, const float* scale0, const float* scale1, const void* residual,
                  int res_dtype, void* out, int out_dtype, bool out_blocked, int64_t m, int64_t n, hipStream_t st);

@@ -570,12 +570,16 @@ int launch_tiles(Params& p, hipStream_t st) {
   p.slabs = nullptr;
   if (p.splits > 1) {
     void* ws = nullptr;
-    const int rc = pto_hip::gemm_workspace((size_t)p.splits * (DUAL ? 2 : 1) * p.m * p.n * sizeof(float), &ws);
+    const int rc = pto_hip::gemm_slabs((size_t)p.splits * (DUAL ? 2 : 1) * p.m * p.n * sizeof(float), st, &ws);
     if (rc) return rc;
     p.slabs = reinterpret_cast<float*>(ws);
+  }
+  if (p.slabs) {
     if (long_rows) return launch<1, DUAL, float, true, true>(p, st);
     return tall ? launch<2, DUAL, float, true>(p, st) : launch<1, DUAL, float, true>(p, st);
   }
+  p.splits = 1;
+  p.k_per_split = p.k;
   if (long_rows) return launch<1, DUAL, OutT, false, true>(p, st);
   return tall ? launch<2, DUAL, OutT>(p, st) : launch<1, DUAL, OutT>(p, st);
 }

@@ -975,9 +975,13 @@ int launch_variant(GemmParams p, hipStream_t st) {
     p.splits = (p.k + p.k_per_split - 1) / p.k_per_split;
     if (p.splits > 1) {
       void* ws = nullptr;
-      const int rc = pto_hip::gemm_workspace((size_t)p.splits * (DUAL ? 2 : 1) * p.m * p.n * sizeof(float), &ws);
+      const int rc = pto_hip::gemm_slabs((size_t)p.splits * (DUAL ? 2 : 1) * p.m * p.n * sizeof(float), st, &ws);
       if (rc) return rc;
       p.slabs = reinterpret_cast<float*>(ws);
+    }
+    if (!p.slabs) {
+      p.splits = 1;
+      p.k_per_split = p.k;
     }
   }
   int rc = PTO_HIP_OK;

@@ -72,8 +72,16 @@ int layer_workspace(size_t bytes, void** ptr) {
   return rc;
 }
 
-int gemm_workspace(size_t bytes, void** ptr) {
+int gemm_slabs(size_t bytes, hipStream_t st, void** ptr) {
   Context& c = ctx();
+  if (bytes > c.gemm_ws_bytes) {
+    hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(st, &capturing) != hipSuccess) (void)hipGetLastError();
+    if (capturing != hipStreamCaptureStatusNone) {
+      *ptr = nullptr;
+      return PTO_HIP_OK;
+    }
+  }
   const int rc = grow_scratch(&c.gemm_ws, &c.gemm_ws_bytes, bytes);
   *ptr = c.gemm_ws;
   return rc;

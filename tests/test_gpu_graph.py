@@ -119,3 +119,55 @@ def test_a_skinny_projection_sizes_its_scratch_for_every_batch(worker):
         h(x, w, out)
     worker.sync()
     assert worker.get_option("workspace_bytes") == sized
+
+
+@pytest.mark.parametrize("kind", ["e4m3", "16-bit"])
+def test_a_split_product_is_captured_unsplit_when_its_slabs_do_not_fit(worker, kind):
+    """No eager call of the split form before the capture: the graph holds the unsplit product, bit for bit, and the
+    scratch has not grown."""
+    from pypto_amd import _lib
+    from pypto_amd.runtime import _dtype_code
+
+    lib, bf16 = _lib.load(), _dtype_code(torch.bfloat16)
+    k, n = 2048, 2048
+    m = worker.get_option("workspace_bytes") // (16 * 2 * 4 * n) + 256  # 8 splits' slabs: beyond half of everything held
+    m *= 2
+    g = torch.Generator(device="cuda").manual_seed(m)
+    x, wg, wu = (torch.randn(s, generator=g, device="cuda") for s in ((m, k), (k, n), (k, n)))
+    out, want = (torch.full((m, n), float("nan"), dtype=torch.bfloat16, device="cuda") for _ in range(2))
+    one = torch.ones(max(m, n), device="cuda")
+    if kind == "e4m3":
+        x, wg, wu = (t.to(torch.float8_e4m3fn) for t in (x, wg.t().contiguous(), wu.t().contiguous()))
+    else:
+        x, wg, wu = (t.to(torch.bfloat16) for t in (x, wg, wu))
+
+    def call(dst, stream):
+        if kind == "e4m3":
+            _lib.check(lib.pto_hip_gate_up_swiglu_fp8(x.data_ptr(), one.data_ptr(), wg.data_ptr(), one.data_ptr(), wu.data_ptr(),
+                                                      one.data_ptr(), dst.data_ptr(), m, k, n, bf16, stream.cuda_stream))
+        else:
+            _lib.check(lib.pto_hip_gate_up_swiglu(x.data_ptr(), wg.data_ptr(), wu.data_ptr(), dst.data_ptr(), m, k, n, bf16,
+                                                  stream.cuda_stream))
+
+    stream = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    worker.set_option("gemm_variant", 5)
+    try:
+        worker.set_option("gemm_splits", 1)
+        call(want, stream)
+        stream.synchronize()
+        held = worker.get_option("workspace_bytes")
+        worker.set_option("gemm_splits", 8)
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=stream):
+            call(out, stream)
+    finally:
+        worker.set_option("gemm_variant", 0)
+        worker.set_option("gemm_splits", 0)
+    assert worker.get_option("workspace_bytes") == held
+    for _ in range(3):
+        out.fill_(float("nan"))
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, want)
