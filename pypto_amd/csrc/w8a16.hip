@@ -5,9 +5,9 @@
 // projection.py:145-177) with int8 weights and one fp32 scale per output channel.  Decode
 // batches are small (M <= 32), so the work is reading the weights once: HBM-bound.
 //
-//   * the (128- or 256-channel slab, 32-row step) units of a launch are shared out evenly over one
-//     workgroup of four wavefronts per CU, whole numbers of workgroups to a slab where that covers the CUs; the
-//     wavefronts take a share's steps in turn.  Per step a lane reads 8 or 16 bytes of 8
+//   * the (128- or 256-channel slab, 32-row step) units of a launch are shared out evenly over workgroups of
+//     four wavefronts, at most one per CU, and whole numbers of them to a slab where that keeps most CUs
+//     busy (skinny_workgroups); the wavefronts take a share's steps in turn.  Per step a lane reads 8 or 16 bytes of 8
 //     k-rows - whole row segments per 16 lanes - keeps the next step's loads in flight,
 //     widens the int8 codes to fp32 and packs them, transposed, straight into MFMA B operands
 //     (the high halves of the fp32 values are exact bf16), then issues its v_mfma_f32_16x16x32;
@@ -28,6 +28,7 @@
 #include <type_traits>
 
 #include "common.h"
+#include "launch_choice.h"
 #include "slab_sum.h"
 
 namespace {
@@ -86,10 +87,10 @@ struct Stage {
 };
 
 // Workgroup w of G takes the units (slab, 32-row step) [w U / G, (w + 1) U / G) of the list that walks the
-// slabs one after the other (SlabMap): every CU streams the same number of bytes, whatever the
-// shape.  A launch lasts as long as the CU with the most bytes: cut into equal k ranges instead, 272
-// workgroups of a 356 MB pair of 16-bit matrices on 256 CUs read at 4.5 TB/s and 544 at 5.3, where 256 even
-// shares reach 6.5 (load-only twins of this kernel).  The four wavefronts take a run's steps in turn; when
+// slabs one after the other (SlabMap): every workgroup streams the same number of bytes.  A launch lasts as
+// long as the CU with the most bytes: cut into equal k ranges instead, 272 workgroups of a 356 MB pair of 16-bit
+// matrices on 256 CUs read at 4.5 TB/s and 544 at 5.3, where 256 even shares reach 6.5 (load-only twins of
+// this kernel).  The four wavefronts take a run's steps in turn; when
 // a run ends (the slab's last step or the workgroup's) their accumulators are summed through LDS, one after
 // the other, and written as the next partial slab of those channels; the next run's first rows
 // are in flight meanwhile.  MT: 16-row groups of activations (M <= 16 needs one: half the MFMAs,
@@ -487,22 +488,11 @@ int w8a16_partials(const void* x, bool x_blocked, const void* wq0, const void* w
   const int cols = wide ? 16 : 8, slab = 16 * cols;
   p.slabs = (int)((n + slab - 1) / slab);
   p.ks = (int)((k + kStep - 1) / kStep);
-  // Workgroups: one per CU at most (a second one on some CUs is what the slowest CU waits for: 17 MB of codes take
-  // 8.2 us on 256 and 9.9 on 288), and where the slabs allow it a whole number of them per slab, so that
-  // a workgroup has one run and its partial sums one slab (117 MB pair at 32 rows: 224 workgroups 29.6 us, 256 33.0).
-  // Of those the smallest number with the same count of rounds per wavefront, at least min_steps of them.
   const int64_t slabs_total = (int64_t)p.slabs * n_mats, units = slabs_total * p.ks;
-  const int64_t most = std::max<int64_t>(1, cx.w8a16_wgs_per_cu * cx.num_cu);
-  int64_t wgs = most;
-  if (slabs_total <= most) {
-    auto rounds = [&](int64_t per_slab) { return ((p.ks + per_slab - 1) / per_slab + kWaves - 1) / kWaves; };
-    int64_t per_slab = std::max<int64_t>(1, std::min<int64_t>(most / slabs_total, p.ks / (kWaves * cx.w8a16_min_steps)));
-    while (per_slab > 1 && rounds(per_slab - 1) == rounds(per_slab)) --per_slab;
-    wgs = slabs_total * per_slab;
-  }
+  int64_t wgs = skinny_workgroups(slabs_total, p.ks, std::max<int64_t>(1, cx.w8a16_wgs_per_cu * cx.num_cu), cx.w8a16_min_steps);
   // (units * wgs is computed in 32 bits by the kernels; shapes beyond that get a workgroup per slab)
   const bool mapped = units * wgs < (1ll << 31);
-  if (!mapped) wgs = (int64_t)p.slabs * n_mats;
+  if (!mapped) wgs = slabs_total;
   p.per_wg = (int)(units / wgs);
   p.extra = (int)(units % wgs);
   p.mapped = mapped ? 1 : 0;
