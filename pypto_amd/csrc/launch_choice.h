@@ -26,4 +26,53 @@ inline int64_t skinny_workgroups(int64_t slabs, int64_t ks, int64_t most, int64_
   return slabs * per_slab;
 }
 
+// Tile height (64 * *height rows, 0: the 256-row tile with eight wavefronts) and k split count of a product with 16-bit
+// weights: the pair with the least estimated time in microseconds, fitted to every pair (with its finish launch) at 33 to
+// 4000 rows of eleven weight shapes; 0.9 % from the best pair on average, 11 % at most.  Whole rounds of
+// workgroups over the CUs cost (a + b) ns per k row a workgroup walks, a last partial one a + b * its share of the CUs -
+// L2 and the clock are shared -, each round c more for its start and its stores; not less than the weights take to
+// stream; a split the finish launch and the slabs' way out and back, dearer once they outgrow the last-level cache.
+// The 256-row form with a ragged last row tile keeps 80 registers in scratch in the single-operand
+// pass, which slows its slab stores (4096 x 4096 at 400 rows 50 us, 34 with eight wavefronts): there the eight-wavefront
+// form is a candidate too, where its loop is the direct one the costs were taken from (k in whole 64-row tiles).  Over several rounds the board's power limit sets the clock and the 256-row tile, with the
+// fewest operand bytes per MFMA, gains what launches timed alone do not show: it wins unless another is 3 % ahead (gate/up
+// 4096 x 10752 at 2709 rows, estimates 0.7 % apart: against eight-wavefront tiles chosen as for other shapes the whole block
+// took 665 us for 652 on 192-row tiles and takes 600 for 625 on 256-row ones).
+// `forced`: height given, only the split count is chosen.
+inline void choose_quad(int m, int n, int k, bool dual, int64_t num_cu, int forced, int* height, int* want) {
+  constexpr int BK = 64, BN = 256, kMaxSplits = 16;
+  struct Cost {
+    double a, b, c;
+  };
+  // [0]: eight wavefronts
+  static constexpr Cost kCost[5] = {{16.84, 7.88, 2.31}, {5.8, 6.58, 2.03}, {10.02, 5.93, 2.83}, {12.72, 5.69, 4.69}, {16.16, 8.28, 3.52}};
+  const double weights_mb = (double)k * n * (dual ? 2 : 1) * 2e-6;
+  double best = 1e30;
+  for (int h = 0; h <= 4; ++h) {
+    if (forced ? h != forced : (h == 0 && (dual || m % 256 == 0 || k % BK != 0))) continue;
+    const int bm = h ? 64 * h : 256;
+    const int64_t tiles = (int64_t)((m + bm - 1) / bm) * (n / (dual ? BN / 2 : BN));
+    for (int s = 1; s <= kMaxSplits; ++s) {
+      if (s > 1 && k < 4 * BK * s) break;
+      const int64_t kps = ((k + s * BK - 1) / (s * BK)) * BK;
+      if ((k + kps - 1) / kps != s) continue;
+      const int64_t full = tiles * s / num_cu, left = tiles * s % num_cu;
+      const Cost& q = kCost[h];
+      double t = (double)kps * 1e-3 * ((double)full * (q.a + q.b) + (left ? q.a + q.b * (double)left / (double)num_cu : 0.0)) +
+                 q.c * (double)(full + (left ? 1 : 0));
+      t = std::max(t, weights_mb / 10.2);
+      if (s > 1) {
+        const double slab_mb = (double)s * m * n * (dual ? 2 : 1) * 4e-6;
+        t += 2.95 + slab_mb * (dual ? 0.177 : 0.374) + std::max(slab_mb - 128.0, 0.0) * 0.29;
+      }
+      if (h == 4 && full >= 2) t *= 0.97;
+      if (t < best) {
+        best = t;
+        *height = h;
+        *want = s;
+      }
+    }
+  }
+}
+
 }  // namespace pto_hip

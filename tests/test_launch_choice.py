@@ -13,6 +13,9 @@ _SOURCE = """
 extern "C" int64_t skinny_workgroups(int64_t slabs, int64_t ks, int64_t most, int64_t min_steps) {
   return pto_hip::skinny_workgroups(slabs, ks, most, min_steps);
 }
+extern "C" void choose_quad(int m, int n, int k, int dual, int64_t num_cu, int forced, int* height, int* splits) {
+  pto_hip::choose_quad(m, n, k, dual != 0, num_cu, forced, height, splits);
+}
 """
 
 
@@ -41,3 +44,28 @@ def test_skinny_workgroups_keep_the_cus_busy(choice):
                 assert wgs == slabs or ks // (wgs // slabs) >= 4 * min_steps, (slabs, ks)
             if ks >= 64 and units >= most * 4 * min_steps:
                 assert wgs * 8 > most * 5 or (ks + wgs // slabs - 1) // (wgs // slabs) <= 8 * min_steps, (slabs, ks, wgs)
+
+
+def _quad(lib, m, n, k, dual, forced=0):
+    height, splits = C.c_int(-1), C.c_int(-1)
+    lib.choose_quad(m, n, k, int(dual), C.c_int64(256), forced, C.byref(height), C.byref(splits))
+    return height.value, splits.value
+
+
+def test_tile_choice_takes_the_eight_wavefront_form_only_where_its_costs_hold(choice):
+    """Height 0 stands for the direct eight-wavefront loop; with k ending in half a 64-row tile that form would stage
+    its tiles through registers, at other costs, while the four-wavefront forms take such k as they are."""
+    seen = 0
+    for m in (65, 130, 257, 300, 400, 643, 900, 1300, 2459, 4000):
+        for n in (256, 1024, 3072, 4096, 6144, 6656):
+            for k in (32, 96, 512, 544, 1056, 3680, 4096, 4128, 6816, 11008):
+                for dual in (False, True):
+                    height, splits = _quad(choice, m, n, k, dual)
+                    assert 0 <= height <= 4 and 1 <= splits <= 16
+                    assert splits == 1 or k >= 4 * 64 * splits
+                    if height == 0:
+                        seen += 1
+                        assert k % 64 == 0 and not dual and m % 256 != 0, (m, n, k)
+                    for forced in (1, 2, 3, 4):
+                        assert _quad(choice, m, n, k, dual, forced)[0] == forced
+    assert seen > 0
