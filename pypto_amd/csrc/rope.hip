@@ -32,35 +32,45 @@ struct RopeParams {
   int* error_flag;
 };
 
+// The value of channel `ch` of sequence `b` - or, V a vector, of the channels from `ch` on, all of one slab: its partial
+// slabs added in order, times the channel scale.
+template <typename V>
+__device__ __forceinline__ V channel_scale(const RopeParams& p, int ch) {
+  return p.scale ? pto_hip::load_floats<V>(p.scale + ch) : V{} + 1.f;
+}
+template <typename V>
+__device__ __forceinline__ V fetch(const RopeParams& p, int b, int ch) {
+  const V scale = channel_scale<V>(p, ch);
+  const float* src[1] = {p.qkv + (size_t)b * (p.hq + 2 * p.hkv) * p.d + ch};
+  V v[1] = {V{}};
+  pto_hip::add_slabs(src, pto_hip::slab_count(p.map, p.splits, 0, ch), (size_t)p.split_stride, v);
+  return v[0] * scale;
+}
+// Two of them (a channel and the one it rotates with), requested together where both have as many slabs.  They need
+// not: the halves of a head wider than a slab, or of one that starts inside a slab, can lie in two.
+template <typename V>
+__device__ __forceinline__ void fetch2(const RopeParams& p, int b, int ch0, int ch1, V& v0, V& v1) {
+  const int n0 = pto_hip::slab_count(p.map, p.splits, 0, ch0), n1 = pto_hip::slab_count(p.map, p.splits, 0, ch1);
+  if (n0 != n1) {
+    v0 = fetch<V>(p, b, ch0);
+    v1 = fetch<V>(p, b, ch1);
+    return;
+  }
+  const V scale0 = channel_scale<V>(p, ch0), scale1 = channel_scale<V>(p, ch1);
+  const float* row = p.qkv + (size_t)b * (p.hq + 2 * p.hkv) * p.d;
+  const float* src[2] = {row + ch0, row + ch1};
+  V v[2] = {V{}, V{}};
+  pto_hip::add_slabs(src, n0, (size_t)p.split_stride, v);
+  v0 = v[0] * scale0;
+  v1 = v[1] * scale1;
+}
+
 template <typename T>
 __global__ __launch_bounds__(128) void rope_kv_kernel(RopeParams p) {
   const int b = blockIdx.x, head = blockIdx.y;
   const int half = p.d / 2;
   const int pos = p.seq_lens[b] - 1;
-  const size_t src = ((size_t)b * (p.hq + 2 * p.hkv) + head) * p.d;
-  // channel values: sum of the partial slabs in split order, times the channel scale
-  auto fetch = [&](int i) {
-    const float* src1[1] = {p.qkv + src + i};
-    float v[1] = {0.f};
-    pto_hip::add_slabs(src1, pto_hip::slab_count(p.map, p.splits, 0, head * p.d + i), (size_t)p.split_stride, v);
-    return p.scale ? v[0] * p.scale[(size_t)head * p.d + i] : v[0];
-  };
-  // the two channels of a rotated pair, requested together
-  auto fetch_pair = [&](int i, float& lo, float& hi) {
-    const int ch = head * p.d + i;
-    const int n_lo = pto_hip::slab_count(p.map, p.splits, 0, ch), n_hi = pto_hip::slab_count(p.map, p.splits, 0, ch + half);
-    if (n_lo == n_hi) {
-      const float s_lo = p.scale ? p.scale[ch] : 1.f, s_hi = p.scale ? p.scale[ch + half] : 1.f;
-      const float* src2[2] = {p.qkv + src + i, p.qkv + src + i + half};
-      float v[2] = {0.f, 0.f};
-      pto_hip::add_slabs(src2, n_lo, (size_t)p.split_stride, v);
-      lo = v[0] * s_lo;
-      hi = v[1] * s_hi;
-    } else {
-      lo = fetch(i);
-      hi = fetch(i + half);
-    }
-  };
+  const int ch = head * p.d;  // first channel of this head
   const bool is_q = head < p.hq, is_k = !is_q && head < p.hq + p.hkv;
   T* dst;
   if (is_q) {
@@ -82,7 +92,7 @@ __global__ __launch_bounds__(128) void rope_kv_kernel(RopeParams p) {
   const int cpos = pos < 0 ? 0 : (pos >= p.max_pos ? p.max_pos - 1 : pos);
   for (int i = threadIdx.x; i < half; i += blockDim.x) {
     float lo, hi;
-    fetch_pair(i, lo, hi);
+    fetch2<float>(p, b, ch + i, ch + i + half, lo, hi);
     if (is_q || is_k) {
       const size_t t_lo = (size_t)cpos * p.rope_w + i, t_hi = p.rope_w == p.d ? t_lo + half : t_lo;
       dst[i] = (T)(lo * p.cos[t_lo] - hi * p.sin[t_lo]);
@@ -111,7 +121,7 @@ struct RopeFp8Params {
 };
 
 constexpr float kE4m3Max = 448.f;
-typedef float f32x4 __attribute__((__vector_size__(4 * sizeof(float)), __aligned__(4)));  // a caller's tensor may start at any float
+typedef __attribute__((__vector_size__(4 * sizeof(float)))) float f32x4;
 
 __device__ __forceinline__ float e4m3_decode(uint32_t word, int byte) {
   switch (byte) {
@@ -135,55 +145,7 @@ __global__ __launch_bounds__(64) void rope_kv_fp8_kernel(RopeFp8Params pp) {
   const int b = blockIdx.x, head = blockIdx.y, lane = threadIdx.x;
   const int half = p.d / 2;
   const int pos = p.seq_lens[b] - 1;
-  const size_t src = ((size_t)b * (p.hq + 2 * p.hkv) + head) * p.d;
-  // channel values: sum of the partial slabs in split order, times the channel scale
-  auto fetch = [&](int i) {
-    const float* src1[1] = {p.qkv + src + i};
-    float v[1] = {0.f};
-    pto_hip::add_slabs(src1, pto_hip::slab_count(p.map, p.splits, 0, head * p.d + i), (size_t)p.split_stride, v);
-    return p.scale ? v[0] * p.scale[(size_t)head * p.d + i] : v[0];
-  };
-  // the two channels of a rotated pair, requested together
-  auto fetch_pair = [&](int i, float& lo, float& hi) {
-    const int ch = head * p.d + i;
-    const int n_lo = pto_hip::slab_count(p.map, p.splits, 0, ch), n_hi = pto_hip::slab_count(p.map, p.splits, 0, ch + half);
-    if (n_lo == n_hi) {
-      const float s_lo = p.scale ? p.scale[ch] : 1.f, s_hi = p.scale ? p.scale[ch + half] : 1.f;
-      const float* src2[2] = {p.qkv + src + i, p.qkv + src + i + half};
-      float v[2] = {0.f, 0.f};
-      pto_hip::add_slabs(src2, n_lo, (size_t)p.split_stride, v);
-      lo = v[0] * s_lo;
-      hi = v[1] * s_hi;
-    } else {
-      lo = fetch(i);
-      hi = fetch(i + half);
-    }
-  };
-  // four channels at a time (head_dim is a multiple of 8, so four never straddle a slab)
-  auto scale4 = [&](int e) {
-    return p.scale ? *reinterpret_cast<const f32x4*>(p.scale + (size_t)head * p.d + e) : f32x4{1.f, 1.f, 1.f, 1.f};
-  };
-  auto fetch4_one = [&](int e) {
-    const f32x4 sc = scale4(e);
-    const f32x4* src1[1] = {reinterpret_cast<const f32x4*>(p.qkv + src + e)};
-    f32x4 v[1] = {f32x4{0.f, 0.f, 0.f, 0.f}};
-    pto_hip::add_slabs(src1, pto_hip::slab_count(p.map, p.splits, 0, head * p.d + e), (size_t)p.split_stride / 4, v);
-    return v[0] * sc;
-  };
-  auto fetch4 = [&](int e, int o, f32x4& own, f32x4& other) {
-    const int n_e = pto_hip::slab_count(p.map, p.splits, 0, head * p.d + e), n_o = pto_hip::slab_count(p.map, p.splits, 0, head * p.d + o);
-    if (n_e == n_o) {
-      const f32x4 sc_e = scale4(e), sc_o = scale4(o);
-      const f32x4* src2[2] = {reinterpret_cast<const f32x4*>(p.qkv + src + e), reinterpret_cast<const f32x4*>(p.qkv + src + o)};
-      f32x4 v[2] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};
-      pto_hip::add_slabs(src2, n_e, (size_t)p.split_stride / 4, v);
-      own = v[0] * sc_e;
-      other = v[1] * sc_o;
-    } else {
-      own = fetch4_one(e);
-      other = fetch4_one(o);
-    }
-  };
+  const int ch = head * p.d;  // first channel of this head
   const bool is_q = head < p.hq, is_k = !is_q && head < p.hq + p.hkv;
   const int cpos = pos < 0 ? 0 : (pos >= p.max_pos ? p.max_pos - 1 : pos);
 
@@ -191,7 +153,7 @@ __global__ __launch_bounds__(64) void rope_kv_fp8_kernel(RopeFp8Params pp) {
     TQ* dst = reinterpret_cast<TQ*>(p.q_out) + ((size_t)b * p.hq + head) * p.d;
     for (int i = lane; i < half; i += 64) {
       float lo, hi;
-      fetch_pair(i, lo, hi);
+      fetch2<float>(p, b, ch + i, ch + i + half, lo, hi);
       const size_t t_lo = (size_t)cpos * p.rope_w + i, t_hi = p.rope_w == p.d ? t_lo + half : t_lo;
       dst[i] = (TQ)(lo * p.cos[t_lo] - hi * p.sin[t_lo]);
       dst[i + half] = (TQ)(hi * p.cos[t_hi] + lo * p.sin[t_hi]);
@@ -223,14 +185,14 @@ __global__ __launch_bounds__(64) void rope_kv_fp8_kernel(RopeFp8Params pp) {
   for (int u = 0; u < kMaxSpans; ++u) {
     const int e0 = u * 256 + lane * 4;
     if (e0 < p.d) {
-      // four channels at a time, each with the other half of its rotated pair: one trip to memory for the row (eight
-      // scalar sums a lane, one after the other: 11.3 us in a layer of 96 ragged sequences, 10.6 before the sums took slabs in batches)
+      // four channels at a time (of one slab: head_dim is a multiple of 8), each with the other half of its rotated
+      // pair: one trip to memory for the row (96 ragged sequences: 8.2 us, 10.8 with eight scalar sums a lane in turn)
       f32x4 own, other;
       if (is_k) {
         const int o0 = e0 < half ? e0 + half : e0 - half;
-        fetch4(e0, o0, own, other);
+        fetch2<f32x4>(p, b, ch + e0, ch + o0, own, other);
       } else {
-        own = fetch4_one(e0);
+        own = fetch<f32x4>(p, b, ch + e0);
       }
 #pragma unroll
       for (int q = 0; q < 4; ++q) {

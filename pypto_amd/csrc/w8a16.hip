@@ -314,15 +314,15 @@ __device__ __forceinline__ void store4_from_f32(void* p, size_t i, int dt, float
 template <int K>
 __device__ __forceinline__ void sum_splits(const float* const (&part)[K], const float* const (&scale)[K], int splits,
                                            size_t stride, int m, int n, int nn, f32x4 (&sum)[K]) {
-  const f32x4* src[K];
+  const float* src[K];
   f32x4 sc[K];
 #pragma unroll
   for (int k = 0; k < K; ++k) {
-    src[k] = reinterpret_cast<const f32x4*>(part[k] + (size_t)m * nn + n);
+    src[k] = part[k] + (size_t)m * nn + n;
     sum[k] = f32x4{0.f, 0.f, 0.f, 0.f};
     sc[k] = scale[k] ? *reinterpret_cast<const f32x4*>(scale[k] + n) : f32x4{1.f, 1.f, 1.f, 1.f};  // none: unquantised weights
   }
-  pto_hip::add_slabs(src, splits, stride / 4, sum);
+  pto_hip::add_slabs(src, splits, stride, sum);
 #pragma unroll
   for (int k = 0; k < K; ++k) sum[k] *= sc[k];
 }

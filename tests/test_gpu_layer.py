@@ -317,6 +317,37 @@ def test_rope_kv_cache_update_fp8(worker, seq, bs, grow):
     assert torch.equal(vc_d.view(torch.uint8)[rows], vc.view(torch.uint8)[rows])
 
 
+@pytest.mark.parametrize("fp8", [False, True])
+def test_rope_reads_projections_from_any_float(worker, fp8):
+    """The typed entries ask no more of qkv than a float's alignment: the same rows, caches and scales from 4, 8 and 12
+    bytes further on."""
+    from pypto_amd import _lib
+    from pypto_amd.runtime import _dtype_code
+
+    lib = _lib.load()
+    inp, qkv, kc, ks, vc, vs, (b, hq, hkv, d) = _fp8_append_case([17, 1, 40, 16], 16, seed=22)
+    if not fp8:
+        kc, vc = inp.key_cache, inp.value_cache
+    got = []
+    for off in (0, 1, 2, 3):
+        flat = torch.zeros(qkv.numel() + 4, device="cuda")
+        flat[off:off + qkv.numel()] = qkv.reshape(-1).cuda()
+        shifted = flat[off:off + qkv.numel()].reshape(qkv.shape)
+        assert shifted.data_ptr() % 16 == 4 * off
+        caches = [t.clone().cuda() for t in ((kc, vc, ks, vs) if fp8 else (kc, vc))]
+        q_out = torch.zeros(b * hq, d, dtype=torch.bfloat16, device="cuda")
+        tables = [t.cuda() for t in (inp.seq_lens, inp.rope_cos, inp.rope_sin, inp.block_table)]
+        max_blocks, max_pos = inp.max_num_blocks_per_req, inp.rope_cos.shape[0]
+        call = lib.pto_hip_rope_kv_cache_update_fp8 if fp8 else lib.pto_hip_rope_kv_cache_update
+        _lib.check(call(shifted.data_ptr(), *(t.data_ptr() for t in (*tables, *caches, q_out)), b, hq, hkv, d, 16, max_blocks,
+                        max_pos, kc.shape[0] // (hkv * 16 if fp8 else 1), _dtype_code(torch.bfloat16), 0))
+        worker.sync()
+        got.append([t.cpu().view(torch.uint8) for t in (q_out, *caches)])
+    assert got[0][0].any()
+    for other in got[1:]:
+        assert all(torch.equal(a, c) for a, c in zip(got[0], other))
+
+
 def test_fp8_append_then_attention_matches_bf16_path(worker):
     """The appended token is visible to the e4m3 attention path: decode over the updated cache
     agrees with the oracle's attention on the oracle-updated cache."""
@@ -726,3 +757,40 @@ def test_partial_slab_counts_are_exact(worker, slabs):
     torch.testing.assert_close(summed, gate + residual, rtol=2 ** -22, atol=8 * 2 ** -23 * float(gate.abs().max()))
     # one bf16 ulp (2^-7) of SwiGLU's value, SiLU's exponential overflowing to zero below
     torch.testing.assert_close(pair.double(), oracle.swiglu(gate.double(), up.double()), rtol=2 ** -7, atol=1e-30)
+
+
+@pytest.mark.parametrize("fp8_kv", [False, True])
+def test_layer_whose_rotated_halves_have_unequal_slab_counts(worker, fp8_kv):
+    """head_dim 256 puts the halves of a head into two output slabs, and 144 slabs are shared out over all CUs, so the
+    halves of some heads are the sum of two partial slabs and of three."""
+    hq, hkv, d, bs, hidden = 64, 4, 256, 32, 2048
+    slabs, ks, wgs = (hq + 2 * hkv) * d // 128, hidden // 32, worker.device_info()["compute_units"]
+    count = [((s + 1) * ks * wgs - 1) // (slabs * ks) - ((s * ks + 1) * wgs - 1) // (slabs * ks) for s in range(slabs)]
+    assert wgs // 2 < slabs <= wgs * 5 // 8 and any(count[s] != count[s + 1] for s in range(0, slabs, 2))
+    inp = workloads.decoder_layer_inputs(batch=3, hidden=hidden, num_heads=hq, kv_head_num=hkv, head_dim=d,
+                                         intermediate=512, block_size=bs, context_lens=[40, 1, 65], seed=13)
+    args = list(inp.args())
+    if fp8_kv:
+        pool_blocks = inp.key_cache.shape[0] // (hkv * bs)
+        kc, ks_ = oracle.quantize_kv_fp8(inp.key_cache, pool_blocks, hkv, bs)
+        vc, vs_ = oracle.quantize_kv_fp8(inp.value_cache, pool_blocks, hkv, bs)
+        w = inp.weights
+        ref_out, ref_k, ref_v, ref_ks, ref_vs = oracle.decoder_layer_decode(
+            inp.hidden, inp.seq_lens, inp.block_table, kc, vc, inp.rope_cos, inp.rope_sin,
+            inp.gamma_in, inp.gamma_post, *w["qkv"], *w["o"], *w["gate"], *w["up"], *w["down"],
+            num_heads=hq, kv_head_num=hkv, head_dim=d, block_size=bs,
+            max_num_blocks_per_req=inp.max_num_blocks_per_req, eps=inp.eps, k_scale=ks_, v_scale=vs_)
+        args[3:5] = [kc.clone(), vc.clone(), ks_.clone(), vs_.clone()]
+        with worker.register(decoder_layer_decode_fp8kv) as h:
+            h(*args)
+        caches = [(oracle.dequant_kv_fp8(args[3], args[5], bs), oracle.dequant_kv_fp8(ref_k, ref_ks, bs), ref_ks.max() * 32.0),
+                  (oracle.dequant_kv_fp8(args[4], args[6], bs), oracle.dequant_kv_fp8(ref_v, ref_vs, bs), ref_vs.max() * 32.0)]
+    else:
+        ref_out, ref_k, ref_v = _oracle_layer(inp)
+        with worker.register(decoder_layer_decode) as h:
+            h(*args)
+        caches = [(inp.key_cache.float(), ref_k.float(), 2e-2), (inp.value_cache.float(), ref_v.float(), 2e-2)]
+    # an e4m3 row differs by a code at most (the largest step is 32 of its 448); a 16-bit one by its rounding
+    for got, want, tol in caches:
+        assert ((got - want).abs() <= tol + 1e-2 * want.abs() + 1e-6).all()
+    validate_golden({"out": inp.out.float()}, {"out": ref_out.float()}, rtol=2e-2, atol=2e-2)

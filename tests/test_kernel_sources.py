@@ -1,7 +1,12 @@
-"""Rules of the hand-written instructions in the kernel sources (CPU: the sources are read, nothing runs)."""
+"""Rules the kernel sources keep (CPU: they are read and checked by the compiler, nothing runs)."""
 
 import re
+import subprocess
 from pathlib import Path
+
+import pytest
+
+from pypto_amd import build
 
 CSRC = Path(__file__).resolve().parent.parent / "pypto_amd" / "csrc"
 _ASM = re.compile(r"asm volatile\(((?:\s*\"(?:[^\"\\]|\\.)*\")+)")
@@ -27,3 +32,13 @@ def test_a_load_into_lds_never_follows_its_m0_write_directly():
                     seen += 1
                     assert "lds" not in after, f"{path.name}: '{before}' is followed by '{after}'"
     assert seen >= 1
+
+
+@pytest.mark.parametrize("name", ["rope.hip", "w8a16.hip"])
+def test_slab_sums_keep_the_alignment_of_their_sources(name):
+    """A caller's qkv may start at any float; a pointer to a 16-byte vector made from it is reported by the compiler
+    where it reaches a parameter that expects the vector's own alignment."""
+    r = subprocess.run([build.HIPCC, "--offload-arch=gfx950", "--cuda-device-only", "-fsyntax-only", "-std=c++17",
+                        "-Werror=align-mismatch", f"-I{build.INCLUDE}", f"-I{CSRC}", str(CSRC / name)],
+                       capture_output=True, text=True)
+    assert r.returncode == 0, r.stderr
