@@ -27,17 +27,22 @@ inline int64_t skinny_workgroups(int64_t slabs, int64_t ks, int64_t most, int64_
 }
 
 // Tile height (64 * *height rows, 0: the 256-row tile with eight wavefronts) and k split count of a product with 16-bit
-// weights: the pair with the least estimated time in microseconds, fitted to every pair (with its finish launch) at 33 to
-// 4000 rows of eleven weight shapes; 0.9 % from the best pair on average, 11 % at most.  Whole rounds of
+// weights: the pair with the least estimated time in microseconds.  Timed against every pair (with its finish launch) at 33
+// to 4000 rows of eighteen weight shapes, 1024 x 3072 to 8192 x 22016, the one it picks is slower than the best by
+// 1.0 % on average and 23 % at most in gate/up passes, by 2.3 % and 20 % in single ones.  Whole rounds of
 // workgroups over the CUs cost (a + b) ns per k row a workgroup walks, a last partial one a + b * its share of the CUs -
 // L2 and the clock are shared -, each round c more for its start and its stores; not less than the weights take to
 // stream; a split the finish launch and the slabs' way out and back, dearer once they outgrow the last-level cache.
 // The 256-row form with a ragged last row tile keeps 80 registers in scratch in the single-operand
 // pass, which slows its slab stores (4096 x 4096 at 400 rows 50 us, 34 with eight wavefronts): there the eight-wavefront
-// form is a candidate too, where its loop is the direct one the costs were taken from (k in whole 64-row tiles).  Over several rounds the board's power limit sets the clock and the 256-row tile, with the
-// fewest operand bytes per MFMA, gains what launches timed alone do not show: it wins unless another is 3 % ahead (gate/up
-// 4096 x 10752 at 2709 rows, estimates 0.7 % apart: against eight-wavefront tiles chosen as for other shapes the whole block
-// took 665 us for 652 on 192-row tiles and takes 600 for 625 on 256-row ones).
+// form is a candidate too, where its loop is the direct one the costs were taken from (k in whole 64-row tiles).
+// Over several rounds the 256-row tile, with the fewest operand bytes per MFMA, is ahead of what its one-round costs say
+// (back to back, 256 / 192 rows a tile: gate/up 5120 x 13824 at 1800 rows 506 / 528 us, 8192 x 22016 at 3000 1816 / 1846,
+// 4096 x 10752 at 2709 417 / 454): it wins unless another is 5 % ahead.  At 0.97 instead of 0.95 the first two are lost, at
+// 0.93 others are (4096 x 14336 at 3000 rows by 5 %).
+// Up to 64 rows a single matrix is bound by its stream, and splits that start a multiple of 8 MiB apart ask the same memory
+// channels at the same time: 11008 x 4096 in 11 splits of 1024 k rows 31.4 us, in 16 of 704 26.5; 14336 x 4096 in 14 of
+// 1024 33.3, in 16 of 896 31.3.
 // `forced`: height given, only the split count is chosen.
 inline void choose_quad(int m, int n, int k, bool dual, int64_t num_cu, int forced, int* height, int* want) {
   constexpr int BK = 64, BN = 256, kMaxSplits = 16;
@@ -64,8 +69,9 @@ inline void choose_quad(int m, int n, int k, bool dual, int64_t num_cu, int forc
       if (s > 1) {
         const double slab_mb = (double)s * m * n * (dual ? 2 : 1) * 4e-6;
         t += 2.95 + slab_mb * (dual ? 0.177 : 0.374) + std::max(slab_mb - 128.0, 0.0) * 0.29;
+        if (!dual && m <= 64 && kps * n % (4 << 20) == 0) t *= 1.05;
       }
-      if (h == 4 && full >= 2) t *= 0.97;
+      if (h == 4 && full >= 2) t *= 0.95;
       if (t < best) {
         best = t;
         *height = h;
