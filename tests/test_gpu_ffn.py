@@ -717,9 +717,10 @@ def test_gemm_fp8_rows_beyond_32_bit_offsets(worker, variant):
         worker.set_option("gemm_variant", 0)
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("variant", [4, 5])
 @pytest.mark.parametrize("m,k,n,splits", [(1, 512, 128, 2), (33, 640, 200, 3), (129, 2048, 384, 16), (300, 896, 260, 4)])
-def test_gate_up_fp8_k_split_and_fused_quantiser(worker, variant, m, k, n, splits):
+def test_gate_up_fp8_k_split_and_fused_quantiser(worker, variant, m, k, n, splits, dtype):
     """The gate/up pass with k split (uneven shares included): the same h as the unsplit pass up to the order of
     the fp32 sums - exact here, small integers - and the block, whose quantiser sums the slabs itself, is
     bit-identical to the chain of stages under the same split."""
@@ -734,24 +735,30 @@ def test_gate_up_fp8_k_split_and_fused_quantiser(worker, variant, m, k, n, split
         worker.set_option("gemm_variant", variant)
         for sp in (1, splits):
             worker.set_option("gemm_splits", sp)
-            h = torch.full((m, n), float("nan"), dtype=torch.bfloat16, device="cuda")
+            h = torch.full((m, n), float("nan"), dtype=dtype, device="cuda")
             _lib.check(lib.pto_hip_gate_up_swiglu_fp8(a.data_ptr(), sa.data_ptr(), wg.data_ptr(), sw.data_ptr(), wu.data_ptr(),
-                                                      sw.data_ptr(), h.data_ptr(), m, k, n, code(torch.bfloat16), 0))
+                                                      sw.data_ptr(), h.data_ptr(), m, k, n, code(dtype), 0))
             worker.sync()
             hs.append(h.cpu())
-        assert torch.equal(hs[0], hs[1])
+        if dtype == torch.bfloat16:
+            assert torch.equal(hs[0], hs[1])
+        else:
+            # the last product and its rounding to fp16 may be one instruction (one rounding) in one kernel and two in the
+            # other: the same value or its neighbour
+            apart = (hs[0].view(torch.int16).int() - hs[1].view(torch.int16).int()).abs()
+            assert ((hs[0] == hs[1]) | (apart <= 1)).all()  # (zeros of either sign are the same value)
         if n % 128 == 0:
-            q, _ = workloads.ffn_fp8_inputs(tokens=m, hidden=k, intermediate=n, seed=3, device="cuda")
+            q, _ = workloads.ffn_fp8_inputs(tokens=m, hidden=k, intermediate=n, seed=3, dtype=dtype, device="cuda")
             with worker.register(ffn_block_fp8) as hd:
                 hd(*q.args())
-            x8, hb = torch.zeros((m, k), dtype=torch.uint8, device="cuda"), torch.zeros((m, n), dtype=torch.bfloat16, device="cuda")
+            x8, hb = torch.zeros((m, k), dtype=torch.uint8, device="cuda"), torch.zeros((m, n), dtype=dtype, device="cuda")
             h8, sx, sh = torch.zeros((m, n), dtype=torch.uint8, device="cuda"), torch.zeros(m, device="cuda"), torch.zeros(m, device="cuda")
             out = torch.zeros_like(q.out)
-            b16 = code(torch.bfloat16)
-            _lib.check(lib.pto_hip_rms_norm_quantize_fp8(q.x.data_ptr(), q.gamma.data_ptr(), x8.data_ptr(), sx.data_ptr(), m, k, q.eps, b16, 0))
+            act = code(dtype)
+            _lib.check(lib.pto_hip_rms_norm_quantize_fp8(q.x.data_ptr(), q.gamma.data_ptr(), x8.data_ptr(), sx.data_ptr(), m, k, q.eps, act, 0))
             _lib.check(lib.pto_hip_gate_up_swiglu_fp8(x8.data_ptr(), sx.data_ptr(), q.w_gate8.data_ptr(), q.w_gate_scale.data_ptr(),
-                                                      q.w_up8.data_ptr(), q.w_up_scale.data_ptr(), hb.data_ptr(), m, k, n, b16, 0))
-            _lib.check(lib.pto_hip_quantize_rows_fp8(hb.data_ptr(), h8.data_ptr(), sh.data_ptr(), m, n, b16, 0))
+                                                      q.w_up8.data_ptr(), q.w_up_scale.data_ptr(), hb.data_ptr(), m, k, n, act, 0))
+            _lib.check(lib.pto_hip_quantize_rows_fp8(hb.data_ptr(), h8.data_ptr(), sh.data_ptr(), m, n, act, 0))
             _lib.check(lib.pto_hip_projection_fp8(h8.data_ptr(), sh.data_ptr(), q.w_down8.data_ptr(), q.w_down_scale.data_ptr(),
                                                   out.data_ptr(), m, n, k, code(torch.float32), 0))
             worker.sync()

@@ -677,7 +677,11 @@ def test_llama_mini_argument_rules(worker):
 @pytest.mark.parametrize("m,k,n,pair", [(1, 48, 33040, False),   # more slabs than CUs: shares of the list cross slabs, k ends in half a step
                                         (17, 112, 20800, True),  # ... of a pair of matrices, two row groups
                                         (16, 1040, 304, False),  # a few slabs, several workgroups on each, a ragged last slab
-                                        (32, 4096, 128, True), (5, 32, 16, False)])
+                                        (32, 4096, 128, True), (5, 32, 16, False),
+                                        (16, 48, 66064, False),  # more 256-channel slabs than CUs too, one row group
+                                        (17, 48, 33040, True),   # ... of a pair, two row groups
+                                        (9, 2080, 18432, False),  # 144 slabs on all CUs: two or three partial slabs each
+                                        (20, 2080, 36864, False)])  # ... of 256 channels
 def test_skinny_projection_shares_are_exact(worker, kind, m, k, n, pair):
     """Every share of the (slab, step) list against the integer product: small-integer operands make every sum exact
     whatever its order, so a row, channel or step counted twice or left out shows."""
@@ -708,6 +712,27 @@ def test_skinny_projection_shares_are_exact(worker, kind, m, k, n, pair):
         torch.testing.assert_close(out.double(), oracle.swiglu(gate, up), rtol=2 ** -7, atol=1e-30)
     else:
         assert torch.equal(out.double(), gate)
+
+
+def test_skinny_projection_whose_list_is_too_long_for_32_bits(worker):
+    """units * workgroups reaches 2^31 (here by sixteen workgroups per CU): one workgroup per slab instead of shares."""
+    cus = worker.device_info()["compute_units"]
+    k, n = 1024, 2_097_224  # 16385 slabs of 32 steps, the last one ragged
+    assert (n + 127) // 128 * (k // 32) * 16 * cus >= 2 ** 31
+    g = torch.Generator(device="cuda").manual_seed(7)
+    x = torch.randint(-2, 3, (3, k), generator=g, device="cuda").to(torch.bfloat16)
+    w = torch.randint(-3, 4, (k, n), generator=g, device="cuda", dtype=torch.int8)
+    out = torch.full((3, n), float("nan"), device="cuda")
+    one = torch.ones(n, device="cuda")
+    worker.set_option("w8a16_wgs_per_cu", 16)
+    try:
+        with worker.register(w8a16_matmul) as h:
+            h(x, w, one, out)
+        worker.sync()
+    finally:
+        worker.set_option("w8a16_wgs_per_cu", 1)
+    for c in range(0, n, 1 << 18):  # integers below 2^24: exact in fp32 whatever the order
+        assert torch.equal(out[:, c:c + (1 << 18)], x.float() @ w[:, c:c + (1 << 18)].float())
 
 
 @pytest.mark.parametrize("n", [86_000_128, 172_000_256])  # 16-bit weights, int8 codes
