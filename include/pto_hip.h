@@ -574,8 +574,9 @@ PTO_HIP_API int pto_hip_backend_handler_query(const char* hook, int32_t arg, cha
  *                               and tests; 4 and 7 give identical bits)
  *  "gemm_quad_rows"             tile height of the four-wavefront form where "gemm_variant" is 0 or 7:
  *                               0 = by estimate (256 under variant 7, default), 64, 128, 192, 256
- *  "gemm_splits"                k splits of the tiled GEMM: 0 = by shape (default), 1..16 = as given
- *                               when k allows (each split at least four 64-row k tiles)
+ *  "gemm_splits"                k splits of the tiled GEMMs: 0 = by shape (default), 1..16 = as given
+ *                               when k allows (16-bit and int8 weights: each split at least four 64-row
+ *                               k tiles; e4m3: at least one tile of 128 codes), under every "gemm_variant"
  *  "w8a16_wgs_per_cu"           most workgroups per CU of the skinny projections (default 1)
  *  "w8a16_wide"                 1 = int8 codes of large matrices (>= 80 MB) are read 16 per lane
  *                               (default), 0 = always 8 per lane, 2 = 16 per lane whenever the

@@ -98,16 +98,16 @@ struct Const {
 // 4*RING - 1 phases to land, and the waits (vmcnt counted, never 0) leave all but the oldest quarter
 // in flight.  What bounds it: with whole tiles double-buffered instead (eight wavefronts of 128 x 64, one
 // barrier and one full wait a k-tile), a k-tile took the 1.3-1.4 us that its 64 KB need to arrive,
-// whatever its height, against 0.86 us of MFMA at the full clock; now the matrix pipes are busy in 75 % of
-// the clocks of the tall tile's loop and epilogue and the shader clock drops to 2.0 GHz under the load.
+// whatever its height, against 0.86 us of MFMA at the full clock; now the matrix pipes are busy in 77 % of
+// the clocks of the gate/up pass and 74 % of the down pass's (SQ_VALU_MFMA_BUSY_CYCLES / 4 / SQ_BUSY_CU_CYCLES), and
+// the shader clock drops to 2.0 GHz under the load.
 // Weights of three blocks in turn, LLaMA-7B shape at 2048 tokens: gate/up pass 171 -> 148 us (2.5 PFLOP/s), down
 // pass 119 -> 92 us, block 313 -> 264 us; at 300 / 512 / 1024 / 4000 tokens 129 -> 107, 148 -> 125, 193 -> 174,
 // 527 -> 491 us.  Holding a whole tile's fragments (A0, A1, B0, B1) takes 96-128 registers next to 256
 // accumulators: hence one wavefront per SIMD, which also reads a third less from LDS per MFMA than
 // two of 128 x 64 would.
 // The weights are the MFMA's first operand, so that an accumulator register holds four consecutive channels of
-// one row: rows are stored 16 bytes at a time without a transpose (the epilogue of a tile, which the matrix
-// pipes wait out: 23 thousand clocks with quad transposes and an address per store, 11 thousand so).
+// one row: rows are stored 16 bytes at a time without a transpose (the matrix pipes wait out a tile's epilogue).
 // In the gate/up pass a B quarter is 64 gate channels followed by the 64 up channels of the same
 // outputs, and the two accumulator columns of a quadrant are gate / up of the same 32 outputs, so
 // SiLU(g) * u is applied on the accumulators.
@@ -117,7 +117,8 @@ struct Const {
 // LDS checks together for bank conflicts (16 consecutive rows, one logical chunk, 256 bytes = all 64
 // banks) then hit 16 different slots of 8 row pairs.
 // LONG: rows so long that a tile's last one starts 2^32 bytes or more after its first (kLongRow): an address per lane
-// and request instead of 32-bit offsets from the tile's base, which costs every other shape up to 0.9 %.
+// and request instead of 32-bit offsets from the tile's base (for all shapes: LLaMA-7B block at 2048 tokens 266.9 -> 269.1
+// us, 1024 x 2816 at 1024 tokens 38.3 -> 38.7).
 template <int MH, int RING, bool DUAL, bool SPLIT, bool LONG, typename OutT>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) void gemm8_kernel(Params p) {
   constexpr int BM = 128 * MH;
@@ -542,8 +543,9 @@ int launch_tiles(Params& p, hipStream_t st) {
     // The pair of tile height and k splits with the least estimated time in microseconds: rounds of
     // workgroups over the CUs x (k-tiles x the time of one, growing with the share of CUs that are busy, plus a
     // tile's start and epilogue), not less than the weights take to arrive; with k split, plus the finish launch
-    // and the slabs' way out and back.  Fitted to timings of every pair at 8 to 4096 rows of four weight
-    // shapes (hidden 1024 to 5120): the pair it picks is 0.9 % from the best one on average, 15 % at worst.
+    // and the slabs' way out and back.  Fitted at 8 to 4096 rows of four weight shapes (hidden
+    // 1024 to 5120).  Timed against every pair at 8 to 4000 rows of five, the one it picks is 2.0 % from the best on
+    // average and 21 % at worst in gate/up passes, 1.7 % and 17 % in single ones.
     const int from = forced > 0 ? splits : 1, to = forced > 0 ? splits : can_split ? std::max(1, std::min(16, nk / 2)) : 1;
     double best = 1e30;
     for (int th = 1; th >= 0; --th) {
