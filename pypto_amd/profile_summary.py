@@ -117,7 +117,7 @@ def by_grid_summary(args) -> None:
     keys = [k for k in keys if not k[0].startswith("torch:") and "rocclr" not in k[0]]
     data: dict = {"commands": args.command, "calibration": {"copy_kib": args.copy_kib, **{f"{c}_read_for_copy": v for c, v in copy_reading.items()}},
                   "launches": []}
-    lines = [f"# {args.title}", "", "Commands (run from /tmp on the GPU box, R = repository root):", "```", *args.command, "```", ""]
+    lines = [f"# {args.title}", "", "Commands (run from /tmp, R = repository root):", "```", *args.command, "```", ""]
     if args.bench_log and args.bench_log.exists():
         js = [ln for ln in args.bench_log.read_text().splitlines() if ln.startswith('{"metric')]
         if js:
@@ -203,7 +203,7 @@ def main() -> None:
                 data["kernels"][k][f"{label}_kib"] = v["mean"]
                 data["kernels"][k][f"{label}_dispatches"] = v["n"]
 
-    lines = [f"# {args.title}", "", "Commands (run from /tmp on the GPU box, R = repository root):", "```", *args.command,
+    lines = [f"# {args.title}", "", "Commands (run from /tmp, R = repository root):", "```", *args.command,
              "```", ""]
     if args.bench_log and args.bench_log.exists():
         js = [ln for ln in args.bench_log.read_text().splitlines() if ln.startswith('{"metric')]
