@@ -563,14 +563,14 @@ PTO_HIP_API int pto_hip_backend_handler_query(const char* hook, int32_t arg, cha
  *  "attn_group_tiles"           cap on the 16-head query tiles one wavefront carries: 0 = the whole KV
  *                               group up to 64 heads (32 at head_dim 256), the cache read once per
  *                               group (default); 1, 2, 4 = at most that many, read once per wavefront
- *  "gemm_variant"               FFN GEMM tiling: 0 = default choice (with 16-bit weights, columns and k in
- *                               whole tiles: four wavefronts, one per SIMD, on 64- to 256-row tiles;
+ *  "gemm_variant"               FFN GEMM tiling: 0 = default choice (with 16-bit weights:
+ *                               four wavefronts, one per SIMD, on 64- to 256-row tiles;
  *                               otherwise eight, two per SIMD, on a 64-row tile up to 64 rows, else the
  *                               256- or 128-row tile; tile height and k split count with the least
  *                               estimated time; skinny projections up to 32 tokens); 4 = 256-row tile with
  *                               eight wavefronts, k split in two when CUs would idle, 5 = 128-row
  *                               tile, 6 = 64-row tile, k split while CUs would idle, 7 = as 4 with
- *                               four wavefronts wherever that form is built (forced forms, for sweeps
+ *                               four wavefronts with 16-bit weights (forced forms, for sweeps
  *                               and tests; 4 and 7 give identical bits)
  *  "gemm_quad_rows"             tile height of the four-wavefront form where "gemm_variant" is 0 or 7:
  *                               0 = by estimate (256 under variant 7, default), 64, 128, 192, 256

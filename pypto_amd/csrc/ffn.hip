@@ -40,8 +40,11 @@ int launch_typed(const GemmParams& p, int dtype, int out_dtype, hipStream_t st) 
   if (p.scale0)  // int8 weight codes
     return DUAL ? pto_hip::gemm_launch_w8_dual(p, dtype, out_dtype, st)
                 : pto_hip::gemm_launch_w8_single(p, dtype, out_dtype, st);
-  return DUAL ? pto_hip::gemm_launch_w16_dual(p, dtype, out_dtype, st)
-              : pto_hip::gemm_launch_w16_single(p, dtype, out_dtype, st);
+  if (dtype == PTO_HIP_BF16)
+    return DUAL ? pto_hip::gemm_launch_w16_dual_bf16(p, out_dtype, st)
+                : pto_hip::gemm_launch_w16_single_bf16(p, out_dtype, st);
+  return DUAL ? pto_hip::gemm_launch_w16_dual_fp16(p, out_dtype, st)
+              : pto_hip::gemm_launch_w16_single_fp16(p, out_dtype, st);
 }
 
 // ---- fp32 operands: the reference's 64x64 teaching example (01_ffn.py:155-160) ---------------

@@ -6,6 +6,7 @@
 
 #include <algorithm>
 #include <atomic>
+#include <type_traits>
 
 #include "common.h"
 #include "launch_choice.h"
@@ -498,7 +499,12 @@ int launch_gemm(GemmParams p, hipStream_t st) {
 // Operands go global -> LDS directly, as in the eight-wavefront form; with four 16-byte chunks to an
 // A row the swizzle key is (row / 4) % 4 (16 consecutive rows of a fragment read then cover all 16
 // slots of four rows' worth of banks), B keeps 64-byte group g ^ (k-row % 8).  Built for 16-bit
-// weights with n and every k range multiples of the tile (EDGE_M: any number of rows).
+// weights; EDGE 0: m, n and k in whole tiles and stages, 1: any number of rows, 2: any n and k that are multiples of 8 too.
+// A request cannot be masked or cleared on its way into LDS: rows and columns past the end read the last ones (their
+// products are not stored), and in the stage k ends in, the lanes whose bytes would lie past it read zeros from memory
+// instead, for both operands (an infinity there must not become a NaN).  Against the staged eight-wavefront form that such n
+// and k had before (with finish): gate/up 4096 x 14400 at 96 / 333 / 1000 rows 78 / 172 / 310 -> 62 / 104 / 233 us, 2056 x 6008 at
+// 128 / 2000 rows 30.8 / 157 -> 28.7 / 128, 6008 x 2056 at 2000 rows 93 -> 76, 5952 x 1984 80 -> 64; from 40 rows on ahead or level.
 //
 // MT: the tile is 64 * MT rows high, a wavefront's part 32 * MT.  The loop's time is the MFMAs of the rows the tile has,
 // padding included: 333 rows are 512 rows' work on 256-row tiles, 384 on 192-row ones.  A stage is 4 KB smaller
@@ -525,7 +531,9 @@ __device__ __forceinline__ void quad_for(F&& f) {
   }
 }
 
-template <int MT, bool DUAL, bool BF16, typename OutT, bool EDGE_M>
+__device__ const u32x4 quad_zeros = {0u, 0u, 0u, 0u};
+
+template <int MT, bool DUAL, bool BF16, typename OutT, int EDGE>
 __global__ __launch_bounds__(256) void gemm_quad_kernel(GemmParams p) {
   constexpr int NT = 4;
   constexpr int BM = 64 * MT;
@@ -546,7 +554,7 @@ __global__ __launch_bounds__(256) void gemm_quad_kernel(GemmParams p) {
   const int klen = min(p.k, k_begin + p.k_per_split) - k_begin;
   const int m0 = tm * BM;
   const int n0 = tn * (DUAL ? BN / 2 : BN);
-  const int nk = klen / QK;
+  const int nk = EDGE == 2 ? (klen + QK - 1) / QK : klen / QK;
 
   // Requests.  A: instruction e brings rows 64 e + 16 wave + lane / 4, the lane's bytes land in slot
   // lane % 4 of its row.  B: instruction e brings k-rows 8 e + 2 wave + lane / 32, slot lane % 32.
@@ -561,12 +569,13 @@ __global__ __launch_bounds__(256) void gemm_quad_kernel(GemmParams p) {
     bsrc = b_chunk < 16 ? p.b0 : p.b1;
     b_col = n0 + (b_chunk & 15) * 8;
   }
+  if (EDGE == 2) b_col = min(b_col, p.n - 8);
   const char* ga[MT];  // this lane's source of request e, for the stage requested next
   const char* gb[4];
 #pragma unroll
   for (int e = 0; e < MT; ++e) {
     int a_row = m0 + 64 * e + 16 * wave + (lane >> 2);
-    if (EDGE_M) a_row = min(a_row, p.m - 1);  // rows past the end read the last row; their products are not stored
+    if (EDGE != 0) a_row = min(a_row, p.m - 1);  // rows past the end read the last row; their products are not stored
     ga[e] = reinterpret_cast<const char*>(p.a + (int64_t)a_row * p.lda + k_begin + a_chunk * 8);
   }
 #pragma unroll
@@ -632,6 +641,16 @@ __global__ __launch_bounds__(256) void gemm_quad_kernel(GemmParams p) {
     if constexpr (E < MT) pto_hip::to_lds<ST * kStageBytes + E * 4096>(ga[E], lds_w);
     else pto_hip::to_lds<ST * kStageBytes + E * 4096>(gb[E - MT], lds_w);
   };
+  // EDGE 2, pointers at the last stage: if k ends inside it, the lanes past k turn to the zeros
+  auto clip = [&] {
+    const int left = klen - (nk - 1) * QK;
+    if (left == QK) return;
+    const char* zeros = reinterpret_cast<const char*>(&quad_zeros);
+#pragma unroll
+    for (int e = 0; e < MT; ++e) ga[e] = a_chunk * 8 < left ? ga[e] : zeros;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) gb[e] = 8 * e + b_krow < left ? gb[e] : zeros;
+  };
   // moves the pointers on to stage `next` unless that is past the end (then the last stage is requested again)
   auto advance = [&](int next) {
     const int64_t da = next < nk ? a_adv : 0, db = next < nk ? b_adv : 0;
@@ -639,7 +658,9 @@ __global__ __launch_bounds__(256) void gemm_quad_kernel(GemmParams p) {
     for (int e = 0; e < MT; ++e) ga[e] += da;
 #pragma unroll
     for (int e = 0; e < 4; ++e) gb[e] += db;
+    if (EDGE == 2 && next == nk - 1) clip();
   };
+  if (EDGE == 2 && nk == 1) clip();
   quad_for<0, QST - 1>([&](auto st_c) {
     quad_for<0, kRequests>([&](auto e_c) { request(st_c, e_c); });
     advance(decltype(st_c)::value + 1);
@@ -688,8 +709,8 @@ __global__ __launch_bounds__(256) void gemm_quad_kernel(GemmParams p) {
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // nothing may land in LDS after the workgroup has gone
 
   // ---- epilogue (row = m0 + wm*32*MT + i*32 + (r/4)*8 + (lane/32)*4 + r%4, column lane%32 + ...) ----
-  // Only the last row tile of a ragged problem checks its rows: the checks keep the stores of a tile
-  // from being issued as one batch, which every other tile should not pay for.
+  // Only the last row tile of a ragged problem checks its rows (EDGE 2: and the last column tile its columns): the checks
+  // keep the stores of a tile from being issued as one batch, which every other tile should not pay for.
   OutT* c = reinterpret_cast<OutT*>(p.c);
   const int row_base = m0 + wm * 32 * MT + (lane >> 5) * 4;
   const int col0 = (DUAL ? n0 + wn * 64 : n0 + wn * 128) + (lane & 31);
@@ -708,6 +729,7 @@ __global__ __launch_bounds__(256) void gemm_quad_kernel(GemmParams p) {
           float* s = lane_s + (int64_t)rr * p.n;
 #pragma unroll
           for (int jn = 0; jn < JN; ++jn) {
+            if (GUARD && EDGE == 2 && col0 + jn * 32 >= p.n) continue;
             s[jn * 32] = acc[i][jn][r];
             if constexpr (DUAL) s[mn + jn * 32] = acc[i][jn + NT / 2][r];
           }
@@ -726,6 +748,7 @@ __global__ __launch_bounds__(256) void gemm_quad_kernel(GemmParams p) {
         OutT* dst = lane_c + (int64_t)rr * p.ldc;
 #pragma unroll
         for (int jn = 0; jn < JN; ++jn) {
+          if (GUARD && EDGE == 2 && col0 + jn * 32 >= p.n) continue;
           if constexpr (DUAL) {
             store_out<OutT>(dst + jn * 32, silu(acc[i][jn][r]) * acc[i][jn + NT / 2][r]);
           } else {
@@ -737,16 +760,17 @@ __global__ __launch_bounds__(256) void gemm_quad_kernel(GemmParams p) {
       }
     }
   };
-  if (EDGE_M && m0 + BM > p.m) epilogue(QuadConst<1>{});
+  if ((EDGE != 0 && m0 + BM > p.m) || (EDGE == 2 && n0 + (DUAL ? BN / 2 : BN) > p.n)) epilogue(QuadConst<1>{});
   else epilogue(QuadConst<0>{});
 }
 
-template <int MT, bool DUAL, bool BF16, typename OutT, bool EDGE_M>
+template <int MT, bool DUAL, bool BF16, typename OutT, int EDGE>
 int launch_quad_e(GemmParams p, hipStream_t st) {
+  constexpr int kCols = DUAL ? BN / 2 : BN;
   p.tiles_m = (p.m + 64 * MT - 1) / (64 * MT);
-  p.tiles_n = p.n / (DUAL ? BN / 2 : BN);
+  p.tiles_n = (p.n + kCols - 1) / kCols;
   const size_t smem = (size_t)quad_stages(MT) * quad_stage_bytes(MT);
-  auto kern = gemm_quad_kernel<MT, DUAL, BF16, OutT, EDGE_M>;
+  auto kern = gemm_quad_kernel<MT, DUAL, BF16, OutT, EDGE>;
   static std::atomic<bool> attr_set{false};  // per instantiation; callers hold the dispatch lock
   if (!attr_set.load(std::memory_order_acquire)) {
     PTO_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
@@ -758,15 +782,23 @@ int launch_quad_e(GemmParams p, hipStream_t st) {
   return PTO_HIP_OK;
 }
 
-// m ragged: the same loop with the A row pointers clamped once and the stores of the missing rows skipped
+// m ragged: the same loop with the A row pointers clamped once and the stores of the missing rows skipped; n or k ragged: see the kernel
 template <bool DUAL, bool BF16, typename OutT>
 int launch_quad(const GemmParams& p, int height, hipStream_t st) {
+  if (p.n % (DUAL ? BN / 2 : BN) != 0 || p.k % QK != 0) {
+    switch (height) {
+      case 1: return launch_quad_e<1, DUAL, BF16, OutT, 2>(p, st);
+      case 2: return launch_quad_e<2, DUAL, BF16, OutT, 2>(p, st);
+      case 3: return launch_quad_e<3, DUAL, BF16, OutT, 2>(p, st);
+      default: return launch_quad_e<4, DUAL, BF16, OutT, 2>(p, st);
+    }
+  }
   switch (height) {
-    case 1: return launch_quad_e<1, DUAL, BF16, OutT, true>(p, st);
-    case 2: return launch_quad_e<2, DUAL, BF16, OutT, true>(p, st);
-    case 3: return launch_quad_e<3, DUAL, BF16, OutT, true>(p, st);
+    case 1: return launch_quad_e<1, DUAL, BF16, OutT, 1>(p, st);
+    case 2: return launch_quad_e<2, DUAL, BF16, OutT, 1>(p, st);
+    case 3: return launch_quad_e<3, DUAL, BF16, OutT, 1>(p, st);
     default:
-      return p.m % 256 == 0 ? launch_quad_e<4, DUAL, BF16, OutT, false>(p, st) : launch_quad_e<4, DUAL, BF16, OutT, true>(p, st);
+      return p.m % 256 == 0 ? launch_quad_e<4, DUAL, BF16, OutT, 0>(p, st) : launch_quad_e<4, DUAL, BF16, OutT, 1>(p, st);
   }
 }
 
@@ -850,31 +882,29 @@ int launch_variant(GemmParams p, hipStream_t st) {
   p.splits = 1;
   p.k_per_split = p.k;
   p.slabs = nullptr;
-  // variant 0 (default): with 16-bit weights and whole tiles in n and k see choose_quad.  Otherwise
+  // variant 0 (default): with 16-bit weights see choose_quad.  Otherwise
   // eight wavefronts (two per SIMD); up to 64 rows a 64x256 tile with k split
   // over up to 16 workgroups per tile while CUs would idle, beyond that the 256x256 or the 128x256
   // tile and the k split count with the least estimated time (below).  Splits write fp32 slabs
   // that a second kernel sums in split order.
   // The other values force a tile height (the sweeps behind the estimate, and the tests, use them):
   // 4 = 256x256 tile, k split in two when CUs would idle; 5 = 128x256 tile; 6 = 64x256 tile, k split
-  // while CUs would idle; 7 = as 4 with four wavefronts per workgroup (16-bit weights, whole tiles).
+  // while CUs would idle; 7 = as 4 with four wavefronts per workgroup (16-bit weights).
   const int64_t tiles_n = (p.n + (DUAL ? 127 : 255)) / (DUAL ? 128 : 256);
   const int64_t big_tiles = (int64_t)((p.m + 255) / 256) * tiles_n;
   const int64_t small_tiles = (int64_t)((p.m + 127) / 128) * tiles_n;
   const bool few = big_tiles < num_cu;
   int want = 1;
-  // 16-bit weights, whole tiles in n and k: the four-wavefront form, its tile height and the k split count by
-  // estimated time (choose_quad); `quad_height` 0 is the eight-wavefront form, also where those are not met.
+  // 16-bit weights: the four-wavefront form, its tile height and the k split count by estimated time (choose_quad);
+  // `quad_height` 0 is the eight-wavefront form.
   int quad_height = 0;
   bool quad_chosen = false;
   if constexpr (!W8) {
-    if (p.n % (DUAL ? BN / 2 : BN) == 0 && p.k % QK == 0) {
-      const int64_t rows = pto_hip::ctx().gemm_quad_rows;
-      if (variant == 7) quad_height = rows ? (int)rows / 64 : 4;
-      if (variant == 0) {
-        quad_chosen = true;
-        choose_quad(p.m, p.n, p.k, DUAL, num_cu, (int)rows / 64, &quad_height, &want);
-      }
+    const int64_t rows = pto_hip::ctx().gemm_quad_rows;
+    if (variant == 7) quad_height = rows ? (int)rows / 64 : 4;
+    if (variant == 0) {
+      quad_chosen = true;
+      choose_quad(p.m, p.n, p.k, DUAL, num_cu, (int)rows / 64, &quad_height, &want);
     }
   }
   bool small_tile = variant == 5;
@@ -941,7 +971,7 @@ int launch_variant(GemmParams p, hipStream_t st) {
   // "gemm_variant" 4 keeps eight wavefronts; both forms give identical bits.
   bool quad = false;
   if constexpr (!W8) {
-    quad = quad_height > 0 && p.k_per_split % QK == 0;
+    quad = quad_height > 0;
     if (quad) rc = launch_quad<DUAL, BF16, OutT>(p, quad_height, st);
   }
   if (!quad) {
@@ -967,24 +997,26 @@ int launch_variant(GemmParams p, hipStream_t st) {
 
 }  // namespace gemm
 
-// The instantiations are spread over four translation units (16-bit weights or int8 codes, one
+// The instantiations are spread over translation units (16-bit weights by type or int8 codes, one
 // operand or the gate/up pair) so that they compile side by side.
-int gemm_launch_w16_single(const gemm::GemmParams& p, int dtype, int out_dtype, hipStream_t st);
-int gemm_launch_w16_dual(const gemm::GemmParams& p, int dtype, int out_dtype, hipStream_t st);
+int gemm_launch_w16_single_bf16(const gemm::GemmParams& p, int out_dtype, hipStream_t st);
+int gemm_launch_w16_single_fp16(const gemm::GemmParams& p, int out_dtype, hipStream_t st);
+int gemm_launch_w16_dual_bf16(const gemm::GemmParams& p, int out_dtype, hipStream_t st);
+int gemm_launch_w16_dual_fp16(const gemm::GemmParams& p, int out_dtype, hipStream_t st);
 int gemm_launch_w8_single(const gemm::GemmParams& p, int dtype, int out_dtype, hipStream_t st);
 int gemm_launch_w8_dual(const gemm::GemmParams& p, int dtype, int out_dtype, hipStream_t st);
 
 namespace gemm {
-// Picks the instantiation for the operand types; output FP32 or the activation type.
-template <bool DUAL, bool W8>
-int launch_by_type(const GemmParams& p, int dtype, int out_dtype, hipStream_t st) {
-  const bool bf16 = dtype == PTO_HIP_BF16;
-  if (out_dtype == PTO_HIP_FP32)
-    return bf16 ? launch_variant<DUAL, true, float, W8>(p, st) : launch_variant<DUAL, false, float, W8>(p, st);
-  if (out_dtype == PTO_HIP_BF16 && bf16) return launch_variant<DUAL, true, __bf16, W8>(p, st);
-  if (out_dtype == PTO_HIP_FP16 && !bf16) return launch_variant<DUAL, false, _Float16, W8>(p, st);
+// Picks the instantiation for the output type: FP32 (not for a 16-bit gate/up pair, whose callers all keep the activation
+// type) or the activation type.
+template <bool DUAL, bool BF16, bool W8>
+int launch_by_out(const GemmParams& p, int out_dtype, hipStream_t st) {
+  if constexpr (!DUAL || W8)
+    if (out_dtype == PTO_HIP_FP32) return launch_variant<DUAL, BF16, float, W8>(p, st);
+  typedef typename std::conditional<BF16, __bf16, _Float16>::type act_t;
+  if (out_dtype == (BF16 ? PTO_HIP_BF16 : PTO_HIP_FP16)) return launch_variant<DUAL, BF16, act_t, W8>(p, st);
   return fail(PTO_HIP_ERR_INVALID_VALUE, "gemm: output dtype %s must be FP32 or the input dtype %s",
-              dtype_name(out_dtype), dtype_name(dtype));
+              dtype_name(out_dtype), dtype_name(BF16 ? PTO_HIP_BF16 : PTO_HIP_FP16));
 }
 }  // namespace gemm
 

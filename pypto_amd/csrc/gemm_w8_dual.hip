@@ -3,6 +3,7 @@
 
 namespace pto_hip {
 int gemm_launch_w8_dual(const gemm::GemmParams& p, int dtype, int out_dtype, hipStream_t st) {
-  return gemm::launch_by_type<true, true>(p, dtype, out_dtype, st);
+  return dtype == PTO_HIP_BF16 ? gemm::launch_by_out<true, true, true>(p, out_dtype, st)
+                               : gemm::launch_by_out<true, false, true>(p, out_dtype, st);
 }
 }  // namespace pto_hip

@@ -35,7 +35,7 @@ inline int64_t skinny_workgroups(int64_t slabs, int64_t ks, int64_t most, int64_
 // stream; a split the finish launch and the slabs' way out and back, dearer once they outgrow the last-level cache.
 // The 256-row form with a ragged last row tile keeps 80 registers in scratch in the single-operand
 // pass, which slows its slab stores (4096 x 4096 at 400 rows 50 us, 34 with eight wavefronts): there the eight-wavefront
-// form is a candidate too, where its loop is the direct one the costs were taken from (k in whole 64-row tiles).
+// form is a candidate too, where its loop is the direct one the costs were taken from (n and k in whole tiles).
 // Over several rounds the 256-row tile, with the fewest operand bytes per MFMA, is ahead of what its one-round costs say
 // (back to back, 256 / 192 rows a tile: gate/up 5120 x 13824 at 1800 rows 506 / 528 us, 8192 x 22016 at 3000 1816 / 1846,
 // 4096 x 10752 at 2709 417 / 454): it wins unless another is 5 % ahead.  At 0.97 instead of 0.95 the first two are lost, at
@@ -54,9 +54,10 @@ inline void choose_quad(int m, int n, int k, bool dual, int64_t num_cu, int forc
   const double weights_mb = (double)k * n * (dual ? 2 : 1) * 2e-6;
   double best = 1e30;
   for (int h = 0; h <= 4; ++h) {
-    if (forced ? h != forced : (h == 0 && (dual || m % 256 == 0 || k % BK != 0))) continue;
+    if (forced ? h != forced : (h == 0 && (dual || m % 256 == 0 || k % BK != 0 || n % BN != 0))) continue;
     const int bm = h ? 64 * h : 256;
-    const int64_t tiles = (int64_t)((m + bm - 1) / bm) * (n / (dual ? BN / 2 : BN));
+    const int bn = dual ? BN / 2 : BN;
+    const int64_t tiles = (int64_t)((m + bm - 1) / bm) * ((n + bn - 1) / bn);
     for (int s = 1; s <= kMaxSplits; ++s) {
       if (s > 1 && k < 4 * BK * s) break;
       const int64_t kps = ((k + s * BK - 1) / (s * BK)) * BK;

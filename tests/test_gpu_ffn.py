@@ -104,6 +104,47 @@ def test_ffn_tiny_fp16(worker, variant):
     validate_golden({"out": inp.out}, {"out": ref32}, rtol=2e-2, atol=1e-2)
 
 
+@pytest.mark.parametrize("m,k,n,splits", [(33, 8, 8, 1), (65, 24, 40, 1), (130, 40, 264, 1), (257, 72, 136, 1), (200, 1032, 1016, 1),
+                                          (200, 1032, 1016, 3), (300, 1096, 1000, 2), (70, 328, 520, 1), (64, 264, 512, 1), (320, 256, 776, 1)])
+def test_four_wavefront_form_on_ragged_columns_and_k(worker, m, k, n, splits):
+    """Columns and k that end anywhere (multiples of 8) in the four-wavefront form, every tile height: the bits of the
+    eight-wavefront form (same 16-wide k steps, zeros past k), the product of the oracle, nothing written beside it, and an
+    infinite weight in the last row of k gives infinities, not NaN (the lanes past k read zeros for both operands)."""
+    from pypto_amd.runtime import gate_up_swiglu, projection
+    g = torch.Generator().manual_seed(m * k + n)
+    x = (torch.randn(m, k, generator=g) / k ** 0.5).to(torch.bfloat16)
+    w = torch.randn(k, n, generator=g).to(torch.bfloat16)
+    wu = torch.randn(k, n, generator=g).to(torch.bfloat16)
+    w_inf = w.clone()
+    w_inf[-1, 0] = w_inf[-1, -1] = float("inf")
+    x_one = x.clone()
+    x_one[:, -1] = 1.0
+    got = {}
+    worker.set_option("gemm_splits", splits)
+    try:
+        for variant, rows in ((4, 0), (7, 64), (7, 128), (7, 192), (7, 256)):
+            worker.set_option("gemm_variant", variant)
+            worker.set_option("gemm_quad_rows", rows)
+            out, h16, out_inf = torch.zeros(m, n), torch.zeros(m, n, dtype=torch.bfloat16), torch.zeros(m, n)
+            with worker.register(projection) as h:
+                h(x, w, out)
+                if variant == 7:
+                    h(x_one, w_inf, out_inf)
+                    assert bool(out_inf[:, 0].isinf().all()) and bool(out_inf[:, -1].isinf().all())
+                    assert bool(out_inf[:, 1:-1].isfinite().all())
+            with worker.register(gate_up_swiglu) as h:
+                h(x, w, wu, h16)
+            got[variant, rows] = (out, h16)
+    finally:
+        for name in ("gemm_splits", "gemm_variant", "gemm_quad_rows"):
+            worker.set_option(name, 0)
+    for key, (out, h16) in got.items():
+        assert torch.equal(out, got[4, 0][0]) and torch.equal(h16, got[4, 0][1]), key
+    validate_golden({"out": got[4, 0][0]}, {"out": oracle.projection(x, w)}, rtol=2e-3, atol=2e-3)
+    want = oracle.swiglu(oracle.projection(x, w), oracle.projection(x, wu)).to(torch.bfloat16)
+    validate_golden({"out": got[4, 0][1].float()}, {"out": want.float()}, rtol=1e-2, atol=1e-2)
+
+
 @pytest.mark.parametrize("variant", [0, 4, 5, 6, 7])
 @pytest.mark.parametrize("t,h,i", [(256, 512, 1024), (100, 264, 520), (512, 1024, 2816)])
 def test_ffn_block_bf16(worker, variant, t, h, i):

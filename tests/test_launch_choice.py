@@ -71,6 +71,15 @@ def test_tile_choice_takes_the_eight_wavefront_form_only_where_its_costs_hold(ch
     assert seen > 0
 
 
+def test_tile_choice_on_ragged_columns(choice):
+    """Columns or k that end inside a tile are never for the eight-wavefront form, whose loop would stage its tiles through registers."""
+    for m in (33, 257, 400, 900, 2459):
+        for n, k in ((8, 8), (1000, 1096), (4160, 4096), (2056, 6008), (25952, 7720)):
+            for dual in (False, True):
+                height, splits = _quad(choice, m, n, k, dual)
+                assert 1 <= height <= 4 and 1 <= splits <= 16 and (splits == 1 or k >= 4 * 64 * splits)
+
+
 @pytest.mark.parametrize("m,n,k", [(1800, 13824, 5120), (3000, 22016, 8192), (2709, 10752, 4096)])
 def test_tile_choice_takes_tall_tiles_over_many_rounds(choice, m, n, k):
     """Gate/up passes that measured ahead of every other height on 256-row tiles, by 2 to 9 %."""
