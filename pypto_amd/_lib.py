@@ -8,6 +8,7 @@ bindings (python/bindings/modules/error.cpp:60-78).
 from __future__ import annotations
 
 import ctypes as C
+import importlib.util
 from pathlib import Path
 
 LIB_PATH = Path(__file__).resolve().parent / "lib" / "libpto_hip.so"
@@ -161,6 +162,28 @@ def load() -> C.CDLL:
         fn.restype = C.c_int
     _lib = lib
     return lib
+
+
+_dispatch = None
+
+
+def dispatch():
+    """The native argument side of a program call (pyext/dispatch.cpp), loaded once."""
+    global _dispatch
+    if _dispatch is None:
+        path = LIB_PATH.parent / "_dispatch.so"
+        if not path.exists():
+            raise RuntimeError(f"{path} is not built. Build it with `python -m pypto_amd.build`.")
+        spec = importlib.util.spec_from_file_location("pypto_amd._dispatch", path)
+        module = importlib.util.module_from_spec(spec)
+        spec.loader.exec_module(module)
+        _dispatch = module
+    return _dispatch
+
+
+def run_address() -> int:
+    """Where pto_hip_run lies in this process."""
+    return C.cast(load().pto_hip_run, C.c_void_p).value
 
 
 def check(status: int) -> None:

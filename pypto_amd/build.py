@@ -1,9 +1,10 @@
-"""Builds libpto_hip.so (HIP kernels + C ABI) for gfx950, in-tree.
+"""Builds libpto_hip.so (HIP kernels + C ABI) for gfx950 and the Python extension beside it, in-tree.
 
     python -m pypto_amd.build [--force]
 
 Every ``csrc/*.hip`` is compiled with hipcc for ``--offload-arch=gfx950`` and linked into
-``pypto_amd/lib/libpto_hip.so``.  hipcc cross-compiles without a GPU present.
+``pypto_amd/lib/libpto_hip.so``; ``pyext/dispatch.cpp`` is host code for torch's Python binding and becomes
+``pypto_amd/lib/_dispatch.so``.  hipcc cross-compiles without a GPU present.
 """
 
 from __future__ import annotations
@@ -12,6 +13,7 @@ import argparse
 import os
 import subprocess
 import sys
+import sysconfig
 from concurrent.futures import ThreadPoolExecutor
 from pathlib import Path
 
@@ -21,8 +23,11 @@ LIB_DIR = PKG / "lib"
 OBJ_DIR = LIB_DIR / "obj"
 LIB_PATH = LIB_DIR / "libpto_hip.so"
 INCLUDE = PKG.parent / "include"
+DISPATCH_SRC = PKG / "pyext" / "dispatch.cpp"
+DISPATCH_PATH = LIB_DIR / "_dispatch.so"
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
+CXX = os.environ.get("CXX", "g++")
 FLAGS = [
     "--offload-arch=gfx950",
     "-O3",
@@ -69,13 +74,30 @@ def _compile(src: Path, force: bool) -> Path:
     return obj
 
 
+def _build_dispatch(force: bool) -> None:
+    if not force and not _stale(DISPATCH_PATH, [DISPATCH_SRC, *INCLUDE.glob("*.h")]):
+        return
+    import torch
+
+    root = Path(torch.__file__).resolve().parent
+    cmd = [CXX, "-O2", "-std=c++17", "-shared", "-fPIC", "-fvisibility=hidden", f"-I{INCLUDE}",
+           f"-I{sysconfig.get_paths()['include']}", f"-I{root / 'include'}", f"-I{root / 'include/torch/csrc/api/include'}",
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", str(DISPATCH_SRC), "-o", str(DISPATCH_PATH),
+           f"-L{root / 'lib'}", "-ltorch_python", "-ltorch_cpu", "-lc10"]
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError(f"{CXX} failed for {DISPATCH_SRC.name}:\n{r.stderr}")
+
+
 def build(force: bool = False, jobs: int | None = None) -> Path:
     """Compile and link; returns the path of the shared library."""
     OBJ_DIR.mkdir(parents=True, exist_ok=True)
     srcs = sources()
     jobs = jobs or min(8, len(srcs))
     with ThreadPoolExecutor(max_workers=jobs) as ex:
+        ext = ex.submit(_build_dispatch, force)
         objs = list(ex.map(lambda s: _compile(s, force), srcs))
+        ext.result()
     if force or _stale(LIB_PATH, objs):
         cmd = [HIPCC, "--offload-arch=gfx950", "-shared", "-fPIC", "-o", str(LIB_PATH), *map(str, objs)]
         r = subprocess.run(cmd, capture_output=True, text=True)

@@ -436,6 +436,10 @@ class RegistrationHandle:
         self._cid = cid
         self._program = program
         self._closed = False
+        # resident tensors go through native code, which hands everything else back (pyext/dispatch.cpp)
+        self._run = _lib.dispatch().run
+        self._plain = (_lib.run_address(), cid, bytes(d == HOST for d in program.signature), program.optional,
+                       len(program.scalars))
 
     @property
     def cid(self) -> int:
@@ -452,7 +456,11 @@ class RegistrationHandle:
     def __call__(self, *args: Any, config: RunConfig | None = None, stream: int = 0) -> None:
         if self._closed:
             raise RuntimeError("RegistrationHandle is closed")
-        self._worker._dispatch(self._cid, self._program, args, stream)
+        status = self._run(*self._plain, args, stream)
+        if status is None:
+            self._worker._dispatch(self._cid, self._program, args, stream)
+        elif status:
+            _lib.check(status)
 
     def unregister(self) -> None:
         if self._closed:
