@@ -82,4 +82,25 @@ inline void choose_quad(int m, int n, int k, bool dual, int64_t num_cu, int forc
   }
 }
 
+// Tokens per context partition of a workgroup-form attention launch (a workgroup per (sequence, KV head) pair, its
+// wavefronts take the partitions) over an e4m3 cache at head_dim 128; `plain` is the rule for 16-bit caches, two wavefronts per
+// CU and at most 2048 tokens.  A chunk of codes is half the bytes of a 16-bit one, so two wavefronts do not keep enough requests in
+// flight, and a partition of 2048 tokens is what the launch waits for when lengths are ragged: from tables of more than 1536
+// tokens on four wavefronts per CU, partitions of equal length, of 512 to 1024 tokens.  Attention call, us, tables for
+// (pairs x tokens) with equal / ragged lengths: 256 x 4096 63.0 / 61.4 -> 42.6 / 34.4, 320 x 2200 49.9 / 48.0 -> 34.1 / 30.0, 768 x 3000
+// 120 / 70.4 -> 98 / 69, 1280 x 2000 108.2 / 81.9 -> 107.6 / 76.9, 272 x 14000 168 / 148 -> 165 / 106, 512 x 6000 128 -> 129; but one partition split, 1024 x 1400
+// 56.2 -> 59.7, hence 1536.  16-bit caches are the other way round: 768 x 3000 113.9 ragged -> 119, 256 x 4096 equal 80.7 -> 82.6.
+// Not more partitions than a workgroup has wavefronts (max_parts: the form needs no scratch), nor than whose partials, should the grid
+// form be taken after all, fit the fixed area of the entry point that allocates nothing.
+inline int64_t attn_e4m3_partition_tokens(int64_t pairs, int64_t max_ctx, int64_t num_cu, int64_t max_parts, int64_t bytes_per_part,
+                                          int64_t scratch, int64_t plain) {
+  if (max_ctx <= 1536) return plain;
+  const int64_t want = std::max<int64_t>(1, (4 * num_cu + pairs - 1) / pairs);
+  const int64_t tokens = std::min<int64_t>(1024, std::max<int64_t>(512, (max_ctx + want - 1) / want));
+  int64_t parts = std::min((max_ctx + tokens - 1) / tokens, max_parts);
+  parts = std::min(parts, scratch / bytes_per_part);
+  if (parts <= (max_ctx + plain - 1) / plain) return plain;
+  return (max_ctx + parts - 1) / parts;
+}
+
 }  // namespace pto_hip

@@ -25,6 +25,7 @@
 #include <type_traits>
 
 #include "common.h"
+#include "launch_choice.h"
 
 namespace {
 
@@ -1507,6 +1508,9 @@ int plan_launch(const int64_t* config, int q_dtype, int kv_dtype, bool have_scal
     if (want < 1) want = 1;
     tpp = (max_ctx + want - 1) / want;
     if (tpp > 2048) tpp = 2048;
+    if (wg_form && cx.attn_variant < 0 && fp8 && gt == 1 && d == 128)
+      tpp = pto_hip::attn_e4m3_partition_tokens(units, max_ctx, cx.num_cu, wg_max_parts((int)d, gt), batch * hq * (d + 2) * 4,
+                                                PTO_HIP_NOALLOC_SCRATCH_BYTES, tpp);
   }
   tpp = (tpp + align - 1) / align * align;
   if (tpp > max_ctx) tpp = (max_ctx + align - 1) / align * align;

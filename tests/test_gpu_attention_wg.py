@@ -75,6 +75,23 @@ def test_workgroup_form_full_small_configuration(worker):
         assert torch.equal(got, _run(worker, inp, 0, tpp))
 
 
+@pytest.mark.parametrize("longest,tokens", [(1536, 768), (1537, 512), (2100, 640), (4000, 1024)])
+def test_e4m3_pair_per_cu_partitions(worker, longest, tokens):
+    """256 pairs over an e4m3 cache: the library's own partitions (lengths at their edges, empty sequences among them) against the
+    oracle, and bit for bit against the grid on the same ones."""
+    edges = [0, 1, 31, 32, 33, tokens - 1, tokens, tokens + 1, 2 * tokens - 1, 2 * tokens, longest - 1, longest]
+    ctxs = [min(edges[i % len(edges)], longest) for i in range(32)]
+    inp = workloads.paged_attention_inputs(batch=32, num_heads=16, kv_head_num=8, block_size=128, context_lens=ctxs,
+                                           ctx_range=(1, longest), fp8_kv=True, seed=longest)
+    worker.set_option("attn_autotune", 0)
+    try:
+        got = _run(worker, inp, -1, 0)
+        assert torch.equal(got, _run(worker, inp, 0, tokens))
+    finally:
+        worker.set_option("attn_autotune", 1)
+    validate_golden({"out": got}, {"out": _golden(inp)}, rtol=RTOL, atol=ATOL)
+
+
 def test_many_sequences_with_64_heads_on_one_kv_head_at_full_size(worker):
     """256 sequences of 2048-4096 tokens, 64 query heads on one KV head (418 MB of cache): a
     (sequence, head) pair per CU, so the library's own rule takes the workgroup form, with four

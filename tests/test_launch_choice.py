@@ -16,6 +16,9 @@ extern "C" int64_t skinny_workgroups(int64_t slabs, int64_t ks, int64_t most, in
 extern "C" void choose_quad(int m, int n, int k, int dual, int64_t num_cu, int forced, int* height, int* splits) {
   pto_hip::choose_quad(m, n, k, dual != 0, num_cu, forced, height, splits);
 }
+extern "C" int64_t e4m3_partition(int64_t pairs, int64_t max_ctx, int64_t bytes_per_part, int64_t scratch, int64_t plain) {
+  return pto_hip::attn_e4m3_partition_tokens(pairs, max_ctx, 256, 8, bytes_per_part, scratch, plain);
+}
 """
 
 
@@ -28,6 +31,8 @@ def choice(tmp_path_factory):
     lib = C.CDLL(str(so))
     lib.skinny_workgroups.restype = C.c_int64
     lib.skinny_workgroups.argtypes = [C.c_int64] * 4
+    lib.e4m3_partition.restype = C.c_int64
+    lib.e4m3_partition.argtypes = [C.c_int64] * 5
     return lib
 
 
@@ -91,3 +96,27 @@ def test_tile_choice_avoids_splits_on_the_same_memory_channels(choice, k):
     """64 rows of a k x 4096 product: splits of 1024 k rows start 8 MiB apart and measured 6 to 18 % behind others."""
     _, splits = _quad(choice, 64, 4096, k, False)
     assert -(-k // (splits * 64)) * 64 % 1024 != 0
+
+
+def test_e4m3_partitions_cover_the_table_within_the_workgroup_form(choice):
+    """Never fewer partitions than a 16-bit cache gets; more only as far as one workgroup's wavefronts and the fixed scratch
+    area go; otherwise that rule's own length."""
+    scratch = 32 << 20
+    for batch in (1, 32, 40, 97, 160, 255, 4000):
+        for hkv, group in ((8, 1), (8, 4), (8, 16), (64, 8)):
+            pairs = batch * hkv
+            if pairs < 256:
+                continue
+            bytes_per_part = pairs * group * 130 * 4
+            for max_ctx in (32, 500, 1024, 1400, 1536, 1537, 2047, 2048, 2049, 2200, 3000, 4096, 6000, 8192, 14000, 32768):
+                plain = min(2048, -(-max_ctx // -(-512 // pairs)))
+                tokens = choice.e4m3_partition(pairs, max_ctx, bytes_per_part, scratch, plain)
+                before, parts = -(-max_ctx // plain), -(-max_ctx // tokens)
+                assert parts >= before
+                if parts == before:
+                    assert tokens == plain
+                else:
+                    assert parts <= 8 and parts * bytes_per_part <= scratch
+                    assert max_ctx > 1536 and 2 * tokens > 512
+                    if parts < 8 and (parts + 1) * bytes_per_part <= scratch and max_ctx > 1536:
+                        assert tokens <= 1024
