@@ -716,12 +716,14 @@ __global__ __launch_bounds__(64) void attn_partition_kernel(AttnParams p) {
 
 // Merge of the per-partition (m, l, o): the online-update algebra of
 // examples/models/04_paged_attention.py:186-215 applied across partitions, then o / l.
-// One wavefront per output row; partitions are read four at a time so that their loads overlap.
-constexpr int kReduceFast = 8;  // partition counts up to this take the single-round-trip path
+// One wavefront per output row.  What bounds it is the chain of memory round trips: one up to 8 partitions, above that one for
+// the first 16 and less than one for every 16 more.
+constexpr int kReduceFast = 8;    // partition counts up to this take the path without a loop
+constexpr int kReduceBatch = 16;  // partials requested together above
 template <int D>
 __global__ __launch_bounds__(256) void attn_reduce_kernel(AttnParams p) {
   const int lane = threadIdx.x & 63;
-  const int row = blockIdx.x * 4 + (threadIdx.x >> 6);  // b*Hq + query head
+  const int row = blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);  // b*Hq + query head
   if (row >= p.batch * p.hq) return;
   const int b = row / p.hq;
   int ctx = p.ctx_lens[b];
@@ -776,39 +778,46 @@ __global__ __launch_bounds__(256) void attn_reduce_kernel(AttnParams p) {
     }
     return;
   }
-  // lane i holds (m, l) of partitions i, i+64, ...
-  float m = kMinMax;
-  for (int i = lane; i < np; i += 64) m = fmaxf(m, ml[2 * i]);
+  // Lane i holds (m, l) of partitions i, i + 64, ...  The first of them and the first batch of partials are requested before
+  // the context length is known, every further batch before the one in front of it is summed; what slots past np hold is
+  // dropped by select.
+  float pv[2][kReduceBatch][D / 64];
+  auto fetch = [&](int set, int first) {
+#pragma unroll
+    for (int u = 0; u < kReduceBatch; ++u)
+#pragma unroll
+      for (int k = 0; k < D / 64; ++k) pv[set][u][k] = po[(size_t)min(first + u, p.n_part - 1) * D + k * 64 + lane];
+  };
+  float2 own = *reinterpret_cast<const float2*>(ml + 2 * min(lane, p.n_part - 1));
+  fetch(0, 0);
+  float m = lane < np ? own.x : kMinMax;
+  for (int i = lane + 64; i < np; i += 64) m = fmaxf(m, ml[2 * i]);
 #pragma unroll
   for (int off = 32; off > 0; off >>= 1) m = fmaxf(m, __shfl_xor(m, off));
-  float l = 0.f;
-  for (int i = lane; i < np; i += 64) l += __builtin_amdgcn_exp2f(ml[2 * i] - m) * ml[2 * i + 1];
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) l += __shfl_xor(l, off);
-  float o[D / 64];
+  float l = 0.f, o[D / 64];
 #pragma unroll
   for (int k = 0; k < D / 64; ++k) o[k] = 0.f;
-  int i = 0;
-  for (; i + 4 <= np; i += 4) {
-    float w[4], v[4][D / 64];
+  for (int base = 0; base < np; base += 64) {
+    if (base > 0) own = *reinterpret_cast<const float2*>(ml + 2 * min(base + lane, p.n_part - 1));
+    const float wgt = base + lane < np ? __builtin_amdgcn_exp2f(own.x - m) : 0.f;
+    l += base + lane < np ? wgt * own.y : 0.f;
+    auto add = [&](int set, int first) {
 #pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      w[u] = ml[2 * (i + u)];
+      for (int u = 0; u < kReduceBatch; ++u) {
+        const float w = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, wgt), (first + u) & 63));
 #pragma unroll
-      for (int k = 0; k < D / 64; ++k) v[u][k] = po[(size_t)(i + u) * D + k * 64 + lane];
-    }
-#pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      const float wgt = __builtin_amdgcn_exp2f(w[u] - m);
-#pragma unroll
-      for (int k = 0; k < D / 64; ++k) o[k] += wgt * v[u][k];
+        for (int k = 0; k < D / 64; ++k) o[k] = first + u < np ? o[k] + w * pv[set][u][k] : o[k];
+      }
+    };
+    for (int first = base; first < min(base + 64, np); first += 2 * kReduceBatch) {
+      if (first + kReduceBatch < np) fetch(1, first + kReduceBatch);
+      add(0, first);
+      if (first + 2 * kReduceBatch < np) fetch(0, first + 2 * kReduceBatch);
+      if (first + kReduceBatch < np) add(1, first + kReduceBatch);
     }
   }
-  for (; i < np; ++i) {
-    const float wgt = __builtin_amdgcn_exp2f(ml[2 * i] - m);
 #pragma unroll
-    for (int k = 0; k < D / 64; ++k) o[k] += wgt * po[(size_t)i * D + k * 64 + lane];
-  }
+  for (int off = 32; off > 0; off >>= 1) l += __shfl_xor(l, off);
   const float inv = l > 0.f ? 1.f / l : 0.f;
 #pragma unroll
   for (int k = 0; k < D / 64; ++k) {
@@ -1101,7 +1110,7 @@ __global__ __launch_bounds__(PAIR ? 128 : lean_max_waves(D, GT) * 64) void attn_
 template <int D>
 __global__ __launch_bounds__(256) void attn_lean_reduce_kernel(AttnParams p, long long wtot) {
   const int lane = threadIdx.x & 63;
-  const int row = blockIdx.x * 4 + (threadIdx.x >> 6);  // b*Hq + query head
+  const int row = blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);  // b*Hq + query head
   if (row >= p.batch * p.hq) return;
   const int b = row / p.hq, hqi = row % p.hq;
   const int h = hqi / p.group, g = hqi % p.group;
@@ -1332,7 +1341,9 @@ int launch(const AttnParams& p, int batch, bool bf16, hipStream_t stream) {
   }
   if (rc) return rc;
   if (p.n_part > 1) {
-    hipLaunchKernelGGL((attn_reduce_kernel<D>), dim3((unsigned)((batch * p.hq + 3) / 4)), dim3(256), 0,
+    // a workgroup per row as far as that gives every row a CU of its own
+    const int rows = batch * p.hq, per_wg = rows <= pto_hip::ctx().num_cu ? 1 : 4;
+    hipLaunchKernelGGL((attn_reduce_kernel<D>), dim3((unsigned)((rows + per_wg - 1) / per_wg)), dim3((unsigned)per_wg * 64), 0,
                        stream, p);
     PTO_CHECK_HIP(hipGetLastError());
   }

@@ -75,6 +75,17 @@ def test_workgroup_form_full_small_configuration(worker):
         assert torch.equal(got, _run(worker, inp, 0, tpp))
 
 
+@pytest.mark.parametrize("most", [17, 64, 100])
+@pytest.mark.parametrize("d,hq", [(128, 8), (256, 32)])
+def test_merge_of_many_partitions(worker, most, d, hq):
+    """Partition counts at the edges of the merge's batches and of a wavefront's lanes, empty sequences beside long ones."""
+    counts = [n for n in (0, 1, 8, 15, 16, 17, 31, 32, 33, 48, 49, 63, 64, 65, 97) if n < most] + [most]
+    inp = workloads.paged_attention_inputs(batch=len(counts), num_heads=hq, kv_head_num=1, head_dim=d, block_size=32,
+                                           context_lens=[max(0, 32 * n - n % 3) for n in counts], ctx_range=(1, 32 * most), seed=most)
+    got = _run(worker, inp, 0, 32)
+    validate_golden({"out": got}, {"out": _golden(inp)}, rtol=RTOL, atol=ATOL)
+
+
 @pytest.mark.parametrize("longest,tokens", [(1536, 768), (1537, 512), (2100, 640), (4000, 1024)])
 def test_e4m3_pair_per_cu_partitions(worker, longest, tokens):
     """256 pairs over an e4m3 cache: the library's own partitions (lengths at their edges, empty sequences among them) against the
