@@ -103,4 +103,20 @@ inline int64_t attn_e4m3_partition_tokens(int64_t pairs, int64_t max_ctx, int64_
   return (max_ctx + parts - 1) / parts;
 }
 
+// What partition lengths are multiples of: the KV block (`block`, or its part that divides a long one), halved down to 64
+// tokens while the table's blocks give fewer than two wavefronts per CU.  A launch of a few pairs is a chain - table, first rows, a
+// chunk of 32 tokens after the other - that halves are two chunks shorter than whole 128-token blocks.  Attention call, us, whole
+// blocks -> halves: 8 pairs x 1531 tokens 10.4 -> 8.9, x 700 10.5 -> 9.1, x 300 7.8 -> 7.2, 32 x 1531 11.8 -> 10.8; blocks of 256: 8 x 2000
+// 13.9 -> 10.8, 24 x 1100 12.8 -> 10.4.  Down to 32 tokens gains nothing more and costs where wavefronts carry several
+// query tiles (3 x 3000 10.8 -> 14.4, head_dim 256 22.4 -> 30.0), up to four wavefronts per CU nothing (64 x 900 11.0 -> 11.4).
+// bytes_per_part, scratch: as above.
+inline int64_t attn_partition_align(int64_t pairs, int64_t max_ctx, int64_t block, int64_t num_cu, int64_t bytes_per_part, int64_t scratch) {
+  while (block >= 128 && block % 64 == 0) {
+    const int64_t parts = (max_ctx + block - 1) / block;
+    if (pairs * parts >= 2 * num_cu || 2 * parts * bytes_per_part > scratch) break;
+    block /= 2;
+  }
+  return block;
+}
+
 }  // namespace pto_hip

@@ -1508,6 +1508,7 @@ int plan_launch(const int64_t* config, int q_dtype, int kv_dtype, bool have_scal
   int64_t tpp = cx.attn_tokens_per_partition;
   if (tpp <= 0) {
     const int64_t units = batch * hkv * p.gtiles;
+    align = pto_hip::attn_partition_align(units, max_ctx, align, cx.num_cu, batch * hq * (d + 2) * 4, PTO_HIP_NOALLOC_SCRATCH_BYTES);
     // With a (sequence, head) pair or more per CU the launch takes the workgroup form (see
     // paged_attention below), where two wavefronts per CU measured best (decoder layer, 32 sequences
     // of 4096 tokens: 182.5 us a step against 184.0 with four).  A wavefront that carries several
@@ -1680,7 +1681,17 @@ int paged_attention(const void* query, const void* key_cache, const void* value_
   const bool bf16 = q_dtype == PTO_HIP_BF16;
   // Where the partition partials live: the caller's fixed area (never grown) or the workspace.
   auto partials_area = [&](size_t bytes, void** ws) -> int {
-    if (!fixed_scratch) return workspace(bytes, ws);
+    if (!fixed_scratch) {
+      // Room for every launch of a few pairs (attn_partition_align), some of which have more partials than ones with more
+      // pairs: what a call was sized for once also fits a smaller batch under capture.
+      size_t ask = std::max(bytes, (size_t)(4 * cx.num_cu) * p.gt_rows * (d + 2) * sizeof(float));
+      if (ask > cx.workspace_bytes) {
+        hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
+        if (hipStreamIsCapturing((hipStream_t)stream, &capturing) != hipSuccess) (void)hipGetLastError();
+        if (capturing != hipStreamCaptureStatusNone) ask = bytes;
+      }
+      return workspace(ask, ws);
+    }
     if (bytes > fixed_scratch_bytes)
       return fail(PTO_HIP_ERR_INVALID_VALUE,
                   "paged_attention_noalloc: this launch needs %zu bytes of partition partials, the fixed scratch "

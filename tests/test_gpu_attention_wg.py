@@ -86,6 +86,16 @@ def test_merge_of_many_partitions(worker, most, d, hq):
     validate_golden({"out": got}, {"out": _golden(inp)}, rtol=RTOL, atol=ATOL)
 
 
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("bs,ctxs", [(128, [1531]), (256, [63, 2000]), (128, [64, 65, 700]), (192, [500, 96])])
+def test_few_pairs_cut_inside_blocks(worker, bs, ctxs, fp8):
+    """So few pairs that partitions are parts of a block: the library's own rule against the oracle."""
+    inp = workloads.paged_attention_inputs(batch=len(ctxs), num_heads=32, kv_head_num=8, block_size=bs, context_lens=ctxs,
+                                           ctx_range=(1, max(ctxs)), fp8_kv=fp8, seed=bs)
+    got = _run(worker, inp, -1, 0)
+    validate_golden({"out": got}, {"out": _golden(inp)}, rtol=RTOL, atol=ATOL)
+
+
 @pytest.mark.parametrize("longest,tokens", [(1536, 768), (1537, 512), (2100, 640), (4000, 1024)])
 def test_e4m3_pair_per_cu_partitions(worker, longest, tokens):
     """256 pairs over an e4m3 cache: the library's own partitions (lengths at their edges, empty sequences among them) against the

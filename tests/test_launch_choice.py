@@ -16,6 +16,9 @@ extern "C" int64_t skinny_workgroups(int64_t slabs, int64_t ks, int64_t most, in
 extern "C" void choose_quad(int m, int n, int k, int dual, int64_t num_cu, int forced, int* height, int* splits) {
   pto_hip::choose_quad(m, n, k, dual != 0, num_cu, forced, height, splits);
 }
+extern "C" int64_t partition_align(int64_t pairs, int64_t max_ctx, int64_t block, int64_t bytes_per_part, int64_t scratch) {
+  return pto_hip::attn_partition_align(pairs, max_ctx, block, 256, bytes_per_part, scratch);
+}
 extern "C" int64_t e4m3_partition(int64_t pairs, int64_t max_ctx, int64_t bytes_per_part, int64_t scratch, int64_t plain) {
   return pto_hip::attn_e4m3_partition_tokens(pairs, max_ctx, 256, 8, bytes_per_part, scratch, plain);
 }
@@ -31,7 +34,8 @@ def choice(tmp_path_factory):
     lib = C.CDLL(str(so))
     lib.skinny_workgroups.restype = C.c_int64
     lib.skinny_workgroups.argtypes = [C.c_int64] * 4
-    lib.e4m3_partition.restype = C.c_int64
+    lib.e4m3_partition.restype = lib.partition_align.restype = C.c_int64
+    lib.partition_align.argtypes = [C.c_int64] * 5
     lib.e4m3_partition.argtypes = [C.c_int64] * 5
     return lib
 
@@ -120,3 +124,18 @@ def test_e4m3_partitions_cover_the_table_within_the_workgroup_form(choice):
                     assert max_ctx > 1536 and 2 * tokens > 512
                     if parts < 8 and (parts + 1) * bytes_per_part <= scratch and max_ctx > 1536:
                         assert tokens <= 1024
+
+
+def test_partition_alignment_divides_the_block(choice):
+    """A divisor of the block in whole 32-token chunks, and halved only while there are too few partitions and their partials fit."""
+    scratch = 32 << 20
+    for block in (16, 32, 48, 64, 96, 128, 192, 256, 320, 512):
+        for pairs in (1, 3, 8, 32, 100, 255, 256, 4000):
+            for max_ctx in (block, 3 * block, 1536, 12000, 32768):
+                for rows in (1, 16, 64):
+                    per_part = pairs * rows * 258 * 4
+                    align = choice.partition_align(pairs, max_ctx, block, per_part, scratch)
+                    assert block % align == 0
+                    if align != block:
+                        parts = -(-max_ctx // (2 * align))
+                        assert align >= 64 and align % 32 == 0 and pairs * parts < 512 and 2 * parts * per_part <= scratch
