@@ -600,7 +600,7 @@ int launch_any(Params p, hipStream_t st) {
 
 // ---- row kernels: (RMSNorm +) per-row e4m3 quantisation -----------------------------------------
 constexpr int kRowThreads = 256;
-constexpr int kRowVecs = 8;  // 8-element groups a thread keeps in registers: rows of up to 16384 columns
+constexpr int kRowVecs = 8;  // most 8-element groups a thread keeps in registers: rows of up to 16384 columns
 
 __device__ __forceinline__ float clamp_e4m3(float v) { return fminf(fmaxf(v, -kE4m3Max), kE4m3Max); }
 
@@ -610,7 +610,6 @@ __device__ __forceinline__ float block_reduce(float v, bool take_max, float* sha
     const float o = __shfl_xor(v, off);
     v = take_max ? fmaxf(v, o) : v + o;
   }
-  __syncthreads();  // the previous use of `shared` is over
   if ((threadIdx.x & 63) == 0) shared[threadIdx.x >> 6] = v;
   __syncthreads();
   float tot = shared[0];
@@ -628,21 +627,35 @@ struct SlabRows {
   int64_t mn;                           // rows * cols
   int splits;
 };
-template <typename TI, bool NORM, bool SLABS = false>
+// VECS: groups of eight a thread holds, 2, 4, 6 or 8.  The work on groups a row does not have and the registers they take are
+// what bounded the kernel (both quantisers of the 2048 x 4096 x 11008 block: 278 -> 265 us for the block; 2048 x 4096 bf16 with
+// RMSNorm by itself 11.5 -> 9.6, of which the memory needs 4).
+template <typename TI, bool NORM, bool SLABS, int VECS>
 __global__ __launch_bounds__(kRowThreads) void row_quant_kernel(const TI* __restrict__ x, const float* __restrict__ gamma,
                                                                 uint8_t* __restrict__ codes, float* __restrict__ scale,
                                                                 int64_t cols, float eps, SlabRows sl) {
   typedef __attribute__((__vector_size__(8 * sizeof(TI)))) TI vec8;
-  __shared__ float red[kRowThreads / 64];
+  __shared__ float red[2][kRowThreads / 64];
   const int64_t row = blockIdx.x;
   const vec8* xr = reinterpret_cast<const vec8*>(x + row * cols);
   const int nvec = (int)(cols / 8);
   // The row stays in registers in its 16-bit form (four registers per group of eight, not eight):
   // with the whole row's workgroups resident at once the kernel is one round of loads, not two.
-  vec8 y[kRowVecs];
+  vec8 y[VECS];
   float ss = 0.f;
+  constexpr bool kGammaAhead = NORM && VECS <= 4;  // requested with the row, as far as the registers for it go
+  float4 ga[kGammaAhead ? 2 * VECS : 1];
+  if constexpr (kGammaAhead) {
 #pragma unroll
-  for (int u = 0; u < kRowVecs; ++u) {
+    for (int u = 0; u < VECS; ++u) {
+      const int i = threadIdx.x + u * kRowThreads;
+#pragma unroll
+      for (int half = 0; half < 2; ++half)
+        ga[2 * u + half] = gamma && i < nvec ? reinterpret_cast<const float4*>(gamma)[2 * i + half] : float4{1.f, 1.f, 1.f, 1.f};
+    }
+  }
+#pragma unroll
+  for (int u = 0; u < VECS; ++u) {
     const int i = threadIdx.x + u * kRowThreads;
     if (i < nvec) {
       if constexpr (SLABS) {
@@ -668,13 +681,19 @@ __global__ __launch_bounds__(kRowThreads) void row_quant_kernel(const TI* __rest
     }
   }
   if constexpr (NORM) {
-    const float inv = rsqrtf(block_reduce(ss, false, red) / (float)cols + eps);
+    const float inv = rsqrtf(block_reduce(ss, false, red[0]) / (float)cols + eps);
 #pragma unroll
-    for (int u = 0; u < kRowVecs; ++u) {
+    for (int u = 0; u < VECS; ++u) {
       const int i = threadIdx.x + u * kRowThreads;
       if (i < nvec) {
-        const float4 g0 = gamma ? reinterpret_cast<const float4*>(gamma)[2 * i] : float4{1.f, 1.f, 1.f, 1.f};
-        const float4 g1 = gamma ? reinterpret_cast<const float4*>(gamma)[2 * i + 1] : float4{1.f, 1.f, 1.f, 1.f};
+        float4 g0, g1;
+        if constexpr (kGammaAhead) {
+          g0 = ga[2 * u];
+          g1 = ga[2 * u + 1];
+        } else {
+          g0 = gamma ? reinterpret_cast<const float4*>(gamma)[2 * i] : float4{1.f, 1.f, 1.f, 1.f};
+          g1 = gamma ? reinterpret_cast<const float4*>(gamma)[2 * i + 1] : float4{1.f, 1.f, 1.f, 1.f};
+        }
         const float g[8] = {g0.x, g0.y, g0.z, g0.w, g1.x, g1.y, g1.z, g1.w};
 #pragma unroll
         for (int e = 0; e < 8; ++e) y[u][e] = (TI)((float)y[u][e] * inv * g[e]);
@@ -683,10 +702,10 @@ __global__ __launch_bounds__(kRowThreads) void row_quant_kernel(const TI* __rest
   }
   float amax = 0.f;
 #pragma unroll
-  for (int u = 0; u < kRowVecs; ++u)
+  for (int u = 0; u < VECS; ++u)
 #pragma unroll
     for (int e = 0; e < 8; ++e) amax = fmaxf(amax, fabsf((float)y[u][e]));
-  amax = block_reduce(amax, true, red);
+  amax = block_reduce(amax, true, red[1]);
   const float s = amax > 0.f ? amax / kE4m3Max : 1.f;
   // y / s, correctly rounded, without the compiler's ten-instruction division per element: the
   // reciprocal of s is refined once per row to within half an ulp (one Newton step on v_rcp_f32), and
@@ -704,7 +723,7 @@ __global__ __launch_bounds__(kRowThreads) void row_quant_kernel(const TI* __rest
   if (threadIdx.x == 0) scale[row] = s;
   uint2* crow = reinterpret_cast<uint2*>(codes + row * cols);
 #pragma unroll
-  for (int u = 0; u < kRowVecs; ++u) {
+  for (int u = 0; u < VECS; ++u) {
     const int i = threadIdx.x + u * kRowThreads;
     if (i < nvec) {
       float q[8];
@@ -719,6 +738,21 @@ __global__ __launch_bounds__(kRowThreads) void row_quant_kernel(const TI* __rest
   }
 }
 
+// Launches the instantiation for a row's length.
+template <typename TI, bool NORM, bool SLABS>
+void launch_row_quant(const void* x, const float* gamma, void* codes, float* scale, int64_t rows, int64_t cols, float eps,
+                      const SlabRows& sl, hipStream_t st) {
+  auto go = [&](auto kern) {
+    hipLaunchKernelGGL(kern, dim3((unsigned)rows), dim3(kRowThreads), 0, st, reinterpret_cast<const TI*>(x), gamma,
+                       reinterpret_cast<uint8_t*>(codes), scale, cols, eps, sl);
+  };
+  const int64_t vecs = (cols / 8 + kRowThreads - 1) / kRowThreads;
+  if (vecs <= 2) go(row_quant_kernel<TI, NORM, SLABS, 2>);
+  else if (vecs <= 4) go(row_quant_kernel<TI, NORM, SLABS, 4>);
+  else if (vecs <= 6) go(row_quant_kernel<TI, NORM, SLABS, 6>);
+  else go(row_quant_kernel<TI, NORM, SLABS, kRowVecs>);
+}
+
 int row_quant(const void* x, const float* gamma, bool norm, void* codes, float* scale, int64_t rows, int64_t cols,
               float eps, int x_dtype, hipStream_t st) {
   PTO_CHECK_ARG(cols % 8 == 0 && cols <= 8 * kRowThreads * kRowVecs,
@@ -728,16 +762,12 @@ int row_quant(const void* x, const float* gamma, bool norm, void* codes, float* 
   PTO_CHECK_ARG(((uintptr_t)x | (uintptr_t)gamma) % 16 == 0 && (uintptr_t)codes % 8 == 0,
                 "quantize_rows_fp8: misaligned operand");
   if (rows == 0) return PTO_HIP_OK;
-  dim3 grid((unsigned)rows), block(kRowThreads);
-  auto go = [&](auto kern, auto* typed) {
-    hipLaunchKernelGGL(kern, grid, block, 0, st, typed, gamma, reinterpret_cast<uint8_t*>(codes), scale, cols, eps, SlabRows{});
-  };
   if (x_dtype == PTO_HIP_BF16) {
-    if (norm) go(row_quant_kernel<__bf16, true>, reinterpret_cast<const __bf16*>(x));
-    else go(row_quant_kernel<__bf16, false>, reinterpret_cast<const __bf16*>(x));
+    if (norm) launch_row_quant<__bf16, true, false>(x, gamma, codes, scale, rows, cols, eps, SlabRows{}, st);
+    else launch_row_quant<__bf16, false, false>(x, gamma, codes, scale, rows, cols, eps, SlabRows{}, st);
   } else if (x_dtype == PTO_HIP_FP16) {
-    if (norm) go(row_quant_kernel<_Float16, true>, reinterpret_cast<const _Float16*>(x));
-    else go(row_quant_kernel<_Float16, false>, reinterpret_cast<const _Float16*>(x));
+    if (norm) launch_row_quant<_Float16, true, false>(x, gamma, codes, scale, rows, cols, eps, SlabRows{}, st);
+    else launch_row_quant<_Float16, false, false>(x, gamma, codes, scale, rows, cols, eps, SlabRows{}, st);
   } else {
     return pto_hip::fail(PTO_HIP_ERR_INVALID_VALUE, "quantize_rows_fp8: dtype %s not in {BF16, FP16}",
                          pto_hip::dtype_name(x_dtype));
@@ -920,11 +950,8 @@ extern "C" int pto_hip_ffn_swiglu_fp8(const void* x, const float* gamma, const v
   if (p1.splits > 1) {
     // k split: the quantiser sums the slabs itself, h is not written
     const gemm8::SlabRows sl{p1.slabs, p1.sa, p1.sb0, p1.sb1, tokens * intermediate, p1.splits};
-    const dim3 grid((unsigned)tokens), block(gemm8::kRowThreads);
-    if (bf16)
-      hipLaunchKernelGGL((gemm8::row_quant_kernel<__bf16, false, true>), grid, block, 0, st, nullptr, nullptr, h8, sh, intermediate, 0.f, sl);
-    else
-      hipLaunchKernelGGL((gemm8::row_quant_kernel<_Float16, false, true>), grid, block, 0, st, nullptr, nullptr, h8, sh, intermediate, 0.f, sl);
+    if (bf16) gemm8::launch_row_quant<__bf16, false, true>(nullptr, nullptr, h8, sh, tokens, intermediate, 0.f, sl, st);
+    else gemm8::launch_row_quant<_Float16, false, true>(nullptr, nullptr, h8, sh, tokens, intermediate, 0.f, sl, st);
     PTO_CHECK_HIP(hipGetLastError());
   } else {
     rc = gemm8::row_quant(h, nullptr, false, h8, sh, tokens, intermediate, 0.f, x_dtype, st);

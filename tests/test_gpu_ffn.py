@@ -464,6 +464,35 @@ def test_quantize_rows_fp8_matches_oracle(worker, dtype, rows, cols):
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("cols", [8, 4088, 4096, 4104, 8192, 8200, 12288, 12296, 16384])
+def test_row_quantisers_at_the_edges_of_their_row_lengths(worker, cols, dtype):
+    """One column group short of, at and past what each instantiation holds.  Behind the RMSNorm a value may be an ulp off the oracle's
+    (the order of the sum of squares), which moves a code by at most one: half a code's step and one step, 3 / 16 of the
+    value, or 1.5 steps of the smallest ones, 2^-9 of the scale."""
+    from pypto_amd import _lib
+    from pypto_amd.runtime import _dtype_code
+
+    rows = 5
+    g = torch.Generator().manual_seed(cols)
+    x = torch.randn((rows, cols), generator=g).to(dtype)
+    gamma = torch.rand(cols, generator=g) + 0.5
+    xd, gd = x.cuda(), gamma.cuda()
+    codes, scale = torch.zeros((rows, cols), dtype=torch.uint8, device="cuda"), torch.zeros(rows, device="cuda")
+    _lib.check(_lib.load().pto_hip_quantize_rows_fp8(xd.data_ptr(), codes.data_ptr(), scale.data_ptr(), rows, cols, _dtype_code(dtype), 0))
+    worker.sync()
+    want_codes, want_scale = oracle.quantize_rows_fp8(x)
+    assert torch.equal(scale.cpu(), want_scale) and torch.equal(codes.cpu(), want_codes.view(torch.uint8))
+    _lib.check(_lib.load().pto_hip_rms_norm_quantize_fp8(xd.data_ptr(), gd.data_ptr(), codes.data_ptr(), scale.data_ptr(), rows, cols,
+                                                         1e-6, _dtype_code(dtype), 0))
+    worker.sync()
+    want = oracle.rms_norm(x, gamma, 1e-6, out_dtype=dtype).float()
+    s = scale.cpu()[:, None]
+    assert torch.allclose(s[:, 0], want.abs().amax(dim=1) / 448, rtol=2**-7, atol=0)
+    got = codes.cpu().view(torch.float8_e4m3fn).float() * s
+    assert ((got - want).abs() <= want.abs() * (3 / 16) + 1.5 * 2**-9 * s).all()
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 def test_quantize_rows_fp8_quotients_are_the_divisions(worker, dtype):
     """The quantiser forms y / scale from a refined reciprocal and two remainder corrections instead of a
     division per element.  Every code must still be the one the division gives: rows spanning 16-bit
