@@ -627,9 +627,10 @@ struct SlabRows {
   int64_t mn;                           // rows * cols
   int splits;
 };
-// VECS: groups of eight a thread holds, 2, 4, 6 or 8.  The work on groups a row does not have and the registers they take are
-// what bounded the kernel (both quantisers of the 2048 x 4096 x 11008 block: 278 -> 265 us for the block; 2048 x 4096 bf16 with
-// RMSNorm by itself 11.5 -> 9.6, of which the memory needs 4).
+// VECS: groups of eight a thread holds, 2, 4 or 8.  The work on groups a row does not have and the registers they take are
+// what bounded short rows.  Eight groups always -> now, bf16, with / without RMSNorm, us: 2048 x 4096 11.2 / 9.0 -> 9.2 / 8.0, 4000 x 2048 12.2
+// / 10.1 -> 9.6 / 8.0, 4096 x 8192 28.6 / 21.1 -> 26.5 / 20.5; e4m3 FFN block of 2048 x 4096 x 11008 258.0 -> 256.6.  Six for rows of 8193 to 12288 columns
+// loses: 2048 x 11008 24.0 / 16.5 -> 25.4 / 20.0.
 template <typename TI, bool NORM, bool SLABS, int VECS>
 __global__ __launch_bounds__(kRowThreads) void row_quant_kernel(const TI* __restrict__ x, const float* __restrict__ gamma,
                                                                 uint8_t* __restrict__ codes, float* __restrict__ scale,
@@ -749,7 +750,6 @@ void launch_row_quant(const void* x, const float* gamma, void* codes, float* sca
   const int64_t vecs = (cols / 8 + kRowThreads - 1) / kRowThreads;
   if (vecs <= 2) go(row_quant_kernel<TI, NORM, SLABS, 2>);
   else if (vecs <= 4) go(row_quant_kernel<TI, NORM, SLABS, 4>);
-  else if (vecs <= 6) go(row_quant_kernel<TI, NORM, SLABS, 6>);
   else go(row_quant_kernel<TI, NORM, SLABS, kRowVecs>);
 }
 
