@@ -3,13 +3,15 @@
     python -m pypto_amd.build [--force]
 
 Every ``csrc/*.hip`` is compiled with hipcc for ``--offload-arch=gfx950`` and linked into
-``pypto_amd/lib/libpto_hip.so``; ``pyext/dispatch.cpp`` is host code for torch's Python binding and becomes
-``pypto_amd/lib/_dispatch.so``.  hipcc cross-compiles without a GPU present.
+``pypto_amd/lib/libpto_hip.so``, which needs neither torch nor Python; hipcc cross-compiles without a GPU present.
+``pyext/dispatch.cpp`` is host code for torch's Python binding and becomes ``pypto_amd/lib/_dispatch.so`` afterwards, where
+torch is installed.
 """
 
 from __future__ import annotations
 
 import argparse
+import importlib.util
 import os
 import subprocess
 import sys
@@ -95,14 +97,16 @@ def build(force: bool = False, jobs: int | None = None) -> Path:
     srcs = sources()
     jobs = jobs or min(8, len(srcs))
     with ThreadPoolExecutor(max_workers=jobs) as ex:
-        ext = ex.submit(_build_dispatch, force)
         objs = list(ex.map(lambda s: _compile(s, force), srcs))
-        ext.result()
     if force or _stale(LIB_PATH, objs):
         cmd = [HIPCC, "--offload-arch=gfx950", "-shared", "-fPIC", "-o", str(LIB_PATH), *map(str, objs)]
         r = subprocess.run(cmd, capture_output=True, text=True)
         if r.returncode != 0:
             raise RuntimeError(f"link failed:\n{r.stderr}")
+    if importlib.util.find_spec("torch") is None:
+        sys.stderr.write(f"torch is not installed: {DISPATCH_SRC.name} is left out\n")
+    else:
+        _build_dispatch(force)
     return LIB_PATH
 
 

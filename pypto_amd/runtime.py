@@ -375,9 +375,10 @@ class ChipWorker:
         self._require_ready("register")
         if not isinstance(program, HipProgram):
             raise TypeError(f"register() expects a HipProgram, got {type(program).__name__}")
+        native = _lib.dispatch()  # before the id exists: a binary that does not load leaves none behind
         cid = C.c_int(-1)
         _lib.check(self._lib.pto_hip_register(program.name.encode(), C.byref(cid)))
-        h = RegistrationHandle(self, cid.value, program)
+        h = RegistrationHandle(self, cid.value, program, native)
         self._handles.append(h)
         return h
 
@@ -431,13 +432,13 @@ class ChipWorker:
 class RegistrationHandle:
     """A program registered once on a worker, callable many times (worker.py:675-773)."""
 
-    def __init__(self, worker: ChipWorker, cid: int, program: HipProgram) -> None:
+    def __init__(self, worker: ChipWorker, cid: int, program: HipProgram, native: Any = None) -> None:
         self._worker = worker
         self._cid = cid
         self._program = program
         self._closed = False
         # resident tensors go through native code, which hands everything else back (pyext/dispatch.cpp)
-        self._run = _lib.dispatch().run
+        self._run = native.run if native else None
         self._plain = (_lib.run_address(), cid, bytes(d == HOST for d in program.signature), program.optional,
                        len(program.scalars))
 
@@ -456,7 +457,7 @@ class RegistrationHandle:
     def __call__(self, *args: Any, config: RunConfig | None = None, stream: int = 0) -> None:
         if self._closed:
             raise RuntimeError("RegistrationHandle is closed")
-        status = self._run(*self._plain, args, stream)
+        status = self._run(*self._plain, args, stream) if self._run else None
         if status is None:
             self._worker._dispatch(self._cid, self._program, args, stream)
         elif status:

@@ -1,12 +1,14 @@
 """The native argument side of a program call against the general path's descriptors (CPU: pto_hip_run is a callback)."""
 
 import ctypes as C
+import subprocess
+import sys
 
 import numpy as np
 import pytest
 import torch
 
-from pypto_amd import _lib, runtime
+from pypto_amd import _lib, build, runtime
 
 _RUN = C.CFUNCTYPE(C.c_int, C.c_int, C.POINTER(_lib.ChipTensor), C.c_int, C.POINTER(C.c_uint64), C.c_int, C.c_void_p)
 
@@ -80,3 +82,30 @@ def test_a_tensor_of_a_transform_is_handed_back():
 
     torch.vmap(f)(torch.zeros(3, 4))
     assert seen == [None] and r.calls == []
+
+
+def test_the_library_is_linked_before_and_without_torch(monkeypatch, tmp_path, capsys):
+    order = []
+
+    def link(cmd, **kw):
+        order.append("link")
+        (tmp_path / "libpto_hip.so").write_bytes(b"")
+        return subprocess.CompletedProcess(cmd, 0, "", "")
+
+    def extension(force):
+        order.append("extension")
+        raise RuntimeError("no headers")
+
+    monkeypatch.setattr(build, "OBJ_DIR", tmp_path)
+    monkeypatch.setattr(build, "LIB_PATH", tmp_path / "libpto_hip.so")
+    monkeypatch.setattr(build, "sources", lambda: [tmp_path / "a.hip"])
+    monkeypatch.setattr(build, "_compile", lambda src, force: src)
+    monkeypatch.setattr(build.subprocess, "run", link)
+    monkeypatch.setattr(build, "_build_dispatch", extension)
+    with pytest.raises(RuntimeError, match="no headers"):
+        build.build(force=True)
+    assert order == ["link", "extension"]
+    order.clear()
+    monkeypatch.setitem(sys.modules, "torch", None)
+    assert build.build(force=True) == tmp_path / "libpto_hip.so" and order == ["link"]
+    assert "torch is not installed" in capsys.readouterr().err
