@@ -4,8 +4,8 @@
 
 Every ``csrc/*.hip`` is compiled with hipcc for ``--offload-arch=gfx950`` and linked into
 ``pypto_amd/lib/libpto_hip.so``, which needs neither torch nor Python; hipcc cross-compiles without a GPU present.
-``pyext/dispatch.cpp`` is host code for torch's Python binding and becomes ``pypto_amd/lib/_dispatch.so`` afterwards, where
-torch is installed.
+``pyext/dispatch.cpp`` is host code for torch's Python binding and becomes ``pypto_amd/lib/_dispatch.<Python
+ABI>.torch-<version>.so`` afterwards, where torch is installed.
 """
 
 from __future__ import annotations
@@ -19,6 +19,8 @@ import sysconfig
 from concurrent.futures import ThreadPoolExecutor
 from pathlib import Path
 
+from ._lib import dispatch_path
+
 PKG = Path(__file__).resolve().parent
 CSRC = PKG / "csrc"
 LIB_DIR = PKG / "lib"
@@ -26,7 +28,6 @@ OBJ_DIR = LIB_DIR / "obj"
 LIB_PATH = LIB_DIR / "libpto_hip.so"
 INCLUDE = PKG.parent / "include"
 DISPATCH_SRC = PKG / "pyext" / "dispatch.cpp"
-DISPATCH_PATH = LIB_DIR / "_dispatch.so"
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 CXX = os.environ.get("CXX", "g++")
@@ -77,14 +78,16 @@ def _compile(src: Path, force: bool) -> Path:
 
 
 def _build_dispatch(force: bool) -> None:
-    if not force and not _stale(DISPATCH_PATH, [DISPATCH_SRC, *INCLUDE.glob("*.h")]):
-        return
     import torch
 
+    # named after the Python and the torch it is compiled for: another one's binary is never taken for up to date
+    target = dispatch_path()
+    if not force and not _stale(target, [DISPATCH_SRC, *INCLUDE.glob("*.h")]):
+        return
     root = Path(torch.__file__).resolve().parent
     cmd = [CXX, "-O2", "-std=c++17", "-shared", "-fPIC", "-fvisibility=hidden", f"-I{INCLUDE}",
            f"-I{sysconfig.get_paths()['include']}", f"-I{root / 'include'}", f"-I{root / 'include/torch/csrc/api/include'}",
-           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", str(DISPATCH_SRC), "-o", str(DISPATCH_PATH),
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", str(DISPATCH_SRC), "-o", str(target),
            f"-L{root / 'lib'}", "-ltorch_python", "-ltorch_cpu", "-lc10"]
     r = subprocess.run(cmd, capture_output=True, text=True)
     if r.returncode != 0:

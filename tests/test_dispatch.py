@@ -84,6 +84,17 @@ def test_a_tensor_of_a_transform_is_handed_back():
     assert seen == [None] and r.calls == []
 
 
+def test_the_binary_is_named_after_the_torch_it_reads(monkeypatch):
+    """Another torch's objects are never read through it, and a build for another torch never passes for up to date."""
+    here = _lib.dispatch_path()
+    assert here.exists() and torch.__version__ in here.name
+    monkeypatch.setattr(torch, "__version__", "0.0.0")
+    monkeypatch.setattr(_lib, "_dispatch", None)
+    assert _lib.dispatch_path() != here
+    with pytest.raises(RuntimeError):
+        _lib.dispatch()
+
+
 def test_the_library_is_linked_before_and_without_torch(monkeypatch, tmp_path, capsys):
     order = []
 
