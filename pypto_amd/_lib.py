@@ -10,6 +10,7 @@ from __future__ import annotations
 import ctypes as C
 import importlib.util
 import sysconfig
+import warnings
 from pathlib import Path
 
 LIB_PATH = Path(__file__).resolve().parent / "lib" / "libpto_hip.so"
@@ -177,12 +178,15 @@ def dispatch_path() -> Path:
 
 
 def dispatch():
-    """The native argument side of a program call (pyext/dispatch.cpp), loaded once."""
+    """The native argument side of a program call (pyext/dispatch.cpp), loaded once; None where it is not built
+    (every call then takes the general path, about a microsecond a tensor more)."""
     global _dispatch
     if _dispatch is None:
         path = dispatch_path()
         if not path.exists():
-            raise RuntimeError(f"{path} is not built. Build it with `python -m pypto_amd.build`.")
+            warnings.warn(f"{path.name} is not built, calls go through ctypes. Build it with `python -m pypto_amd.build`.",
+                          RuntimeWarning, stacklevel=2)
+            return None
         spec = importlib.util.spec_from_file_location("pypto_amd._dispatch", path)
         module = importlib.util.module_from_spec(spec)
         spec.loader.exec_module(module)

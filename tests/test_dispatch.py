@@ -91,8 +91,39 @@ def test_the_binary_is_named_after_the_torch_it_reads(monkeypatch):
     monkeypatch.setattr(torch, "__version__", "0.0.0")
     monkeypatch.setattr(_lib, "_dispatch", None)
     assert _lib.dispatch_path() != here
-    with pytest.raises(RuntimeError):
-        _lib.dispatch()
+    with pytest.warns(RuntimeWarning):
+        assert _lib.dispatch() is None
+
+
+class _Library:
+    """Stands for the C library of a worker: counts the ids it hands out."""
+
+    def __init__(self):
+        self.registered = 0
+
+    def pto_hip_register(self, name, out):
+        self.registered += 1
+        return 0
+
+
+def _worker():
+    w = runtime.ChipWorker.__new__(runtime.ChipWorker)
+    w._lib, w._initialized, w._handles, w._owned = _Library(), True, [], {}
+    return w
+
+
+def test_programs_are_called_without_the_binary(monkeypatch, tmp_path):
+    monkeypatch.setattr(_lib, "_dispatch", None)
+    monkeypatch.setattr(_lib, "dispatch_path", lambda: tmp_path / "absent.so")
+    monkeypatch.setattr(_lib, "run_address", lambda: 0)
+    w = _worker()
+    seen = []
+    w._dispatch = lambda cid, program, args, stream: seen.append((program, args, stream))
+    with pytest.warns(RuntimeWarning):
+        h = w.register(runtime.rms_norm)
+    t = torch.zeros(2)
+    h(t, t, t, 1e-5, stream=3)
+    assert seen == [(runtime.rms_norm, (t, t, t, 1e-5), 3)]
 
 
 def test_the_library_is_linked_before_and_without_torch(monkeypatch, tmp_path, capsys):
