@@ -375,9 +375,10 @@ class ChipWorker:
         self._require_ready("register")
         if not isinstance(program, HipProgram):
             raise TypeError(f"register() expects a HipProgram, got {type(program).__name__}")
+        native = _lib.dispatch()  # before the id exists: a binary that does not load leaves none behind
         cid = C.c_int(-1)
         _lib.check(self._lib.pto_hip_register(program.name.encode(), C.byref(cid)))
-        h = RegistrationHandle(self, cid.value, program, _lib.dispatch())
+        h = RegistrationHandle(self, cid.value, program, native)
         self._handles.append(h)
         return h
 

@@ -126,6 +126,17 @@ def test_programs_are_called_without_the_binary(monkeypatch, tmp_path):
     assert seen == [(runtime.rms_norm, (t, t, t, 1e-5), 3)]
 
 
+def test_a_binary_that_does_not_load_leaves_no_program_registered(monkeypatch, tmp_path):
+    broken = tmp_path / "broken.so"
+    broken.write_bytes(b"no library")
+    monkeypatch.setattr(_lib, "_dispatch", None)
+    monkeypatch.setattr(_lib, "dispatch_path", lambda: broken)
+    w = _worker()
+    with pytest.raises(ImportError):
+        w.register(runtime.rms_norm)
+    assert w._lib.registered == 0 and w._handles == []
+
+
 def test_the_library_is_linked_before_and_without_torch(monkeypatch, tmp_path, capsys):
     order = []
 
