@@ -1,12 +1,13 @@
 """Rules the kernel sources keep (CPU: they are read and checked by the compiler, nothing runs)."""
 
 import re
+import struct
 import subprocess
 from pathlib import Path
 
 import pytest
 
-from pypto_amd import build
+from pypto_amd import _lib, build
 
 CSRC = Path(__file__).resolve().parent.parent / "pypto_amd" / "csrc"
 _ASM = re.compile(r"asm volatile\(((?:\s*\"(?:[^\"\\]|\\.)*\")+)")
@@ -42,3 +43,31 @@ def test_slab_sums_keep_the_alignment_of_their_sources(name):
                         "-Werror=align-mismatch", f"-I{build.INCLUDE}", f"-I{CSRC}", str(CSRC / name)],
                        capture_output=True, text=True)
     assert r.returncode == 0, r.stderr
+
+
+def _registers(pattern: str, tmp_path) -> dict[str, int]:
+    """Vector registers of the built kernels whose mangled name matches, from the notes of the library's code objects."""
+    data, magic, found = _lib.LIB_PATH.read_bytes(), b"__CLANG_OFFLOAD_BUNDLE__", {}
+    at = data.find(magic)
+    while at >= 0:
+        (entries,), pos = struct.unpack_from("<Q", data, at + len(magic)), at + len(magic) + 8
+        for _ in range(entries):
+            offset, size, length = struct.unpack_from("<QQQ", data, pos)
+            target, pos = data[pos + 24:pos + 24 + length], pos + 24 + length
+            code = data[at + offset:at + offset + size]
+            if b"gfx950" in target and re.search(pattern.encode(), code):
+                (tmp_path / "code.elf").write_bytes(code)
+                notes = subprocess.run([str(Path(build.HIPCC).parent.parent / "llvm/bin/llvm-readelf"), "--notes", str(tmp_path / "code.elf")],
+                                       capture_output=True, text=True, check=True).stdout
+                for name, count in re.findall(r"\.name:\s+(\S+)[\s\S]*?\.vgpr_count:\s+(\d+)", notes):
+                    if re.search(pattern, name):
+                        found[name] = int(count)
+        at = data.find(magic, at + 1)
+    return found
+
+
+@pytest.mark.parametrize("head_dim", [128, 256])
+def test_the_merge_of_few_partitions_leaves_room_for_eight_wavefronts_per_simd(head_dim, tmp_path):
+    """Its launches have thousands of rows; the registers of the path for many partitions must not be charged to it."""
+    found = _registers(f"attn_reduce_kernelILi{head_dim}E", tmp_path)
+    assert found and min(found.values()) <= 64, found
