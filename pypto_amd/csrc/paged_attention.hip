@@ -717,13 +717,12 @@ __global__ __launch_bounds__(64) void attn_partition_kernel(AttnParams p) {
 // Merge of the per-partition (m, l, o): the online-update algebra of
 // examples/models/04_paged_attention.py:186-215 applied across partitions, then o / l.
 // One wavefront per output row.  What bounds it is the chain of memory round trips: one up to 8 partitions, above that one for
-// the first 16 and less than one for every 16 more.  FEW: launches of up to kReduceFast partitions, a kernel of its own: beside the
-// other path's two batches of partials it would hold 132 registers instead of 50 (head_dim 256: 226 instead of 64), two or three
+// the context length, one for the first BATCH partials and less than one for every BATCH more.  BATCH 0: launches of up to kReduceFast partitions, a kernel
+// of its own: beside the other path's two batches of partials (16 then) it held 132 registers instead of 50 (head_dim 256: 226 instead of 64), two or three
 // wavefronts per SIMD instead of eight.  Attention call of 128 sequences, 32 heads on one KV head, one kernel for both -> two, us: 16-bit
 // cache of 1024 tokens 30.3 -> 29.0, of 64 to 4096 42.7 -> 38.0, e4m3 27.9 -> 25.5 and 45.2 -> 36.1.
-constexpr int kReduceFast = 8;    // most partitions of the path without a loop
-constexpr int kReduceBatch = 16;  // partials requested together above
-template <int D, bool FEW>
+constexpr int kReduceFast = 8;  // most partitions of the path without a loop
+template <int D, int BATCH>
 __global__ __launch_bounds__(256) void attn_reduce_kernel(AttnParams p) {
   const int lane = threadIdx.x & 63;
   const int row = blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);  // b*Hq + query head
@@ -735,7 +734,7 @@ __global__ __launch_bounds__(256) void attn_reduce_kernel(AttnParams p) {
   const int np = (ctx + p.tpp - 1) / p.tpp;
   const float* ml = p.part_ml + (size_t)row * p.n_part * 2;
   const float* po = p.part_o + (size_t)row * p.n_part * D;
-  if constexpr (FEW) {
+  if constexpr (BATCH == 0) {
     // Few partitions: every slot the row could use is fetched at once, before the context length
     // is known, so the launch is one memory round trip instead of three; slots past np (never
     // written, or stale) are dropped by select, not by a zero weight.
@@ -781,17 +780,19 @@ __global__ __launch_bounds__(256) void attn_reduce_kernel(AttnParams p) {
     }
     return;
   }
-  // Lane i holds (m, l) of partitions i, i + 64, ...  The first of them and the first batch of partials are requested before
-  // the context length is known, every further batch before the one in front of it is summed; what slots past np hold is
-  // dropped by select.
-  float pv[2][kReduceBatch][D / 64];
+  // Lane i holds (m, l) of partitions i, i + 64, ...  Every batch of partials is requested before the one in front of it is summed.
+  // Slots past the row's own partitions repeat its last one, a line that is asked for anyway, and are dropped by select: all slots asked for before
+  // the length is known cost the other rows' bandwidth (100 sequences of 16 to 2500 tokens, 32 heads on one KV head at head_dim 256, 50.5 -> 49.3 us).
+  constexpr int kBatch = BATCH == 0 ? 1 : BATCH;  // (not instantiated past the return above)
+  const int last = max(np - 1, 0);
+  float pv[2][kBatch][D / 64];
   auto fetch = [&](int set, int first) {
 #pragma unroll
-    for (int u = 0; u < kReduceBatch; ++u)
+    for (int u = 0; u < kBatch; ++u)
 #pragma unroll
-      for (int k = 0; k < D / 64; ++k) pv[set][u][k] = po[(size_t)min(first + u, p.n_part - 1) * D + k * 64 + lane];
+      for (int k = 0; k < D / 64; ++k) pv[set][u][k] = po[(size_t)min(first + u, last) * D + k * 64 + lane];
   };
-  float2 own = *reinterpret_cast<const float2*>(ml + 2 * min(lane, p.n_part - 1));
+  float2 own = *reinterpret_cast<const float2*>(ml + 2 * min(lane, last));
   fetch(0, 0);
   float m = lane < np ? own.x : kMinMax;
   for (int i = lane + 64; i < np; i += 64) m = fmaxf(m, ml[2 * i]);
@@ -801,22 +802,22 @@ __global__ __launch_bounds__(256) void attn_reduce_kernel(AttnParams p) {
 #pragma unroll
   for (int k = 0; k < D / 64; ++k) o[k] = 0.f;
   for (int base = 0; base < np; base += 64) {
-    if (base > 0) own = *reinterpret_cast<const float2*>(ml + 2 * min(base + lane, p.n_part - 1));
+    if (base > 0) own = *reinterpret_cast<const float2*>(ml + 2 * min(base + lane, last));
     const float wgt = base + lane < np ? __builtin_amdgcn_exp2f(own.x - m) : 0.f;
     l += base + lane < np ? wgt * own.y : 0.f;
     auto add = [&](int set, int first) {
 #pragma unroll
-      for (int u = 0; u < kReduceBatch; ++u) {
+      for (int u = 0; u < kBatch; ++u) {
         const float w = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, wgt), (first + u) & 63));
 #pragma unroll
         for (int k = 0; k < D / 64; ++k) o[k] = first + u < np ? o[k] + w * pv[set][u][k] : o[k];
       }
     };
-    for (int first = base; first < min(base + 64, np); first += 2 * kReduceBatch) {
-      if (first + kReduceBatch < np) fetch(1, first + kReduceBatch);
+    for (int first = base; first < min(base + 64, np); first += 2 * kBatch) {
+      if (first + kBatch < np) fetch(1, first + kBatch);
       add(0, first);
-      if (first + 2 * kReduceBatch < np) fetch(0, first + 2 * kReduceBatch);
-      if (first + kReduceBatch < np) add(1, first + kReduceBatch);
+      if (first + 2 * kBatch < np) fetch(0, first + 2 * kBatch);
+      if (first + kBatch < np) add(1, first + kBatch);
     }
   }
 #pragma unroll
@@ -1344,11 +1345,19 @@ int launch(const AttnParams& p, int batch, bool bf16, hipStream_t stream) {
   }
   if (rc) return rc;
   if (p.n_part > 1) {
-    // a workgroup per row as far as that gives every row a CU of its own
-    const int rows = batch * p.hq, per_wg = rows <= pto_hip::ctx().num_cu ? 1 : 4;
-    const dim3 rgrid((unsigned)((rows + per_wg - 1) / per_wg)), rblock((unsigned)per_wg * 64);
-    if (p.n_part <= kReduceFast) hipLaunchKernelGGL((attn_reduce_kernel<D, true>), rgrid, rblock, 0, stream, p);
-    else hipLaunchKernelGGL((attn_reduce_kernel<D, false>), rgrid, rblock, 0, stream, p);
+    // Up to 8 partitions a workgroup per row as far as that gives every row a CU of its own (128 rows, 4 partitions 7.46 -> 7.20 us a call, head_dim 256
+    // 9.35 -> 8.93; level from 384 rows on).  Above: for a few rows the longest batches and a workgroup each (8 rows of 47 partitions, batches of
+    // 16 / 8 8.9 / 9.2 us, 32 rows level); then 4 rows to a workgroup and batches of 8 (256 rows of 16 partitions 13.7 -> 13.0 us against one each, 2048
+    // rows of up to 16 26.7 -> 26.5 against batches of 16); many rows want the wavefronts per SIMD that batches of 4 leave room
+    // for (6400 rows of up to 11, 16 / 8 / 4 48.1 / 46.3 / 45.6, at head_dim 256 3200 rows of up to 10 49.3 / 47.4 / 46.2).
+    const int rows = batch * p.hq;
+    auto merge = [&](auto kern, int per_wg) {
+      hipLaunchKernelGGL(kern, dim3((unsigned)((rows + per_wg - 1) / per_wg)), dim3((unsigned)per_wg * 64), 0, stream, p);
+    };
+    if (p.n_part <= kReduceFast) merge(attn_reduce_kernel<D, 0>, rows <= pto_hip::ctx().num_cu ? 1 : 4);
+    else if (rows <= 32) merge(attn_reduce_kernel<D, 16>, 1);
+    else if ((int64_t)rows * D <= (1 << 19)) merge(attn_reduce_kernel<D, 8>, 4);
+    else merge(attn_reduce_kernel<D, 4>, 4);
     PTO_CHECK_HIP(hipGetLastError());
   }
   return PTO_HIP_OK;

@@ -86,6 +86,17 @@ def test_merge_of_many_partitions(worker, most, d, hq):
     validate_golden({"out": got}, {"out": _golden(inp)}, rtol=RTOL, atol=ATOL)
 
 
+@pytest.mark.parametrize("d,hq,batch", [(128, 8, 4), (128, 64, 66), (256, 8, 4), (256, 32, 66)])
+def test_merge_of_many_partitions_by_rows(worker, d, hq, batch):
+    """The merge's kernels for at most 32 rows and for those beyond 2^19 / head_dim, at the edges of their batches."""
+    counts = [33, 0, 17, 9, 8, 7, 5, 4, 3, 1, 16, 31, 32]
+    inp = workloads.paged_attention_inputs(batch=batch, num_heads=hq, kv_head_num=1, head_dim=d, block_size=32,
+                                           context_lens=[max(0, 32 * counts[i % 13] - i % 3) for i in range(batch)],
+                                           ctx_range=(1, 32 * 33), seed=batch + d)
+    got = _run(worker, inp, 0, 32)
+    validate_golden({"out": got}, {"out": _golden(inp)}, rtol=RTOL, atol=ATOL)
+
+
 @pytest.mark.parametrize("fp8", [False, True])
 @pytest.mark.parametrize("bs,ctxs", [(128, [1531]), (256, [63, 2000]), (128, [64, 65, 700]), (192, [500, 96])])
 def test_few_pairs_cut_inside_blocks(worker, bs, ctxs, fp8):

@@ -71,3 +71,11 @@ def test_the_merge_of_few_partitions_leaves_room_for_eight_wavefronts_per_simd(h
     """Its launches have thousands of rows; the registers of the path for many partitions must not be charged to it."""
     found = _registers(f"attn_reduce_kernelILi{head_dim}E", tmp_path)
     assert found and min(found.values()) <= 64, found
+
+
+@pytest.mark.parametrize("head_dim", [128, 256])
+def test_the_merge_of_many_rows_leaves_room_for_five_wavefronts_per_simd(head_dim, tmp_path):
+    """Thousands of rows of more partitions: a kernel that holds two batches of four partials, not of sixteen (512 registers
+    over five wavefronts, in granules of eight)."""
+    found = _registers(f"attn_reduce_kernelILi{head_dim}ELi4E", tmp_path)
+    assert len(found) == 1 and max(found.values()) <= 96, found
