@@ -103,20 +103,42 @@ inline int64_t attn_e4m3_partition_tokens(int64_t pairs, int64_t max_ctx, int64_
   return (max_ctx + parts - 1) / parts;
 }
 
-// What partition lengths are multiples of: the KV block (`block`, or its part that divides a long one), halved down to 64
-// tokens while the table's blocks give fewer than two wavefronts per CU.  A launch of a few pairs is a chain - table, first rows, a
-// chunk of 32 tokens after the other - that halves are two chunks shorter than whole 128-token blocks.  Attention call, us, whole
-// blocks -> halves: 8 pairs x 1531 tokens 10.4 -> 8.9, x 700 10.5 -> 9.1, x 300 7.8 -> 7.2, 32 x 1531 11.8 -> 10.8; blocks of 256: 8 x 2000
-// 13.9 -> 10.8, 24 x 1100 12.8 -> 10.4.  Down to 32 tokens gains nothing more and costs where wavefronts carry several
-// query tiles (3 x 3000 10.8 -> 14.4, head_dim 256 22.4 -> 30.0), up to four wavefronts per CU nothing (64 x 900 11.0 -> 11.4).
-// bytes_per_part, scratch: as above.
-inline int64_t attn_partition_align(int64_t pairs, int64_t max_ctx, int64_t block, int64_t num_cu, int64_t bytes_per_part, int64_t scratch) {
-  while (block >= 128 && block % 64 == 0) {
-    const int64_t parts = (max_ctx + block - 1) / block;
-    if (pairs * parts >= 2 * num_cu || 2 * parts * bytes_per_part > scratch) break;
-    block /= 2;
+// What partition lengths are multiples of: the KV block (`block`, or its part that divides a long one) or a half, quarter ... of it down to 64
+// tokens.  A launch of a few pairs is a chain - table, first rows, a chunk of 32 tokens after the other - that halves are two
+// chunks shorter than whole 128-token blocks; what they cost is another partial per query row (written, read by the merge) and, from one
+// partition to two, the merge itself.  So a partition is halved as far as the wavefronts it gives leave that hidden, by the `weight` of a partial beside its
+// part of the cache: query rows per KV head (`rows`, as far as one wavefront carries them) against the length, squared since a short
+// partition is also the shorter chain.  Measured against whole blocks and every halving at 2 to 250 pairs, tables of 1 to 24
+// blocks of 128, 256 and 512 tokens, 1 to 64 query heads per KV head, equal and ragged lengths (3828 calls, whole blocks -> this rule):
+// -14.1 % on average, 27 calls more than 3 % slower, by 6 % at most; 0.8 % behind the best of each.  Us, whole blocks -> halved:
+// one partition: 64 pairs x 384 of a 512-token block, 16 heads 14.1 -> 12.5, quarters 9.1, but 8 x 96 of a 128-token block 6.1 -> 6.9 (kept whole);
+// two, the four of which a workgroup's wavefronts can merge (head_dim 256 with few heads only as far as CUs idle): 160 x 224, 16 heads 9.2 -> 8.0;
+// more: 8 x 1504, 16 heads 10.7 -> 9.8; but 96 x 480, 32 heads 12.2 -> 19.6, 8 heads at head_dim 256 16.2 -> 18.7 (kept whole).
+// Halves as long as the table's blocks gave fewer than two wavefronts per CU, whatever the rows, as before: -11.1 % on average, 729 calls more than
+// 3 % slower, by up to 88 %.
+// `wg_parts` > 0: the workgroup form is asked for, which up to that many partitions stay within.  bytes_per_part, scratch: as above.
+inline int64_t attn_partition_align(int64_t pairs, int64_t max_ctx, int64_t block, int64_t num_cu, int64_t bytes_per_part, int64_t scratch,
+                                    int64_t rows = 1, int64_t head_dim = 128, bool e4m3 = false, int64_t wg_parts = 0) {
+  const bool long_rows = head_dim * (e4m3 ? 1 : 2) > 256;  // of the cache: more of the time is its stream
+  const bool short_rows = e4m3 && head_dim == 128 && rows <= 16;
+  int64_t align = block;
+  for (int64_t len = block; len >= 128 && len % 64 == 0; len /= 2) {
+    const int64_t parts = (max_ctx + len - 1) / len;
+    if (2 * parts * bytes_per_part > scratch || (parts <= wg_parts && 2 * parts > wg_parts)) break;
+    const double weight = (double)(rows * head_dim) / 128.0 * (128.0 / (double)len) * (128.0 / (double)len);
+    int quarters;  // wavefronts up to which a partition is halved, in quarters of the CUs
+    if (parts == 1) quarters = weight <= 4.0 ? 4 : 0;
+    else if (parts == 2) quarters = long_rows && rows < 8 && len <= 128 ? 3 : 8;
+    else if (parts <= 4 && short_rows) quarters = 8;  // (eight of which a workgroup can merge)
+    else if (weight >= 16.0) quarters = short_rows ? 3 : 2;
+    else if (weight > 4.0) quarters = e4m3 && rows <= 8 ? 4 : 3;
+    else if (len <= 128) quarters = short_rows ? 6 : long_rows ? 3 : 4;
+    else if (long_rows) quarters = 4;
+    else quarters = weight <= (e4m3 ? 2.0 : 1.0) ? 6 : 5;
+    if (pairs * parts * 4 <= quarters * num_cu && pairs * parts < 2 * num_cu) align = len / 2;
+    else if (parts > 1) break;  // (one partition: four can still be ahead where two are not)
   }
-  return block;
+  return align;
 }
 
 }  // namespace pto_hip

@@ -1348,14 +1348,14 @@ int launch(const AttnParams& p, int batch, bool bf16, hipStream_t stream) {
     // Up to 8 partitions a workgroup per row as far as that gives every row a CU of its own (128 rows, 4 partitions 7.46 -> 7.20 us a call, head_dim 256
     // 9.35 -> 8.93; level from 384 rows on).  Above: for a few rows the longest batches and a workgroup each (8 rows of 47 partitions, batches of
     // 16 / 8 8.9 / 9.2 us, 32 rows level); then 4 rows to a workgroup and batches of 8 (256 rows of 16 partitions 13.7 -> 13.0 us against one each, 2048
-    // rows of up to 16 26.7 -> 26.5 against batches of 16); many rows want the wavefronts per SIMD that batches of 4 leave room
+    // rows of up to 16 26.7 -> 26.5 against batches of 16; up to 256 rows of more than 32 partitions the long ones, 64 of 163 20.6 -> 18.8); many rows want the wavefronts per SIMD that batches of 4 leave room
     // for (6400 rows of up to 11, 16 / 8 / 4 48.1 / 46.3 / 45.6, at head_dim 256 3200 rows of up to 10 49.3 / 47.4 / 46.2).
     const int rows = batch * p.hq;
     auto merge = [&](auto kern, int per_wg) {
       hipLaunchKernelGGL(kern, dim3((unsigned)((rows + per_wg - 1) / per_wg)), dim3((unsigned)per_wg * 64), 0, stream, p);
     };
     if (p.n_part <= kReduceFast) merge(attn_reduce_kernel<D, 0>, rows <= pto_hip::ctx().num_cu ? 1 : 4);
-    else if (rows <= 32) merge(attn_reduce_kernel<D, 16>, 1);
+    else if (rows <= 32 || (rows <= pto_hip::ctx().num_cu && p.n_part > 32)) merge(attn_reduce_kernel<D, 16>, 1);
     else if ((int64_t)rows * D <= (1 << 19)) merge(attn_reduce_kernel<D, 8>, 4);
     else merge(attn_reduce_kernel<D, 4>, 4);
     PTO_CHECK_HIP(hipGetLastError());
@@ -1521,7 +1521,9 @@ int plan_launch(const int64_t* config, int q_dtype, int kv_dtype, bool have_scal
   int64_t tpp = cx.attn_tokens_per_partition;
   if (tpp <= 0) {
     const int64_t units = batch * hkv * p.gtiles;
-    align = pto_hip::attn_partition_align(units, max_ctx, align, cx.num_cu, batch * hq * (d + 2) * 4, PTO_HIP_NOALLOC_SCRATCH_BYTES);
+    // (from the whole table: a launch's own bound on the blocks then moves no partition, and its result is that of clipped lengths)
+    align = pto_hip::attn_partition_align(units, max_blocks * bs, align, cx.num_cu, batch * hq * (d + 2) * 4, PTO_HIP_NOALLOC_SCRATCH_BYTES,
+                                          std::min(p.group, p.gt_rows), d, fp8, cx.attn_variant == 2 ? wg_max_parts((int)d, gt) : 0);
     // With a (sequence, head) pair or more per CU the launch takes the workgroup form (see
     // paged_attention below), where two wavefronts per CU measured best (decoder layer, 32 sequences
     // of 4096 tokens: 182.5 us a step against 184.0 with four).  A wavefront that carries several

@@ -19,6 +19,9 @@ extern "C" void choose_quad(int m, int n, int k, int dual, int64_t num_cu, int f
 extern "C" int64_t partition_align(int64_t pairs, int64_t max_ctx, int64_t block, int64_t bytes_per_part, int64_t scratch) {
   return pto_hip::attn_partition_align(pairs, max_ctx, block, 256, bytes_per_part, scratch);
 }
+extern "C" int64_t partition_align_shape(int64_t pairs, int64_t max_ctx, int64_t block, int64_t rows, int64_t head_dim, int e4m3, int64_t wg_parts) {
+  return pto_hip::attn_partition_align(pairs, max_ctx, block, 256, pairs * rows * (head_dim + 2) * 4, 32 << 20, rows, head_dim, e4m3 != 0, wg_parts);
+}
 extern "C" int64_t e4m3_partition(int64_t pairs, int64_t max_ctx, int64_t bytes_per_part, int64_t scratch, int64_t plain) {
   return pto_hip::attn_e4m3_partition_tokens(pairs, max_ctx, 256, 8, bytes_per_part, scratch, plain);
 }
@@ -37,6 +40,8 @@ def choice(tmp_path_factory):
     lib.e4m3_partition.restype = lib.partition_align.restype = C.c_int64
     lib.partition_align.argtypes = [C.c_int64] * 5
     lib.e4m3_partition.argtypes = [C.c_int64] * 5
+    lib.partition_align_shape.restype = C.c_int64
+    lib.partition_align_shape.argtypes = [C.c_int64] * 5 + [C.c_int, C.c_int64]
     return lib
 
 
@@ -139,3 +144,24 @@ def test_partition_alignment_divides_the_block(choice):
                     if align != block:
                         parts = -(-max_ctx // (2 * align))
                         assert align >= 64 and align % 32 == 0 and pairs * parts < 512 and 2 * parts * per_part <= scratch
+
+
+@pytest.mark.parametrize("pairs,tokens,block,rows,d,e4m3,want", [
+    (8, 1536, 128, 4, 128, False, 64), (8, 1536, 128, 16, 128, False, 64), (8, 768, 128, 4, 128, False, 64),
+    (160, 256, 128, 16, 128, False, 64), (128, 256, 128, 32, 128, True, 64), (64, 512, 512, 16, 128, False, 128), (8, 256, 256, 64, 128, False, 64),
+    # a second partial per row costs more than the shorter chain gives
+    (8, 128, 128, 16, 128, False, 128), (200, 128, 128, 32, 128, False, 128), (100, 512, 128, 8, 256, False, 128), (96, 512, 128, 32, 128, False, 128),
+    (160, 384, 128, 32, 128, False, 128), (160, 384, 128, 16, 256, True, 128), (16, 3072, 128, 16, 256, False, 128), (200, 256, 128, 4, 256, False, 128)])
+def test_partitions_are_cut_where_the_partials_cost_less_than_the_chain(choice, pairs, tokens, block, rows, d, e4m3, want):
+    """Calls that measured 5 % or more ahead with the partition length given here."""
+    assert choice.partition_align_shape(pairs, tokens, block, rows, d, int(e4m3), 0) == want
+
+
+@pytest.mark.parametrize("d,most", [(128, 8), (256, 4)])
+def test_partition_alignment_stays_within_the_workgroup_form(choice, d, most):
+    """Asked for, that form is kept wherever whole blocks allow it: no cut takes the count past its wavefronts."""
+    for pairs in (1, 8, 100, 255):
+        for blocks in range(1, 24):
+            for block in (64, 128, 256, 512):
+                align = choice.partition_align_shape(pairs, blocks * block, block, 8, d, 0, most)
+                assert blocks > most or blocks * block // align <= most
