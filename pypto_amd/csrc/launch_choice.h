@@ -86,20 +86,26 @@ inline void choose_quad(int m, int n, int k, bool dual, int64_t num_cu, int forc
 // wavefronts take the partitions) over an e4m3 cache at head_dim 128; `plain` is the rule for 16-bit caches, two wavefronts per
 // CU and at most 2048 tokens.  A chunk of codes is half the bytes of a 16-bit one, so two wavefronts do not keep enough requests in
 // flight, and a partition of 2048 tokens is what the launch waits for when lengths are ragged: from tables of more than 1536
-// tokens on four wavefronts per CU, partitions of equal length, of 512 to 1024 tokens.  Attention call, us, tables for
+// tokens on four wavefronts per CU, partitions of equal length: of 512 to 1024 tokens but for whole blocks (416 of a 1568-token table of 32-token
+// ones) and max_parts (1536 of a 12000-token table).  Attention call, us, tables for
 // (pairs x tokens) with equal / ragged lengths: 256 x 4096 63.0 / 61.4 -> 42.6 / 34.4, 320 x 2200 49.9 / 48.0 -> 34.1 / 30.0, 768 x 3000
-// 120 / 70.4 -> 98 / 69, 1280 x 2000 108.2 / 81.9 -> 107.6 / 76.9, 272 x 14000 168 / 148 -> 165 / 106, 512 x 6000 128 -> 129; but one partition split, 1024 x 1400
-// 56.2 -> 59.7, hence 1536.  16-bit caches are the other way round: 768 x 3000 113.9 ragged -> 119, 256 x 4096 equal 80.7 -> 82.6.
+// 120 / 70.4 -> 98 / 69; but one partition split, 1024 x 1400 56.2 -> 59.7, hence 1536.  16-bit caches are the other way round: 768 x 3000 113.9 ragged
+// -> 119, 256 x 4096 equal 80.7 -> 82.6.  The plain rule stays where its own wavefronts fill the CUs as well, lengths equal / down to half / to a tenth:
+// from four partitions on (plain -> more: 320 x 8000 108 / 85 / 79 -> 119 / 100 / 78), between 3.5 and 6 times 2048 tokens per CU (320 x 6000
+// 80 / 69 / 66 -> 88 / 75 / 56, 800 x 2600 96 / 75 / 70 -> 99 / 82 / 65; below they are ahead, 512 x 3500 81 / 72 / 66 -> 78 / 65 / 51, and above, 1600 x 3500
+// 263 / 198 / 159 -> 250 / 190 / 149), and for one partition of four pairs per CU (1600 x 2000 143 / 119 / 96 -> 150 / 119 / 92).
 // Not more partitions than a workgroup has wavefronts (max_parts: the form needs no scratch), nor than whose partials, should the grid
 // form be taken after all, fit the fixed area of the entry point that allocates nothing.
 inline int64_t attn_e4m3_partition_tokens(int64_t pairs, int64_t max_ctx, int64_t num_cu, int64_t max_parts, int64_t bytes_per_part,
                                           int64_t scratch, int64_t plain) {
   if (max_ctx <= 1536) return plain;
+  const int64_t before = (max_ctx + plain - 1) / plain, load = pairs * max_ctx / 2048;
+  if (before >= 4 || (2 * load > 7 * num_cu && load < 6 * num_cu) || (before == 1 && pairs >= 4 * num_cu)) return plain;
   const int64_t want = std::max<int64_t>(1, (4 * num_cu + pairs - 1) / pairs);
   const int64_t tokens = std::min<int64_t>(1024, std::max<int64_t>(512, (max_ctx + want - 1) / want));
   int64_t parts = std::min((max_ctx + tokens - 1) / tokens, max_parts);
   parts = std::min(parts, scratch / bytes_per_part);
-  if (parts <= (max_ctx + plain - 1) / plain) return plain;
+  if (parts <= before) return plain;
   return (max_ctx + parts - 1) / parts;
 }
 

@@ -1348,7 +1348,7 @@ int launch(const AttnParams& p, int batch, bool bf16, hipStream_t stream) {
     // Up to 8 partitions a workgroup per row as far as that gives every row a CU of its own (128 rows, 4 partitions 7.46 -> 7.20 us a call, head_dim 256
     // 9.35 -> 8.93; level from 384 rows on).  Above: for a few rows the longest batches and a workgroup each (8 rows of 47 partitions, batches of
     // 16 / 8 8.9 / 9.2 us, 32 rows level); then 4 rows to a workgroup and batches of 8 (256 rows of 16 partitions 13.7 -> 13.0 us against one each, 2048
-    // rows of up to 16 26.7 -> 26.5 against batches of 16; up to 256 rows of more than 32 partitions the long ones, 64 of 163 20.6 -> 18.8); many rows want the wavefronts per SIMD that batches of 4 leave room
+    // rows of up to 16 26.7 -> 26.5 against batches of 16; up to 256 rows of more than 32 partitions the long ones, 64 of 163 20.6 -> 19.0); many rows want the wavefronts per SIMD that batches of 4 leave room
     // for (6400 rows of up to 11, 16 / 8 / 4 48.1 / 46.3 / 45.6, at head_dim 256 3200 rows of up to 10 49.3 / 47.4 / 46.2).
     const int rows = batch * p.hq;
     auto merge = [&](auto kern, int per_wg) {
