@@ -1449,8 +1449,9 @@ namespace {
 // load-only probe, so that both walk the cache in the same pieces.
 // active_blocks >= 0 bounds the KV loop of every sequence to that many blocks, as the SPMD form's
 // config slot does (09_paged_attention_spmd.py:482: max_bn = min(max_bn, active_block_num)); < 0: no bound.
+// whole_blocks: no partition is cut inside a block for the sake of a shorter chain.
 int plan_launch(const int64_t* config, int q_dtype, int kv_dtype, bool have_scales, int64_t active_blocks,
-                AttnParams& p, int& gt, bool& lean) {
+                AttnParams& p, int& gt, bool& lean, bool whole_blocks = false) {
   pto_hip::Context& cx = pto_hip::ctx();
   using pto_hip::dtype_name;
   using pto_hip::fail;
@@ -1522,8 +1523,9 @@ int plan_launch(const int64_t* config, int q_dtype, int kv_dtype, bool have_scal
   if (tpp <= 0) {
     const int64_t units = batch * hkv * p.gtiles;
     // (from the whole table: a launch's own bound on the blocks then moves no partition, and its result is that of clipped lengths)
-    align = pto_hip::attn_partition_align(units, max_blocks * bs, align, cx.num_cu, batch * hq * (d + 2) * 4, PTO_HIP_NOALLOC_SCRATCH_BYTES,
-                                          std::min(p.group, p.gt_rows), d, fp8, cx.attn_variant == 2 ? wg_max_parts((int)d, gt) : 0);
+    if (!whole_blocks)
+      align = pto_hip::attn_partition_align(units, max_blocks * bs, align, cx.num_cu, batch * hq * (d + 2) * 4, PTO_HIP_NOALLOC_SCRATCH_BYTES,
+                                            std::min(p.group, p.gt_rows), d, fp8, cx.attn_variant == 2 ? wg_max_parts((int)d, gt) : 0);
     // With a (sequence, head) pair or more per CU the launch takes the workgroup form (see
     // paged_attention below), where two wavefronts per CU measured best (decoder layer, 32 sequences
     // of 4096 tokens: 182.5 us a step against 184.0 with four).  A wavefront that carries several
@@ -1696,17 +1698,7 @@ int paged_attention(const void* query, const void* key_cache, const void* value_
   const bool bf16 = q_dtype == PTO_HIP_BF16;
   // Where the partition partials live: the caller's fixed area (never grown) or the workspace.
   auto partials_area = [&](size_t bytes, void** ws) -> int {
-    if (!fixed_scratch) {
-      // Room for every launch of a few pairs (attn_partition_align), some of which have more partials than ones with more
-      // pairs: what a call was sized for once also fits a smaller batch under capture.
-      size_t ask = std::max(bytes, (size_t)(4 * cx.num_cu) * p.gt_rows * (d + 2) * sizeof(float));
-      if (ask > cx.workspace_bytes) {
-        hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
-        if (hipStreamIsCapturing((hipStream_t)stream, &capturing) != hipSuccess) (void)hipGetLastError();
-        if (capturing != hipStreamCaptureStatusNone) ask = bytes;
-      }
-      return workspace(ask, ws);
-    }
+    if (!fixed_scratch) return workspace(bytes, ws);
     if (bytes > fixed_scratch_bytes)
       return fail(PTO_HIP_ERR_INVALID_VALUE,
                   "paged_attention_noalloc: this launch needs %zu bytes of partition partials, the fixed scratch "
@@ -1720,8 +1712,36 @@ int paged_attention(const void* query, const void* key_cache, const void* value_
   // workgroup from the (sequence, KV head, query tile) pairs alone; "attn_variant" 2 asks for it
   // whenever the partition count allows.
   const int64_t pairs = batch * hkv * p.gtiles;
-  const bool wg_possible = !lean && p.n_part > 1 && p.n_part <= wg_max_parts((int)d, gt);
-  p.wg_merge = wg_possible && (cx.attn_variant == 2 || (cx.attn_variant < 0 && pairs >= cx.num_cu));
+  bool wg_possible = false;
+  auto choose_form = [&] {
+    wg_possible = !lean && p.n_part > 1 && p.n_part <= wg_max_parts((int)d, gt);
+    p.wg_merge = wg_possible && (cx.attn_variant == 2 || (cx.attn_variant < 0 && pairs >= cx.num_cu));
+  };
+  choose_form();
+  if (!fixed_scratch) {
+    // A call leaves room for the partials of every smaller batch with its heads and table, whatever form it takes itself, since the workspace cannot
+    // grow while a graph is recorded: below a pair per CU pairs * partitions stay under five wavefronts per CU, or, past the 2048 tokens that a
+    // partition has at most, under the evenly split form's gigabyte.  A recorded call that still has no room (nothing ran before it)
+    // takes whole blocks, fewer partials or none.
+    const size_t slot = (size_t)std::min(p.group, p.gt_rows) * (d + 2) * sizeof(float);
+    const size_t room = slot * (size_t)std::max<int64_t>(5 * cx.num_cu, (1ll << 30) / (2 * d * (fp8 ? 1 : 2)) / 2048 + cx.num_cu);
+    const size_t need = p.n_part > 1 && !lean && !p.wg_merge ? (size_t)batch * hq * p.n_part * (d + 2) * sizeof(float) : 0;
+    if (std::max(room, need) > cx.workspace_bytes) {
+      hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
+      if (hipStreamIsCapturing((hipStream_t)stream, &capturing) != hipSuccess) {
+        (void)hipGetLastError();
+        capturing = hipStreamCaptureStatusActive;  // unknown: allocate only what the call itself needs
+      }
+      void* ws = nullptr;
+      if (capturing == hipStreamCaptureStatusNone) {
+        if (workspace(std::max(room, need), &ws) != PTO_HIP_OK) (void)hipGetLastError();  // what the call needs is asked for below
+      } else if (need > cx.workspace_bytes) {
+        const int rc = plan_launch(config, q_dtype, kv_dtype, k_scale && v_scale, active_blocks, p, gt, lean, true);
+        if (rc != PTO_HIP_OK) return rc;
+        choose_form();
+      }
+    }
+  }
 
   // Launch shape by measurement (see TuneState): only while the caller has not fixed the shape.
   hipStream_t hs = (hipStream_t)stream;

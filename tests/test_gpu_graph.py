@@ -121,6 +121,67 @@ def test_a_skinny_projection_sizes_its_scratch_for_every_batch(worker):
     assert worker.get_option("workspace_bytes") == sized
 
 
+def _without_scratch(worker):
+    """The library's scratch areas are given back, as in a process that has just started."""
+    torch.cuda.synchronize()
+    worker.close()
+    worker.init()
+    assert worker.get_option("workspace_bytes") == 0
+
+
+@pytest.mark.parametrize("hi", [100, 1500, 8000])
+@pytest.mark.parametrize("fp8", [False, True])
+def test_an_attention_call_sizes_its_scratch_for_smaller_batches(worker, fp8, hi):
+    """One eager call is what a caller owes before it captures, whatever form that call took: here a workgroup per pair or one
+    partition, without partials of its own."""
+    _without_scratch(worker)
+
+    def call(batch):
+        inp = workloads.paged_attention_inputs(batch=batch, num_heads=32, kv_head_num=8, context_lens=[hi] * batch, ctx_range=(1, hi), fp8_kv=fp8,
+                                               seed=batch, device="cuda")
+        with worker.register(paged_attention) as h:
+            h(*inp.args())
+        worker.sync()
+        return worker.get_option("workspace_bytes")
+
+    sized = call(32)
+    assert sized > 0
+    for batch in (31, 30, 17, 13, 9, 8, 5, 3, 2, 1):
+        assert call(batch) == sized, batch
+
+
+@pytest.mark.parametrize("ctx,d", [(100, 128), (250, 256)])
+def test_a_captured_attention_call_without_scratch_takes_whole_blocks(worker, ctx, d):
+    """Nothing ran before the capture, so there is no room for partials: the graph holds the call on whole blocks, bit for bit."""
+    inp = workloads.paged_attention_inputs(batch=1, num_heads=8, kv_head_num=8, head_dim=d, block_size=256, context_lens=[ctx], ctx_range=(1, 256), seed=ctx,
+                                           device="cuda")
+    args = inp.args()
+    with worker.register(paged_attention) as h:
+        worker.set_option("attn_tokens_per_partition", 256)
+        try:
+            h(*args)
+        finally:
+            worker.set_option("attn_tokens_per_partition", 0)
+        worker.sync()
+        want = inp.out.clone()
+        h(*args)  # (loads the kernels of the cut form)
+        worker.sync()
+    _without_scratch(worker)
+    stream = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with worker.register(paged_attention) as h:
+        with torch.cuda.graph(graph, stream=stream):
+            h(*args, stream=stream.cuda_stream)
+    assert worker.get_option("workspace_bytes") == 0
+    for _ in range(3):
+        inp.out.fill_(float("nan"))
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(inp.out, want)
+
+
 @pytest.mark.parametrize("kind", ["e4m3", "16-bit"])
 def test_a_split_product_is_captured_unsplit_when_its_slabs_do_not_fit(worker, kind):
     """No eager call of the split form before the capture: the graph holds the unsplit product, bit for bit, and the
