@@ -1114,7 +1114,7 @@ __global__ __launch_bounds__(PAIR ? 128 : lean_max_waves(D, GT) * 64) void attn_
 template <int D>
 __global__ __launch_bounds__(256) void attn_lean_reduce_kernel(AttnParams p, long long wtot) {
   const int lane = threadIdx.x & 63;
-  const int row = blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);  // b*Hq + query head
+  const int row = blockIdx.x * 4 + (threadIdx.x >> 6);  // b*Hq + query head
   if (row >= p.batch * p.hq) return;
   const int b = row / p.hq, hqi = row % p.hq;
   const int h = hqi / p.group, g = hqi % p.group;
