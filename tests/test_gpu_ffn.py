@@ -108,7 +108,7 @@ def test_ffn_tiny_fp16(worker, variant):
                                           (200, 1032, 1016, 3), (300, 1096, 1000, 2), (70, 328, 520, 1), (64, 264, 512, 1), (320, 256, 776, 1)])
 def test_four_wavefront_form_on_ragged_columns_and_k(worker, m, k, n, splits):
     """Columns and k that end anywhere (multiples of 8) in the four-wavefront form, every tile height: the bits of the
-    eight-wavefront form (same 16-wide k steps, zeros past k), the product of the oracle, nothing written beside it, and an
+    eight-wavefront form (same 16-wide k steps, zeros past k), the product of the oracle, and an
     infinite weight in the last row of k gives infinities, not NaN (the lanes past k read zeros for both operands)."""
     from pypto_amd.runtime import gate_up_swiglu, projection
     g = torch.Generator().manual_seed(m * k + n)
@@ -143,6 +143,43 @@ def test_four_wavefront_form_on_ragged_columns_and_k(worker, m, k, n, splits):
     validate_golden({"out": got[4, 0][0]}, {"out": oracle.projection(x, w)}, rtol=2e-3, atol=2e-3)
     want = oracle.swiglu(oracle.projection(x, w), oracle.projection(x, wu)).to(torch.bfloat16)
     validate_golden({"out": got[4, 0][1].float()}, {"out": want.float()}, rtol=1e-2, atol=1e-2)
+
+
+@pytest.mark.parametrize("m,k,n,splits", [(1, 8, 8, 1), (65, 24, 40, 1), (130, 40, 264, 1), (257, 72, 136, 1), (200, 1032, 1016, 1),
+                                          (200, 1032, 1016, 3), (300, 1096, 1000, 2), (64, 264, 512, 1), (320, 256, 776, 1)])
+def test_four_wavefront_form_stays_inside_its_operands(worker, m, k, n, splits):
+    """Every operand lies between NaN, every output between values that have to stay: what a load past the last row, column or k
+    brings must not reach a product, and no store may land beside the output."""
+    from pypto_amd.runtime import gate_up_swiglu, projection
+    g = torch.Generator(device="cuda").manual_seed(m * k + n)
+    pad = 512  # elements on either side: 16-byte aligned for both types
+
+    def between(shape, dtype, fill):
+        buf = torch.full((2 * pad + shape[0] * shape[1],), fill, dtype=dtype, device="cuda")
+        return buf, buf[pad:pad + shape[0] * shape[1]].view(shape)
+
+    (_, x), (_, w), (_, wu) = (between(s, torch.bfloat16, float("nan")) for s in ((m, k), (k, n), (k, n)))
+    x.copy_(torch.randn((m, k), generator=g, device="cuda") / k ** 0.5)
+    w.copy_(torch.randn((k, n), generator=g, device="cuda"))
+    wu.copy_(torch.randn((k, n), generator=g, device="cuda"))
+    ref, ref_up = oracle.projection(x.cpu(), w.cpu()), oracle.projection(x.cpu(), wu.cpu())
+    want = oracle.swiglu(ref, ref_up).to(torch.bfloat16)
+    worker.set_option("gemm_splits", splits)
+    worker.set_option("gemm_variant", 7)
+    try:
+        for rows in (64, 128, 192, 256):
+            worker.set_option("gemm_quad_rows", rows)
+            for program, weights, dtype, expected, tol in ((projection, (w,), torch.float32, ref, 2e-3), (projection, (w,), torch.bfloat16, ref, 1e-2),
+                                                           (gate_up_swiglu, (w, wu), torch.bfloat16, want, 1e-2)):
+                buf, out = between((m, n), dtype, -77.0)
+                with worker.register(program) as h:
+                    h(x, *weights, out)
+                worker.sync()
+                validate_golden({"out": out.cpu().float()}, {"out": expected.float()}, rtol=tol, atol=tol)
+                assert bool((buf[:pad] == -77.0).all()) and bool((buf[pad + m * n:] == -77.0).all()), (rows, program.name)
+    finally:
+        for name in ("gemm_splits", "gemm_variant", "gemm_quad_rows"):
+            worker.set_option(name, 0)
 
 
 @pytest.mark.parametrize("variant", [0, 4, 5, 6, 7])
