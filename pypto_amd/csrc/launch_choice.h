@@ -35,7 +35,10 @@ inline int64_t skinny_workgroups(int64_t slabs, int64_t ks, int64_t most, int64_
 // stream; a split the finish launch and the slabs' way out and back, dearer once they outgrow the last-level cache.
 // The 256-row form with a ragged last row tile keeps 80 registers in scratch in the single-operand
 // pass, which slows its slab stores (4096 x 4096 at 400 rows 50 us, 34 with eight wavefronts): there the eight-wavefront
-// form is a candidate too, where its loop is the direct one the costs were taken from (n and k in whole tiles).
+// form is a candidate too, where its loop is the direct one the costs were taken from (n and k in whole tiles).  With ragged columns or k
+// the 256-row form always keeps them and that loop is never ahead (at 33 to 1800 rows of fourteen such weight shapes, every tile and split timed, its best is
+// behind the best of the four-wavefront forms in all 230 passes): there it is dearer by what was measured beside its cost, 1.1 times up to
+// two rounds and 1.2 with slabs.  8192 x 8128 at 400 / 900 rows 99 / 151 -> 73 / 121 us, 8192 x 7232 90 / 141 -> 68 / 114.
 // Over several rounds the 256-row tile, with the fewest operand bytes per MFMA, is ahead of what its one-round costs say
 // (back to back, 256 / 192 rows a tile: gate/up 5120 x 13824 at 1800 rows 506 / 528 us, 8192 x 22016 at 3000 1816 / 1846,
 // 4096 x 10752 at 2709 417 / 454): it wins unless another is 5 % ahead.  At 0.97 instead of 0.95 the first two are lost, at
@@ -52,6 +55,7 @@ inline void choose_quad(int m, int n, int k, bool dual, int64_t num_cu, int forc
   // [0]: eight wavefronts
   static constexpr Cost kCost[5] = {{16.84, 7.88, 2.31}, {5.8, 6.58, 2.03}, {10.02, 5.93, 2.83}, {12.72, 5.69, 4.69}, {16.16, 8.28, 3.52}};
   const double weights_mb = (double)k * n * (dual ? 2 : 1) * 2e-6;
+  const bool spills = !dual && (n % BN != 0 || k % 32 != 0);  // the 256-row form, whatever m
   double best = 1e30;
   for (int h = 0; h <= 4; ++h) {
     if (forced ? h != forced : (h == 0 && (dual || m % 256 == 0 || k % BK != 0 || n % BN != 0))) continue;
@@ -73,6 +77,8 @@ inline void choose_quad(int m, int n, int k, bool dual, int64_t num_cu, int forc
         if (!dual && m <= 64 && kps * n % (4 << 20) == 0) t *= 1.05;
       }
       if (h == 4 && full >= 2) t *= 0.95;
+      else if (h == 4 && spills) t *= 1.1;
+      if (h == 4 && spills && s > 1) t *= 1.2;
       if (t < best) {
         best = t;
         *height = h;
