@@ -97,8 +97,8 @@ inline void choose_quad(int m, int n, int k, bool dual, int64_t num_cu, int forc
 // (pairs x tokens) with equal / ragged lengths: 256 x 4096 63.0 / 61.4 -> 42.6 / 34.4, 320 x 2200 49.9 / 48.0 -> 34.1 / 30.0, 768 x 3000
 // 120 / 70.4 -> 98 / 69; but one partition split, 1024 x 1400 56.2 -> 59.7, hence 1536.  16-bit caches are the other way round: 768 x 3000 113.9 ragged
 // -> 119, 256 x 4096 equal 80.7 -> 82.6.  The plain rule stays where its own wavefronts fill the CUs as well, lengths equal / down to half / to a tenth:
-// from four partitions on (plain -> more: 320 x 8000 108 / 85 / 79 -> 119 / 100 / 78), between 3.5 and 6 times 2048 tokens per CU (320 x 6000
-// 80 / 69 / 66 -> 88 / 75 / 56, 800 x 2600 96 / 75 / 70 -> 99 / 82 / 65; below they are ahead, 512 x 3500 81 / 72 / 66 -> 78 / 65 / 51, and above, 1600 x 3500
+// from four partitions on (plain -> more: 320 x 8000 108 / 85 / 79 -> 119 / 100 / 78), between 4.5 and 6 times 2048 tokens per CU (448 x 6000
+// 115 / 92 / 82 -> 117 / 100 / 85, 1024 x 2600 114 / 92 / 77 -> 118 / 96 / 81; below they are ahead with ragged lengths, 512 x 3500 81 / 72 / 66 -> 78 / 65 / 51, 768 x 3000 100 / 84 / 73 -> 106 / 88 / 68, and above, 1600 x 3500
 // 263 / 198 / 159 -> 250 / 190 / 149), and for one partition of four pairs per CU (1600 x 2000 143 / 119 / 96 -> 150 / 119 / 92).
 // Not more partitions than a workgroup has wavefronts (max_parts: the form needs no scratch), nor than whose partials, should the grid
 // form be taken after all, fit the fixed area of the entry point that allocates nothing.
@@ -106,7 +106,7 @@ inline int64_t attn_e4m3_partition_tokens(int64_t pairs, int64_t max_ctx, int64_
                                           int64_t scratch, int64_t plain) {
   if (max_ctx <= 1536) return plain;
   const int64_t before = (max_ctx + plain - 1) / plain, load = pairs * max_ctx / 2048;
-  if (before >= 4 || (2 * load > 7 * num_cu && load < 6 * num_cu) || (before == 1 && pairs >= 4 * num_cu)) return plain;
+  if (before >= 4 || (2 * load > 9 * num_cu && load < 6 * num_cu) || (before == 1 && pairs >= 4 * num_cu)) return plain;
   const int64_t want = std::max<int64_t>(1, (4 * num_cu + pairs - 1) / pairs);
   const int64_t tokens = std::min<int64_t>(1024, std::max<int64_t>(512, (max_ctx + want - 1) / want));
   int64_t parts = std::min((max_ctx + tokens - 1) / tokens, max_parts);

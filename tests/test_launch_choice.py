@@ -168,8 +168,8 @@ def test_partition_alignment_stays_within_the_workgroup_form(choice, d, most):
 
 
 @pytest.mark.parametrize("pairs,tokens,split", [
-    (256, 2048, True), (256, 4096, True), (320, 4992, True), (512, 3584, True), (640, 2048, True), (1600, 3584, True),
-    (256, 8064, False), (320, 6016, False), (320, 8064, False), (400, 6016, False), (800, 2688, False), (1096, 2048, False), (1600, 2048, False)])
+    (256, 2048, True), (256, 4096, True), (320, 4992, True), (512, 3584, True), (640, 2048, True), (768, 3072, True), (1600, 3584, True),
+    (256, 8064, False), (448, 6016, False), (320, 8064, False), (400, 6016, False), (1024, 2688, False), (1096, 2048, False), (1600, 2048, False)])
 def test_e4m3_partitions_stay_where_the_cus_are_full(choice, pairs, tokens, split):
     """Pairs and tables that measured ahead with more partitions or not."""
     plain = min(2048, -(-tokens // -(-512 // pairs)))
