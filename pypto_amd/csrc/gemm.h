@@ -504,12 +504,14 @@ int launch_gemm(GemmParams p, hipStream_t st) {
 // products are not stored), and in the stage k ends in, the lanes whose bytes would lie past it read zeros from memory
 // instead, for both operands (an infinity there must not become a NaN).  Against the staged eight-wavefront form that such n
 // and k had before (with finish): gate/up 4096 x 14400 at 96 / 333 / 1000 rows 78 / 172 / 310 -> 62 / 104 / 233 us, 2056 x 6008 at
-// 128 / 2000 rows 30.8 / 157 -> 28.7 / 128, 6008 x 2056 at 2000 rows 93 -> 76, 5952 x 1984 80 -> 64; from 40 rows on ahead or level.
+// 128 / 2000 rows 30.8 / 157 -> 28.7 / 128, 6008 x 2056 at 2000 rows 93 -> 76, 5952 x 1984 80 -> 64; from one row on
+// ahead or level (1000 x 2736 at 8 / 33 rows 18.4 / 20.1 -> 10.1 / 11.5, gate/up 4104 x 4096 19.5 / 22.2 -> 19.1 / 21.9).  The staged form is left to the forced
+// variants, for sweeps and as the other side of a comparison bit for bit.
 //
 // MT: the tile is 64 * MT rows high, a wavefront's part 32 * MT.  The loop's time is the MFMAs of the rows the tile has,
 // padding included: 333 rows are 512 rows' work on 256-row tiles, 384 on 192-row ones.  A stage is 4 KB smaller
 // per 64 rows, and what that leaves of the LDS goes into more stages in flight.  The low tiles replace eight-wavefront
-// ones wherever n and k allow; passes with their finish, best split count of each: 4096 x 14336 gate/up at 128 / 333 /
+// ones; passes with their finish, best split count of each: 4096 x 14336 gate/up at 128 / 333 /
 // 700 rows 67 / 97 / 193 -> 60 / 88 / 167 us, 14336 x 4096 at 96 / 333 / 2500 rows 37 / 65 / 282 -> 33 / 56 / 245,
 // 1024 x 3072 gate/up at 96 / 512 rows 14.5 / 16.5 -> 12.3 / 12.8.
 constexpr int QK = 32;   // k extent of a stage
