@@ -124,6 +124,7 @@ inline int64_t attn_e4m3_partition_tokens(int64_t pairs, int64_t max_ctx, int64_
 // blocks of 128, 256 and 512 tokens, 1 to 64 query heads per KV head, equal and ragged lengths (3828 calls, whole blocks -> this rule):
 // -14.1 % on average, 27 calls more than 3 % slower, by 6 % at most; 0.8 % behind the best of each.  Us, whole blocks -> halved:
 // one partition: 64 pairs x 384 of a 512-token block, 16 heads 14.1 -> 12.5, quarters 9.1, but 8 x 96 of a 128-token block 6.1 -> 6.9 (kept whole);
+// above a pair per CU 300 x 512 of one block 21.6 -> 18.4, e4m3 18.0 -> 15.5, but of a 128-token one 8.1 -> 7.9 and 16-bit head_dim 256 29.9 -> 33.8;
 // two, the four of which a workgroup's wavefronts can merge (head_dim 256 with few heads only as far as CUs idle): 160 x 224, 16 heads 9.2 -> 8.0;
 // more: 8 x 1504, 16 heads 10.7 -> 9.8; but 96 x 480, 32 heads 12.2 -> 19.6, 8 heads at head_dim 256 16.2 -> 18.7 (kept whole).
 // Halves as long as the table's blocks gave fewer than two wavefronts per CU, whatever the rows, as before: -11.1 % on average, 729 calls more than
@@ -139,7 +140,7 @@ inline int64_t attn_partition_align(int64_t pairs, int64_t max_ctx, int64_t bloc
     if (2 * parts * bytes_per_part > scratch || (parts <= wg_parts && 2 * parts > wg_parts)) break;
     const double weight = (double)(rows * head_dim) / 128.0 * (128.0 / (double)len) * (128.0 / (double)len);
     int quarters;  // wavefronts up to which a partition is halved, in quarters of the CUs
-    if (parts == 1) quarters = weight <= 4.0 ? 4 : 0;
+    if (parts == 1) quarters = weight > 4.0 ? 0 : weight > 1.0 || len <= 128 || long_rows ? 4 : e4m3 ? 7 : 6;
     else if (parts == 2) quarters = long_rows && rows < 8 && len <= 128 ? 3 : 8;
     else if (parts <= 4 && short_rows) quarters = 8;  // (eight of which a workgroup can merge)
     else if (weight >= 16.0) quarters = short_rows ? 3 : 2;

@@ -149,6 +149,7 @@ def test_partition_alignment_divides_the_block(choice):
 @pytest.mark.parametrize("pairs,tokens,block,rows,d,e4m3,want", [
     (8, 1536, 128, 4, 128, False, 64), (8, 1536, 128, 16, 128, False, 64), (8, 768, 128, 4, 128, False, 64),
     (160, 256, 128, 16, 128, False, 64), (128, 256, 128, 32, 128, True, 64), (64, 512, 512, 16, 128, False, 128), (8, 256, 256, 64, 128, False, 64),
+    (300, 512, 512, 4, 128, False, 256), (440, 256, 256, 1, 128, True, 128), (300, 512, 512, 1, 256, False, 512), (300, 256, 256, 16, 128, False, 256),
     # a second partial per row costs more than the shorter chain gives
     (8, 128, 128, 16, 128, False, 128), (200, 128, 128, 32, 128, False, 128), (100, 512, 128, 8, 256, False, 128), (96, 512, 128, 32, 128, False, 128),
     (160, 384, 128, 32, 128, False, 128), (160, 384, 128, 16, 256, True, 128), (16, 3072, 128, 16, 256, False, 128), (200, 256, 128, 4, 256, False, 128)])
