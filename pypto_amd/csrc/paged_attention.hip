@@ -1346,16 +1346,18 @@ int launch(const AttnParams& p, int batch, bool bf16, hipStream_t stream) {
   if (rc) return rc;
   if (p.n_part > 1) {
     // Up to 8 partitions a workgroup per row as far as that gives every row a CU of its own (128 rows, 4 partitions 7.46 -> 7.20 us a call, head_dim 256
-    // 9.35 -> 8.93; level from 384 rows on).  Above: for a few rows the longest batches and a workgroup each (8 rows of 47 partitions, batches of
-    // 16 / 8 8.9 / 9.2 us, 32 rows level); then 4 rows to a workgroup and batches of 8 (256 rows of 16 partitions 13.7 -> 13.0 us against one each, 2048
-    // rows of up to 16 26.7 -> 26.5 against batches of 16; up to 256 rows of more than 32 partitions the long ones, 64 of 163 20.6 -> 19.0); many rows want the wavefronts per SIMD that batches of 4 leave room
+    // 9.35 -> 8.93; level from 384 rows on).  Above, as far as that too the longest batches (96 rows of 32 partitions 8.7 us, batches of 8 and four rows
+    // to a workgroup 9.3), but for rows whose four are a KV head's group: with a multiple of eight pairs their workgroup then runs on the
+    // XCD that wrote the partials, ahead from some 1200 of them on (64 rows of 20 11.5 -> 10.8, 256 of 16 9.9 -> 9.4, of 40 19.3 -> 17.0).  Beyond, four rows to a workgroup:
+    // 2048 rows of up to 16 26.5 us, batches of 16 26.7; many rows want the wavefronts per SIMD that batches of 4 leave room
     // for (6400 rows of up to 11, 16 / 8 / 4 48.1 / 46.3 / 45.6, at head_dim 256 3200 rows of up to 10 49.3 / 47.4 / 46.2).
     const int rows = batch * p.hq;
     auto merge = [&](auto kern, int per_wg) {
       hipLaunchKernelGGL(kern, dim3((unsigned)((rows + per_wg - 1) / per_wg)), dim3((unsigned)per_wg * 64), 0, stream, p);
     };
     if (p.n_part <= kReduceFast) merge(attn_reduce_kernel<D, 0>, rows <= pto_hip::ctx().num_cu ? 1 : 4);
-    else if (rows <= 32 || (rows <= pto_hip::ctx().num_cu && p.n_part > 32)) merge(attn_reduce_kernel<D, 16>, 1);
+    else if (rows <= pto_hip::ctx().num_cu && !(p.group == 4 && batch * p.hkv % 8 == 0 && rows * p.n_part >= 1200))
+      merge(attn_reduce_kernel<D, 16>, 1);
     else if ((int64_t)rows * D <= (1 << 19)) merge(attn_reduce_kernel<D, 8>, 4);
     else merge(attn_reduce_kernel<D, 4>, 4);
     PTO_CHECK_HIP(hipGetLastError());
