@@ -147,7 +147,7 @@ inline int64_t attn_partition_align(int64_t pairs, int64_t max_ctx, int64_t bloc
     else if (weight > 4.0) quarters = e4m3 && rows <= 8 ? 4 : 3;
     else if (len <= 128) quarters = short_rows ? 6 : long_rows ? 3 : 4;
     else if (long_rows) quarters = 4;
-    else quarters = weight <= (e4m3 ? 2.0 : 1.0) ? 6 : 5;
+    else quarters = weight > (e4m3 ? 2.0 : 1.0) ? 5 : short_rows && weight <= 1.0 ? 8 : 6;
     if (pairs * parts * 4 <= quarters * num_cu && pairs * parts < 2 * num_cu) align = len / 2;
     else if (parts > 1) break;  // (one partition: four can still be ahead where two are not)
   }
