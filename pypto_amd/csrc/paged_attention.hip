@@ -1736,7 +1736,11 @@ int paged_attention(const void* query, const void* key_cache, const void* value_
       }
       void* ws = nullptr;
       if (capturing == hipStreamCaptureStatusNone) {
+        // (a capture on another stream must not be broken by what this call could do without)
+        hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+        const bool relaxed = hipThreadExchangeStreamCaptureMode(&mode) == hipSuccess;
         if (workspace(std::max(room, need), &ws) != PTO_HIP_OK) (void)hipGetLastError();  // what the call needs is asked for below
+        if (relaxed) (void)hipThreadExchangeStreamCaptureMode(&mode);
       } else if (need > cx.workspace_bytes) {
         const int rc = plan_launch(config, q_dtype, kv_dtype, k_scale && v_scale, active_blocks, p, gt, lean, true);
         if (rc != PTO_HIP_OK) return rc;

@@ -150,6 +150,36 @@ def test_an_attention_call_sizes_its_scratch_for_smaller_batches(worker, fp8, hi
         assert call(batch) == sized, batch
 
 
+def test_an_eager_attention_call_leaves_another_streams_capture_alone(worker):
+    """The room it makes for smaller batches is its own affair: a capture that is going on elsewhere ends and replays as recorded."""
+    inp = workloads.paged_attention_inputs(batch=32, num_heads=32, kv_head_num=8, context_lens=[300] * 32, ctx_range=(1, 300), seed=9, device="cuda")
+    with worker.register(paged_attention) as h:
+        h(*inp.args())  # (loads the kernels)
+    _without_scratch(worker)
+    x = torch.zeros(64, device="cuda")
+    recorded, eager = torch.cuda.Stream(), torch.cuda.Stream()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    worker.set_option("attn_autotune", 0)
+    try:
+        with worker.register(paged_attention) as h:
+            with torch.cuda.graph(graph, stream=recorded):
+                x.add_(1.0)
+                h(*inp.args(), stream=eager.cuda_stream)
+                x.mul_(2.0)
+            worker.sync()
+            got = inp.out.clone()
+            h(*inp.args())
+            worker.sync()
+    finally:
+        worker.set_option("attn_autotune", 1)
+    assert torch.equal(got, inp.out) and bool(got.isfinite().all())
+    for step in range(3):
+        graph.replay()
+        torch.cuda.synchronize()
+        assert bool((x == 2.0 ** (step + 2) - 2.0).all())
+
+
 @pytest.mark.parametrize("ctx,d", [(100, 128), (250, 256)])
 def test_a_captured_attention_call_without_scratch_takes_whole_blocks(worker, ctx, d):
     """Nothing ran before the capture, so there is no room for partials: the graph holds the call on whole blocks, bit for bit."""
