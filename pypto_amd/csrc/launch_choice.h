@@ -98,8 +98,8 @@ inline void choose_quad(int m, int n, int k, bool dual, int64_t num_cu, int forc
 // 120 / 70.4 -> 98 / 69; but one partition split, 1024 x 1400 56.2 -> 59.7, hence 1536.  16-bit caches are the other way round: 768 x 3000 113.9 ragged
 // -> 119, 256 x 4096 equal 80.7 -> 82.6.  The plain rule stays where its own wavefronts fill the CUs as well, lengths equal / down to half / to a tenth:
 // from four partitions on (plain -> more: 320 x 8000 108 / 85 / 79 -> 119 / 100 / 78), between 4.5 and 6 times 2048 tokens per CU (448 x 6000
-// 115 / 92 / 82 -> 117 / 100 / 85, 1024 x 2600 114 / 92 / 77 -> 118 / 96 / 81; below they are ahead with ragged lengths, 512 x 3500 81 / 72 / 66 -> 78 / 65 / 51, 768 x 3000 100 / 84 / 73 -> 106 / 88 / 68, and above, 1600 x 3500
-// 263 / 198 / 159 -> 250 / 190 / 149), and for one partition of four pairs per CU (1600 x 2000 143 / 119 / 96 -> 150 / 119 / 92).
+// 115 / 92 / 82 -> 117 / 100 / 85, 1024 x 2600 114 / 92 / 77 -> 118 / 96 / 81; below they are ahead with ragged lengths, 512 x 3500
+// 81 / 72 / 66 -> 78 / 65 / 51, 768 x 3000 100 / 84 / 73 -> 106 / 88 / 68, and above, 1600 x 3500 263 / 198 / 159 -> 250 / 190 / 149), and for one partition of four pairs per CU (1600 x 2000 143 / 119 / 96 -> 150 / 119 / 92).
 // Not more partitions than a workgroup has wavefronts (max_parts: the form needs no scratch), nor than whose partials, should the grid
 // form be taken after all, fit the fixed area of the entry point that allocates nothing.
 inline int64_t attn_e4m3_partition_tokens(int64_t pairs, int64_t max_ctx, int64_t num_cu, int64_t max_parts, int64_t bytes_per_part,
