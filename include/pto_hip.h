@@ -574,6 +574,10 @@ PTO_HIP_API int pto_hip_backend_handler_query(const char* hook, int32_t arg, cha
  *                               and tests; 4 and 7 give identical bits)
  *  "gemm_quad_rows"             tile height of the four-wavefront form where "gemm_variant" is 0 or 7:
  *                               0 = by estimate (256 under variant 7, default), 64, 128, 192, 256
+ *  "gemm_narrow"                products with 16-bit weights in tiles of 16 to 64 rows x 32 or 64 channels, one launch
+ *                               each: 0 = where estimated faster than the tiled GEMM, and up to 32 rows for at most
+ *                               1.6 million weights (default), -1 = never, 1..4 = always, with that tile
+ *                               ("gemm_variant", "gemm_quad_rows" or "gemm_splits" other than 0 switch it off)
  *  "gemm_splits"                k splits of the tiled GEMMs: 0 = by shape (default), 1..16 = as given
  *                               when k allows (16-bit and int8 weights: each split at least four 64-row
  *                               k tiles; e4m3: at least one tile of 128 codes), under every "gemm_variant"

@@ -23,7 +23,9 @@
 //     workgroups per tile, each writing an fp32 slab, and a finish kernel sums the slabs in
 //     split order (plus SwiGLU for the gate/up pass);
 //   * at decode-size token counts (at most 32 rows) the block is bound by reading the weights
-//     once and runs as skinny projections instead (ffn_skinny below).
+//     once and runs as skinny projections instead (ffn_skinny below);
+//   * products of a small call, whose time is a chain of launches and round trips, run in narrow tiles
+//     with k split inside the workgroup, one launch each (narrow_gemm.h).
 #include <hip/hip_runtime.h>
 #include <algorithm>
 
@@ -35,8 +37,37 @@ namespace {
 
 using namespace pto_hip::gemm;
 
+constexpr int64_t kSkinnyMaxTokens = 32;
+constexpr int kNarrowMinK = 32;
+
+// Products of up to kSkinnyMaxTokens rows that take the small-call form instead of the skinny one (every k of a block's at least 32).
+bool narrow_not_skinny(int64_t k, int64_t n, bool dual) {
+  return pto_hip::ctx().gemm_narrow >= 0 && pto_hip::ctx().gemm_splits == 0 && pto_hip::ctx().gemm_quad_rows == 0 && k >= kNarrowMinK &&
+         pto_hip::narrow_beats_skinny(k, n, dual);
+}
+
+// Tile of the small-call form for a product with 16-bit weights, 0 for the tiled GEMM.  A forced tile form, height or split
+// count asks for the tiled GEMM.  Whoever sums the slabs of partials_out spares that product its finish launch.
+int narrow_tile(const GemmParams& p, bool dual) {
+  const pto_hip::Context& cx = pto_hip::ctx();
+  if (cx.gemm_variant != 0 || cx.gemm_splits != 0 || cx.gemm_quad_rows != 0 || cx.gemm_narrow < 0 || p.k < kNarrowMinK) return 0;
+  if (cx.gemm_narrow > 0) return (int)cx.gemm_narrow;
+  int height = 0, splits = 1;
+  double us = pto_hip::choose_quad(p.m, p.n, p.k, dual, cx.num_cu, 0, &height, &splits);
+  if (splits > 1 && p.partials_out) us -= 2.95;
+  if (p.m <= kSkinnyMaxTokens && pto_hip::narrow_beats_skinny(p.k, p.n, dual)) us = 1e9;
+  return pto_hip::choose_narrow(p.m, p.n, p.k, dual, cx.num_cu, us);
+}
+
 template <bool DUAL>
 int launch_typed(const GemmParams& p, int dtype, int out_dtype, hipStream_t st) {
+  const bool built = dtype == out_dtype || (!DUAL && out_dtype == PTO_HIP_FP32);
+  if (const int tile = !p.scale0 && built ? narrow_tile(p, DUAL) : 0) {
+    if (p.partials_out) *p.partials_out = pto_hip::finished_slab(reinterpret_cast<const float*>(p.c));
+    if (DUAL) return dtype == PTO_HIP_BF16 ? pto_hip::narrow_dual_bf16(p, tile, st) : pto_hip::narrow_dual_fp16(p, tile, st);
+    return dtype == PTO_HIP_BF16 ? pto_hip::narrow_single_bf16(p, tile, out_dtype, st)
+                                 : pto_hip::narrow_single_fp16(p, tile, out_dtype, st);
+  }
   if (p.scale0)  // int8 weight codes
     return DUAL ? pto_hip::gemm_launch_w8_dual(p, dtype, out_dtype, st)
                 : pto_hip::gemm_launch_w8_single(p, dtype, out_dtype, st);
@@ -85,8 +116,6 @@ __global__ __launch_bounds__(256) void activation_kernel(const float* __restrict
   for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (size_t)gridDim.x * 256)
     h[i] = (TO)activate(act, gate[i]);
 }
-
-constexpr int64_t kSkinnyMaxTokens = 32;
 
 int ffn_skinny(const void* x, const float* gamma, const void* w_gate, const void* w_up, const void* w_down,
                void* out, int64_t tokens, int64_t hidden, int64_t intermediate, float eps, int dtype,
@@ -203,7 +232,7 @@ extern "C" int pto_hip_ffn_swiglu(const void* x, const float* gamma, const void*
       intermediate % 16 == 0 && intermediate >= 32 &&
       ((uintptr_t)x | (uintptr_t)w_gate | (uintptr_t)w_up | (uintptr_t)w_down | (uintptr_t)out |
        (uintptr_t)gamma) % 16 == 0 &&
-      (out_dtype == PTO_HIP_FP32 || out_dtype == dtype))
+      (out_dtype == PTO_HIP_FP32 || out_dtype == dtype) && !narrow_not_skinny(hidden, intermediate, true))
     return ffn_skinny(x, gamma, w_gate, w_up, w_down, out, tokens, hidden, intermediate, eps, dtype, out_dtype, st);
 
   const size_t xn_bytes = gamma ? ((size_t)tokens * hidden * eb + 255) / 256 * 256 : 0;
@@ -350,7 +379,7 @@ extern "C" int pto_hip_projection(const void* x, const void* w, const void* resi
   PTO_CHECK_ARG(((uintptr_t)x | (uintptr_t)w | (uintptr_t)out | (uintptr_t)residual) % 16 == 0,
                 "projection: operand pointers must be 16-byte aligned");
   hipStream_t st = (hipStream_t)stream;
-  if (m <= kSkinnyMaxTokens && ctx().gemm_variant == 0 && k % 16 == 0 && k >= 32) {
+  if (m <= kSkinnyMaxTokens && ctx().gemm_variant == 0 && k % 16 == 0 && k >= 32 && !narrow_not_skinny(k, n, false)) {
     W8Partials parts{};
     int rc = w8a16_partials(x, false, w, nullptr, m, k, n, dtype, st, &parts, true);
     if (rc) return rc;
@@ -391,7 +420,7 @@ extern "C" int pto_hip_gate_up_swiglu(const void* x, const void* w_gate, const v
   PTO_CHECK_ARG(((uintptr_t)x | (uintptr_t)w_gate | (uintptr_t)w_up | (uintptr_t)out) % 16 == 0,
                 "gate_up_swiglu: operand pointers must be 16-byte aligned");
   hipStream_t st = (hipStream_t)stream;
-  if (m <= kSkinnyMaxTokens && ctx().gemm_variant == 0 && k % 16 == 0 && k >= 32) {
+  if (m <= kSkinnyMaxTokens && ctx().gemm_variant == 0 && k % 16 == 0 && k >= 32 && !narrow_not_skinny(k, n, true)) {
     W8Partials parts{};
     int rc = w8a16_partials(x, false, w_gate, w_up, m, k, n, dtype, st, &parts, true);
     if (rc) return rc;

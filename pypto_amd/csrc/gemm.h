@@ -1007,6 +1007,11 @@ int gemm_launch_w16_dual_bf16(const gemm::GemmParams& p, int out_dtype, hipStrea
 int gemm_launch_w16_dual_fp16(const gemm::GemmParams& p, int out_dtype, hipStream_t st);
 int gemm_launch_w8_single(const gemm::GemmParams& p, int dtype, int out_dtype, hipStream_t st);
 int gemm_launch_w8_dual(const gemm::GemmParams& p, int dtype, int out_dtype, hipStream_t st);
+// The products of a small call (narrow_gemm.h), 16-bit weights; tile 1 to 4 as choose_narrow numbers them, k at least 32.
+int narrow_single_bf16(const gemm::GemmParams& p, int tile, int out_dtype, hipStream_t st);
+int narrow_single_fp16(const gemm::GemmParams& p, int tile, int out_dtype, hipStream_t st);
+int narrow_dual_bf16(const gemm::GemmParams& p, int tile, hipStream_t st);
+int narrow_dual_fp16(const gemm::GemmParams& p, int tile, hipStream_t st);
 
 namespace gemm {
 // Picks the instantiation for the output type: FP32 (not for a 16-bit gate/up pair, whose callers all keep the activation

@@ -47,7 +47,8 @@ inline int64_t skinny_workgroups(int64_t slabs, int64_t ks, int64_t most, int64_
 // channels at the same time: 11008 x 4096 in 11 splits of 1024 k rows 31.4 us, in 16 of 704 26.5; 14336 x 4096 in 14 of
 // 1024 33.3, in 16 of 896 31.3.
 // `forced`: height given, only the split count is chosen.
-inline void choose_quad(int m, int n, int k, bool dual, int64_t num_cu, int forced, int* height, int* want) {
+// Returns the estimate (without the launch's own time).
+inline double choose_quad(int m, int n, int k, bool dual, int64_t num_cu, int forced, int* height, int* want) {
   constexpr int BK = 64, BN = 256, kMaxSplits = 16;
   struct Cost {
     double a, b, c;
@@ -86,6 +87,42 @@ inline void choose_quad(int m, int n, int k, bool dual, int64_t num_cu, int forc
       }
     }
   }
+  return best;
+}
+
+// Tile of the small-call form (narrow_gemm.h) for a product with 16-bit weights: 1: 16 rows x 32 channels, 2: 32 x 32, 3: 32 x 64, 4: 64 x 64;
+// 0: the tiled GEMM.  Estimated microseconds, fitted to 40 to 1024 rows of nineteen weight shapes from 512 x 512 to 2048 x 5632
+// (rms 5 to 11 %): a launch, the operand KB of a tile once per round of workgroups over the CUs, and what the weights take to
+// arrive.  tiled_us: choose_quad's estimate, which takes 1.11 of itself and 2 us in the same measure; the form has to be 5 % ahead.  Over the
+// 175 products of 33 and more rows among them the rule is 1.35 times as fast as the tiled GEMM, the best of all tiles and forms 1.38; two
+// are slower, by 9 % at most (3584 x 1024 at 700 rows), and at 512 rows and more of wide pairs nothing changes.
+// Up to 32 rows a product in the skinny form streams its weights once, in two launches; this form is ahead up to 1.6 million weights
+// (us, skinny -> this, 1 / 32 rows: 512 x 1024 pair 6.1 / 7.3 -> 4.2 / 4.5, 1024 x 1024 5.7 / 7.3 -> 4.1 / 4.7, 2048 x 768 6.1 / 7.5 ->
+// 5.6 / 6.8; but 768 x 2048 pair 7.0 / 8.4 -> 7.7 / 7.7, 1024 x 2048 pair 7.0 / 8.6 -> 9.3 / 9.5).
+inline bool narrow_beats_skinny(int64_t k, int64_t n, bool dual) { return k * n * (dual ? 2 : 1) <= 1600000; }
+
+inline int choose_narrow(int64_t m, int64_t n, int64_t k, bool dual, int64_t num_cu, double tiled_us) {
+  struct Tile {
+    int rows, channels;
+    double us[2], round[2], mb[2];  // of a single product and of a pair
+  };
+  static constexpr Tile kTiles[4] = {{16, 32, {2.31, 2.40}, {0.0171, 0.0154}, {0.394, 0.371}},
+                                     {32, 32, {2.33, 2.22}, {0.0201, 0.0226}, {0.313, 0.274}},
+                                     {32, 64, {1.83, 1.67}, {0.0226, 0.0257}, {0.070, 0.084}},
+                                     {64, 64, {2.80, 2.77}, {0.0191, 0.0275}, {0.165, 0.0}}};
+  double best = (1.112 * tiled_us + 2.05) * 0.95;
+  int tile = 0;
+  for (int i = 0; i < 4; ++i) {
+    const Tile& t = kTiles[i];
+    const int64_t wgs = ((m + t.rows - 1) / t.rows) * ((n + t.channels - 1) / t.channels);
+    const double kb = (double)k * 2.0 * (t.channels * (dual ? 2 : 1) + t.rows) * 1e-3;
+    const double us = t.us[dual] + t.round[dual] * (double)((wgs + num_cu - 1) / num_cu) * kb + t.mb[dual] * (double)k * n * (dual ? 2 : 1) * 2e-6;
+    if (us < best) {
+      best = us;
+      tile = i + 1;
+    }
+  }
+  return tile;
 }
 
 // Tokens per context partition of a workgroup-form attention launch (a workgroup per (sequence, KV head) pair, its

@@ -1060,6 +1060,9 @@ int pto_hip_set_option(const char* name, int64_t value) {
   } else if (!std::strcmp(name, "gemm_quad_rows")) {
     PTO_CHECK_ARG(value >= 0 && value <= 256 && value % 64 == 0, "gemm_quad_rows must be 0, 64, 128, 192 or 256");
     c.gemm_quad_rows = value;
+  } else if (!std::strcmp(name, "gemm_narrow")) {
+    PTO_CHECK_ARG(value >= -1 && value <= 4, "gemm_narrow must be in [-1, 4]");
+    c.gemm_narrow = value;
   } else if (!std::strcmp(name, "gemm_variant")) {
     PTO_CHECK_ARG(value == 0 || (value >= 4 && value <= 7), "gemm_variant must be 0, 4, 5, 6 or 7");
     c.gemm_variant = value;
@@ -1113,6 +1116,7 @@ int pto_hip_get_option(const char* name, int64_t* value) {
   if (!std::strcmp(name, "attn_tokens_per_partition")) *value = c.attn_tokens_per_partition;
   else if (!std::strcmp(name, "gemm_quad_rows")) *value = c.gemm_quad_rows;
   else if (!std::strcmp(name, "gemm_variant")) *value = c.gemm_variant;
+  else if (!std::strcmp(name, "gemm_narrow")) *value = c.gemm_narrow;
   else if (!std::strcmp(name, "gemm_splits")) *value = c.gemm_splits;
   else if (!std::strcmp(name, "attn_waves_per_cu")) *value = c.attn_waves_per_cu;
   else if (!std::strcmp(name, "attn_kernel_timing")) *value = c.attn_kernel_timing;
