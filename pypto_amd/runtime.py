@@ -329,10 +329,15 @@ class ChipWorker:
 
     def free(self, ptr: int) -> None:
         self._require_ready("free")
-        if ptr not in self._owned:
+        # the entry goes first: once the memory is released, another thread's malloc may be given its address
+        nbytes = self._owned.pop(ptr, None)
+        if nbytes is None:
             raise ValueError(f"pointer 0x{ptr:x} was not allocated by this worker")
-        _lib.check(self._lib.pto_hip_free(ptr))
-        del self._owned[ptr]
+        try:
+            _lib.check(self._lib.pto_hip_free(ptr))
+        except Exception:
+            self._owned[ptr] = nbytes
+            raise
 
     def copy_to(self, dst_dev_ptr: int, src_host_ptr: int, nbytes: int) -> None:
         self._require_ready("copy_to")
