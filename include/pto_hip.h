@@ -587,6 +587,10 @@ PTO_HIP_API int pto_hip_backend_handler_query(const char* hook, int32_t arg, cha
  *                               channel count is a multiple of 16
  *  "w8a16_min_steps"            fewest 32-row steps per wavefront before k is split further
  *                               (default 2)
+ *  "skinny_fuse"                skinny projections of up to four rows whose workgroups make their activations
+ *                               themselves, where that is faster than a launch in front (same bits): 1 = the
+ *                               input RMSNorm, 2 = SwiGLU of the pair in front, 4 = the merge of the attention
+ *                               partials (a sum of these; default 7, 0 = never)
  *  "w8a16_gemm_rows"            rows from which the int8 projections run as one tiled GEMM (codes
  *                               widened inside the kernel, weights read once) instead of 32-row
  *                               passes (default 33; 0 = never)

@@ -73,6 +73,7 @@ struct Context {
   int64_t gemm_splits = 0;       // k splits of the tiled GEMM: 0 = by shape, 1..16 = as given (when k allows)
   int64_t w8a16_wgs_per_cu = 1;  // most workgroups of the skinny projection kernel per compute unit
   int64_t w8a16_wide = 1;        // int8 codes read 16 per lane: 0 never, 1 for large matrices, 2 whenever shapes allow
+  int64_t skinny_fuse = 7;         // skinny projections of up to four rows make their activations themselves: 1 norm, 2 SwiGLU, 4 merge
   int64_t w8a16_min_steps = 2;   // fewest 32-row steps per wavefront before k is split further
   int64_t w8a16_gemm_rows = 33;  // rows from which int8 projections run as a tiled GEMM (0 = never)
 };
@@ -125,13 +126,43 @@ inline W8Partials finished_slab(const float* product) {
   p.splits = 1;
   return p;
 }
+// Unmerged partials of an attention launch: per (sequence, query head) and partition the running maximum and sum, and the
+// unnormalised result; partition i of a sequence holds tokens [i tpp, (i + 1) tpp) of its first ctx_cap.
+struct AttnPartials {
+  const float* ml;  // [B * Hq, n_part, 2]
+  const float* o;   // [B * Hq, n_part, D]
+  const int32_t* ctx_lens;
+  int n_part, tpp, ctx_cap;
+};
+// What the workgroups of a skinny projection of up to kSkinnyFusedRows rows make their activations from (skinny.h).
+constexpr int kSkinnyFusedRows = 4;
+struct ProjectionSource {
+  enum Kind { kTensor, kNorm, kSwiglu, kMerge } kind;
+  const float* gamma;  // kNorm: x is the row-major input of the norm
+  float eps;
+  W8Partials pair;  // kSwiglu: the gate/up pair's partial slabs and scales
+  const float* scale0;
+  const float* scale1;
+  AttnPartials attn;  // kMerge
+  int head_dim;
+};
+// Whether a projection [m, k] @ [k, n] may be given the source (head_dim: kMerge only).
+bool skinny_fuses(ProjectionSource::Kind kind, int64_t m, int64_t k, int64_t n, const void* wq0, const void* wq1, bool w16, int64_t head_dim = 0);
+constexpr int kMergeHeld = 40;  // most partitions per row of a kMerge source
+// Bytes of the partial slabs of such a projection (up to kSkinnyFusedRows rows), for callers that provide the area: what a source is
+// read from lies in workspace() itself.
+size_t skinny_fused_bytes(int64_t k, int64_t n, const void* wq0, const void* wq1, bool w16);
 // Launches the partial kernel for x[M, K] @ wq0[K, N] (and wq1 when non-null).  x_blocked: x is
 // stored [K/8][32][8] - element (m, k) at ((k/8)*32 + m)*8 + k%8 - the layout the layer's own
 // producers write so that a wavefront's activation reads are whole consecutive cache lines.
 // w16: the weights are 16-bit values of the activation type instead of int8 codes (the finish
 // kernels then take null scales).
+// src: the activations are made by the workgroups (x unused but for kNorm); area: where the slabs go instead of workspace().
 int w8a16_partials(const void* x, bool x_blocked, const void* wq0, const void* wq1, int64_t m, int64_t k,
-                   int64_t n, int x_dtype, hipStream_t st, W8Partials* out, bool w16 = false);
+                   int64_t n, int x_dtype, hipStream_t st, W8Partials* out, bool w16 = false,
+                   const ProjectionSource* src = nullptr, float* area = nullptr);
+// Whether `st` is being captured (or that cannot be told).
+bool stream_capturing(hipStream_t st);
 // Grow-only device scratch for intermediates that must survive calls which use workspace().
 int layer_workspace(size_t bytes, void** ptr);
 // Grow-only device scratch for the split-K slabs of the tiled GEMMs.  Null when `st` is being captured and the area
@@ -192,7 +223,9 @@ int paged_attention(const void* query, const void* key_cache, const void* value_
                     bool want_blocked, bool* wrote_blocked,
                     const int64_t* config, int q_dtype, int kv_dtype, const float* k_scale,
                     const float* v_scale, int64_t pool_blocks, void* stream, void* fixed_scratch = nullptr,
-                    size_t fixed_scratch_bytes = 0, int64_t active_blocks = -1);
+                    size_t fixed_scratch_bytes = 0, int64_t active_blocks = -1, AttnPartials* unmerged = nullptr);
+// unmerged: the caller can take the partials as they are, up to unmerged->n_part per row.  A launch that has a merge kernel and is
+// not being measured then leaves it out and describes them there, `out` and `out16` unwritten; otherwise n_part comes back 0.
 // Forgets every measured launch shape (and releases the events of measurements in flight).
 void attention_tuning_reset();
 // Residency cap and form (1 = workgroup form) the last launch's signature was tuned to; -1 while untuned.

@@ -125,27 +125,43 @@ int ffn_skinny(const void* x, const float* gamma, const void* w_gate, const void
   auto up = [](size_t n) { return (n + 255) / 256 * 256; };
   // intermediates of one 32-row pass, in the blocked activation layout [K/8][32][8]
   const size_t sz_xn = up((size_t)kW8MaxM * hidden * eb), sz_h = up((size_t)kW8MaxM * intermediate * eb);
+  // slabs of a down projection that reads the pair's from workspace() (none where the area would have to grow under capture)
+  size_t sz_slabs = skinny_fused_bytes(intermediate, hidden, w_down, nullptr, true);
+  if (sz_xn + sz_h + sz_slabs > ctx().layer_ws_bytes && stream_capturing(st)) sz_slabs = 0;
   void* lws = nullptr;
-  int rc = layer_workspace(sz_xn + sz_h, &lws);
+  int rc = layer_workspace(sz_xn + sz_h + sz_slabs, &lws);
   if (rc) return rc;
   void* xn = lws;
   void* hbuf = reinterpret_cast<char*>(lws) + sz_xn;
+  float* slabs = sz_slabs ? reinterpret_cast<float*>(reinterpret_cast<char*>(hbuf) + sz_h) : nullptr;
   const bool blk_x = gamma != nullptr && rms_norm_blocked_fits(kW8MaxM, hidden);
   for (int64_t r0 = 0; r0 < tokens; r0 += kW8MaxM) {
     const int64_t m = tokens - r0 < kW8MaxM ? tokens - r0 : kW8MaxM;
     const void* xr = reinterpret_cast<const char*>(x) + (size_t)r0 * hidden * eb;
     const void* a1 = xr;
-    if (gamma) {
+    ProjectionSource src{};
+    if (blk_x && skinny_fuses(ProjectionSource::kNorm, m, hidden, intermediate, w_gate, w_up, true)) {
+      src.kind = ProjectionSource::kNorm;
+      src.gamma = gamma;
+      src.eps = eps;
+    } else if (gamma) {
       if (blk_x) rc = rms_norm_blocked(xr, gamma, xn, m, hidden, eps, dtype, st);
       else rc = pto_hip_rms_norm(xr, gamma, xn, m, hidden, eps, dtype, dtype, st);
       if (rc) return rc;
       a1 = xn;
     }
     W8Partials parts{};
-    if ((rc = w8a16_partials(a1, gamma && blk_x, w_gate, w_up, m, hidden, intermediate, dtype, st, &parts, true)))
+    if ((rc = w8a16_partials(a1, a1 == xn && blk_x, w_gate, w_up, m, hidden, intermediate, dtype, st, &parts, true, &src)))
       return rc;
-    if ((rc = w8a16_finish(parts, nullptr, nullptr, nullptr, 0, hbuf, dtype, true, m, intermediate, st))) return rc;
-    if ((rc = w8a16_partials(hbuf, true, w_down, nullptr, m, intermediate, hidden, dtype, st, &parts, true))) return rc;
+    if (slabs && skinny_fuses(ProjectionSource::kSwiglu, m, intermediate, hidden, w_down, nullptr, true)) {
+      src.kind = ProjectionSource::kSwiglu;
+      src.pair = parts;
+      rc = w8a16_partials(nullptr, false, w_down, nullptr, m, intermediate, hidden, dtype, st, &parts, true, &src, slabs);
+    } else {
+      if ((rc = w8a16_finish(parts, nullptr, nullptr, nullptr, 0, hbuf, dtype, true, m, intermediate, st))) return rc;
+      rc = w8a16_partials(hbuf, true, w_down, nullptr, m, intermediate, hidden, dtype, st, &parts, true);
+    }
+    if (rc) return rc;
     void* outr = reinterpret_cast<char*>(out) + (size_t)r0 * hidden * ob;
     if ((rc = w8a16_finish(parts, nullptr, nullptr, nullptr, 0, outr, out_dtype, false, m, hidden, st))) return rc;
   }

@@ -24,6 +24,7 @@
 #include <vector>
 #include <type_traits>
 
+#include "attn_merge.h"
 #include "common.h"
 #include "launch_choice.h"
 
@@ -36,7 +37,8 @@ typedef __attribute__((__vector_size__(8 * sizeof(_Float16)))) _Float16 f16x8;
 
 constexpr int kChunk = 32;  // tokens per wave iteration: two 16-token MFMA tiles
 constexpr float kLog2e = 1.4426950408889634f;
-constexpr float kMinMax = -1e30f;  // clamp of the running maximum (04_paged_attention.py:521)
+using pto_hip::attn::kMinMax;
+using pto_hip::attn::kReduceFast;
 
 struct AttnParams {
   const void* q;
@@ -64,6 +66,7 @@ struct AttnParams {
   int n_wg;        // evenly split form: resident workgroups (one per CU); 0 = partition grid
   int lean_waves;  // ... and wavefronts in each
   float scale_log2e;
+  int no_merge;    // partition grid: the partials are left as they are
 };
 
 template <bool BF16>
@@ -714,14 +717,7 @@ __global__ __launch_bounds__(64) void attn_partition_kernel(AttnParams p) {
   }
 }
 
-// Merge of the per-partition (m, l, o): the online-update algebra of
-// examples/models/04_paged_attention.py:186-215 applied across partitions, then o / l.
-// One wavefront per output row.  What bounds it is the chain of memory round trips: one up to 8 partitions, above that one for
-// the context length, one for the first BATCH partials and less than one for every BATCH more.  BATCH 0: launches of up to kReduceFast partitions, a kernel
-// of its own: beside the other path's two batches of partials (16 then) it held 132 registers instead of 50 (head_dim 256: 226 instead of 64), two or three
-// wavefronts per SIMD instead of eight.  Attention call of 128 sequences, 32 heads on one KV head, one kernel for both -> two, us: 16-bit
-// cache of 1024 tokens 30.3 -> 29.0, of 64 to 4096 42.7 -> 38.0, e4m3 27.9 -> 25.5 and 45.2 -> 36.1.
-constexpr int kReduceFast = 8;  // most partitions of the path without a loop
+// Merge launch: one wavefront per output row (merge_row).
 template <int D, int BATCH>
 __global__ __launch_bounds__(256) void attn_reduce_kernel(AttnParams p) {
   const int lane = threadIdx.x & 63;
@@ -732,100 +728,11 @@ __global__ __launch_bounds__(256) void attn_reduce_kernel(AttnParams p) {
   const int max_ctx = p.ctx_cap;
   ctx = ctx < 0 ? 0 : (ctx > max_ctx ? max_ctx : ctx);
   const int np = (ctx + p.tpp - 1) / p.tpp;
-  const float* ml = p.part_ml + (size_t)row * p.n_part * 2;
-  const float* po = p.part_o + (size_t)row * p.n_part * D;
-  if constexpr (BATCH == 0) {
-    // Few partitions: every slot the row could use is fetched at once, before the context length
-    // is known, so the launch is one memory round trip instead of three; slots past np (never
-    // written, or stale) are dropped by select, not by a zero weight.
-    float pm[kReduceFast], pl[kReduceFast], pv[kReduceFast][D / 64];
-#pragma unroll
-    for (int u = 0; u < kReduceFast; ++u) {
-      const int i = min(u, p.n_part - 1);
-      pm[u] = ml[2 * i];
-      pl[u] = ml[2 * i + 1];
-#pragma unroll
-      for (int k = 0; k < D / 64; ++k) pv[u][k] = po[(size_t)i * D + k * 64 + lane];
-    }
-    float m = kMinMax;
-#pragma unroll
-    for (int u = 0; u < kReduceFast; ++u) m = u < np ? fmaxf(m, pm[u]) : m;
-    float l = 0.f, o[D / 64];
-#pragma unroll
-    for (int k = 0; k < D / 64; ++k) o[k] = 0.f;
-#pragma unroll
-    for (int u = 0; u < kReduceFast; ++u) {
-      const float wgt = __builtin_amdgcn_exp2f(pm[u] - m);
-      if (u < np) {
-        l += wgt * pl[u];
-#pragma unroll
-        for (int k = 0; k < D / 64; ++k) o[k] += wgt * pv[u][k];
-      }
-    }
-    const float inv = l > 0.f ? 1.f / l : 0.f;
-#pragma unroll
-    for (int k = 0; k < D / 64; ++k) {
-      const float y = o[k] * inv;
-      const size_t idx = (size_t)row * D + k * 64 + lane;
-      p.out[idx] = y;
-      if (p.out16) {
-        size_t i16 = idx;
-        if (p.out16_blocked) {
-          const int bb = row / p.hq, kk = (row % p.hq) * D + k * 64 + lane;
-          i16 = ((size_t)(kk >> 3) * 32 + bb) * 8 + (kk & 7);
-        }
-        if (p.out16_bf16) reinterpret_cast<__bf16*>(p.out16)[i16] = (__bf16)y;
-        else reinterpret_cast<_Float16*>(p.out16)[i16] = (_Float16)y;
-      }
-    }
-    return;
-  }
-  // Lane i holds (m, l) of partitions i, i + 64, ...  Every batch of partials is requested before the one in front of it is summed.
-  // Slots past the row's own partitions repeat its last one, a line that is asked for anyway, and are dropped by select: all slots asked for before
-  // the length is known cost the other rows' bandwidth (100 sequences of 16 to 2500 tokens, 32 heads on one KV head at head_dim 256, 50.5 -> 49.3 us).
-  constexpr int kBatch = BATCH == 0 ? 1 : BATCH;  // (not instantiated past the return above)
-  const int last = max(np - 1, 0);
-  float pv[2][kBatch][D / 64];
-  auto fetch = [&](int set, int first) {
-#pragma unroll
-    for (int u = 0; u < kBatch; ++u)
-#pragma unroll
-      for (int k = 0; k < D / 64; ++k) pv[set][u][k] = po[(size_t)min(first + u, last) * D + k * 64 + lane];
-  };
-  float2 own = *reinterpret_cast<const float2*>(ml + 2 * min(lane, last));
-  fetch(0, 0);
-  float m = lane < np ? own.x : kMinMax;
-  for (int i = lane + 64; i < np; i += 64) m = fmaxf(m, ml[2 * i]);
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) m = fmaxf(m, __shfl_xor(m, off));
-  float l = 0.f, o[D / 64];
-#pragma unroll
-  for (int k = 0; k < D / 64; ++k) o[k] = 0.f;
-  for (int base = 0; base < np; base += 64) {
-    if (base > 0) own = *reinterpret_cast<const float2*>(ml + 2 * min(base + lane, last));
-    const float wgt = base + lane < np ? __builtin_amdgcn_exp2f(own.x - m) : 0.f;
-    l += base + lane < np ? wgt * own.y : 0.f;
-    auto add = [&](int set, int first) {
-#pragma unroll
-      for (int u = 0; u < kBatch; ++u) {
-        const float w = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, wgt), (first + u) & 63));
-#pragma unroll
-        for (int k = 0; k < D / 64; ++k) o[k] = first + u < np ? o[k] + w * pv[set][u][k] : o[k];
-      }
-    };
-    for (int first = base; first < min(base + 64, np); first += 2 * kBatch) {
-      if (first + kBatch < np) fetch(1, first + kBatch);
-      add(0, first);
-      if (first + 2 * kBatch < np) fetch(0, first + 2 * kBatch);
-      if (first + kBatch < np) add(1, first + kBatch);
-    }
-  }
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) l += __shfl_xor(l, off);
-  const float inv = l > 0.f ? 1.f / l : 0.f;
+  float o[D / 64];
+  pto_hip::attn::merge_row<D, BATCH>(p.part_ml + (size_t)row * p.n_part * 2, p.part_o + (size_t)row * p.n_part * D, p.n_part, np, lane, o);
 #pragma unroll
   for (int k = 0; k < D / 64; ++k) {
-    const float y = o[k] * inv;
+    const float y = o[k];
     const size_t idx = (size_t)row * D + k * 64 + lane;
     p.out[idx] = y;
     if (p.out16) {
@@ -1344,7 +1251,7 @@ int launch(const AttnParams& p, int batch, bool bf16, hipStream_t stream) {
     else rc = launch_streaming(attn_partition_kernel<D, false, FP8, GT>, grid, dim3(64), lds, stream, p);
   }
   if (rc) return rc;
-  if (p.n_part > 1) {
+  if (p.n_part > 1 && !p.no_merge) {
     // Up to 8 partitions a workgroup per row as far as that gives every row a CU of its own (128 rows, 4 partitions 7.46 -> 7.20 us a call, head_dim 256
     // 9.35 -> 8.93; level from 384 rows on).  Above, as far as that too the longest batches (96 rows of 32 partitions 8.7 us, batches of 8 and four rows
     // to a workgroup 9.3), but for rows whose four are a KV head's group: with a multiple of eight pairs their workgroup then runs on the
@@ -1657,8 +1564,10 @@ int paged_attention(const void* query, const void* key_cache, const void* value_
                     const int32_t* block_table, const int32_t* context_lens, float* out, void* out16,
                     bool want_blocked, bool* wrote_blocked, const int64_t* config, int q_dtype, int kv_dtype, const float* k_scale,
                     const float* v_scale, int64_t pool_blocks, void* stream, void* fixed_scratch,
-                    size_t fixed_scratch_bytes, int64_t active_blocks) {
+                    size_t fixed_scratch_bytes, int64_t active_blocks, AttnPartials* unmerged) {
   Context& cx = ctx();
+  const int most_unmerged = unmerged ? unmerged->n_part : 0;
+  if (unmerged) *unmerged = AttnPartials{};
   if (!cx.initialized) return fail(PTO_HIP_ERR_NOT_INITIALIZED, "pto_hip_init has not been called");
   PTO_CHECK_ARG(config != nullptr, "paged_attention: config is null");
   const int64_t batch = config[0], hq = config[1], hkv = config[2], d = config[3];
@@ -1802,6 +1711,10 @@ int paged_attention(const void* query, const void* key_cache, const void* value_
     if (rc != PTO_HIP_OK) return rc;
     p.part_o = reinterpret_cast<float*>(ws);
     p.part_ml = reinterpret_cast<float*>(reinterpret_cast<char*>(ws) + o_bytes);
+    if (p.n_part <= most_unmerged && measuring < 0) {  // (a measured launch shape is compared with its merge)
+      p.no_merge = 1;
+      *unmerged = AttnPartials{p.part_ml, p.part_o, context_lens, p.n_part, p.tpp, p.ctx_cap};
+    }
   }
   // "attn_variant" 1 selects the evenly split form (one pinned workgroup per CU).
   p.n_wg = 0;

@@ -72,6 +72,12 @@ int layer_workspace(size_t bytes, void** ptr) {
   return rc;
 }
 
+bool stream_capturing(hipStream_t st) {
+  hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(st, &capturing) == hipSuccess) return capturing != hipStreamCaptureStatusNone;
+  (void)hipGetLastError();
+  return true;
+}
 int gemm_slabs(size_t bytes, hipStream_t st, void** ptr) {
   Context& c = ctx();
   if (bytes > c.gemm_ws_bytes) {
@@ -1096,6 +1102,9 @@ int pto_hip_set_option(const char* name, int64_t value) {
   } else if (!std::strcmp(name, "w8a16_wide")) {
     PTO_CHECK_ARG(value >= 0 && value <= 2, "w8a16_wide must be 0, 1 or 2");
     c.w8a16_wide = value;
+  } else if (!std::strcmp(name, "skinny_fuse")) {
+    PTO_CHECK_ARG(value >= 0 && value <= 7, "skinny_fuse must be in [0, 7]");
+    c.skinny_fuse = value;
   } else if (!std::strcmp(name, "w8a16_min_steps")) {
     PTO_CHECK_ARG(value >= 1 && value <= 1024, "w8a16_min_steps must be in [1, 1024]");
     c.w8a16_min_steps = value;
@@ -1159,6 +1168,7 @@ int pto_hip_get_option(const char* name, int64_t* value) {
   else if (!std::strcmp(name, "attn_group_tiles")) *value = c.attn_group_tiles;
   else if (!std::strcmp(name, "w8a16_wgs_per_cu")) *value = c.w8a16_wgs_per_cu;
   else if (!std::strcmp(name, "w8a16_min_steps")) *value = c.w8a16_min_steps;
+  else if (!std::strcmp(name, "skinny_fuse")) *value = c.skinny_fuse;
   else if (!std::strcmp(name, "w8a16_wide")) *value = c.w8a16_wide;
   else if (!std::strcmp(name, "w8a16_gemm_rows")) *value = c.w8a16_gemm_rows;
   else return fail(PTO_HIP_ERR_NOT_FOUND, "unknown option '%s'", name);

@@ -29,247 +29,13 @@
 
 #include "common.h"
 #include "launch_choice.h"
-#include "slab_sum.h"
+#include "skinny.h"
 
 namespace {
 
-typedef __attribute__((__vector_size__(4 * sizeof(float)))) float f32x4;
-typedef __attribute__((__vector_size__(4 * sizeof(uint32_t)))) uint32_t u32x4;
-typedef __attribute__((__vector_size__(8 * sizeof(__bf16)))) __bf16 bf16x8;
-typedef __attribute__((__vector_size__(8 * sizeof(_Float16)))) _Float16 f16x8;
-
-constexpr int kStep = 32;                // k rows per step
-constexpr int kMaxM = pto_hip::kW8MaxM;
-constexpr int kWaves = 4;                // wavefronts per workgroup of the partial kernel
-
-struct GemvParams {
-  const uint16_t* x;    // [M, K] 16-bit activations
-  const void* wq[2];    // [K, N] each (int8 codes or 16-bit weights); the second is the up projection of a pair
-  float* part[2];       // [partial slabs, M, N] each
-  int m, k, n, x_blocked;  // x_blocked: activations stored [K/8][32][8] (see w8a16_partials) instead of row-major
-  int slabs, ks;        // output slabs of one matrix, 32-row steps of one slab
-  int per_wg, extra;    // units / workgroups and its remainder (see SlabMap)
-  int mapped;           // 0: a workgroup per slab
-};
-
-template <bool BF16>
-__device__ __forceinline__ f32x4 mfma16(u32x4 a, u32x4 b, f32x4 c) {
-  if constexpr (BF16) {
-    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a),
-                                                   __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
-  } else {
-    return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, a),
-                                                  __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
-  }
-}
-
-// Two small integers held as fp32 -> packed pair of 16-bit floats, exact.
-template <bool BF16>
-__device__ __forceinline__ uint32_t pack_pair(float lo, float hi) {
-  if constexpr (BF16) {
-    // |value| <= 128 has at most 8 significant bits: the upper half of the fp32 pattern is the bf16.
-    return __builtin_amdgcn_perm(__builtin_bit_cast(uint32_t, hi), __builtin_bit_cast(uint32_t, lo),
-                                 0x07060302u);
-  } else {
-    return __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(lo, hi));
-  }
-}
-
-typedef uint32_t u32x2 __attribute__((__vector_size__(2 * sizeof(uint32_t))));
-
-// One register stage of a lane: kCols channels of the k rows kg*8 .. kg*8+7, and the activations.
-// W8: int8 weight codes, 8 bytes (kCols 8) or 16 bytes (kCols 16) per row and lane; otherwise
-// 16-bit weights of the activation type (16 bytes = 8 channels).
-template <bool W8, int kCols, int MT>
-struct Stage {
-  typename std::conditional<(W8 && kCols == 8), u32x2, u32x4>::type w[8];
-  u32x4 xa[MT];  // activations of rows c (and c+16), k = kg*8 .. +8
-};
-
-// Workgroup w of G takes the units (slab, 32-row step) [w U / G, (w + 1) U / G) of the list that walks the
-// slabs one after the other (SlabMap): every workgroup streams the same number of bytes.  A launch lasts as
-// long as the CU with the most bytes: cut into equal k ranges instead, 272 workgroups of a 356 MB pair of 16-bit
-// matrices on 256 CUs read at 4.5 TB/s and 544 at 5.3, where 256 even shares reach 6.5 (load-only twins of
-// this kernel).  The four wavefronts take a run's steps in turn; when
-// a run ends (the slab's last step or the workgroup's) their accumulators are summed through LDS, one after
-// the other, and written as the next partial slab of those channels; the next run's first rows
-// are in flight meanwhile.  MT: 16-row groups of activations (M <= 16 needs one: half the MFMAs,
-// activations and partial sums).  Rows past M are computed on row M - 1 and not written.
-template <bool BF16, bool W8, int kCols, int MT, bool NT>
-__global__ __launch_bounds__(kWaves * 64) __attribute__((amdgpu_waves_per_eu(1, 2))) void w8a16_partial_kernel(GemvParams p) {
-  static_assert(kCols == 8 || (W8 && kCols == 16), "16 channels per lane only with int8 codes");
-  constexpr int kSlab = 16 * kCols;  // output channels of a slab: 16 lanes of kCols channels
-  constexpr int kRows = 16 * MT;
-  extern __shared__ __attribute__((aligned(16))) float red[];  // [kWaves][kRows][kSlab]
-  const int tid = threadIdx.x, lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // uniform: row addresses stay scalar
-  const int c = lane & 15, kg = lane >> 4;
-
-  // this workgroup's units, and a cursor over them in rounds of kWaves steps of one slab
-  const int wg = blockIdx.x, wgs = gridDim.x;
-  const int u_begin = wg * p.per_wg + wg * p.extra / wgs, u_end = (wg + 1) * p.per_wg + (wg + 1) * p.extra / wgs;
-  struct Cursor {
-    int slab, step, end;  // the round's first step and the end of its run
-  };
-  auto run_end = [&](int slab) { return min(p.ks, u_end - slab * p.ks); };
-  auto last_of_run = [&](const Cursor& cur) { return cur.step + kWaves >= cur.end; };
-  auto last = [&](const Cursor& cur) { return last_of_run(cur) && cur.slab * p.ks + cur.end >= u_end; };
-  auto advance = [&](Cursor& cur) {
-    if (!last_of_run(cur)) {
-      cur.step += kWaves;
-    } else {
-      cur.slab += 1;
-      cur.step = 0;
-      cur.end = run_end(cur.slab);
-    }
-  };
-
-  // Row-major x: lane (c, kg) reads 16 bytes of rows c and c+16 at k = kstep + 8*kg.  Blocked x
-  // keeps the 32 rows of each 8-k group together, so the same reads of a wavefront cover
-  // consecutive bytes instead of half cache lines.
-  const int x_step = p.x_blocked ? kMaxM : 1;  // elements per unit of k
-  const uint16_t* xp[MT];
-#pragma unroll
-  for (int h = 0; h < MT; ++h) {
-    const int row = min(c + 16 * h, p.m - 1);
-    xp[h] = p.x_blocked ? p.x + (size_t)(kg * kMaxM + row) * 8 : p.x + (size_t)row * p.k + kg * 8;
-  }
-
-  f32x4 acc[kCols][MT];
-  auto clear = [&] {
-#pragma unroll
-    for (int i = 0; i < kCols; ++i)
-#pragma unroll
-      for (int h = 0; h < MT; ++h) acc[i][h] = f32x4{0.f, 0.f, 0.f, 0.f};
-  };
-  clear();
-
-  // Loads never depend on a condition, so the number of requests in flight is known at compile
-  // time: a wavefront without a step of its own in a round reads the run's last one again, and a last step
-  // that would reach past row k is moved back to end at row k - the rows it then repeats are
-  // multiplied by zeroed activations.  A row address is a wavefront-uniform row base plus a
-  // per-lane offset.
-  constexpr int kWBytes = W8 ? 1 : 2;  // bytes per weight
-  typedef typename std::conditional<(W8 && kCols == 8), u32x2, u32x4>::type wvec_t;
-  auto load = [&](Stage<W8, kCols, MT>& s, const Cursor& cur) {
-    const int row0 = min(min(cur.step + wave, cur.end - 1) * kStep, p.k - kStep);
-    const int mat = cur.slab >= p.slabs ? 1 : 0;
-    const int n0 = min((cur.slab - mat * p.slabs) * kSlab + c * kCols, p.n - kCols);
-    const size_t lane_off = ((size_t)n0 + (size_t)(kg * 8) * p.n) * kWBytes;
-    const char* wbase = reinterpret_cast<const char*>(p.wq[mat]) + (size_t)row0 * p.n * kWBytes;
-#pragma unroll
-    for (int h = 0; h < MT; ++h) s.xa[h] = *reinterpret_cast<const u32x4*>(xp[h] + (size_t)row0 * x_step);
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      const char* row = wbase + (size_t)e * p.n * kWBytes;  // uniform
-      if constexpr (NT) s.w[e] = __builtin_nontemporal_load(reinterpret_cast<const wvec_t*>(row + lane_off));
-      else s.w[e] = *reinterpret_cast<const wvec_t*>(row + lane_off);
-    }
-  };
-  auto compute = [&](const Stage<W8, kCols, MT>& s, const Cursor& cur) {
-    const int step = cur.step + wave;
-    if (step >= cur.end) return;  // uniform: no step for this wavefront in this round
-    const bool k_ok = min(step * kStep, p.k - kStep) + kg * 8 >= step * kStep;
-    u32x4 a[MT];
-#pragma unroll
-    for (int h = 0; h < MT; ++h) a[h] = k_ok ? s.xa[h] : u32x4{0u, 0u, 0u, 0u};
-#pragma unroll
-    for (int i = 0; i < kCols; ++i) {
-      // channel n0 + i: its 8 k-values, as packed pairs (k, k+1)
-      u32x4 b;
-      if constexpr (W8) {
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          const uint32_t w0 = s.w[2 * q][i >> 2];
-          const uint32_t w1 = s.w[2 * q + 1][i >> 2];
-          const float f0 = (float)(int8_t)(w0 >> ((i & 3) * 8));
-          const float f1 = (float)(int8_t)(w1 >> ((i & 3) * 8));
-          b[q] = pack_pair<BF16>(f0, f1);
-        }
-      } else {
-        // 16-bit weights: element i of rows 2q and 2q+1 (an 8x8 transpose in registers)
-        const uint32_t sel = (i & 1) ? 0x07060302u : 0x05040100u;
-#pragma unroll
-        for (int q = 0; q < 4; ++q) b[q] = __builtin_amdgcn_perm(s.w[2 * q + 1][i >> 1], s.w[2 * q][i >> 1], sel);
-      }
-#pragma unroll
-      for (int h = 0; h < MT; ++h) acc[i][h] = mfma16<BF16>(a[h], b, acc[i][h]);
-      __builtin_amdgcn_sched_barrier(0);  // keep the conversions next to their MFMAs
-    }
-  };
-
-  // End of a run: the wavefronts' accumulators through LDS into one partial slab.  acc[i][h][r] is row
-  // h*16 + 4*kg + r, channel c*kCols + i; the float4s of a row are kept in the order (v, c) - channels c*kCols + 4v .. -
-  // so that neither the writes nor the reads of 16 lanes collide in a bank.
-  constexpr int kQuads = kSlab / 4;
-  auto finish_run = [&](const Cursor& cur) {
-    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");  // the last run's sums have been read
-    float4* mine = reinterpret_cast<float4*>(red) + wave * (kRows * kQuads) + c;
-#pragma unroll
-    for (int h = 0; h < MT; ++h)
-#pragma unroll
-      for (int r = 0; r < 4; ++r)
-#pragma unroll
-        for (int v = 0; v < kCols / 4; ++v)
-          mine[(h * 16 + 4 * kg + r) * kQuads + v * 16] =
-              float4{acc[4 * v][h][r], acc[4 * v + 1][h][r], acc[4 * v + 2][h][r], acc[4 * v + 3][h][r]};
-    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-    const int mat = cur.slab >= p.slabs ? 1 : 0;
-    // partial slab number: how many workgroups before this one hold steps of the slab (the one
-    // that holds its first unit has number 0)
-    const int first = cur.slab * p.ks;
-    const int owner = p.mapped ? (int)(((unsigned)(first + 1) * (unsigned)wgs - 1) / (unsigned)(p.per_wg * wgs + p.extra)) : wg;
-    const int q = tid % kQuads, n = (cur.slab - mat * p.slabs) * kSlab + (q & 15) * kCols + (q >> 4) * 4;
-    float* out = p.part[mat] + (size_t)(wg - owner) * p.m * p.n + n;
-    if (n < p.n) {
-      for (int row = tid / kQuads; row < p.m; row += kWaves * 64 / kQuads) {
-        const float4* src = reinterpret_cast<const float4*>(red) + row * kQuads + q;
-        float4 a = src[0];
-#pragma unroll
-        for (int w = 1; w < kWaves; ++w) {
-          const float4 v = src[w * (kRows * kQuads)];
-          a.x += v.x; a.y += v.y; a.z += v.z; a.w += v.w;
-        }
-        *reinterpret_cast<float4*>(out + (size_t)row * p.n) = a;
-      }
-    }
-    clear();
-  };
-
-  Cursor use, ahead;
-  use.slab = u_begin / p.ks;
-  use.step = u_begin - use.slab * p.ks;
-  use.end = run_end(use.slab);
-  ahead = use;
-  // Two register stages, one of them in flight while the other is multiplied (three and four measured slower: one
-  // sequence's layer 75.2 -> 77.8 / 79.2 us).  The last round is a copy of its own that requests nothing:
-  // behind a branch around the loads the compiler would wait for all of them in every round, and reading
-  // the last rows again costs as much as a new round.
-  Stage<W8, kCols, MT> st[2];
-  load(st[0], ahead);
-  auto round = [&](const Stage<W8, kCols, MT>& cur) {
-    compute(cur, use);
-    if (last_of_run(use)) finish_run(use);
-  };
-  for (;;) {
-    if (last(use)) {
-      round(st[0]);
-      break;
-    }
-    advance(ahead);
-    load(st[1], ahead);
-    round(st[0]);
-    advance(use);
-    if (last(use)) {
-      round(st[1]);
-      break;
-    }
-    advance(ahead);
-    load(st[0], ahead);
-    round(st[1]);
-    advance(use);
-  }
-}
+using namespace pto_hip::skinny;
+using pto_hip::SlabMap;
+using pto_hip::slab_count;
 
 struct FinishParams {
   const float* part0;   // [splits, 32 or M, N]: `stride` elements between splits
@@ -281,7 +47,7 @@ struct FinishParams {
   int m, n, splits, res_dtype, out_dtype;
   int out_blocked;  // write out as [N/8][32][8] for the next projection
   int64_t stride;
-  pto_hip::SlabMap map;
+  SlabMap map;
 };
 
 // Element index of (row m, channel n) in the blocked activation layout [N/8][32][8].
@@ -310,35 +76,6 @@ __device__ __forceinline__ void store4_from_f32(void* p, size_t i, int dt, float
   }
 }
 
-// Sums of the k splits of four channels of K matrices with `splits` slabs each, in split order, times the channel scales.
-template <int K>
-__device__ __forceinline__ void sum_splits(const float* const (&part)[K], const float* const (&scale)[K], int splits,
-                                           size_t stride, int m, int n, int nn, f32x4 (&sum)[K]) {
-  const float* src[K];
-  f32x4 sc[K];
-#pragma unroll
-  for (int k = 0; k < K; ++k) {
-    src[k] = part[k] + (size_t)m * nn + n;
-    sum[k] = f32x4{0.f, 0.f, 0.f, 0.f};
-    sc[k] = scale[k] ? *reinterpret_cast<const f32x4*>(scale[k] + n) : f32x4{1.f, 1.f, 1.f, 1.f};  // none: unquantised weights
-  }
-  pto_hip::add_slabs(src, splits, stride, sum);
-#pragma unroll
-  for (int k = 0; k < K; ++k) sum[k] *= sc[k];
-}
-__device__ __forceinline__ float4 sum_splits(const float* part, const float* scale, int splits, size_t stride, int m,
-                                             int n, int nn) {
-  const float* parts[1] = {part};
-  const float* scales[1] = {scale};
-  f32x4 sum[1];
-  sum_splits<1>(parts, scales, splits, stride, m, n, nn, sum);
-  return float4{sum[0][0], sum[0][1], sum[0][2], sum[0][3]};
-}
-
-__device__ __forceinline__ float silu_mul(float g, float u) {
-  return g * __frcp_rn(1.f + __expf(-g)) * u;  // SiLU(gate) * up, device form of 01_ffn.py:70-75
-}
-
 __global__ __launch_bounds__(256) void w8a16_finish_kernel(FinishParams p) {
   const int n = (blockIdx.x * 256 + threadIdx.x) * 4;
   const int m = blockIdx.y;
@@ -346,25 +83,11 @@ __global__ __launch_bounds__(256) void w8a16_finish_kernel(FinishParams p) {
   const size_t idx = (size_t)m * p.n + n;
   float4 r = {0.f, 0.f, 0.f, 0.f};  // requested with the slabs
   if (p.residual) r = load4_as_f32(p.residual, idx, p.res_dtype);
-  const int splits0 = pto_hip::slab_count(p.map, p.splits, 0, n);
   float4 a;
   if (p.part1) {
-    const int splits1 = pto_hip::slab_count(p.map, p.splits, 1, n);
-    float4 u;
-    if (splits0 == splits1) {
-      const float* parts[2] = {p.part0, p.part1};
-      const float* scales[2] = {p.scale0, p.scale1};
-      f32x4 sum[2];
-      sum_splits<2>(parts, scales, splits0, (size_t)p.stride, m, n, p.n, sum);
-      a = float4{sum[0][0], sum[0][1], sum[0][2], sum[0][3]};
-      u = float4{sum[1][0], sum[1][1], sum[1][2], sum[1][3]};
-    } else {
-      a = sum_splits(p.part0, p.scale0, splits0, (size_t)p.stride, m, n, p.n);
-      u = sum_splits(p.part1, p.scale1, splits1, (size_t)p.stride, m, n, p.n);
-    }
-    a = float4{silu_mul(a.x, u.x), silu_mul(a.y, u.y), silu_mul(a.z, u.z), silu_mul(a.w, u.w)};
+    a = swiglu_quad(p.part0, p.part1, p.scale0, p.scale1, p.map, p.splits, (size_t)p.stride, m, n, p.n);
   } else {
-    a = sum_splits(p.part0, p.scale0, splits0, (size_t)p.stride, m, n, p.n);
+    a = sum_splits(p.part0, p.scale0, slab_count(p.map, p.splits, 0, n), (size_t)p.stride, m, n, p.n);
   }
   if (p.residual) {
     a.x += r.x; a.y += r.y; a.z += r.z; a.w += r.w;
@@ -388,7 +111,7 @@ struct FinishNormParams {
   int out_blocked;
   float eps;
   int64_t stride;  // elements between splits
-  pto_hip::SlabMap map;
+  SlabMap map;
 };
 
 __global__ __launch_bounds__(kNormThreads) void w8a16_finish_norm_kernel(FinishNormParams p) {
@@ -402,7 +125,7 @@ __global__ __launch_bounds__(kNormThreads) void w8a16_finish_norm_kernel(FinishN
     if (n < p.n) {
       g[u] = *reinterpret_cast<const float4*>(p.gamma + n);
       const float4 r = load4_as_f32(p.residual, (size_t)m * p.n + n, p.res_dtype);
-      float4 a = sum_splits(p.part, p.scale, pto_hip::slab_count(p.map, p.splits, 0, n), (size_t)p.stride, m, n, p.n);
+      float4 a = sum_splits(p.part, p.scale, slab_count(p.map, p.splits, 0, n), (size_t)p.stride, m, n, p.n);
       a.x += r.x; a.y += r.y; a.z += r.z; a.w += r.w;
       v[u] = a;
       *reinterpret_cast<float4*>(p.sum_out + (size_t)m * p.n + n) = a;
@@ -465,8 +188,82 @@ int launch_partial(const GemvParams& p, int wgs, bool nt, hipStream_t st) {
 
 namespace pto_hip {
 
+int skinny_norm_launch(const skinny::GemvParams& p, bool bf16, bool w16, bool wide, int wgs, size_t smem, hipStream_t st);
+int skinny_swiglu_launch(const skinny::GemvParams& p, bool bf16, bool w16, bool wide, int wgs, size_t smem, hipStream_t st);
+int skinny_merge_launch(const skinny::GemvParams& p, bool bf16, bool w16, bool wide, int wgs, size_t smem, hipStream_t st);
+
+namespace {
+// How a projection's units fall to workgroups.
+struct SkinnyPlan {
+  bool wide, mapped;
+  int cols, slabs, ks, splits, per_slab;  // per_slab: workgroups of every slab; 0: shares cross slabs
+  int64_t units, wgs;
+};
+SkinnyPlan plan_skinny(int64_t k, int64_t n, const void* wq0, const void* wq1, bool w16) {
+  const Context& cx = ctx();
+  const int n_mats = wq1 ? 2 : 1;
+  SkinnyPlan q{};
+  // int8 codes are read 16 per lane (256-channel slabs, 256-byte row pieces instead of 128) when rows and base
+  // addresses allow 16-byte loads and the matrices are large.  Twice the channels in a slab are twice the partial
+  // sums at the same number of workgroups, and 32 instead of 16 KB per wavefront through LDS at the end of a run.
+  // Measured with their finish at 1 / 16 / 32 rows: 178 MB 36.0 / 38.8 / 44.6 us (8 per lane: 36.4 / 42.0 / 50.2), 117 MB
+  // 24.1 / 26.0 / 29.6 (25.6 / 29.2 / 34.0), 89 MB 20.4 / 22.1 / 25.7 (21.9 / 24.9 / 28.6); but 67 MB 16.5 / 18.2 / 21.7
+  // (15.6 / 17.7 / 20.7), 59 MB 15.8 / 17.5 / 20.7 (14.7 / 16.5 / 19.2), 17 MB 9.0 / 10.5 / 12.7 (8.2 / 9.3 / 10.8).
+  q.wide = !w16 && cx.w8a16_wide != 0 && n % 16 == 0 && ((uintptr_t)wq0 | (uintptr_t)wq1) % 16 == 0 &&
+           (cx.w8a16_wide == 2 || k * n * n_mats >= (int64_t)80 * 1000 * 1000);
+  q.cols = q.wide ? 16 : 8;
+  const int slab = 16 * q.cols;
+  q.slabs = (int)((n + slab - 1) / slab);
+  q.ks = (int)((k + kStep - 1) / kStep);
+  const int64_t slabs_total = (int64_t)q.slabs * n_mats;
+  q.units = slabs_total * q.ks;
+  q.wgs = skinny_workgroups(slabs_total, q.ks, std::max<int64_t>(1, cx.w8a16_wgs_per_cu * cx.num_cu), cx.w8a16_min_steps);
+  // (units * wgs is computed in 32 bits by the kernels; shapes beyond that get a workgroup per slab)
+  q.mapped = q.units * q.wgs < (1ll << 31);
+  if (!q.mapped) q.wgs = slabs_total;
+  q.splits = q.mapped ? (int)((q.ks * q.wgs + q.units - 1) / q.units) + 1 : 1;  // at most
+  q.per_slab = q.wgs % slabs_total == 0 && q.wgs / slabs_total <= q.ks ? (int)(q.wgs / slabs_total) : 0;
+  return q;
+}
+// LDS of the fused form: the sums and m rows of a share.
+size_t fused_lds(const SkinnyPlan& q, int64_t m) {
+  const size_t span = ((size_t)q.ks + q.per_slab - 1) / q.per_slab * kStep + kStep;
+  return (size_t)kWaves * 16 * 16 * q.cols * sizeof(float) + (size_t)m * (span + 8) * 2;
+}
+}  // namespace
+
+// The launch saved is 2 to 5 us of a chain of ten; what is made instead is made by every workgroup, so it pays while a thread's part is
+// held in registers at once, one round trip to the caches (decoder layer, us, one / two rows, separate launch -> made here):
+// kNorm, up to 4 rows: 4096 wide int8 71.9 / 75.1 -> 70.4 / 73.1, 2048 wide 48.5 / 49.9 -> 46.8 / 48.3.
+// kSwiglu: 5632 -> 2048 channels (352 k rows a share) 48.5 / 49.9 -> 46.9 / 48.6; 14336 -> 4096 (1792) 55.2 -> 54.4 in one round trip, but 75.1 -> 76.7
+// for two rows in two; 20032 -> 8192 (5008) 142.9 -> 144.0.
+// kMerge: a head a wavefront (32 heads, 4096 wide) 71.9 -> 69.7, two 75.1 -> 75.0, three (40 heads, 8192 wide) 142.9 -> 145.4; 63 partitions, a loop
+// past the 32 held, 38.3 -> 42.6.
+bool skinny_fuses(ProjectionSource::Kind kind, int64_t m, int64_t k, int64_t n, const void* wq0, const void* wq1, bool w16, int64_t head_dim) {
+  const Context& cx = ctx();
+  if (!(cx.skinny_fuse >> (kind - 1) & 1) || cx.w8a16_nt == 0 || m > kSkinnyFusedRows || k % 16 != 0 || k < kStep) return false;
+  const SkinnyPlan q = plan_skinny(k, n, wq0, wq1, w16);
+  if (q.per_slab == 0 || fused_lds(q, m) > (size_t)kFusedLds) return false;
+  const int64_t share = ((int64_t)q.ks + q.per_slab - 1) / q.per_slab * kStep;
+  switch (kind) {
+    case ProjectionSource::kNorm: return k <= 8 * 256 * kNormVecs && share + (k % kStep ? kStep : 0) <= 8 * 256 * kNormOwn;
+    case ProjectionSource::kSwiglu: return m * share <= 1536;
+    case ProjectionSource::kMerge: {
+      const bool whole = q.ks % q.per_slab == 0 && share % head_dim == 0;
+      return m * (whole ? share / head_dim : share / head_dim + 2) <= kWaves;
+    }
+    default: return false;
+  }
+}
+
+size_t skinny_fused_bytes(int64_t k, int64_t n, const void* wq0, const void* wq1, bool w16) {
+  const SkinnyPlan q = plan_skinny(k, n, wq0, wq1, w16);
+  return (size_t)q.splits * kSkinnyFusedRows * n * sizeof(float) * (wq1 ? 2 : 1);
+}
+
 int w8a16_partials(const void* x, bool x_blocked, const void* wq0, const void* wq1, int64_t m, int64_t k, int64_t n,
-                   int x_dtype, hipStream_t st, W8Partials* out, bool w16) {
+                   int x_dtype, hipStream_t st, W8Partials* out, bool w16, const ProjectionSource* src, float* area) {
+  const SkinnyPlan q = plan_skinny(k, n, wq0, wq1, w16);
   GemvParams p{};
   p.x = reinterpret_cast<const uint16_t*>(x);
   p.wq[0] = wq0;
@@ -475,46 +272,46 @@ int w8a16_partials(const void* x, bool x_blocked, const void* wq0, const void* w
   p.k = (int)k;
   p.n = (int)n;
   p.x_blocked = x_blocked ? 1 : 0;
-  const Context& cx = ctx();
-  const int n_mats = wq1 ? 2 : 1;
-  // int8 codes are read 16 per lane (256-channel slabs, 256-byte row pieces instead of 128) when rows and base
-  // addresses allow 16-byte loads and the matrices are large.  Twice the channels in a slab are twice the partial
-  // sums at the same number of workgroups, and 32 instead of 16 KB per wavefront through LDS at the end of a run.
-  // Measured with their finish at 1 / 16 / 32 rows: 178 MB 36.0 / 38.8 / 44.6 us (8 per lane: 36.4 / 42.0 / 50.2), 117 MB
-  // 24.1 / 26.0 / 29.6 (25.6 / 29.2 / 34.0), 89 MB 20.4 / 22.1 / 25.7 (21.9 / 24.9 / 28.6); but 67 MB 16.5 / 18.2 / 21.7
-  // (15.6 / 17.7 / 20.7), 59 MB 15.8 / 17.5 / 20.7 (14.7 / 16.5 / 19.2), 17 MB 9.0 / 10.5 / 12.7 (8.2 / 9.3 / 10.8).
-  const bool wide = !w16 && cx.w8a16_wide != 0 && n % 16 == 0 && ((uintptr_t)wq0 | (uintptr_t)wq1) % 16 == 0 &&
-                    (cx.w8a16_wide == 2 || k * n * n_mats >= (int64_t)80 * 1000 * 1000);
-  const int cols = wide ? 16 : 8, slab = 16 * cols;
-  p.slabs = (int)((n + slab - 1) / slab);
-  p.ks = (int)((k + kStep - 1) / kStep);
-  const int64_t slabs_total = (int64_t)p.slabs * n_mats, units = slabs_total * p.ks;
-  int64_t wgs = skinny_workgroups(slabs_total, p.ks, std::max<int64_t>(1, cx.w8a16_wgs_per_cu * cx.num_cu), cx.w8a16_min_steps);
-  // (units * wgs is computed in 32 bits by the kernels; shapes beyond that get a workgroup per slab)
-  const bool mapped = units * wgs < (1ll << 31);
-  if (!mapped) wgs = slabs_total;
-  p.per_wg = (int)(units / wgs);
-  p.extra = (int)(units % wgs);
-  p.mapped = mapped ? 1 : 0;
-  out->map = mapped ? SlabMap{(unsigned)units, (unsigned)wgs, (unsigned)p.ks, wide ? 8 : 7, p.slabs} : SlabMap{};
-  out->splits = mapped ? (int)((p.ks * wgs + units - 1) / units) + 1 : 1;  // at most
+  p.slabs = q.slabs;
+  p.ks = q.ks;
+  p.per_wg = (int)(q.units / q.wgs);
+  p.extra = (int)(q.units % q.wgs);
+  p.mapped = q.mapped ? 1 : 0;
+  p.per_slab = q.per_slab;
+  out->map = q.mapped ? SlabMap{(unsigned)q.units, (unsigned)q.wgs, (unsigned)q.ks, q.wide ? 8 : 7, q.slabs} : SlabMap{};
+  out->splits = q.splits;
   // scratch for 32 rows whatever m: a call sized once fits every smaller and larger batch of the shape, also under capture
-  const size_t one = (size_t)out->splits * kMaxM * n * sizeof(float);
-  void* ws = nullptr;
-  int rc = workspace(one * n_mats, &ws);
-  if (rc) return rc;
-  p.part[0] = reinterpret_cast<float*>(ws);
-  p.part[1] = reinterpret_cast<float*>(reinterpret_cast<char*>(ws) + one);
+  size_t one = (size_t)q.splits * kMaxM * n * sizeof(float);
+  int rc = PTO_HIP_OK;
+  if (area) {
+    one = (size_t)q.splits * kSkinnyFusedRows * n * sizeof(float);
+  } else {
+    void* ws = nullptr;
+    if ((rc = workspace(one * (wq1 ? 2 : 1), &ws))) return rc;
+    area = reinterpret_cast<float*>(ws);
+  }
+  p.part[0] = area;
+  p.part[1] = reinterpret_cast<float*>(reinterpret_cast<char*>(area) + one);
+  const Context& cx = ctx();
   const bool bf = x_dtype == PTO_HIP_BF16, nt = cx.w8a16_nt != 0, two = m > 16;
-  auto go = [&](auto w8, auto kcols) {
-    constexpr bool W8 = decltype(w8)::value;
-    constexpr int C = decltype(kcols)::value;
-    if (bf) return two ? launch_partial<true, W8, C, 2>(p, (int)wgs, nt, st) : launch_partial<true, W8, C, 1>(p, (int)wgs, nt, st);
-    return two ? launch_partial<false, W8, C, 2>(p, (int)wgs, nt, st) : launch_partial<false, W8, C, 1>(p, (int)wgs, nt, st);
-  };
-  typedef std::integral_constant<int, 8> C8;
-  typedef std::integral_constant<int, 16> C16;
-  rc = w16 ? go(std::false_type{}, C8{}) : wide ? go(std::true_type{}, C16{}) : go(std::true_type{}, C8{});
+  const int wgs = (int)q.wgs;
+  if (src && src->kind != ProjectionSource::kTensor) {
+    p.src = *src;
+    const size_t smem = fused_lds(q, m);
+    rc = src->kind == ProjectionSource::kNorm     ? skinny_norm_launch(p, bf, w16, q.wide, wgs, smem, st)
+         : src->kind == ProjectionSource::kSwiglu ? skinny_swiglu_launch(p, bf, w16, q.wide, wgs, smem, st)
+                                                  : skinny_merge_launch(p, bf, w16, q.wide, wgs, smem, st);
+  } else {
+    auto go = [&](auto w8, auto kcols) {
+      constexpr bool W8 = decltype(w8)::value;
+      constexpr int C = decltype(kcols)::value;
+      if (bf) return two ? launch_partial<true, W8, C, 2>(p, wgs, nt, st) : launch_partial<true, W8, C, 1>(p, wgs, nt, st);
+      return two ? launch_partial<false, W8, C, 2>(p, wgs, nt, st) : launch_partial<false, W8, C, 1>(p, wgs, nt, st);
+    };
+    typedef std::integral_constant<int, 8> C8;
+    typedef std::integral_constant<int, 16> C16;
+    rc = w16 ? go(std::false_type{}, C8{}) : q.wide ? go(std::true_type{}, C16{}) : go(std::true_type{}, C8{});
+  }
   if (rc) return rc;
   out->part[0] = p.part[0];
   out->part[1] = wq1 ? p.part[1] : nullptr;
