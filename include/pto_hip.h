@@ -547,6 +547,10 @@ PTO_HIP_API int pto_hip_backend_handler_query(const char* hook, int32_t arg, cha
  *                               loaded with the non-temporal hint so that they do not displace what other
  *                               kernels keep in the caches (default); 0 = ordinary loads
  *  "attn_tuned_waves_per_cu"    read only: the cap the last launch's signature settled on (-1 = not yet)
+ *  "attn_order"                 sequences worked through by length, so that every CU gets long and short ones
+ *                               (partition grid and workgroup form, up to 256 sequences; same bits): -1 = where
+ *                               the first calls of a shape measure it faster (default), 0 = never, 1 = always
+ *  "attn_tuned_order"           read only: 1 when the last launch's shape settled on that order, 0 not, -1 = not yet
  *  "attn_tuned_workgroup_form"  read only: 1 when it settled on the workgroup form, 0 the grid, -1 = not yet
  *  "workspace_bytes"            read only: bytes of device memory the library's grow-only scratch areas hold
  *  "attn_kernel_timing"         1 = every paged-attention launch gives its streaming kernel a start and a stop

@@ -75,6 +75,7 @@ struct Context {
   int64_t w8a16_wide = 1;        // int8 codes read 16 per lane: 0 never, 1 for large matrices, 2 whenever shapes allow
   int64_t skinny_fuse = 7;         // skinny projections of up to four rows make their activations themselves: 1 norm, 2 SwiGLU, 4 merge
   int64_t w8a16_min_steps = 2;   // fewest 32-row steps per wavefront before k is split further
+  int64_t attn_order = -1;         // sequences by length: -1 where measured faster, 0 never, 1 always (partition grid and workgroup form)
   int64_t w8a16_gemm_rows = 33;  // rows from which int8 projections run as a tiled GEMM (0 = never)
 };
 
@@ -228,8 +229,8 @@ int paged_attention(const void* query, const void* key_cache, const void* value_
 // not being measured then leaves it out and describes them there, `out` and `out16` unwritten; otherwise n_part comes back 0.
 // Forgets every measured launch shape (and releases the events of measurements in flight).
 void attention_tuning_reset();
-// Residency cap and form (1 = workgroup form) the last launch's signature was tuned to; -1 while untuned.
-void attention_tuning_last(int64_t* cap, int64_t* wg);
+// Residency cap, form (1 = workgroup form) and order (1 = sequences by length) the last launch's signature was tuned to; -1 while untuned.
+void attention_tuning_last(int64_t* cap, int64_t* wg, int64_t* ordered);
 // The same contract for the shapes the tiled kernels are not built for (head_dim other than 128 / 256
 // up to 256, block sizes off the 16-token grid); attention_needs_generic says which launches take it.
 bool attention_needs_generic(const int64_t* config, int kv_dtype);

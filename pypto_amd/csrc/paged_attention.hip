@@ -67,6 +67,8 @@ struct AttnParams {
   int lean_waves;  // ... and wavefronts in each
   float scale_log2e;
   int no_merge;    // partition grid: the partials are left as they are
+  int order_band;  // partition grid and workgroup form: sequences by length, in bands of this many pairs (ordered_pair); 0: as they come
+  int order_bits, order_shift;  // bits of a key and of a sequence's number in it
 };
 
 template <bool BF16>
@@ -652,6 +654,42 @@ __device__ __forceinline__ void attend_range_pair(const AttnParams& p, int b, in
   }
 }
 
+// The pair a workgroup takes when sequences are worked through by length.  The hardware places workgroups in order and, as a CU
+// takes several at once or one after the other, what a CU streams is the sum of what a stride of the pairs holds: of sequences as they come,
+// long ones meet on some CUs by chance and the launch waits for those.  Here the pairs are dealt in bands of one per CU, the sequences of
+// falling length and every other band backwards, so that the sums are alike.  A sequence's place is found by every wavefront for itself:
+// key = (32-token chunks, number), unique; the wanted-th largest key bit by bit, one comparison of all keys and a
+// count per bit: about 20 rounds, half a microsecond, behind one load of the lengths.  That is what a launch of equal lengths would lose, so it is one
+// of the shapes the first calls measure.  Attention call, us, lengths in random order as they come -> so: 96 x 8 pairs of 200 to 3000
+// tokens e4m3 67.5 -> 57.4; 225 pairs of 667 to 3121 e4m3, head_dim 256 54.3 -> 47.8; 63 x 8 of 877 to 2373, 128 heads, head_dim 256 147 -> 135;
+// no gain where a launch streams at the memory's rate anyway (16-bit, head_dim 128: 96 x 8 of 200 to 3000 108.2 -> 107.5).
+constexpr int kOrderKeys = 4;  // sequences / 64 at most
+__device__ __forceinline__ int ordered_pair(const AttnParams& p, int pos, int lane) {
+  const int per = p.hkv * p.gtiles, pairs = p.batch * per;
+  const int band = pos / p.order_band, first = band * p.order_band;
+  const int place = band & 1 ? first + min(p.order_band, pairs - first) - 1 - (pos - first) : pos;
+  const int rank = place / per;
+  const uint32_t mask = (1u << p.order_shift) - 1;
+  uint32_t key[kOrderKeys];
+#pragma unroll
+  for (int i = 0; i < kOrderKeys; ++i) {
+    const int seq = i * 64 + lane;
+    int len = p.ctx_lens[min(seq, p.batch - 1)];
+    len = len < 0 ? 0 : (len > p.ctx_cap ? p.ctx_cap : len);
+    key[i] = seq < p.batch ? (uint32_t)((len + kChunk - 1) / kChunk) << p.order_shift | (mask - (uint32_t)seq) : 0u;
+  }
+  // (a key of 0, the last number with no tokens, is never counted and is what remains when the last place is asked for)
+  uint32_t found = 0;
+  for (int bit = p.order_bits - 1; bit >= 0; --bit) {
+    const uint32_t probe = found | 1u << bit;
+    int count = 0;
+#pragma unroll
+    for (int i = 0; i < kOrderKeys; ++i) count += __builtin_popcountll(__builtin_amdgcn_ballot_w64(key[i] >= probe));
+    if (count > rank) found = probe;
+  }
+  return (int)(mask - (found & mask)) * per + place % per;
+}
+
 template <int D, bool BF16, bool FP8, int GT, bool ONCE = true>
 __global__ __launch_bounds__(64) void attn_partition_kernel(AttnParams p) {
   const int lane = threadIdx.x;
@@ -663,7 +701,8 @@ __global__ __launch_bounds__(64) void attn_partition_kernel(AttnParams p) {
   // tail of the grid is dispatched last.
   const int pairs = p.batch * p.hkv * p.gtiles;
   const int part = blockIdx.x / pairs;
-  const int pair = blockIdx.x % pairs;
+  const int pos = blockIdx.x % pairs;
+  const int pair = p.order_band ? __builtin_amdgcn_readfirstlane(ordered_pair(p, pos, lane)) : pos;
   const int b = pair / (p.hkv * p.gtiles);
   const int h = (pair / p.gtiles) % p.hkv;
   const int gt = pair % p.gtiles;
@@ -773,7 +812,7 @@ __global__ __launch_bounds__(wg_max_parts(D, GT) * 64) void attn_wg_kernel(AttnP
   const int lane = threadIdx.x & 63;
   const int part = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int c = lane & 15, j = lane >> 4;
-  const int pair = blockIdx.x;
+  const int pair = p.order_band ? __builtin_amdgcn_readfirstlane(ordered_pair(p, blockIdx.x, lane)) : blockIdx.x;
   const int b = pair / (p.hkv * p.gtiles);
   const int h = (pair / p.gtiles) % p.hkv;
   const int gt = pair % p.gtiles;
@@ -1476,13 +1515,14 @@ namespace {
 // How a launch spreads over the CUs depends on how ragged the context lengths are, which the host
 // does not see (they live in device memory).  For every launch signature the first calls therefore
 // time a short list of shapes that all give bit-identical results - residency caps of the
-// partition grid and, where the partition count allows it, the workgroup form - with a pair of
+// partition grid and, where the partition count allows it, the workgroup form, both also with the sequences by length - with a pair of
 // events around each call's launches, read back without blocking on later calls; once every
 // candidate has kTuneReps readings the fastest is used from then on.  Calls made while a stream
 // is being captured, and the entry point that allocates nothing, never measure.
 struct TuneCandidate {
   int cap;      // residency cap of the partition grid (0 = none)
   bool wg;      // workgroup form
+  bool ordered; // sequences by length (ordered_pair)
 };
 struct TunePending {
   int cand;
@@ -1497,7 +1537,7 @@ struct TuneState {
 };
 constexpr int kTuneReps = 4;
 constexpr size_t kTuneMaxSignatures = 512;  // signatures beyond this many run the fixed rule
-typedef std::array<int64_t, 12> TuneKey;
+typedef std::array<int64_t, 13> TuneKey;
 std::map<TuneKey, TuneState>& tune_table() {
   static std::map<TuneKey, TuneState> t;
   return t;
@@ -1532,8 +1572,14 @@ void tune_harvest(TuneState& ts) {
     for (int d : ts.done) all = all && d >= kTuneReps;
     if (all) {
       ts.chosen = 0;
+      // a candidate must win by 1 %; an order by length, behind the others in the list, by 4: what it gains at all is more
+      // (with 1 % two of 37 drawn calls took it and were 1 and 3 % slower)
+      float beat = ts.best_us[0];
       for (size_t c = 1; c < ts.cands.size(); ++c)
-        if (ts.best_us[c] < ts.best_us[ts.chosen] * 0.99f) ts.chosen = (int)c;  // a candidate must win by 1 %
+        if (ts.best_us[c] < beat * (ts.cands[c].ordered && !ts.cands[ts.chosen].ordered ? 0.96f : 0.99f)) {
+          ts.chosen = (int)c;
+          beat = ts.best_us[c];
+        }
     }
   }
 }
@@ -1549,13 +1595,14 @@ void attention_tuning_reset() {
   tune_table().clear();
   g_last_tuned = nullptr;
 }
-void attention_tuning_last(int64_t* cap, int64_t* wg) {
-  *cap = *wg = -1;
+void attention_tuning_last(int64_t* cap, int64_t* wg, int64_t* ordered) {
+  *cap = *wg = *ordered = -1;
   if (!g_last_tuned) return;
   tune_harvest(*g_last_tuned);  // readings that have arrived since the last launch
   if (g_last_tuned->chosen < 0) return;
   *cap = g_last_tuned->cands[g_last_tuned->chosen].cap;
   *wg = g_last_tuned->cands[g_last_tuned->chosen].wg ? 1 : 0;
+  *ordered = g_last_tuned->cands[g_last_tuned->chosen].ordered ? 1 : 0;
 }
 }  // namespace pto_hip
 
@@ -1658,13 +1705,22 @@ int paged_attention(const void* query, const void* key_cache, const void* value_
     }
   }
 
+  // Sequences by length: a few that fit the keys, and a key of 31 bits.
+  auto bits = [](int64_t n) {
+    int k = 0;
+    while ((1ll << k) <= n) ++k;
+    return k;
+  };
+  const int len_bits = bits((p.ctx_cap + kChunk - 1) / kChunk), seq_bits = bits(batch - 1);
+  const bool may_order = !lean && batch > 1 && batch <= 64 * kOrderKeys && len_bits + seq_bits <= 31 && cx.attn_order != 0;
+  bool ordered = may_order && cx.attn_order > 0;
   // Launch shape by measurement (see TuneState): only while the caller has not fixed the shape.
   hipStream_t hs = (hipStream_t)stream;
   TuneState* ts = nullptr;
   int measuring = -1;
-  if (cx.attn_autotune != 0 && cx.attn_waves_per_cu == 0 && cx.attn_variant < 0 && !lean) {
+  if (cx.attn_autotune != 0 && cx.attn_waves_per_cu == 0 && cx.attn_variant < 0 && cx.attn_order <= 0 && !lean) {
     const TuneKey key = {batch, hq, hkv, d, config[4], config[5], (int64_t)q_dtype, (int64_t)kv_dtype, (int64_t)p.ctx_cap,
-                         (int64_t)p.tpp, (int64_t)gt, (int64_t)(out16 != nullptr)};
+                         (int64_t)p.tpp, (int64_t)gt, (int64_t)(out16 != nullptr), (int64_t)may_order};
     auto& table_ = tune_table();
     auto it = table_.find(key);
     if (it == table_.end() && table_.size() < kTuneMaxSignatures) it = table_.emplace(key, TuneState{}).first;
@@ -1672,9 +1728,13 @@ int paged_attention(const void* query, const void* key_cache, const void* value_
   }
   if (ts) {
     if (ts->cands.empty()) {
-      ts->cands.push_back({0, p.wg_merge != 0});  // the rule's own choice first
-      if (wg_possible) ts->cands.push_back({0, p.wg_merge == 0});
-      for (int cap : {3, 2, 4}) ts->cands.push_back({cap, false});
+      ts->cands.push_back({0, p.wg_merge != 0, false});  // the rule's own choice first
+      if (wg_possible) ts->cands.push_back({0, p.wg_merge == 0, false});
+      for (int cap : {3, 2, 4}) ts->cands.push_back({cap, false, false});
+      if (may_order && pairs * 2 >= cx.num_cu) {  // (fewer pairs than half the CUs never gained)
+        if (wg_possible) ts->cands.push_back({0, true, true});
+        for (int cap : {0, 2, 4}) ts->cands.push_back({cap, false, true});
+      }
       ts->best_us.assign(ts->cands.size(), 1e30f);
       ts->issued.assign(ts->cands.size(), 0);
       ts->done.assign(ts->cands.size(), 0);
@@ -1700,7 +1760,13 @@ int paged_attention(const void* query, const void* key_cache, const void* value_
     }
     p.resident_cap = ts->cands[use].cap;
     p.wg_merge = ts->cands[use].wg ? 1 : 0;
+    ordered = ts->cands[use].ordered;
     g_last_tuned = ts;
+  }
+  if (ordered) {
+    p.order_band = cx.num_cu;
+    p.order_shift = seq_bits;
+    p.order_bits = len_bits + seq_bits;
   }
   if (p.n_part > 1 && !lean && !p.wg_merge) {
     const size_t rows = (size_t)batch * hq;

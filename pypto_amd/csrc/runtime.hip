@@ -1088,6 +1088,9 @@ int pto_hip_set_option(const char* name, int64_t value) {
   } else if (!std::strcmp(name, "w8a16_nt")) {
     PTO_CHECK_ARG(value == 0 || value == 1, "w8a16_nt must be 0 or 1");
     c.w8a16_nt = value;
+  } else if (!std::strcmp(name, "attn_order")) {
+    PTO_CHECK_ARG(value >= -1 && value <= 1, "attn_order must be -1, 0 or 1");
+    c.attn_order = value;
   } else if (!std::strcmp(name, "attn_lean_siblings")) {
     PTO_CHECK_ARG(value >= 0 && value <= 2, "attn_lean_siblings must be 0, 1 or 2");
     c.attn_lean_siblings = value;
@@ -1157,13 +1160,15 @@ int pto_hip_get_option(const char* name, int64_t* value) {
   else if (!std::strcmp(name, "attn_variant")) *value = c.attn_variant;
   else if (!std::strcmp(name, "attn_autotune")) *value = c.attn_autotune;
   else if (!std::strcmp(name, "attn_lean_siblings")) *value = c.attn_lean_siblings;
+  else if (!std::strcmp(name, "attn_order")) *value = c.attn_order;
   else if (!std::strcmp(name, "w8a16_nt")) *value = c.w8a16_nt;
   else if (!std::strcmp(name, "workspace_bytes"))  // read only: device memory the three grow-only scratch areas hold
     *value = (int64_t)(c.workspace_bytes + c.layer_ws_bytes + c.gemm_ws_bytes);
-  else if (!std::strcmp(name, "attn_tuned_waves_per_cu") || !std::strcmp(name, "attn_tuned_workgroup_form")) {
-    int64_t cap = -1, wg = -1;
-    attention_tuning_last(&cap, &wg);
-    *value = !std::strcmp(name, "attn_tuned_waves_per_cu") ? cap : wg;
+  else if (!std::strcmp(name, "attn_tuned_waves_per_cu") || !std::strcmp(name, "attn_tuned_workgroup_form") ||
+           !std::strcmp(name, "attn_tuned_order")) {
+    int64_t cap = -1, wg = -1, ordered = -1;
+    attention_tuning_last(&cap, &wg, &ordered);
+    *value = !std::strcmp(name, "attn_tuned_waves_per_cu") ? cap : !std::strcmp(name, "attn_tuned_order") ? ordered : wg;
   }
   else if (!std::strcmp(name, "attn_group_tiles")) *value = c.attn_group_tiles;
   else if (!std::strcmp(name, "w8a16_wgs_per_cu")) *value = c.w8a16_wgs_per_cu;
