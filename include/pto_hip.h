@@ -582,6 +582,10 @@ PTO_HIP_API int pto_hip_backend_handler_query(const char* hook, int32_t arg, cha
  *                               each: 0 = where estimated faster than the tiled GEMM, and up to 32 rows for at most
  *                               1.6 million weights (default), -1 = never, 1..4 = always, with that tile
  *                               ("gemm_variant", "gemm_quad_rows" or "gemm_splits" other than 0 switch it off)
+ *  "gemm_stream"                projections of 33 to 96 rows inside a decoder layer or an FFN block with a norm that
+ *                               stream their weights into registers: 1 = where measured ahead of the tiled GEMM
+ *                               (default), 0 = never, 2 = whenever shapes allow ("gemm_variant", "gemm_quad_rows"
+ *                               or "gemm_splits" other than 0 switch it off)
  *  "gemm_splits"                k splits of the tiled GEMMs: 0 = by shape (default), 1..16 = as given
  *                               when k allows (16-bit and int8 weights: each split at least four 64-row
  *                               k tiles; e4m3: at least one tile of 128 codes), under every "gemm_variant"

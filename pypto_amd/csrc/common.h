@@ -75,6 +75,7 @@ struct Context {
   int64_t w8a16_wide = 1;        // int8 codes read 16 per lane: 0 never, 1 for large matrices, 2 whenever shapes allow
   int64_t skinny_fuse = 7;         // skinny projections of up to four rows make their activations themselves: 1 norm, 2 SwiGLU, 4 merge
   int64_t w8a16_min_steps = 2;   // fewest 32-row steps per wavefront before k is split further
+  int64_t gemm_stream = 1;         // projections of 33 to 96 rows that stream their weights: 0 never, 1 where measured ahead, 2 whenever shapes allow
   int64_t attn_order = -1;         // sequences by length: -1 where measured faster, 0 never, 1 always (partition grid and workgroup form)
   int64_t w8a16_gemm_rows = 33;  // rows from which int8 projections run as a tiled GEMM (0 = never)
 };
@@ -108,6 +109,13 @@ __device__ __forceinline__ int slab_count(const SlabMap& s, int splits, int mat,
   if (s.units == 0) return splits;
   const unsigned first = (unsigned)(mat * s.slabs + (ch >> s.shift)) * s.ks;
   return (int)(((first + s.ks) * s.wgs - 1) / s.units - ((first + 1) * s.wgs - 1) / s.units) + 1;
+}
+// Row a workgroup takes where one writes a row of the blocked layout [K/8][rows][8]: its 128-byte lines are eight rows' pieces, and
+// eight rows whose workgroups run on one XCD (workgroup id mod 8) meet in that XCD's L2.  A permutation of 0 .. rows - 1.
+__device__ __forceinline__ int blocked_row(int id, int rows) {
+  const int base = id & ~63, groups = min(rows - base, 64) >> 3;  // groups of eight rows among the next 64
+  if (groups == 0 || id - base >= groups * 8) return id;
+  return base + (id - base) % groups * 8 + (id - base) / groups;
 }
 // fp32 partial sums of a projection: element (s, m, n) of projection i is part[i][s * slab_stride + m * N + n] for
 // s below slab_count(map, splits, i, n).  The skinny kernels write [M, N] slabs into the shared workspace; the
@@ -169,13 +177,14 @@ int layer_workspace(size_t bytes, void** ptr);
 // Grow-only device scratch for the split-K slabs of the tiled GEMMs.  Null when `st` is being captured and the area
 // would have to grow: the product then runs unsplit.
 int gemm_slabs(size_t bytes, hipStream_t st, void** ptr);
+// out_rows of these and of the kernels below: 0 writes rows, otherwise the blocked layout [N/8][out_rows][8] of the next projection.
 // out = cast(sum_s(part0) * scale0 [-> SiLU(.) * (sum_s(part1) * scale1)] [+ residual]).
 int w8a16_finish(const W8Partials& parts, const float* scale0, const float* scale1, const void* residual,
-                 int res_dtype, void* out, int out_dtype, bool out_blocked, int64_t m, int64_t n, hipStream_t st);
+                 int res_dtype, void* out, int out_dtype, int out_rows, int64_t m, int64_t n, hipStream_t st);
 // sum_out = sum_s(part) * scale + residual (fp32); normed_out = cast(RMSNorm(sum_out) * gamma).
 bool w8a16_finish_norm_fits(int64_t n);
 int w8a16_finish_norm(const W8Partials& parts, const float* scale, const void* residual, int res_dtype,
-                      float* sum_out, const float* gamma, void* normed_out, int out_dtype, bool out_blocked,
+                      float* sum_out, const float* gamma, void* normed_out, int out_dtype, int out_rows,
                       int64_t m, int64_t n, float eps, hipStream_t st);
 // The tiled GEMM with int8 weight codes (widened on their way into LDS, scales applied to the
 // accumulators): out = (x @ codes0) * scale0 (+ residual), or with codes1 / scale1 given
@@ -186,6 +195,12 @@ bool gemm_w8_fits(const void* x, const void* wq0, const void* wq1, const void* r
 int gemm_w8(const void* x, const void* wq0, const float* scale0, const void* wq1, const float* scale1,
             const void* residual, int res_dtype, void* out, int64_t m, int64_t k, int64_t n, int x_dtype,
             int out_dtype, hipStream_t st);
+// Projections of some tens of rows bound by reading their weights (stream_rows.h), left as fp32 slabs of k splits.  stream_rows_for
+// says whether one is to run so - row count of the blocked layout its activations should have, 0 otherwise - and has made room
+// for its slabs; x_rows: 0 for activations in rows.
+int stream_rows_for(int64_t m, int64_t k, int64_t n, const void* wq0, const void* wq1, bool w16, hipStream_t st);
+int stream_partials(const void* x, int x_rows, const void* wq0, const void* wq1, int64_t m, int64_t k, int64_t n, int x_dtype,
+                    hipStream_t st, W8Partials* out, bool w16);
 // x[M, K] @ w[K, N] through the tiled GEMM, left as k-split partial sums for a fused consumer
 // (scale null: 16-bit weights).  With one split the product, scales applied, is written to
 // `direct` (fp32 [M, N]) and returned as a single slab.
@@ -207,13 +222,13 @@ int rope_kv_cache_update_fp8(const W8Partials& qkv, const float* qkv_scale,
                              float* v_scale, void* q_out, int64_t batch, int64_t num_heads, int64_t kv_head_num,
                              int64_t head_dim, int64_t block_size, int64_t max_num_blocks_per_req,
                              int64_t max_pos, int rope_width, int64_t pool_blocks, int q_dtype, void* stream);
-// RMSNorm of at most 32 rows written in the blocked activation layout [H/8][32][8].
-bool rms_norm_blocked_fits(int64_t rows, int64_t hidden);
+// RMSNorm of at most out_rows rows written in the blocked activation layout [H/8][out_rows][8].
+bool rms_norm_blocked_fits(int64_t rows, int64_t hidden, int out_rows = kW8MaxM);
 int rms_norm_blocked(const void* x, const float* gamma, void* out, int64_t rows, int64_t hidden, float eps,
-                     int dtype, hipStream_t st);
+                     int dtype, hipStream_t st, int out_rows = kW8MaxM);
 int cast_from_f32(const float* in, void* out, size_t n, int out_dtype, hipStream_t st);
 // pto_hip_paged_attention with an optional second output: the result rounded to the query dtype.
-// want_blocked asks for the copy as [Hq*D/8][32][8] over the batch rows (batch <= 32);
+// out16_rows asks for the copy as [Hq*D/8][out16_rows][8] over the batch rows (at most so many);
 // *wrote_blocked says whether that is how it was written (only a launch with a merge kernel can).
 // pool_blocks > 0: the number of physical blocks in the caches; a table entry beyond it that a
 // sequence uses reads block 0 instead and is reported by the next pto_hip_sync.
@@ -221,7 +236,7 @@ int cast_from_f32(const float* in, void* out, size_t n, int out_dtype, hipStream
 // form of the orchestration carries in its config, 09_paged_attention_spmd.py:468,482); < 0: no bound.
 int paged_attention(const void* query, const void* key_cache, const void* value_cache,
                     const int32_t* block_table, const int32_t* context_lens, float* out, void* out16,
-                    bool want_blocked, bool* wrote_blocked,
+                    int out16_rows, bool* wrote_blocked,
                     const int64_t* config, int q_dtype, int kv_dtype, const float* k_scale,
                     const float* v_scale, int64_t pool_blocks, void* stream, void* fixed_scratch = nullptr,
                     size_t fixed_scratch_bytes = 0, int64_t active_blocks = -1, AttnPartials* unmerged = nullptr);

@@ -158,14 +158,30 @@ int ffn_skinny(const void* x, const float* gamma, const void* w_gate, const void
       src.pair = parts;
       rc = w8a16_partials(nullptr, false, w_down, nullptr, m, intermediate, hidden, dtype, st, &parts, true, &src, slabs);
     } else {
-      if ((rc = w8a16_finish(parts, nullptr, nullptr, nullptr, 0, hbuf, dtype, true, m, intermediate, st))) return rc;
+      if ((rc = w8a16_finish(parts, nullptr, nullptr, nullptr, 0, hbuf, dtype, kW8MaxM, m, intermediate, st))) return rc;
       rc = w8a16_partials(hbuf, true, w_down, nullptr, m, intermediate, hidden, dtype, st, &parts, true);
     }
     if (rc) return rc;
     void* outr = reinterpret_cast<char*>(out) + (size_t)r0 * hidden * ob;
-    if ((rc = w8a16_finish(parts, nullptr, nullptr, nullptr, 0, outr, out_dtype, false, m, hidden, st))) return rc;
+    if ((rc = w8a16_finish(parts, nullptr, nullptr, nullptr, 0, outr, out_dtype, 0, m, hidden, st))) return rc;
   }
   return PTO_HIP_OK;
+}
+
+int ffn_stream(const void* x, const float* gamma, const void* w_gate, const void* w_up, const void* w_down, void* out, int64_t tokens,
+               int64_t hidden, int64_t intermediate, float eps, int dtype, int out_dtype, int rows, hipStream_t st) {
+  using namespace pto_hip;
+  const size_t xn_bytes = ((size_t)rows * hidden * 2 + 255) / 256 * 256;
+  void* ws = nullptr;
+  int rc = workspace(xn_bytes + (size_t)rows * intermediate * 2, &ws);
+  if (rc) return rc;
+  void* h = reinterpret_cast<char*>(ws) + xn_bytes;
+  if ((rc = rms_norm_blocked(x, gamma, ws, tokens, hidden, eps, dtype, st, rows))) return rc;
+  W8Partials parts{};
+  if ((rc = stream_partials(ws, rows, w_gate, w_up, tokens, hidden, intermediate, dtype, st, &parts, true))) return rc;
+  if ((rc = w8a16_finish(parts, nullptr, nullptr, nullptr, 0, h, dtype, rows, tokens, intermediate, st))) return rc;
+  if ((rc = stream_partials(h, rows, w_down, nullptr, tokens, intermediate, hidden, dtype, st, &parts, true))) return rc;
+  return w8a16_finish(parts, nullptr, nullptr, nullptr, 0, out, out_dtype, 0, tokens, hidden, st);
 }
 
 }  // namespace
@@ -250,6 +266,13 @@ extern "C" int pto_hip_ffn_swiglu(const void* x, const float* gamma, const void*
        (uintptr_t)gamma) % 16 == 0 &&
       (out_dtype == PTO_HIP_FP32 || out_dtype == dtype) && !narrow_not_skinny(hidden, intermediate, true))
     return ffn_skinny(x, gamma, w_gate, w_up, w_down, out, tokens, hidden, intermediate, eps, dtype, out_dtype, st);
+
+  // Some tens of tokens: the block streams its weights, from activations that the norm and the pair's finish leave in blocked form.
+  if (sixteen && gamma && ((uintptr_t)x | (uintptr_t)gamma | (uintptr_t)out) % 16 == 0 && (out_dtype == PTO_HIP_FP32 || out_dtype == dtype)) {
+    const int rows = stream_rows_for(tokens, hidden, intermediate, w_gate, w_up, true, st);
+    if (rows && rms_norm_blocked_fits(tokens, hidden, rows) && stream_rows_for(tokens, intermediate, hidden, w_down, nullptr, true, st))
+      return ffn_stream(x, gamma, w_gate, w_up, w_down, out, tokens, hidden, intermediate, eps, dtype, out_dtype, rows, st);
+  }
 
   const size_t xn_bytes = gamma ? ((size_t)tokens * hidden * eb + 255) / 256 * 256 : 0;
   const size_t h_bytes = (size_t)tokens * intermediate * eb;
@@ -399,7 +422,7 @@ extern "C" int pto_hip_projection(const void* x, const void* w, const void* resi
     W8Partials parts{};
     int rc = w8a16_partials(x, false, w, nullptr, m, k, n, dtype, st, &parts, true);
     if (rc) return rc;
-    return w8a16_finish(parts, nullptr, nullptr, residual, res_dtype, out, out_dtype, false, m, n, st);
+    return w8a16_finish(parts, nullptr, nullptr, residual, res_dtype, out, out_dtype, 0, m, n, st);
   }
   GemmParams p{};
   p.a = reinterpret_cast<const uint16_t*>(x);
@@ -440,7 +463,7 @@ extern "C" int pto_hip_gate_up_swiglu(const void* x, const void* w_gate, const v
     W8Partials parts{};
     int rc = w8a16_partials(x, false, w_gate, w_up, m, k, n, dtype, st, &parts, true);
     if (rc) return rc;
-    return w8a16_finish(parts, nullptr, nullptr, nullptr, 0, out, dtype, false, m, n, st);
+    return w8a16_finish(parts, nullptr, nullptr, nullptr, 0, out, dtype, 0, m, n, st);
   }
   GemmParams p{};
   p.a = reinterpret_cast<const uint16_t*>(x);

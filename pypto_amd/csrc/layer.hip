@@ -36,10 +36,20 @@ int layer_large_batch(const PtoHipDecoderLayerArgs* a, int rope_w, void* stream)
   const bool fp8kv = a->kv_dtype == PTO_HIP_FP8E4M3FN;
   const int64_t qkv_n = (hq + 2 * hkv) * d;
   auto up = [](size_t n) { return (n + 255) / 256 * 256; };
-  const size_t sz_normed = up((size_t)b * h * 2), sz_qkv = up((size_t)b * std::max(qkv_n, h) * 4),  // also holds an unsplit o_proj product
+  const bool w16 = !a->wg_s;
+  const bool vec = ((uintptr_t)a->hidden_states | (uintptr_t)a->gamma_in | (uintptr_t)a->gamma_post) % 16 == 0;
+  hipStream_t st = (hipStream_t)stream;
+  // Rows of the blocked layout of the activations in front of a projection that streams its weights; 0: rows, and the tiled GEMM.
+  const int qkv_rows = vec ? stream_rows_for(b, h, qkv_n, a->wqkv_q, nullptr, w16, st) : 0;
+  const int o_rows = stream_rows_for(b, hq * d, h, a->wo_q, nullptr, w16, st);
+  const int gu_rows = stream_rows_for(b, h, inter, a->wg_q, a->wu_q, w16, st);
+  const int down_rows = gu_rows ? stream_rows_for(b, inter, h, a->wd_q, nullptr, w16, st) : 0;
+  const bool fused_norm = w8a16_finish_norm_fits(h);
+  const size_t rows16 = std::max<int64_t>(b, std::max(std::max(qkv_rows, o_rows), std::max(gu_rows, down_rows)));
+  const size_t sz_normed = up(rows16 * h * 2), sz_qkv = up((size_t)b * std::max(qkv_n, h) * 4),  // also holds an unsplit o_proj product
                sz_q = up((size_t)b * hq * d * 2), sz_attn = up((size_t)b * hq * d * 4),
-               sz_attn16 = up((size_t)b * hq * d * 2), sz_resid = up((size_t)b * h * 4),
-               sz_h = up((size_t)b * inter * 2);
+               sz_attn16 = up(rows16 * hq * d * 2), sz_resid = up((size_t)b * h * 4),
+               sz_h = up(rows16 * inter * 2);
   void* lws = nullptr;
   int rc = layer_workspace(sz_normed + sz_qkv + sz_q + sz_attn + sz_attn16 + sz_resid + sz_normed + sz_h, &lws);
   if (rc) return rc;
@@ -53,12 +63,16 @@ int layer_large_batch(const PtoHipDecoderLayerArgs* a, int rope_w, void* stream)
   void* normed2 = w;             w += sz_normed;
   void* hbuf = w;
 
-  hipStream_t st = (hipStream_t)stream;
-  if ((rc = pto_hip_rms_norm(a->hidden_states, a->gamma_in, normed, b, h, a->eps, dt, dt, stream))) return rc;
+  const int norm_rows = rms_norm_blocked_fits(b, h, qkv_rows) ? qkv_rows : 0;
+  if (norm_rows) rc = rms_norm_blocked(a->hidden_states, a->gamma_in, normed, b, h, a->eps, dt, st, norm_rows);
+  else rc = pto_hip_rms_norm(a->hidden_states, a->gamma_in, normed, b, h, a->eps, dt, dt, stream);
+  if (rc) return rc;
   // The k-split slabs of the q/k/v and o projections go unsummed to the kernels that follow them
   // (RoPE + append; residual + RMSNorm), as the partial sums of the skinny projections do.
   W8Partials parts{};
-  if ((rc = gemm_partials(normed, a->wqkv_q, a->wqkv_s, b, h, qkv_n, dt, qkv, st, &parts))) return rc;
+  if (qkv_rows) rc = stream_partials(normed, norm_rows, a->wqkv_q, nullptr, b, h, qkv_n, dt, st, &parts, w16);
+  else rc = gemm_partials(normed, a->wqkv_q, a->wqkv_s, b, h, qkv_n, dt, qkv, st, &parts);
+  if (rc) return rc;
   const float* qkv_scale = parts.scaled ? nullptr : a->wqkv_s;
   const int64_t pool_blocks = a->pool_rows / (hkv * a->block_size);
   if (fp8kv)
@@ -75,24 +89,42 @@ int layer_large_batch(const PtoHipDecoderLayerArgs* a, int rope_w, void* stream)
   uint32_t scale_bits;
   __builtin_memcpy(&scale_bits, &scale, 4);
   const int64_t cfg[7] = {b, hq, hkv, d, a->block_size, a->max_num_blocks_per_req, (int64_t)scale_bits};
-  if ((rc = paged_attention(q16, a->key_cache, a->value_cache, a->block_table, a->seq_lens, attn, attn16, false, nullptr,
+  bool blk_attn = false;
+  if ((rc = paged_attention(q16, a->key_cache, a->value_cache, a->block_table, a->seq_lens, attn, attn16, o_rows, &blk_attn,
                             cfg, dt, fp8kv ? PTO_HIP_FP8E4M3FN : dt, fp8kv ? a->k_scale : nullptr,
                             fp8kv ? a->v_scale : nullptr, pool_blocks, stream)))
     return rc;
-  if (w8a16_finish_norm_fits(h)) {
-    // o_proj into the buffer the q/k/v product no longer needs, then sum + residual + RMSNorm in one kernel
-    if ((rc = gemm_partials(attn16, a->wo_q, a->wo_s, b, hq * d, h, dt, qkv, st, &parts))) return rc;
-    if ((rc = w8a16_finish_norm(parts, parts.scaled ? nullptr : a->wo_s, a->hidden_states, dt, resid1, a->gamma_post,
-                                normed2, dt, false, b, h, a->eps, st)))
-      return rc;
-  } else {
-    if ((rc = project(attn16, a->wo_q, a->wo_s, a->hidden_states, resid1, b, hq * d, h, dt, dt, PTO_HIP_FP32, stream)))
-      return rc;
-    if ((rc = pto_hip_rms_norm(resid1, a->gamma_post, normed2, b, h, a->eps, PTO_HIP_FP32, dt, stream))) return rc;
+  // o_proj, unstreamed into the buffer the q/k/v product no longer needs
+  if (o_rows || fused_norm) {
+    if (o_rows) rc = stream_partials(attn16, blk_attn ? o_rows : 0, a->wo_q, nullptr, b, hq * d, h, dt, st, &parts, w16);
+    else rc = gemm_partials(attn16, a->wo_q, a->wo_s, b, hq * d, h, dt, qkv, st, &parts);
+    if (rc) return rc;
   }
-  if (a->wg_s) rc = pto_hip_w8a16_swiglu(normed2, a->wg_q, a->wg_s, a->wu_q, a->wu_s, hbuf, b, h, inter, dt, dt, stream);
-  else rc = pto_hip_gate_up_swiglu(normed2, a->wg_q, a->wu_q, hbuf, b, h, inter, dt, stream);
+  const float* o_scale = parts.scaled ? nullptr : a->wo_s;
+  int normed2_rows = gu_rows;
+  if (fused_norm) {  // sum + residual + RMSNorm in one kernel
+    rc = w8a16_finish_norm(parts, o_scale, a->hidden_states, dt, resid1, a->gamma_post, normed2, dt, gu_rows, b, h, a->eps, st);
+  } else {
+    if (o_rows) rc = w8a16_finish(parts, o_scale, nullptr, a->hidden_states, dt, resid1, PTO_HIP_FP32, 0, b, h, st);
+    else rc = project(attn16, a->wo_q, a->wo_s, a->hidden_states, resid1, b, hq * d, h, dt, dt, PTO_HIP_FP32, stream);
+    if (rc) return rc;
+    normed2_rows = 0;
+    rc = pto_hip_rms_norm(resid1, a->gamma_post, normed2, b, h, a->eps, PTO_HIP_FP32, dt, stream);
+  }
   if (rc) return rc;
+  if (gu_rows) {
+    if ((rc = stream_partials(normed2, normed2_rows, a->wg_q, a->wu_q, b, h, inter, dt, st, &parts, w16))) return rc;
+    rc = w8a16_finish(parts, a->wg_s, a->wu_s, nullptr, 0, hbuf, dt, down_rows, b, inter, st);
+  } else if (a->wg_s) {
+    rc = pto_hip_w8a16_swiglu(normed2, a->wg_q, a->wg_s, a->wu_q, a->wu_s, hbuf, b, h, inter, dt, dt, stream);
+  } else {
+    rc = pto_hip_gate_up_swiglu(normed2, a->wg_q, a->wu_q, hbuf, b, h, inter, dt, stream);
+  }
+  if (rc) return rc;
+  if (down_rows) {
+    if ((rc = stream_partials(hbuf, down_rows, a->wd_q, nullptr, b, inter, h, dt, st, &parts, w16))) return rc;
+    return w8a16_finish(parts, a->wd_s, nullptr, resid1, PTO_HIP_FP32, a->out, dt, 0, b, h, st);
+  }
   return project(hbuf, a->wd_q, a->wd_s, resid1, a->out, b, inter, h, dt, PTO_HIP_FP32, dt, stream);
 }
 
@@ -236,7 +268,7 @@ extern "C" int pto_hip_decoder_layer_decode(const PtoHipDecoderLayerArgs* a, voi
   AttnPartials unmerged{};
   const bool may_merge = slabs && skinny_fuses(ProjectionSource::kMerge, b, hq * d, h, a->wo_q, nullptr, w16, d);
   unmerged.n_part = kMergeHeld;
-  if ((rc = paged_attention(q16, a->key_cache, a->value_cache, a->block_table, a->seq_lens, attn, attn16, blk,
+  if ((rc = paged_attention(q16, a->key_cache, a->value_cache, a->block_table, a->seq_lens, attn, attn16, blk ? kW8MaxM : 0,
                             &blk_attn, cfg, dt, fp8kv ? PTO_HIP_FP8E4M3FN : dt, fp8kv ? a->k_scale : nullptr,
                             fp8kv ? a->v_scale : nullptr, a->pool_rows / (hkv * a->block_size), stream, nullptr, 0, -1,
                             may_merge ? &unmerged : nullptr)))
@@ -252,11 +284,11 @@ extern "C" int pto_hip_decoder_layer_decode(const PtoHipDecoderLayerArgs* a, voi
   }
   if (rc) return rc;
   if (w8a16_finish_norm_fits(h)) {
-    if ((rc = w8a16_finish_norm(parts, a->wo_s, a->hidden_states, dt, resid1, a->gamma_post, normed2, dt, blk, b, h,
+    if ((rc = w8a16_finish_norm(parts, a->wo_s, a->hidden_states, dt, resid1, a->gamma_post, normed2, dt, blk ? kW8MaxM : 0, b, h,
                                 a->eps, st)))
       return rc;
   } else {
-    if ((rc = w8a16_finish(parts, a->wo_s, nullptr, a->hidden_states, dt, resid1, PTO_HIP_FP32, false, b, h, st)))
+    if ((rc = w8a16_finish(parts, a->wo_s, nullptr, a->hidden_states, dt, resid1, PTO_HIP_FP32, 0, b, h, st)))
       return rc;
     if ((rc = pto_hip_rms_norm(resid1, a->gamma_post, normed2, b, h, a->eps, PTO_HIP_FP32, dt, stream))) return rc;
   }
@@ -269,8 +301,8 @@ extern "C" int pto_hip_decoder_layer_decode(const PtoHipDecoderLayerArgs* a, voi
     src.scale1 = a->wu_s;
     if ((rc = w8a16_partials(nullptr, false, a->wd_q, nullptr, b, inter, h, dt, st, &parts, w16, &src, slabs))) return rc;
   } else {
-    if ((rc = w8a16_finish(parts, a->wg_s, a->wu_s, nullptr, 0, hbuf, dt, blk, b, inter, st))) return rc;
+    if ((rc = w8a16_finish(parts, a->wg_s, a->wu_s, nullptr, 0, hbuf, dt, blk ? kW8MaxM : 0, b, inter, st))) return rc;
     if ((rc = w8a16_partials(hbuf, blk, a->wd_q, nullptr, b, inter, h, dt, st, &parts, w16))) return rc;
   }
-  return w8a16_finish(parts, a->wd_s, nullptr, resid1, PTO_HIP_FP32, a->out, dt, false, b, h, st);
+  return w8a16_finish(parts, a->wd_s, nullptr, resid1, PTO_HIP_FP32, a->out, dt, 0, b, h, st);
 }

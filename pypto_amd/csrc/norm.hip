@@ -62,13 +62,13 @@ template <typename TI, typename T, bool BLOCKED>
 __global__ __launch_bounds__(kThreads) void rms_norm_vec_kernel(const TI* __restrict__ x,
                                                                 const float* __restrict__ gamma,
                                                                 T* __restrict__ out, int64_t hidden,
-                                                                float eps) {
+                                                                float eps, int out_rows) {
   typedef __attribute__((__vector_size__(8 * sizeof(T)))) T vec8;
   typedef __attribute__((__vector_size__(8 * sizeof(TI)))) TI vec8i;
-  const int64_t row = blockIdx.x;
+  const int64_t row = BLOCKED ? pto_hip::blocked_row(blockIdx.x, gridDim.x) : blockIdx.x;
   const vec8i* xr = reinterpret_cast<const vec8i*>(x + row * hidden);
   vec8* orow = BLOCKED ? reinterpret_cast<vec8*>(out) + row : reinterpret_cast<vec8*>(out + row * hidden);
-  constexpr int kOutStride = BLOCKED ? 32 : 1;  // vec8 units between consecutive 8-element groups
+  const int out_stride = BLOCKED ? out_rows : 1;  // vec8 units between consecutive 8-element groups
   const int nvec = (int)(hidden / 8);
   vec8i v[kVecPerThread];
   float4 g0[kVecPerThread], g1[kVecPerThread];  // requested with the row, so that the second pass waits for nothing
@@ -104,7 +104,7 @@ __global__ __launch_bounds__(kThreads) void rms_norm_vec_kernel(const TI* __rest
       const float g[8] = {g0[u].x, g0[u].y, g0[u].z, g0[u].w, g1[u].x, g1[u].y, g1[u].z, g1[u].w};
 #pragma unroll
       for (int e = 0; e < 8; ++e) o[e] = (T)((float)v[u][e] * inv * g[e]);
-      orow[(size_t)i * kOutStride] = o;
+      orow[(size_t)i * out_stride] = o;
     }
   }
 }
@@ -137,22 +137,22 @@ int launch_out(const void* x, const float* gamma, void* out, int64_t rows, int64
 }  // namespace
 
 namespace pto_hip {
-bool rms_norm_blocked_fits(int64_t rows, int64_t hidden) {
-  return rows <= 32 && hidden % 8 == 0 && hidden <= 8 * kThreads * kVecPerThread;
+bool rms_norm_blocked_fits(int64_t rows, int64_t hidden, int out_rows) {
+  return rows <= out_rows && hidden % 8 == 0 && hidden <= 8 * kThreads * kVecPerThread;
 }
 int rms_norm_blocked(const void* x, const float* gamma, void* out, int64_t rows, int64_t hidden, float eps,
-                     int dtype, hipStream_t st) {
-  PTO_CHECK_ARG(rms_norm_blocked_fits(rows, hidden) && (dtype == PTO_HIP_BF16 || dtype == PTO_HIP_FP16) &&
+                     int dtype, hipStream_t st, int out_rows) {
+  PTO_CHECK_ARG(rms_norm_blocked_fits(rows, hidden, out_rows) && (dtype == PTO_HIP_BF16 || dtype == PTO_HIP_FP16) &&
                     ((uintptr_t)x | (uintptr_t)out | (uintptr_t)gamma) % 16 == 0 && gamma != nullptr,
                 "rms_norm (blocked): unsupported shape [%lld, %lld] or operands", (long long)rows, (long long)hidden);
   if (rows == 0) return PTO_HIP_OK;
   dim3 grid((unsigned)rows), block(kThreads);
   if (dtype == PTO_HIP_BF16)
     hipLaunchKernelGGL((rms_norm_vec_kernel<__bf16, __bf16, true>), grid, block, 0, st, (const __bf16*)x, gamma,
-                       (__bf16*)out, hidden, eps);
+                       (__bf16*)out, hidden, eps, out_rows);
   else
     hipLaunchKernelGGL((rms_norm_vec_kernel<_Float16, _Float16, true>), grid, block, 0, st, (const _Float16*)x, gamma,
-                       (_Float16*)out, hidden, eps);
+                       (_Float16*)out, hidden, eps, out_rows);
   PTO_CHECK_HIP(hipGetLastError());
   return PTO_HIP_OK;
 }
@@ -177,16 +177,16 @@ extern "C" int pto_hip_rms_norm(const void* x, const float* gamma, void* out, in
     const bool bf = out_dtype == PTO_HIP_BF16;
     if (x_dtype == PTO_HIP_FP32 && bf)
       hipLaunchKernelGGL((rms_norm_vec_kernel<float, __bf16, false>), grid, block, 0, st, (const float*)x, gamma,
-                         (__bf16*)out, hidden, eps);
+                         (__bf16*)out, hidden, eps, 0);
     else if (x_dtype == PTO_HIP_FP32)
       hipLaunchKernelGGL((rms_norm_vec_kernel<float, _Float16, false>), grid, block, 0, st, (const float*)x, gamma,
-                         (_Float16*)out, hidden, eps);
+                         (_Float16*)out, hidden, eps, 0);
     else if (bf)
       hipLaunchKernelGGL((rms_norm_vec_kernel<__bf16, __bf16, false>), grid, block, 0, st, (const __bf16*)x, gamma,
-                         (__bf16*)out, hidden, eps);
+                         (__bf16*)out, hidden, eps, 0);
     else
       hipLaunchKernelGGL((rms_norm_vec_kernel<_Float16, _Float16, false>), grid, block, 0, st, (const _Float16*)x,
-                         gamma, (_Float16*)out, hidden, eps);
+                         gamma, (_Float16*)out, hidden, eps, 0);
     PTO_CHECK_HIP(hipGetLastError());
     return PTO_HIP_OK;
   }

@@ -49,7 +49,7 @@ struct AttnParams {
   float* out;
   void* out16;     // optional second copy of the result in the 16-bit activation type
   int out16_bf16;
-  int out16_blocked;  // copy stored [Hq*D/8][32][8] over the batch rows instead of [B, Hq*D]
+  int out16_rows;  // copy stored [Hq*D/8][out16_rows][8] over the batch rows; 0: [B, Hq*D]
   float* part_o;   // [B*Hq, n_part, D]
   float* part_ml;  // [B*Hq, n_part, 2]  (running max in log2 units, row sum)
   const float* k_scale;  // [pool_blocks, Hkv] for an e4m3 cache, else null
@@ -776,9 +776,9 @@ __global__ __launch_bounds__(256) void attn_reduce_kernel(AttnParams p) {
     p.out[idx] = y;
     if (p.out16) {
       size_t i16 = idx;
-      if (p.out16_blocked) {
+      if (p.out16_rows) {
         const int bb = row / p.hq, kk = (row % p.hq) * D + k * 64 + lane;  // element kk of batch row bb
-        i16 = ((size_t)(kk >> 3) * 32 + bb) * 8 + (kk & 7);
+        i16 = ((size_t)(kk >> 3) * p.out16_rows + bb) * 8 + (kk & 7);
       }
       if (p.out16_bf16) reinterpret_cast<__bf16*>(p.out16)[i16] = (__bf16)y;
       else reinterpret_cast<_Float16*>(p.out16)[i16] = (_Float16)y;
@@ -876,9 +876,9 @@ __global__ __launch_bounds__(wg_max_parts(D, GT) * 64) void attn_wg_kernel(AttnP
     *reinterpret_cast<float4*>(p.out + idx) = y;
     if (p.out16) {
       size_t i16 = idx;
-      if (p.out16_blocked) {
+      if (p.out16_rows) {
         const int bb = row / p.hq, kk = (row % p.hq) * D + e;  // elements kk .. kk+3 of batch row bb
-        i16 = ((size_t)(kk >> 3) * 32 + bb) * 8 + (kk & 7);
+        i16 = ((size_t)(kk >> 3) * p.out16_rows + bb) * 8 + (kk & 7);
       }
       if (p.out16_bf16) {
         typedef __bf16 b4 __attribute__((ext_vector_type(4)));
@@ -1163,9 +1163,9 @@ __global__ __launch_bounds__(256) void attn_lean_reduce_kernel(AttnParams p, lon
     p.out[idx] = y;
     if (p.out16) {
       size_t i16 = idx;
-      if (p.out16_blocked) {
+      if (p.out16_rows) {
         const int bb = row / p.hq, kk = (row % p.hq) * D + k * 64 + lane;  // element kk of batch row bb
-        i16 = ((size_t)(kk >> 3) * 32 + bb) * 8 + (kk & 7);
+        i16 = ((size_t)(kk >> 3) * p.out16_rows + bb) * 8 + (kk & 7);
       }
       if (p.out16_bf16) reinterpret_cast<__bf16*>(p.out16)[i16] = (__bf16)y;
       else reinterpret_cast<_Float16*>(p.out16)[i16] = (_Float16)y;
@@ -1609,7 +1609,7 @@ void attention_tuning_last(int64_t* cap, int64_t* wg, int64_t* ordered) {
 namespace pto_hip {
 int paged_attention(const void* query, const void* key_cache, const void* value_cache,
                     const int32_t* block_table, const int32_t* context_lens, float* out, void* out16,
-                    bool want_blocked, bool* wrote_blocked, const int64_t* config, int q_dtype, int kv_dtype, const float* k_scale,
+                    int out16_rows, bool* wrote_blocked, const int64_t* config, int q_dtype, int kv_dtype, const float* k_scale,
                     const float* v_scale, int64_t pool_blocks, void* stream, void* fixed_scratch,
                     size_t fixed_scratch_bytes, int64_t active_blocks, AttnPartials* unmerged) {
   Context& cx = ctx();
@@ -1648,7 +1648,7 @@ int paged_attention(const void* query, const void* key_cache, const void* value_
   p.out = out;
   p.out16 = nullptr;
   p.out16_bf16 = q_dtype == PTO_HIP_BF16;
-  p.out16_blocked = 0;
+  p.out16_rows = 0;
   if (wrote_blocked) *wrote_blocked = false;
   p.k_scale = k_scale;
   p.v_scale = v_scale;
@@ -1814,8 +1814,8 @@ int paged_attention(const void* query, const void* key_cache, const void* value_
   if (merged) {
     // the merge kernel writes the copy, blocked on request; without a merge a cast kernel writes it row-major
     p.out16 = out16;
-    p.out16_blocked = (out16 && want_blocked) ? 1 : 0;
-    if (wrote_blocked) *wrote_blocked = p.out16_blocked != 0;
+    p.out16_rows = out16 ? out16_rows : 0;
+    if (wrote_blocked) *wrote_blocked = p.out16_rows != 0;
   }
   int rc;
   const int nb = (int)batch;
@@ -1890,7 +1890,7 @@ extern "C" int pto_hip_paged_attention_noalloc(const void* query, const void* ke
   if (!area)
     return pto_hip::fail(PTO_HIP_ERR_NOT_INITIALIZED, "the static scratch area of device %d was not set up by pto_hip_init",
                          cx.device);
-  return pto_hip::paged_attention(query, key_cache, value_cache, block_table, context_lens, out, nullptr, false, nullptr,
+  return pto_hip::paged_attention(query, key_cache, value_cache, block_table, context_lens, out, nullptr, 0, nullptr,
                                   config, q_dtype, kv_dtype, k_scale, v_scale, 0, stream, area,
                                   PTO_HIP_NOALLOC_SCRATCH_BYTES);
 }
@@ -1902,7 +1902,7 @@ extern "C" int pto_hip_paged_attention(const void* query, const void* key_cache,
                                        const float* k_scale, const float* v_scale, void* stream) {
   PTO_DISPATCH_LOCK();
   // The size of the caches is not part of this signature: table entries are used as given.
-  return pto_hip::paged_attention(query, key_cache, value_cache, block_table, context_lens, out, nullptr, false, nullptr, config,
+  return pto_hip::paged_attention(query, key_cache, value_cache, block_table, context_lens, out, nullptr, 0, nullptr, config,
                                   q_dtype, kv_dtype, k_scale, v_scale, 0, stream);
 }
 

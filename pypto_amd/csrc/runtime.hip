@@ -1088,6 +1088,9 @@ int pto_hip_set_option(const char* name, int64_t value) {
   } else if (!std::strcmp(name, "w8a16_nt")) {
     PTO_CHECK_ARG(value == 0 || value == 1, "w8a16_nt must be 0 or 1");
     c.w8a16_nt = value;
+  } else if (!std::strcmp(name, "gemm_stream")) {
+    PTO_CHECK_ARG(value >= 0 && value <= 2, "gemm_stream must be 0, 1 or 2");
+    c.gemm_stream = value;
   } else if (!std::strcmp(name, "attn_order")) {
     PTO_CHECK_ARG(value >= -1 && value <= 1, "attn_order must be -1, 0 or 1");
     c.attn_order = value;
@@ -1161,6 +1164,7 @@ int pto_hip_get_option(const char* name, int64_t* value) {
   else if (!std::strcmp(name, "attn_autotune")) *value = c.attn_autotune;
   else if (!std::strcmp(name, "attn_lean_siblings")) *value = c.attn_lean_siblings;
   else if (!std::strcmp(name, "attn_order")) *value = c.attn_order;
+  else if (!std::strcmp(name, "gemm_stream")) *value = c.gemm_stream;
   else if (!std::strcmp(name, "w8a16_nt")) *value = c.w8a16_nt;
   else if (!std::strcmp(name, "workspace_bytes"))  // read only: device memory the three grow-only scratch areas hold
     *value = (int64_t)(c.workspace_bytes + c.layer_ws_bytes + c.gemm_ws_bytes);

@@ -45,13 +45,13 @@ struct FinishParams {
   const void* residual; // [M, N] in res_dtype, or null
   void* out;            // [M, N]
   int m, n, splits, res_dtype, out_dtype;
-  int out_blocked;  // write out as [N/8][32][8] for the next projection
+  int out_rows;  // write out as [N/8][out_rows][8] for the next projection; 0: row-major
   int64_t stride;
   SlabMap map;
 };
 
-// Element index of (row m, channel n) in the blocked activation layout [N/8][32][8].
-__device__ __forceinline__ size_t blocked_index(int m, int n) { return ((size_t)(n >> 3) * kMaxM + m) * 8 + (n & 7); }
+// Element index of (row m, channel n) in the blocked activation layout [N/8][rows][8].
+__device__ __forceinline__ size_t blocked_index(int rows, int m, int n) { return ((size_t)(n >> 3) * rows + m) * 8 + (n & 7); }
 
 __device__ __forceinline__ float4 load4_as_f32(const void* p, size_t i, int dt) {
   if (dt == PTO_HIP_FP32) return *reinterpret_cast<const float4*>(reinterpret_cast<const float*>(p) + i);
@@ -76,10 +76,13 @@ __device__ __forceinline__ void store4_from_f32(void* p, size_t i, int dt, float
   }
 }
 
+// BLOCKED: eight rows and 128 channels a workgroup, a wavefront's 64 quads whole 128-byte lines of the blocked layout (8 rows x 8
+// channels); rows of the layout written one a workgroup, its lines are put together from eight XCDs' caches.
+template <bool BLOCKED>
 __global__ __launch_bounds__(256) void w8a16_finish_kernel(FinishParams p) {
-  const int n = (blockIdx.x * 256 + threadIdx.x) * 4;
-  const int m = blockIdx.y;
-  if (n >= p.n) return;
+  const int n = BLOCKED ? blockIdx.x * 128 + (threadIdx.x >> 3) * 4 : (blockIdx.x * 256 + threadIdx.x) * 4;
+  const int m = BLOCKED ? blockIdx.y * 8 + (threadIdx.x & 7) : blockIdx.y;
+  if (n >= p.n || m >= p.m) return;
   const size_t idx = (size_t)m * p.n + n;
   float4 r = {0.f, 0.f, 0.f, 0.f};  // requested with the slabs
   if (p.residual) r = load4_as_f32(p.residual, idx, p.res_dtype);
@@ -92,7 +95,7 @@ __global__ __launch_bounds__(256) void w8a16_finish_kernel(FinishParams p) {
   if (p.residual) {
     a.x += r.x; a.y += r.y; a.z += r.z; a.w += r.w;
   }
-  store4_from_f32(p.out, p.out_blocked ? blocked_index(m, n) : idx, p.out_dtype, a);
+  store4_from_f32(p.out, BLOCKED ? blocked_index(p.out_rows, m, n) : idx, p.out_dtype, a);
 }
 
 // Finish of a projection followed by RMSNorm of the sum with the residual: one workgroup per
@@ -108,14 +111,14 @@ struct FinishNormParams {
   const float* gamma;    // [N]
   void* normed_out;      // [M, N] in out_dtype
   int n, splits, res_dtype, out_dtype;
-  int out_blocked;
+  int out_rows;
   float eps;
   int64_t stride;  // elements between splits
   SlabMap map;
 };
 
 __global__ __launch_bounds__(kNormThreads) void w8a16_finish_norm_kernel(FinishNormParams p) {
-  const int m = blockIdx.x;
+  const int m = p.out_rows ? pto_hip::blocked_row(blockIdx.x, gridDim.x) : blockIdx.x;
   float4 v[kNormVec];
   float4 g[kNormVec];  // requested with the row, so that the second pass waits for nothing
   float ss = 0.f;
@@ -146,7 +149,7 @@ __global__ __launch_bounds__(kNormThreads) void w8a16_finish_norm_kernel(FinishN
     const int n = (threadIdx.x + u * kNormThreads) * 4;
     if (n < p.n) {
       const float4 y = {v[u].x * inv * g[u].x, v[u].y * inv * g[u].y, v[u].z * inv * g[u].z, v[u].w * inv * g[u].w};
-      store4_from_f32(p.normed_out, p.out_blocked ? blocked_index(m, n) : (size_t)m * p.n + n, p.out_dtype, y);
+      store4_from_f32(p.normed_out, p.out_rows ? blocked_index(p.out_rows, m, n) : (size_t)m * p.n + n, p.out_dtype, y);
     }
   }
 }
@@ -321,7 +324,7 @@ int w8a16_partials(const void* x, bool x_blocked, const void* wq0, const void* w
 }
 
 int w8a16_finish(const W8Partials& parts, const float* scale0, const float* scale1, const void* residual,
-                 int res_dtype, void* out, int out_dtype, bool out_blocked, int64_t m, int64_t n, hipStream_t st) {
+                 int res_dtype, void* out, int out_dtype, int out_rows, int64_t m, int64_t n, hipStream_t st) {
   FinishParams f{};
   f.part0 = parts.part[0];
   f.part1 = parts.part[1];
@@ -334,10 +337,13 @@ int w8a16_finish(const W8Partials& parts, const float* scale0, const float* scal
   f.splits = parts.splits;
   f.res_dtype = res_dtype;
   f.out_dtype = out_dtype;
-  f.out_blocked = out_blocked ? 1 : 0;
+  f.out_rows = out_rows;
   f.stride = parts.slab_stride;
   f.map = parts.map;
-  hipLaunchKernelGGL(w8a16_finish_kernel, dim3((unsigned)((n / 4 + 255) / 256), (unsigned)m), dim3(256), 0, st, f);
+  if (out_rows)
+    hipLaunchKernelGGL(w8a16_finish_kernel<true>, dim3((unsigned)((n + 127) / 128), (unsigned)((m + 7) / 8)), dim3(256), 0, st, f);
+  else
+    hipLaunchKernelGGL(w8a16_finish_kernel<false>, dim3((unsigned)((n / 4 + 255) / 256), (unsigned)m), dim3(256), 0, st, f);
   PTO_CHECK_HIP(hipGetLastError());
   return PTO_HIP_OK;
 }
@@ -345,7 +351,7 @@ int w8a16_finish(const W8Partials& parts, const float* scale0, const float* scal
 bool w8a16_finish_norm_fits(int64_t n) { return n % 4 == 0 && n <= 4 * kNormThreads * kNormVec; }
 
 int w8a16_finish_norm(const W8Partials& parts, const float* scale, const void* residual, int res_dtype,
-                      float* sum_out, const float* gamma, void* normed_out, int out_dtype, bool out_blocked,
+                      float* sum_out, const float* gamma, void* normed_out, int out_dtype, int out_rows,
                       int64_t m, int64_t n, float eps, hipStream_t st) {
   FinishNormParams f{};
   f.part = parts.part[0];
@@ -358,7 +364,7 @@ int w8a16_finish_norm(const W8Partials& parts, const float* scale, const void* r
   f.splits = parts.splits;
   f.res_dtype = res_dtype;
   f.out_dtype = out_dtype;
-  f.out_blocked = out_blocked ? 1 : 0;
+  f.out_rows = out_rows;
   f.eps = eps;
   f.stride = parts.slab_stride;
   f.map = parts.map;
@@ -398,7 +404,7 @@ extern "C" int pto_hip_w8a16_matmul(const void* x, const void* w_q, const float*
     if (rc) return rc;
     rc = w8a16_finish(parts, w_scale, nullptr,
                       residual ? byte_offset(residual, r0 * n * dtype_bytes(res_dtype)) : nullptr, res_dtype,
-                      byte_offset(out, r0 * n * dtype_bytes(out_dtype)), out_dtype, false, rows, n, st);
+                      byte_offset(out, r0 * n * dtype_bytes(out_dtype)), out_dtype, 0, rows, n, st);
     if (rc) return rc;
   }
   return PTO_HIP_OK;
@@ -426,7 +432,7 @@ extern "C" int pto_hip_w8a16_swiglu(const void* x, const void* wg_q, const float
     rc = w8a16_partials(byte_offset(x, r0 * k * 2), false, wg_q, wu_q, rows, k, n, x_dtype, st, &parts);
     if (rc) return rc;
     rc = w8a16_finish(parts, wg_scale, wu_scale, nullptr, 0, byte_offset(out, r0 * n * dtype_bytes(out_dtype)),
-                      out_dtype, false, rows, n, st);
+                      out_dtype, 0, rows, n, st);
     if (rc) return rc;
   }
   return PTO_HIP_OK;

@@ -1,0 +1,86 @@
+"""Projections of 33 to 96 rows that stream their weights (stream_rows.h), inside decoder layers and FFN blocks."""
+
+import pytest
+import torch
+
+import oracle
+from pypto_amd import runtime, workloads
+
+pytestmark = pytest.mark.gpu
+
+
+def _error(got, want):
+    return ((got.double() - want.double()).norm() / want.double().norm()).item()
+
+
+# row groups of 16 full and not, 3, 4 and 6 of them; k that ends inside a 32-row step, fewer steps than wavefronts, columns
+# that end inside a slab and inside a matrix of a pair
+@pytest.mark.parametrize("batch", [33, 48, 49, 64, 65, 96])
+@pytest.mark.parametrize("hidden,heads,kv_heads,inter,int8,dtype", [
+    (512, 4, 2, 1040, True, torch.float16), (1040, 8, 1, 2064, True, torch.bfloat16), (1040, 8, 1, 2064, False, torch.bfloat16),
+    (48, 2, 1, 80, False, torch.float16), (2048, 5, 5, 4112, False, torch.float16), (4096, 32, 8, 1344, True, torch.bfloat16)])
+def test_decoder_layer_streamed_beside_tiled(worker, batch, hidden, heads, kv_heads, inter, int8, dtype):
+    """Both are fp32 sums of the same products, rounded to the activation type at the same places: they differ by what a sum in another
+    order moves across a rounding boundary, under two units of the type in the norm (2^-8 bf16, 2^-11 fp16)."""
+    lens = [1 + (37 * i) % 130 for i in range(batch)]
+    d = workloads.decoder_layer_inputs(batch=batch, hidden=hidden, num_heads=heads, kv_head_num=kv_heads, intermediate=inter, block_size=64,
+                                       context_lens=lens, dtype=dtype, seed=batch, device="cuda", int8_weights=int8, weight_std=None)
+    before = d.key_cache.clone(), d.value_cache.clone()
+    program = runtime.decoder_layer_decode if int8 else runtime.decoder_layer_decode_w16
+    got = []
+    try:
+        for stream in (0, 2, 2):
+            worker.set_option("gemm_stream", stream)
+            d.key_cache.copy_(before[0])
+            d.value_cache.copy_(before[1])
+            d.out.fill_(float("nan"))
+            with worker.register(program) as h:
+                h(*d.args())
+            worker.sync()
+            got.append((d.out.clone(), d.key_cache.clone(), d.value_cache.clone()))
+    finally:
+        worker.set_option("gemm_stream", 1)
+    unit = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11
+    assert all(torch.equal(a, b) for a, b in zip(got[1], got[2]))
+    for a, b in zip(got[1], got[0]):
+        assert bool(a.isfinite().all()) and _error(a, b) < 2 * unit
+
+
+@pytest.mark.parametrize("tokens,hidden,inter", [(33, 1040, 4112), (64, 2048, 1032), (90, 48, 200), (96, 4096, 11008)])
+@pytest.mark.parametrize("out_dtype", [torch.float32, torch.bfloat16])
+def test_ffn_block_streamed_against_the_oracle(worker, tokens, hidden, inter, out_dtype):
+    f = workloads.ffn_inputs(tokens=tokens, hidden=hidden, intermediate=inter, out_dtype=out_dtype, seed=tokens, device="cuda")
+    buf = torch.full((tokens * hidden + 1024,), -77.0, dtype=out_dtype, device="cuda")
+    out = buf[512:512 + tokens * hidden].view(tokens, hidden)
+    worker.set_option("gemm_stream", 2)
+    try:
+        with worker.register(runtime.ffn_block) as h:
+            h(f.x, f.gamma, f.w_gate, f.w_up, f.w_down, out, f.eps)
+        worker.sync()
+    finally:
+        worker.set_option("gemm_stream", 1)
+    ref = oracle.ffn_block(f.x.cpu(), f.gamma.cpu(), f.w_gate.cpu(), f.w_up.cpu(), f.w_down.cpu(), f.eps)
+    runtime.validate_golden({"out": out.cpu().float()}, {"out": ref.float()}, rtol=2e-2, atol=1e-2)
+    assert bool((buf[:512] == -77.0).all()) and bool((buf[512 + tokens * hidden:] == -77.0).all())
+
+
+def test_replays_of_a_captured_block(worker):
+    """Recorded after one eager call; every replay, between eager calls that use the same scratch, gives its result."""
+    small = workloads.ffn_inputs(tokens=40, hidden=4096, intermediate=11008, seed=1, device="cuda")
+    with worker.register(runtime.ffn_block) as h:
+        stream = torch.cuda.Stream()
+        with torch.cuda.stream(stream):
+            h(small.x, small.gamma, small.w_gate, small.w_up, small.w_down, small.out, small.eps, stream=stream.cuda_stream)
+            stream.synchronize()
+            want = small.out.clone()
+            graph = torch.cuda.CUDAGraph()
+            graph.capture_begin()
+            h(small.x, small.gamma, small.w_gate, small.w_up, small.w_down, small.out, small.eps, stream=stream.cuda_stream)
+            graph.capture_end()
+            for _ in range(3):
+                small.out.zero_()
+                graph.replay()
+                stream.synchronize()
+                assert torch.equal(small.out, want)
+                h(small.x, small.gamma, small.w_gate, small.w_up, small.w_down, torch.empty_like(small.out), small.eps, stream=stream.cuda_stream)
+                stream.synchronize()
