@@ -69,7 +69,7 @@ struct Context {
   int64_t w8a16_nt = 1;            // skinny projections: weight rows read with non-temporal loads
   int64_t gemm_variant = 0;
   int64_t gemm_quad_rows = 0;    // tile height of the four-wavefront form: 0 = by estimate
-  int64_t gemm_narrow = 0;       // small-call form of products with 16-bit weights: -1 never, 0 by estimate, 1..4 its tile
+  int64_t gemm_narrow = 0;       // small-call form of products with 16-bit or e4m3 weights: -1 never, 0 by estimate, 1..4 its tile
   int64_t gemm_splits = 0;       // k splits of the tiled GEMM: 0 = by shape, 1..16 = as given (when k allows)
   int64_t w8a16_wgs_per_cu = 1;  // most workgroups of the skinny projection kernel per compute unit
   int64_t w8a16_wide = 1;        // int8 codes read 16 per lane: 0 never, 1 for large matrices, 2 whenever shapes allow

@@ -12,6 +12,7 @@
 // transpose of the 16-bit layout) plus one fp32 scale per output channel, so both GEMM operands
 // are k-major and go global -> LDS -> registers without any transpose.  The GEMM uses
 // v_mfma_f32_32x32x64_f8f6f4: lane l holds row/column l % 32 and the 32 codes k = 32 * (l / 32) .. +32.
+// Products of a small call go to narrow_gemm8.h instead (choose_narrow8).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -19,6 +20,7 @@
 #include <type_traits>
 
 #include "common.h"
+#include "launch_choice.h"
 #include "lds_load.h"
 
 namespace pto_hip {
@@ -529,10 +531,18 @@ __global__ __launch_bounds__(256) void gemm8_finish_kernel(const float* __restri
   }
 }
 
+}  // namespace gemm8
+}  // namespace pto_hip
+
+#include "narrow_gemm8.h"
+
+namespace pto_hip {
+namespace gemm8 {
+
 // Picks the tile height and the k splits and launches the tiles.  With p.splits > 1 afterwards the slabs
-// hold the raw sums and the caller finishes them.
+// hold the raw sums and the caller finishes them: in a launch of its own, or (sums_on_the_way) in one that it makes anyway.
 template <bool DUAL, typename OutT>
-int launch_tiles(Params& p, hipStream_t st) {
+int launch_tiles(Params& p, bool sums_on_the_way, hipStream_t st) {
   const int64_t num_cu = pto_hip::ctx().num_cu, variant = pto_hip::ctx().gemm_variant, forced = pto_hip::ctx().gemm_splits;
   const int64_t tiles_n = (p.n + (DUAL ? 127 : 255)) / (DUAL ? 128 : 256);
   const int nk = p.k / BK;
@@ -564,6 +574,16 @@ int launch_tiles(Params& p, hipStream_t st) {
         }
       }
     }
+    // Small calls in narrow tiles, one launch.  The estimate's 3 us for the launch that sums the slabs do not count against a caller that has one anyway.
+    const int64_t narrow = pto_hip::ctx().gemm_narrow;
+    if (can_split && forced == 0 && narrow >= 0) {
+      const double tiled_us = best - (sums_on_the_way && splits > 1 ? 3.0 : 0.0);
+      const int tile = narrow > 0 ? (int)std::min<int64_t>(narrow, 3) : pto_hip::choose_narrow8(p.m, p.n, p.k, DUAL, num_cu, tiled_us);
+      if (tile > 0) {
+        p.splits = 1;
+        return launch_narrow8<DUAL, OutT>(p, tile, st);
+      }
+    }
   }
   const bool long_rows = std::max(p.lda, p.ldb) >= kLongRow;  // built on 128-row tiles
   const int per = (nk + splits - 1) / splits;
@@ -588,7 +608,7 @@ int launch_tiles(Params& p, hipStream_t st) {
 
 template <bool DUAL, typename OutT>
 int launch_any(Params p, hipStream_t st) {
-  const int rc = launch_tiles<DUAL, OutT>(p, st);
+  const int rc = launch_tiles<DUAL, OutT>(p, false, st);
   if (rc || p.splits == 1) return rc;
   const unsigned bx = (unsigned)((p.n / 4 + 255) / 256);
   const unsigned by = (unsigned)std::min<int64_t>(p.m, std::max<int64_t>(1, 4096 / bx));
@@ -945,7 +965,7 @@ extern "C" int pto_hip_ffn_swiglu_fp8(const void* x, const float* gamma, const v
   p1.n = (int)intermediate;
   p1.k = (int)hidden;
   const bool bf16 = x_dtype == PTO_HIP_BF16;
-  rc = bf16 ? gemm8::launch_tiles<true, __bf16>(p1, st) : gemm8::launch_tiles<true, _Float16>(p1, st);
+  rc = bf16 ? gemm8::launch_tiles<true, __bf16>(p1, true, st) : gemm8::launch_tiles<true, _Float16>(p1, true, st);
   if (rc) return rc;
   if (p1.splits > 1) {
     // k split: the quantiser sums the slabs itself, h is not written

@@ -125,6 +125,34 @@ inline int choose_narrow(int64_t m, int64_t n, int64_t k, bool dual, int64_t num
   return tile;
 }
 
+// Tile of the small-call form of e4m3 products (narrow_gemm8.h): 1: 16 rows x 16 channels, 2: 32 x 32, 3: 64 x 32; 0: the tiled GEMM.
+// Estimated microseconds, fitted to 1 to 1024 rows of sixteen weight shapes from 512 x 1024 to 13824 x 5120 (rms 10 to 19 %): a launch, the operand
+// KB of a tile once per round of workgroups over the CUs, and what the weights take to arrive.  tiled_us: what the tiled form's own
+// estimate says; this form has to be 5 % ahead.  Timed at other row counts, and with six other weight shapes among them, the rule is 1.45 times as
+// fast as the tiled form alone, the best of all four 1.48, and nothing is slower by more than the noise of 2 %.
+inline int choose_narrow8(int64_t m, int64_t n, int64_t k, bool dual, int64_t num_cu, double tiled_us) {
+  struct Tile {
+    int rows, channels;
+    double us[2], round[2], kb[2], mb[2];  // of a single product and of a pair
+  };
+  static constexpr Tile kTiles[3] = {{16, 16, {1.78, 1.83}, {0.39, 1.68}, {0.0306, 0.0057}, {0.0, 0.170}},
+                                     {32, 32, {1.36, 2.61}, {0.72, 1.02}, {0.0286, 0.0219}, {0.0, 0.111}},
+                                     {64, 32, {0.0, 1.56}, {5.09, 0.64}, {0.0198, 0.0361}, {0.0, 0.0}}};
+  double best = 0.95 * tiled_us;
+  int tile = 0;
+  for (int i = 0; i < 3; ++i) {
+    const Tile& t = kTiles[i];
+    const int64_t wgs = ((m + t.rows - 1) / t.rows) * ((n + t.channels - 1) / t.channels);
+    const double kb = (double)k * (t.channels * (dual ? 2 : 1) + t.rows) * 1e-3;
+    const double us = t.us[dual] + (double)((wgs + num_cu - 1) / num_cu) * (t.round[dual] + t.kb[dual] * kb) + t.mb[dual] * (double)k * n * (dual ? 2 : 1) * 1e-6;
+    if (us < best) {
+      best = us;
+      tile = i + 1;
+    }
+  }
+  return tile;
+}
+
 // Whether a projection of m rows inside a decoder layer or block streams its weights (stream_rows.h) instead of running as a tiled GEMM.
 // Measured in whole layers with each projection switched, 36 / 56 / 80 / 96 rows of twelve models from 1024 x 3072 to 8192 x 28672, us gained:
 // 16-bit weights: pairs from 30 million on (4096 x 14336 4 / 5 / 4 / 6, 3072 x 8192 9 / 14 / 13 / 14, 8192 x 16384 10 / 10 / 11 / 12; 2048 x 5632, 23 million,

@@ -13,6 +13,7 @@ extern "C" int choose_narrow(int m, int n, int k, int dual) {
   int height = 0, splits = 0;
   return pto_hip::choose_narrow(m, n, k, dual != 0, 256, pto_hip::choose_quad(m, n, k, dual != 0, 256, 0, &height, &splits));
 }
+extern "C" int choose_narrow8(int m, int n, int k, int dual, double tiled_us) { return pto_hip::choose_narrow8(m, n, k, dual != 0, 256, tiled_us); }
 extern "C" int beats_skinny(int64_t k, int64_t n, int dual) { return pto_hip::narrow_beats_skinny(k, n, dual != 0); }
 """
 
@@ -24,6 +25,7 @@ def choice(tmp_path_factory):
     so = d / "choice.so"
     subprocess.run(["g++", "-std=c++17", "-O1", "-shared", "-fPIC", f"-I{CSRC}", str(d / "choice.cpp"), "-o", str(so)], check=True)
     lib = C.CDLL(str(so))
+    lib.choose_narrow8.argtypes = [C.c_int] * 4 + [C.c_double]
     lib.beats_skinny.argtypes = [C.c_int64, C.c_int64, C.c_int]
     return lib
 
@@ -45,3 +47,11 @@ def test_large_products_keep_the_tiled_form(choice):
 def test_up_to_32_rows_only_small_weights(choice):
     assert choice.beats_skinny(512, 1536, 1) and choice.beats_skinny(2048, 768, 0) and choice.beats_skinny(1024, 1024, 0)
     assert not choice.beats_skinny(768, 2048, 1) and not choice.beats_skinny(2048, 1024, 0) and not choice.beats_skinny(1 << 29, 1 << 29, 1)
+
+
+# (m, n, k, pair): the tiled GEMM's measured us and the fastest measured tile of the form (0: none)
+@pytest.mark.parametrize("m,n,k,dual,us,tile", [(8, 1024, 512, 1, 7.7, 1), (128, 512, 1024, 0, 11.5, 1), (64, 2816, 768, 1, 8.9, 2), (512, 1024, 512, 1, 8.0, 3),
+                                                (192, 768, 2816, 0, 14.0, 2), (512, 2816, 1024, 1, 12.4, 0), (64, 5120, 13824, 0, 25.6, 0),
+                                                (8, 11008, 4096, 1, 22.4, 0), (2048, 4096, 11008, 0, 93.0, 0)])
+def test_small_e4m3_products_take_the_measured_tile(choice, m, n, k, dual, us, tile):
+    assert choice.choose_narrow8(m, n, k, dual, us) == tile
