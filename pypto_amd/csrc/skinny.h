@@ -432,7 +432,7 @@ struct Activations<BF16, kSwiglu> {
         auto get = [&](int b) { t[u][mat][b] = *reinterpret_cast<const f32x4*>(src + (size_t)min(b, last) * s.pair.slab_stride); };
         get(0);
         get(1);
-        if (s.pair.splits > 3) {  // (at most; two whole shares per slab count three)
+        if (s.pair.splits > 2) {  // (at most: shares that cross slabs give a slab of two shares' work three parts)
           get(2);
           get(3);
         }

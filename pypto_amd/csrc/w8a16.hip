@@ -224,8 +224,9 @@ SkinnyPlan plan_skinny(int64_t k, int64_t n, const void* wq0, const void* wq1, b
   // (units * wgs is computed in 32 bits by the kernels; shapes beyond that get a workgroup per slab)
   q.mapped = q.units * q.wgs < (1ll << 31);
   if (!q.mapped) q.wgs = slabs_total;
-  q.splits = q.mapped ? (int)((q.ks * q.wgs + q.units - 1) / q.units) + 1 : 1;  // at most
   q.per_slab = q.wgs % slabs_total == 0 && q.wgs / slabs_total <= q.ks ? (int)(q.wgs / slabs_total) : 0;
+  // at most; whole shares are as many for every slab
+  q.splits = q.per_slab ? q.per_slab : (int)((q.ks * q.wgs + q.units - 1) / q.units) + 1;
   return q;
 }
 // LDS of the fused form: the sums and m rows of a share.

@@ -63,7 +63,8 @@ def test_decoder_layer_has_the_bits_of_separate_launches(worker, batch, hidden, 
         worker.set_option("w8a16_wide", 1)
 
 
-@pytest.mark.parametrize("tokens,hidden,inter", [(1, 4096, 11008), (2, 1040, 4112), (3, 2048, 5632), (4, 1024, 3072), (4, 8192, 2048), (1, 48, 40000)])
+@pytest.mark.parametrize("tokens,hidden,inter", [(1, 4096, 11008), (2, 1040, 4112), (3, 2048, 5632), (4, 1024, 3072), (4, 8192, 2048), (1, 48, 40000),
+                                                 (1, 2496, 8448), (2, 2560, 8448)])  # the pair's channels have two or three partial sums
 def test_ffn_block_has_the_bits_of_separate_launches(worker, tokens, hidden, inter):
     f = workloads.ffn_inputs(tokens=tokens, hidden=hidden, intermediate=inter, seed=tokens, device="cuda")
     args = (f.x, f.gamma, f.w_gate, f.w_up, f.w_down, f.out, f.eps)
