@@ -159,14 +159,15 @@ inline int choose_narrow8(int64_t m, int64_t n, int64_t k, bool dual, int64_t nu
 // lost 1 / 2 / 4 / 4), deep single ones from 40 million on (14336 x 4096 7 / 10 / 9 / 11, 13824 x 5120 9 / 11 / 10 / 9; 8192 x 3072 lost 2 to 6,
 // square ones 0 to 7).
 // int8: pairs from 80 million on (4096 x 14336 10 / 9 / 7 / 4, 4096 x 11008 11 / 8 / 6 / 6; 3072 x 8192 lost 0 to 3), deep single ones of 5120 channels
-// and 60 million up, with few slabs a channel (13824 x 5120 3 / 3 / 2 / 2, 16384 x 8192 7 / 5 / 4 / 3; 14336 x 4096 lost 0 to 2); and up to 64 rows of few k, whose 64-row
-// tiles found no k split: singles up to 4096 (4096 x 4096 2, 3072 x 3072 26 / 25, 2048 x 2048 18, 3072 x 1024 35) and pairs up to 1536 (1024 x 3072 7 / 4; 2048 x 5632 lost 1).
+// and 60 million up, with few slabs a channel (13824 x 5120 3 / 3 / 2 / 2, 16384 x 8192 7 / 5 / 4 / 3; 14336 x 4096 lost 0 to 2).
+// Few k, up to 64 rows (layers with these projections tiled -> streamed, k split in both, 36 / 48 / 64 rows, us gained): hidden 1024 5 / 4 / 2,
+// 1280 4 / 3 / 0, 1536 4 / 2 / -1, 1792 2 / 1 / 0, 2048 2 / 1 / 0, 2304 2 / 1 / 0, 3072 3 / 2 / 2, 3584 8 / 9 / 8.
 constexpr int kStreamRowsMax = 96;
 inline bool stream_rows_ahead(int64_t m, int64_t k, int64_t n, bool dual, bool w16) {
   const int64_t weights = k * n * (dual ? 2 : 1);
   if (w16) return dual ? weights >= 30000000 : weights >= 40000000 && k >= 2 * n;
-  if (dual) return weights >= 80000000 || (m <= 64 && k <= 1536);
-  return (m <= 64 && k <= 4096) || (n >= 5120 && weights >= 60000000 && k >= 2 * n);
+  if (dual) return weights >= 80000000 || (m <= 64 && k <= (m <= 48 ? 1536 : 1280));
+  return (m <= 64 && k <= 4096 && (m <= 48 || k <= 1280 || k >= 3072)) || (n >= 5120 && weights >= 60000000 && k >= 2 * n);
 }
 
 // Tokens per context partition of a workgroup-form attention launch (a workgroup per (sequence, KV head) pair, its
