@@ -1515,9 +1515,11 @@ namespace {
 // How a launch spreads over the CUs depends on how ragged the context lengths are, which the host
 // does not see (they live in device memory).  For every launch signature the first calls therefore
 // time a short list of shapes that all give bit-identical results - residency caps of the
-// partition grid and, where the partition count allows it, the workgroup form, both also with the sequences by length - with a pair of
+// partition grid and, where the partition count allows it, the workgroup form - with a pair of
 // events around each call's launches, read back without blocking on later calls; once every
-// candidate has kTuneReps readings the fastest is used from then on.  Calls made while a stream
+// candidate has kTuneReps readings the fastest is used from then on.  Then, where an order by length may gain, that shape is timed again beside
+// itself with the sequences by length and one more ordered shape: as a second round, since all in one kept a program on the rule's choice for
+// 36 calls instead of 20 (a graph recorded after 32 calls of a 16-sequence layer ran 171.1 us, not 168.9).  Calls made while a stream
 // is being captured, and the entry point that allocates nothing, never measure.
 struct TuneCandidate {
   int cap;      // residency cap of the partition grid (0 = none)
@@ -1533,7 +1535,17 @@ struct TuneState {
   std::vector<float> best_us;
   std::vector<int> issued, done;
   std::vector<TunePending> pending;
-  int chosen = -1;
+  int chosen = -1;     // of the rounds that are over
+  size_t settled = 0;  // candidates of the rounds that are over
+  bool order = false;  // a round of orders by length is to come
+  bool wg_possible = false;
+
+  void add(TuneCandidate c) {
+    cands.push_back(c);
+    best_us.push_back(1e30f);
+    issued.push_back(0);
+    done.push_back(0);
+  }
 };
 constexpr int kTuneReps = 4;
 constexpr size_t kTuneMaxSignatures = 512;  // signatures beyond this many run the fixed rule
@@ -1567,20 +1579,26 @@ void tune_harvest(TuneState& ts) {
     ts.pending[i] = ts.pending.back();
     ts.pending.pop_back();
   }
-  if (ts.chosen < 0) {
-    bool all = true;
-    for (int d : ts.done) all = all && d >= kTuneReps;
-    if (all) {
-      ts.chosen = 0;
-      // a candidate must win by 1 %; an order by length, behind the others in the list, by 4: what it gains at all is more
-      // (with 1 % two of 37 drawn calls took it and were 1 and 3 % slower)
-      float beat = ts.best_us[0];
-      for (size_t c = 1; c < ts.cands.size(); ++c)
-        if (ts.best_us[c] < beat * (ts.cands[c].ordered && !ts.cands[ts.chosen].ordered ? 0.96f : 0.99f)) {
-          ts.chosen = (int)c;
-          beat = ts.best_us[c];
-        }
+  bool all = ts.settled < ts.cands.size();
+  for (size_t c = ts.settled; c < ts.cands.size(); ++c) all = all && ts.done[c] >= kTuneReps;
+  if (!all) return;
+  // A candidate must win by 1 %; an order by length by 4: what it gains at all is more (with 1 % two of 37 drawn calls took it
+  // and were 1 and 3 % slower).  The first of a round is what the others are measured against.
+  ts.chosen = (int)ts.settled;
+  float beat = ts.best_us[ts.chosen];
+  for (size_t c = ts.settled + 1; c < ts.cands.size(); ++c)
+    if (ts.best_us[c] < beat * (ts.cands[c].ordered && !ts.cands[ts.chosen].ordered ? 0.96f : 0.99f)) {
+      ts.chosen = (int)c;
+      beat = ts.best_us[c];
     }
+  ts.settled = ts.cands.size();
+  if (ts.order) {
+    ts.order = false;
+    const TuneCandidate best = ts.cands[ts.chosen];
+    ts.add(best);  // (again: the clocks ramp up during the first calls)
+    ts.add({best.cap, best.wg, true});
+    if (ts.wg_possible && !best.wg) ts.add({0, true, true});
+    else if (best.wg || best.cap != 0) ts.add({0, false, true});
   }
 }
 }  // namespace
@@ -1728,16 +1746,11 @@ int paged_attention(const void* query, const void* key_cache, const void* value_
   }
   if (ts) {
     if (ts->cands.empty()) {
-      ts->cands.push_back({0, p.wg_merge != 0, false});  // the rule's own choice first
-      if (wg_possible) ts->cands.push_back({0, p.wg_merge == 0, false});
-      for (int cap : {3, 2, 4}) ts->cands.push_back({cap, false, false});
-      if (may_order && pairs * 2 >= cx.num_cu) {  // (fewer pairs than half the CUs never gained)
-        if (wg_possible) ts->cands.push_back({0, true, true});
-        for (int cap : {0, 2, 4}) ts->cands.push_back({cap, false, true});
-      }
-      ts->best_us.assign(ts->cands.size(), 1e30f);
-      ts->issued.assign(ts->cands.size(), 0);
-      ts->done.assign(ts->cands.size(), 0);
+      ts->add({0, p.wg_merge != 0, false});  // the rule's own choice first
+      if (wg_possible) ts->add({0, p.wg_merge == 0, false});
+      for (int cap : {3, 2, 4}) ts->add({cap, false, false});
+      ts->order = may_order && pairs * 2 >= cx.num_cu;  // (fewer pairs than half the CUs never gained)
+      ts->wg_possible = wg_possible;
     }
     hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
     if (hipStreamIsCapturing(hs, &capturing) != hipSuccess) {
@@ -1747,7 +1760,7 @@ int paged_attention(const void* query, const void* key_cache, const void* value_
     const bool may_measure = capturing == hipStreamCaptureStatusNone && !fixed_scratch;
     if (may_measure) tune_harvest(*ts);
     int use = ts->chosen >= 0 ? ts->chosen : 0;
-    if (ts->chosen < 0 && may_measure) {
+    if (may_measure) {
       // the candidate measured least so far: the readings of every candidate are spread over the
       // first calls alike (the clocks ramp up during them; a block of early calls per candidate
       // would favour whichever comes last)
