@@ -94,8 +94,11 @@ inline double choose_quad(int m, int n, int k, bool dual, int64_t num_cu, int fo
 // 0: the tiled GEMM.  Estimated microseconds, fitted to 40 to 1024 rows of nineteen weight shapes from 512 x 512 to 2048 x 5632
 // (rms 5 to 11 %): a launch, the operand KB of a tile once per round of workgroups over the CUs, and what the weights take to
 // arrive.  tiled_us: choose_quad's estimate, which takes 1.11 of itself and 2 us in the same measure; the form has to be 5 % ahead.  Over the
-// 175 products of 33 and more rows among them the rule is 1.35 times as fast as the tiled GEMM, the best of all tiles and forms 1.38; two
-// are slower, by 9 % at most (3584 x 1024 at 700 rows), and at 512 rows and more of wide pairs nothing changes.
+// 175 products of 33 and more rows among them the estimate was 1.35 times as fast as the tiled GEMM, the best of all tiles and forms 1.38.  Timed alone: in a
+// block the activations of the down projection have just been written by other XCDs, and every tile of channels fetches them again.  Hence
+// the last term, 1.3 us per MB of a single product's activations: without it blocks of 333 to 1000 rows lost up to 17 % (768 x 2560 at 768 rows 25.7
+// -> 30.2 us, 1024 x 3072 at 640 30.3 -> 35.4).  With it, over 110 blocks of 64 to 1300 rows of
+// ten shapes, 512 x 1024 to 1280 x 4096: 1.13 times as fast as the tiled form, five slower, by 2 to 4 %.
 // Up to 32 rows a product in the skinny form streams its weights once, in two launches; this form is ahead up to 1.6 million weights
 // (us, skinny -> this, 1 / 32 rows: 512 x 1024 pair 6.1 / 7.3 -> 4.2 / 4.5, 1024 x 1024 5.7 / 7.3 -> 4.1 / 4.7, 2048 x 768 6.1 / 7.5 ->
 // 5.6 / 6.8; but 768 x 2048 pair 7.0 / 8.4 -> 7.7 / 7.7, 1024 x 2048 pair 7.0 / 8.6 -> 9.3 / 9.5).
@@ -116,7 +119,8 @@ inline int choose_narrow(int64_t m, int64_t n, int64_t k, bool dual, int64_t num
     const Tile& t = kTiles[i];
     const int64_t wgs = ((m + t.rows - 1) / t.rows) * ((n + t.channels - 1) / t.channels);
     const double kb = (double)k * 2.0 * (t.channels * (dual ? 2 : 1) + t.rows) * 1e-3;
-    const double us = t.us[dual] + t.round[dual] * (double)((wgs + num_cu - 1) / num_cu) * kb + t.mb[dual] * (double)k * n * (dual ? 2 : 1) * 2e-6;
+    const double us = t.us[dual] + t.round[dual] * (double)((wgs + num_cu - 1) / num_cu) * kb + t.mb[dual] * (double)k * n * (dual ? 2 : 1) * 2e-6 +
+                      (dual ? 0.0 : 1.3 * (double)m * k * 2e-6);
     if (us < best) {
       best = us;
       tile = i + 1;
