@@ -111,9 +111,10 @@ __device__ __forceinline__ int slab_count(const SlabMap& s, int splits, int mat,
   return (int)(((first + s.ks) * s.wgs - 1) / s.units - ((first + 1) * s.wgs - 1) / s.units) + 1;
 }
 // Row a workgroup takes where one writes a row of the blocked layout [K/8][rows][8]: its 128-byte lines are eight rows' pieces, and
-// eight rows whose workgroups run on one XCD (workgroup id mod 8) meet in that XCD's L2.  A permutation of 0 .. rows - 1.
+// eight rows whose workgroups run on one XCD (workgroup id mod 8) meet in that XCD's L2.  A permutation of 0 .. rows - 1; rows 0, for up to
+// 32 rows, where nothing is gained: as they come.
 __device__ __forceinline__ int blocked_row(int id, int rows) {
-  if (rows <= kW8MaxM) return id;  // (nothing gained, and the division below delays a launch of 3 us by 0.1)
+  if (rows == 0) return id;
   const int base = id & ~63, groups = min(rows - base, 64) >> 3;  // groups of eight rows among the next 64
   if (groups == 0 || id - base >= groups * 8) return id;
   return base + (id - base) % groups * 8 + (id - base) / groups;

@@ -208,7 +208,7 @@ extern "C" int pto_hip_decoder_layer_decode(const PtoHipDecoderLayerArgs* a, voi
   const size_t total = sz_normed + sz_q + sz_attn + sz_attn16 + sz_resid + sz_normed + sz_h;
   // Slabs of projections that read partials from workspace(); left out, and those projections given their activations, where
   // the area would have to grow under capture.
-  size_t sz_slabs = up(std::max(skinny_fused_bytes(hq * d, h, a->wo_q, nullptr, w16), skinny_fused_bytes(inter, h, a->wd_q, nullptr, w16)));
+  size_t sz_slabs = b > kSkinnyFusedRows ? 0 : up(std::max(skinny_fused_bytes(hq * d, h, a->wo_q, nullptr, w16), skinny_fused_bytes(inter, h, a->wd_q, nullptr, w16)));
   if (total + sz_slabs > cx.layer_ws_bytes && stream_capturing((hipStream_t)stream)) sz_slabs = 0;
   void* lws = nullptr;
   {

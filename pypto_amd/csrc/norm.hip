@@ -62,10 +62,10 @@ template <typename TI, typename T, bool BLOCKED>
 __global__ __launch_bounds__(kThreads) void rms_norm_vec_kernel(const TI* __restrict__ x,
                                                                 const float* __restrict__ gamma,
                                                                 T* __restrict__ out, int64_t hidden,
-                                                                float eps, int out_rows) {
+                                                                float eps, int out_rows, int spread_rows) {
   typedef __attribute__((__vector_size__(8 * sizeof(T)))) T vec8;
   typedef __attribute__((__vector_size__(8 * sizeof(TI)))) TI vec8i;
-  const int64_t row = BLOCKED ? pto_hip::blocked_row(blockIdx.x, gridDim.x) : blockIdx.x;
+  const int64_t row = BLOCKED ? pto_hip::blocked_row(blockIdx.x, spread_rows) : blockIdx.x;
   const vec8i* xr = reinterpret_cast<const vec8i*>(x + row * hidden);
   vec8* orow = BLOCKED ? reinterpret_cast<vec8*>(out) + row : reinterpret_cast<vec8*>(out + row * hidden);
   const int out_stride = BLOCKED ? out_rows : 1;  // vec8 units between consecutive 8-element groups
@@ -147,12 +147,13 @@ int rms_norm_blocked(const void* x, const float* gamma, void* out, int64_t rows,
                 "rms_norm (blocked): unsupported shape [%lld, %lld] or operands", (long long)rows, (long long)hidden);
   if (rows == 0) return PTO_HIP_OK;
   dim3 grid((unsigned)rows), block(kThreads);
+  const int spread = rows > kW8MaxM ? (int)rows : 0;
   if (dtype == PTO_HIP_BF16)
     hipLaunchKernelGGL((rms_norm_vec_kernel<__bf16, __bf16, true>), grid, block, 0, st, (const __bf16*)x, gamma,
-                       (__bf16*)out, hidden, eps, out_rows);
+                       (__bf16*)out, hidden, eps, out_rows, spread);
   else
     hipLaunchKernelGGL((rms_norm_vec_kernel<_Float16, _Float16, true>), grid, block, 0, st, (const _Float16*)x, gamma,
-                       (_Float16*)out, hidden, eps, out_rows);
+                       (_Float16*)out, hidden, eps, out_rows, spread);
   PTO_CHECK_HIP(hipGetLastError());
   return PTO_HIP_OK;
 }
@@ -177,16 +178,16 @@ extern "C" int pto_hip_rms_norm(const void* x, const float* gamma, void* out, in
     const bool bf = out_dtype == PTO_HIP_BF16;
     if (x_dtype == PTO_HIP_FP32 && bf)
       hipLaunchKernelGGL((rms_norm_vec_kernel<float, __bf16, false>), grid, block, 0, st, (const float*)x, gamma,
-                         (__bf16*)out, hidden, eps, 0);
+                         (__bf16*)out, hidden, eps, 0, 0);
     else if (x_dtype == PTO_HIP_FP32)
       hipLaunchKernelGGL((rms_norm_vec_kernel<float, _Float16, false>), grid, block, 0, st, (const float*)x, gamma,
-                         (_Float16*)out, hidden, eps, 0);
+                         (_Float16*)out, hidden, eps, 0, 0);
     else if (bf)
       hipLaunchKernelGGL((rms_norm_vec_kernel<__bf16, __bf16, false>), grid, block, 0, st, (const __bf16*)x, gamma,
-                         (__bf16*)out, hidden, eps, 0);
+                         (__bf16*)out, hidden, eps, 0, 0);
     else
       hipLaunchKernelGGL((rms_norm_vec_kernel<_Float16, _Float16, false>), grid, block, 0, st, (const _Float16*)x,
-                         gamma, (_Float16*)out, hidden, eps, 0);
+                         gamma, (_Float16*)out, hidden, eps, 0, 0);
     PTO_CHECK_HIP(hipGetLastError());
     return PTO_HIP_OK;
   }

@@ -113,13 +113,14 @@ struct FinishNormParams {
   void* normed_out;      // [M, N] in out_dtype
   int n, splits, res_dtype, out_dtype;
   int out_rows;
+  int spread_rows;  // see blocked_row
   float eps;
   int64_t stride;  // elements between splits
   SlabMap map;
 };
 
 __global__ __launch_bounds__(kNormThreads) void w8a16_finish_norm_kernel(FinishNormParams p) {
-  const int m = p.out_rows ? pto_hip::blocked_row(blockIdx.x, gridDim.x) : blockIdx.x;
+  const int m = pto_hip::blocked_row(blockIdx.x, p.spread_rows);
   float4 v[kNormVec];
   float4 g[kNormVec];  // requested with the row, so that the second pass waits for nothing
   float ss = 0.f;
@@ -362,6 +363,7 @@ int w8a16_finish_norm(const W8Partials& parts, const float* scale, const void* r
   f.sum_out = sum_out;
   f.gamma = gamma;
   f.normed_out = normed_out;
+  f.spread_rows = out_rows && m > kW8MaxM ? (int)m : 0;
   f.n = (int)n;
   f.splits = parts.splits;
   f.res_dtype = res_dtype;
