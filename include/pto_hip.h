@@ -583,7 +583,7 @@ PTO_HIP_API int pto_hip_backend_handler_query(const char* hook, int32_t arg, cha
  *                               1.6 million weights (default), -1 = never, 1..4 = always, with that tile
  *                               ("gemm_variant", "gemm_quad_rows" or "gemm_splits" other than 0 switch it off).
  *                               e4m3 products likewise, tiles of 16 x 16, 32 x 32 and 64 x 32 (4 counts as 3)
- *  "gemm_stream"                projections of 33 to 96 rows inside a decoder layer or an FFN block with a norm that
+ *  "gemm_stream"                projections of 33 to 96 rows inside a decoder layer or an FFN block that
  *                               stream their weights into registers: 1 = where measured ahead of the tiled GEMM
  *                               (default), 0 = never, 2 = whenever shapes allow ("gemm_variant", "gemm_quad_rows"
  *                               or "gemm_splits" other than 0 switch it off)

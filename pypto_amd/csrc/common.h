@@ -228,6 +228,8 @@ int rope_kv_cache_update_fp8(const W8Partials& qkv, const float* qkv_scale,
 bool rms_norm_blocked_fits(int64_t rows, int64_t hidden, int out_rows = kW8MaxM);
 int rms_norm_blocked(const void* x, const float* gamma, void* out, int64_t rows, int64_t hidden, float eps,
                      int dtype, hipStream_t st, int out_rows = kW8MaxM);
+// Rows of 16-bit values in that layout, as they are (hidden % 8 == 0, 16-byte aligned).
+int rows_blocked(const void* x, void* out, int64_t rows, int64_t hidden, hipStream_t st, int out_rows);
 int cast_from_f32(const float* in, void* out, size_t n, int out_dtype, hipStream_t st);
 // pto_hip_paged_attention with an optional second output: the result rounded to the query dtype.
 // out16_rows asks for the copy as [Hq*D/8][out16_rows][8] over the batch rows (at most so many);

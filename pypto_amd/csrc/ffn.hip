@@ -176,7 +176,8 @@ int ffn_stream(const void* x, const float* gamma, const void* w_gate, const void
   int rc = workspace(xn_bytes + (size_t)rows * intermediate * 2, &ws);
   if (rc) return rc;
   void* h = reinterpret_cast<char*>(ws) + xn_bytes;
-  if ((rc = rms_norm_blocked(x, gamma, ws, tokens, hidden, eps, dtype, st, rows))) return rc;
+  rc = gamma ? rms_norm_blocked(x, gamma, ws, tokens, hidden, eps, dtype, st, rows) : rows_blocked(x, ws, tokens, hidden, st, rows);
+  if (rc) return rc;
   W8Partials parts{};
   if ((rc = stream_partials(ws, rows, w_gate, w_up, tokens, hidden, intermediate, dtype, st, &parts, true))) return rc;
   if ((rc = w8a16_finish(parts, nullptr, nullptr, nullptr, 0, h, dtype, rows, tokens, intermediate, st))) return rc;
@@ -267,10 +268,10 @@ extern "C" int pto_hip_ffn_swiglu(const void* x, const float* gamma, const void*
       (out_dtype == PTO_HIP_FP32 || out_dtype == dtype) && !narrow_not_skinny(hidden, intermediate, true))
     return ffn_skinny(x, gamma, w_gate, w_up, w_down, out, tokens, hidden, intermediate, eps, dtype, out_dtype, st);
 
-  // Some tens of tokens: the block streams its weights, from activations that the norm and the pair's finish leave in blocked form.
-  if (sixteen && gamma && ((uintptr_t)x | (uintptr_t)gamma | (uintptr_t)out) % 16 == 0 && (out_dtype == PTO_HIP_FP32 || out_dtype == dtype)) {
+  // Some tens of tokens: the block streams its weights, from activations that the norm (or a copy) and the pair's finish leave in blocked form.
+  if (sixteen && ((uintptr_t)x | (uintptr_t)gamma | (uintptr_t)out) % 16 == 0 && (out_dtype == PTO_HIP_FP32 || out_dtype == dtype)) {
     const int rows = stream_rows_for(tokens, hidden, intermediate, w_gate, w_up, true, st);
-    if (rows && rms_norm_blocked_fits(tokens, hidden, rows) && stream_rows_for(tokens, intermediate, hidden, w_down, nullptr, true, st))
+    if (rows && (!gamma || rms_norm_blocked_fits(tokens, hidden, rows)) && stream_rows_for(tokens, intermediate, hidden, w_down, nullptr, true, st))
       return ffn_stream(x, gamma, w_gate, w_up, w_down, out, tokens, hidden, intermediate, eps, dtype, out_dtype, rows, st);
   }
 

@@ -64,6 +64,27 @@ def test_ffn_block_streamed_against_the_oracle(worker, tokens, hidden, inter, ou
     assert bool((buf[:512] == -77.0).all()) and bool((buf[512 + tokens * hidden:] == -77.0).all())
 
 
+@pytest.mark.parametrize("tokens,hidden,inter", [(33, 1040, 4112), (47, 264, 1032), (65, 48, 200), (96, 20488, 512)])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_ffn_without_a_norm_streamed_beside_tiled(worker, tokens, hidden, inter, dtype):
+    """The copy into the blocked layout moves values as they are (rows beyond the norm's limit too): the two routes differ by the order of
+    fp32 sums and, through it, by single roundings of h to 16 bits, of which a sum over `inter` averages most."""
+    f = workloads.ffn_inputs(tokens=tokens, hidden=hidden, intermediate=inter, dtype=dtype, with_norm=False, out_dtype=torch.float32, seed=tokens, device="cuda")
+    got = {}
+    try:
+        for stream in (0, 2):
+            worker.set_option("gemm_stream", stream)
+            f.out.fill_(float("nan"))
+            with worker.register(runtime.ffn_swiglu) as h:
+                h(f.x, f.w_gate, f.w_up, f.w_down, f.out)
+            worker.sync()
+            got[stream] = f.out.clone()
+    finally:
+        worker.set_option("gemm_stream", 1)
+    unit = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11
+    assert bool(got[2].isfinite().all()) and _error(got[2], got[0]) < unit
+
+
 def test_replays_of_a_captured_block(worker):
     """Recorded after one eager call; every replay, between eager calls that use the same scratch, gives its result."""
     small = workloads.ffn_inputs(tokens=40, hidden=4096, intermediate=11008, seed=1, device="cuda")
