@@ -600,6 +600,7 @@ PTO_HIP_API int pto_hip_backend_handler_query(const char* hook, int32_t arg, cha
  *                               themselves, where that is faster than a launch in front (same bits): 1 = the
  *                               input RMSNorm, 2 = SwiGLU of the pair in front, 4 = the merge of the attention
  *                               partials (a sum of these; default 7, 0 = never)
+ *  "skinny_fused"               read only: which of these the last decoder layer or FFN block (pto_hip_ffn_swiglu) took
  *  "w8a16_gemm_rows"            rows from which the int8 projections run as one tiled GEMM (codes
  *                               widened inside the kernel, weights read once) instead of 32-row
  *                               passes (default 33; 0 = never)

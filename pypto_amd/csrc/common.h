@@ -74,6 +74,7 @@ struct Context {
   int64_t w8a16_wgs_per_cu = 1;  // most workgroups of the skinny projection kernel per compute unit
   int64_t w8a16_wide = 1;        // int8 codes read 16 per lane: 0 never, 1 for large matrices, 2 whenever shapes allow
   int64_t skinny_fuse = 7;         // skinny projections of up to four rows make their activations themselves: 1 norm, 2 SwiGLU, 4 merge
+  int64_t skinny_fused = 0;        // read only: the sources that the last layer or FFN block took (bits as in skinny_fuse)
   int64_t w8a16_min_steps = 2;   // fewest 32-row steps per wavefront before k is split further
   int64_t gemm_stream = 1;         // projections of 33 to 96 rows that stream their weights: 0 never, 1 where measured ahead, 2 whenever shapes allow
   int64_t attn_order = -1;         // sequences by length: -1 where measured faster, 0 never, 1 always (partition grid and workgroup form)

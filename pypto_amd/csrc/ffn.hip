@@ -253,6 +253,7 @@ extern "C" int pto_hip_ffn_swiglu(const void* x, const float* gamma, const void*
   PTO_CHECK_ARG(tokens < (1 << 30) && hidden < (1 << 30) && intermediate < (1 << 30), "ffn: shape too large");
   if (tokens == 0) return PTO_HIP_OK;
   PTO_CHECK_ARG(x && w_gate && w_up && w_down && out, "ffn: null tensor pointer");
+  ctx().skinny_fused = 0;
   hipStream_t st = (hipStream_t)stream;
   const int eb = dtype_bytes(dtype);
   PTO_CHECK_ARG(dtype == PTO_HIP_BF16 || dtype == PTO_HIP_FP16 || dtype == PTO_HIP_FP32,

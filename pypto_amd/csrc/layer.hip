@@ -140,6 +140,7 @@ extern "C" int pto_hip_decoder_layer_decode(const PtoHipDecoderLayerArgs* a, voi
                 inter = a->intermediate;
   PTO_CHECK_ARG(b >= 0 && b < (1 << 20), "decoder_layer_decode: batch %lld out of range", (long long)b);
   if (b == 0) return PTO_HIP_OK;
+  cx.skinny_fused = 0;
   PTO_CHECK_ARG(h > 0 && hq > 0 && hkv > 0 && d > 0 && inter > 0 && hq % hkv == 0,
                 "decoder_layer_decode: bad model dimensions");
   PTO_CHECK_ARG(a->dtype == PTO_HIP_BF16 || a->dtype == PTO_HIP_FP16,

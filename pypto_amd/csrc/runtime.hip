@@ -1178,6 +1178,7 @@ int pto_hip_get_option(const char* name, int64_t* value) {
   else if (!std::strcmp(name, "w8a16_wgs_per_cu")) *value = c.w8a16_wgs_per_cu;
   else if (!std::strcmp(name, "w8a16_min_steps")) *value = c.w8a16_min_steps;
   else if (!std::strcmp(name, "skinny_fuse")) *value = c.skinny_fuse;
+  else if (!std::strcmp(name, "skinny_fused")) *value = c.skinny_fused;
   else if (!std::strcmp(name, "w8a16_wide")) *value = c.w8a16_wide;
   else if (!std::strcmp(name, "w8a16_gemm_rows")) *value = c.w8a16_gemm_rows;
   else return fail(PTO_HIP_ERR_NOT_FOUND, "unknown option '%s'", name);

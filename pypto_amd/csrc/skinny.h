@@ -546,7 +546,11 @@ struct MergeActivations {
 #pragma unroll
     for (int k = 0; k < D / 64; ++k) {
       const int kk = head * D + k * 64 + lane;
-      if (kk >= k_lo && kk < k_hi) reinterpret_cast<T*>(xs)[m * pitch + kk - k_lo] = (T)(o[k] * inv);
+      // Rounded to fp32 first, as the merge launch writes it: left to itself the compiler makes product and cast one v_fma_mixlo_f16, which
+      // rounds once, and a call then differed from the measured ones of its signature, which merge in a launch.
+      float y = o[k] * inv;
+      asm("" : "+v"(y));
+      if (kk >= k_lo && kk < k_hi) reinterpret_cast<T*>(xs)[m * pitch + kk - k_lo] = (T)y;
     }
   }
   static __device__ __forceinline__ float read(float v, int lane) {

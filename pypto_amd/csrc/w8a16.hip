@@ -303,6 +303,7 @@ int w8a16_partials(const void* x, bool x_blocked, const void* wq0, const void* w
   const int wgs = (int)q.wgs;
   if (src && src->kind != ProjectionSource::kTensor) {
     p.src = *src;
+    ctx().skinny_fused |= 1 << (src->kind - 1);
     const size_t smem = fused_lds(q, m);
     rc = src->kind == ProjectionSource::kNorm     ? skinny_norm_launch(p, bf, w16, q.wide, wgs, smem, st)
          : src->kind == ProjectionSource::kSwiglu ? skinny_swiglu_launch(p, bf, w16, q.wide, wgs, smem, st)

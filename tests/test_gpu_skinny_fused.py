@@ -9,7 +9,7 @@ pytestmark = pytest.mark.gpu
 
 
 def _run(worker, program, args, outputs, fuse):
-    """The outputs of one call, its caches put back afterwards."""
+    """The outputs of one call and the sources its projections took, its caches put back afterwards."""
     before = [t.clone() for t in outputs]
     worker.set_option("skinny_fuse", fuse)
     try:
@@ -19,12 +19,13 @@ def _run(worker, program, args, outputs, fuse):
                     t.copy_(b)
                 h(*args)
         worker.sync()
+        took = worker.get_option("skinny_fused")
     finally:
         worker.set_option("skinny_fuse", 7)
     got = [t.clone() for t in outputs]
     for t, b in zip(outputs, before):
         t.copy_(b)
-    return got
+    return got, took
 
 
 def _same(a, b):
@@ -32,15 +33,17 @@ def _same(a, b):
 
 
 # hidden with a half last step and without, shares of one and several pieces; head_dim 128 and 256; one partition, up to 8, up
-# to 40 and more (which keeps its merge launch); an empty sequence beside long ones; 8 and 16 codes a lane
-@pytest.mark.parametrize("batch,hidden,heads,kv_heads,head_dim,inter,block,lens,int8,e4m3,wide", [
-    (1, 4096, 32, 8, 128, 14336, 128, [2049], True, False, 1), (2, 1040, 8, 2, 128, 2064, 64, [1, 700], True, False, 1),
-    (4, 1040, 8, 1, 128, 2064, 64, [0, 33, 1300, 2500], False, False, 1), (3, 512, 4, 4, 256, 1040, 128, [400, 0, 3000], False, False, 1),
-    (1, 2048, 8, 2, 256, 4096, 64, [1111], True, True, 1), (4, 2048, 16, 4, 128, 5632, 128, [600, 599, 1, 128], False, False, 1),
-    (2, 2048, 16, 4, 128, 5632, 128, [600, 5000], True, True, 2), (1, 48, 2, 1, 128, 80, 16, [17], True, False, 1),
-    (1, 8192, 64, 8, 128, 8192, 128, [900], True, False, 2)])
+# to 40 and more (which keeps its merge launch); an empty sequence beside long ones; 8 and 16 codes a lane.  The calls are not measured: a
+# measured call keeps its merge launch.  takes: the sources that the dispatch takes
+@pytest.mark.parametrize("batch,hidden,heads,kv_heads,head_dim,inter,block,lens,int8,e4m3,wide,takes", [
+    (1, 4096, 32, 8, 128, 14336, 128, [2049], True, False, 1, 5), (2, 1040, 8, 2, 128, 2064, 64, [1, 700], True, False, 1, 7),
+    (4, 1040, 8, 1, 128, 2064, 64, [0, 33, 1300, 2500], False, False, 1, 3), (3, 512, 4, 4, 256, 1040, 128, [400, 0, 3000], False, False, 1, 7),
+    (1, 2048, 8, 2, 256, 4096, 64, [1111], True, True, 1, 7), (4, 2048, 16, 4, 128, 5632, 128, [600, 599, 1, 128], False, False, 1, 3),
+    (2, 2048, 16, 4, 128, 5632, 128, [600, 5000], True, True, 2, 3), (1, 48, 2, 1, 128, 80, 16, [17], True, False, 1, 3),
+    (1, 8192, 64, 8, 128, 8192, 128, [900], True, False, 2, 3), (1, 2048, 8, 2, 256, 4096, 64, [450], False, False, 1, 7),
+    (1, 2048, 8, 2, 256, 4096, 64, [5000], True, False, 1, 3)])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
-def test_decoder_layer_has_the_bits_of_separate_launches(worker, batch, hidden, heads, kv_heads, head_dim, inter, block, lens, int8, e4m3, wide, dtype):
+def test_decoder_layer_has_the_bits_of_separate_launches(worker, batch, hidden, heads, kv_heads, head_dim, inter, block, lens, int8, e4m3, wide, takes, dtype):
     d = workloads.decoder_layer_inputs(batch=batch, hidden=hidden, num_heads=heads, kv_head_num=kv_heads, head_dim=head_dim, intermediate=inter,
                                        block_size=block, context_lens=lens, dtype=dtype, seed=hidden + batch, device="cuda", int8_weights=int8,
                                        weight_std=None)
@@ -54,25 +57,54 @@ def test_decoder_layer_has_the_bits_of_separate_launches(worker, batch, hidden, 
     else:
         program = runtime.decoder_layer_decode if int8 else runtime.decoder_layer_decode_w16
     worker.set_option("w8a16_wide", wide)
+    worker.set_option("attn_autotune", 0)
     try:
-        ref = _run(worker, program, args, outputs, 0)
-        assert bool(ref[0].isfinite().all())
+        ref, none = _run(worker, program, args, outputs, 0)
+        assert bool(ref[0].isfinite().all()) and none == 0
         for fuse in (1, 2, 4, 7):
-            assert _same(_run(worker, program, args, outputs, fuse), ref), fuse
+            got, took = _run(worker, program, args, outputs, fuse)
+            assert _same(got, ref), fuse
+            assert took == fuse & takes, fuse
     finally:
+        worker.set_option("attn_autotune", 1)
         worker.set_option("w8a16_wide", 1)
+
+
+@pytest.mark.parametrize("hidden,heads,lens,int8", [(4096, 32, [2049], True), (2048, 16, [1500, 900], False)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_measured_and_settled_calls_have_the_same_bits(worker, hidden, heads, lens, int8, dtype):
+    """The calls that measure a signature merge its partitions in a launch, the later ones inside the o projection."""
+    d = workloads.decoder_layer_inputs(batch=len(lens), hidden=hidden, num_heads=heads, kv_head_num=heads // 4, intermediate=3 * hidden, block_size=128,
+                                       context_lens=lens, dtype=dtype, seed=5, device="cuda", int8_weights=int8, weight_std=None)
+    worker.set_option("attn_autotune", 0)  # forget what earlier tests settled
+    worker.set_option("attn_autotune", 1)
+    outs, merged = [], []
+    with worker.register(runtime.decoder_layer_decode if int8 else runtime.decoder_layer_decode_w16) as h:
+        for _ in range(32):
+            h(*d.args())
+            worker.sync()
+            outs.append(d.out.clone())
+            merged.append(bool(worker.get_option("skinny_fused") & 4))
+    assert not merged[0] and merged[-1]
+    assert all(torch.equal(o, outs[0]) for o in outs)
 
 
 @pytest.mark.parametrize("tokens,hidden,inter", [(1, 4096, 11008), (2, 1040, 4112), (3, 2048, 5632), (4, 1024, 3072), (4, 8192, 2048), (1, 48, 40000),
                                                  (1, 2496, 8448), (2, 2560, 8448)])  # the pair's channels have two or three partial sums
-def test_ffn_block_has_the_bits_of_separate_launches(worker, tokens, hidden, inter):
-    f = workloads.ffn_inputs(tokens=tokens, hidden=hidden, intermediate=inter, seed=tokens, device="cuda")
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_ffn_block_has_the_bits_of_separate_launches(worker, tokens, hidden, inter, dtype):
+    f = workloads.ffn_inputs(tokens=tokens, hidden=hidden, intermediate=inter, dtype=dtype, seed=tokens, device="cuda")
     args = (f.x, f.gamma, f.w_gate, f.w_up, f.w_down, f.out, f.eps)
     worker.set_option("gemm_narrow", -1)
     try:
-        ref = _run(worker, runtime.ffn_block, args, [f.out], 0)
+        ref, none = _run(worker, runtime.ffn_block, args, [f.out], 0)
+        assert none == 0
+        seen = 0
         for fuse in (1, 2, 7):
-            assert _same(_run(worker, runtime.ffn_block, args, [f.out], fuse), ref), fuse
+            got, took = _run(worker, runtime.ffn_block, args, [f.out], fuse)
+            assert _same(got, ref), fuse
+            seen |= took
+        assert seen
     finally:
         worker.set_option("gemm_narrow", 0)
 
@@ -81,7 +113,7 @@ def test_replays_of_a_captured_layer(worker):
     """Recorded after one eager call, replayed between eager calls that use the same scratch."""
     d = workloads.decoder_layer_inputs(batch=1, hidden=2048, num_heads=16, kv_head_num=4, intermediate=5632, context_lens=[700], seed=3, device="cuda")
     big = workloads.decoder_layer_inputs(batch=8, hidden=2048, num_heads=16, kv_head_num=4, intermediate=5632, context=900, seed=4, device="cuda")
-    want = _run(worker, runtime.decoder_layer_decode, d.args(), [d.out, d.key_cache, d.value_cache], 0)
+    want = _run(worker, runtime.decoder_layer_decode, d.args(), [d.out, d.key_cache, d.value_cache], 0)[0]
     stream = torch.cuda.Stream()
     with worker.register(runtime.decoder_layer_decode) as h:
         with torch.cuda.stream(stream):
@@ -91,6 +123,7 @@ def test_replays_of_a_captured_layer(worker):
             graph.capture_begin()
             h(*d.args(), stream=stream.cuda_stream)
             graph.capture_end()
+            assert worker.get_option("skinny_fused") & 4
             for _ in range(3):
                 d.out.zero_()
                 graph.replay()
