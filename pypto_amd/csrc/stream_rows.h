@@ -68,7 +68,7 @@ __global__ __launch_bounds__(kWaves * 64) __attribute__((amdgpu_waves_per_eu(1, 
 
   // Loads never depend on a condition, so that the requests in flight are known at compile time: past its last step a
   // wavefront asks for one address over and over.  A last step that would reach past row k ends at row k; the rows it then repeats
-  // are multiplied by zeroed activations.
+  // are cleared in the activations, and in 16-bit weights too: an infinity there must not become a NaN.
   auto load = [&](Held<W8, MT>& s, int round) {
     const int step = s0 + round * kWaves + wave;
     const bool real = step < s1;
@@ -82,9 +82,16 @@ __global__ __launch_bounds__(kWaves * 64) __attribute__((amdgpu_waves_per_eu(1, 
 #pragma unroll
     for (int h = 0; h < MT; ++h) s.xa[h] = *reinterpret_cast<const u32x4*>(xbase + x_off[h]);
   };
-  auto compute = [&](const Held<W8, MT>& s, int round) {
+  auto compute = [&](Held<W8, MT>& s, int round) {
     const int step = s0 + round * kWaves + wave;
     if (step >= s1) return;  // uniform
+    if constexpr (!W8) {
+      if (step * kStep > p.k - kStep) {  // uniform
+        const uint32_t keep = p.k - kStep + kg * 8 >= step * kStep ? ~0u : 0u;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) s.w[e] &= u32x4{keep, keep, keep, keep};
+      }
+    }
     const bool k_ok = min(step * kStep, p.k - kStep) + kg * 8 >= step * kStep;
     u32x4 a[MT];
 #pragma unroll

@@ -85,6 +85,37 @@ def test_ffn_without_a_norm_streamed_beside_tiled(worker, tokens, hidden, inter,
     assert bool(got[2].isfinite().all()) and _error(got[2], got[0]) < unit
 
 
+@pytest.mark.parametrize("tokens,hidden,inter", [(33, 40, 264), (64, 1032, 48), (96, 264, 1048)])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_a_step_that_ends_inside_keeps_infinities_apart(worker, tokens, hidden, inter, dtype):
+    """The last step of a k that is no multiple of 32 repeats rows: an infinite weight among them must not become NaN.  The gate is one on
+    every channel (SiLU(8) is nearly 8, an infinite gate stays infinite), so that h is finite and positive but for its infinite channels."""
+    x = torch.ones(tokens, hidden, dtype=dtype, device="cuda")
+    wg = torch.full((hidden, inter), 8.0 / hidden, dtype=dtype, device="cuda")
+    wu, wd = wg.clone(), torch.full((inter, hidden), 1.0 / inter, dtype=dtype, device="cuda")
+    out = torch.zeros(tokens, hidden, dtype=torch.float32, device="cuda")
+
+    def call(wu, wd):
+        out.fill_(float("nan"))
+        h(x, wg, wu, wd, out)
+        worker.sync()
+        return out.clone()
+
+    worker.set_option("gemm_stream", 2)
+    try:
+        with worker.register(runtime.ffn_swiglu) as h:
+            assert bool(call(wu, wd).isfinite().all())
+            wd_inf = wd.clone()
+            wd_inf[-32, 0] = wd_inf[-1, -1] = float("inf")
+            got = call(wu, wd_inf)
+            assert bool((got[:, 0] == float("inf")).all()) and bool((got[:, -1] == float("inf")).all()) and bool(got[:, 1:-1].isfinite().all())
+            wu_inf = wu.clone()
+            wu_inf[-32, 3] = float("inf")
+            assert bool((call(wu_inf, wd) == float("inf")).all())
+    finally:
+        worker.set_option("gemm_stream", 1)
+
+
 def test_replays_of_a_captured_block(worker):
     """Recorded after one eager call; every replay, between eager calls that use the same scratch, gives its result."""
     small = workloads.ffn_inputs(tokens=40, hidden=4096, intermediate=11008, seed=1, device="cuda")
