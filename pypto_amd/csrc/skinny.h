@@ -86,8 +86,15 @@ struct Stage {
 };
 
 // acc += activations x one stage of weights: 8 k rows of kCols channels a lane, transposed in registers into MFMA operands.
+// keep false: rows that a last step repeats, zero in both operands - an infinite 16-bit weight there must not become a NaN.  They
+// are cleared by the transposing v_perm_b32 itself (selector 12 gives a zero byte): behind a branch of their own in the last step layers of one
+// to four rows were 0.2 us slower, and the 32-row form took 280 registers instead of 256.
 template <bool BF16, bool W8, int kCols, int MT, typename W>
-__device__ __forceinline__ void multiply(const W (&w)[8], const u32x4 (&a)[MT], f32x4 (&acc)[kCols][MT]) {
+__device__ __forceinline__ void multiply(const W (&w)[8], const u32x4 (&x)[MT], bool keep, f32x4 (&acc)[kCols][MT]) {
+  const uint32_t even = keep ? 0x05040100u : 0x0c0c0c0cu, odd = keep ? 0x07060302u : 0x0c0c0c0cu;
+  u32x4 a[MT];
+#pragma unroll
+  for (int h = 0; h < MT; ++h) a[h] = keep ? x[h] : u32x4{0u, 0u, 0u, 0u};
 #pragma unroll
   for (int i = 0; i < kCols; ++i) {
     // channel n0 + i: its 8 k-values, as packed pairs (k, k+1)
@@ -103,7 +110,7 @@ __device__ __forceinline__ void multiply(const W (&w)[8], const u32x4 (&a)[MT], 
       }
     } else {
       // 16-bit weights: element i of rows 2q and 2q+1 (an 8x8 transpose in registers)
-      const uint32_t sel = (i & 1) ? 0x07060302u : 0x05040100u;
+      const uint32_t sel = (i & 1) ? odd : even;
 #pragma unroll
       for (int q = 0; q < 4; ++q) b[q] = __builtin_amdgcn_perm(w[2 * q + 1][i >> 1], w[2 * q][i >> 1], sel);
     }
@@ -208,7 +215,7 @@ __global__ __launch_bounds__(kWaves * 64) __attribute__((amdgpu_waves_per_eu(1, 
   // Loads never depend on a condition, so the number of requests in flight is known at compile
   // time: a wavefront without a step of its own in a round reads the run's last one again, and a last step
   // that would reach past row k is moved back to end at row k - the rows it then repeats are
-  // multiplied by zeroed activations.  A row address is a wavefront-uniform row base plus a
+  // cleared in the activations and in 16-bit weights.  A row address is a wavefront-uniform row base plus a
   // per-lane offset.
   constexpr int kWBytes = W8 ? 1 : 2;  // bytes per weight
   typedef typename std::conditional<(W8 && kCols == 8), u32x2, u32x4>::type wvec_t;
@@ -231,10 +238,7 @@ __global__ __launch_bounds__(kWaves * 64) __attribute__((amdgpu_waves_per_eu(1, 
     const int step = cur.step + wave;
     if (step >= cur.end) return;  // uniform: no step for this wavefront in this round
     const bool k_ok = min(step * kStep, p.k - kStep) + kg * 8 >= step * kStep;
-    u32x4 a[MT];
-#pragma unroll
-    for (int h = 0; h < MT; ++h) a[h] = k_ok ? s.xa[h] : u32x4{0u, 0u, 0u, 0u};
-    multiply<BF16, W8, kCols, MT>(s.w, a, acc);
+    multiply<BF16, W8, kCols, MT>(s.w, s.xa, k_ok, acc);
   };
 
   auto finish_run = [&](const Cursor& cur) {
@@ -599,8 +603,8 @@ __global__ __launch_bounds__(kWaves * 64) __attribute__((amdgpu_waves_per_eu(1, 
     if (step >= s1) return;  // uniform
     const int k = row_of(round) + kg * 8;
     const u32x4 act = *reinterpret_cast<const u32x4*>(xs + min(c, p.m - 1) * pitch + k - k_lo);
-    const u32x4 a[1] = {k >= step * kStep ? act : u32x4{0u, 0u, 0u, 0u}};
-    multiply<BF16, W8, kCols, 1>(w, a, acc);
+    const u32x4 a[1] = {act};
+    multiply<BF16, W8, kCols, 1>(w, a, k >= step * kStep, acc);
   };
 
   wvec_t w0[8], w1[8];

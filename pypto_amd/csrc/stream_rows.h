@@ -82,21 +82,11 @@ __global__ __launch_bounds__(kWaves * 64) __attribute__((amdgpu_waves_per_eu(1, 
 #pragma unroll
     for (int h = 0; h < MT; ++h) s.xa[h] = *reinterpret_cast<const u32x4*>(xbase + x_off[h]);
   };
-  auto compute = [&](Held<W8, MT>& s, int round) {
+  auto compute = [&](const Held<W8, MT>& s, int round) {
     const int step = s0 + round * kWaves + wave;
     if (step >= s1) return;  // uniform
-    if constexpr (!W8) {
-      if (step * kStep > p.k - kStep) {  // uniform
-        const uint32_t keep = p.k - kStep + kg * 8 >= step * kStep ? ~0u : 0u;
-#pragma unroll
-        for (int e = 0; e < 8; ++e) s.w[e] &= u32x4{keep, keep, keep, keep};
-      }
-    }
     const bool k_ok = min(step * kStep, p.k - kStep) + kg * 8 >= step * kStep;
-    u32x4 a[MT];
-#pragma unroll
-    for (int h = 0; h < MT; ++h) a[h] = k_ok ? s.xa[h] : u32x4{0u, 0u, 0u, 0u};
-    multiply<BF16, W8, kCols, MT>(s.w, a, acc);
+    multiply<BF16, W8, kCols, MT>(s.w, s.xa, k_ok, acc);
   };
   Held<W8, MT> st[NS];
 #pragma unroll

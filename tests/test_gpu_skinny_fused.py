@@ -109,6 +109,39 @@ def test_ffn_block_has_the_bits_of_separate_launches(worker, tokens, hidden, int
         worker.set_option("gemm_narrow", 0)
 
 
+@pytest.mark.parametrize("tokens", [1, 4, 7, 32])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_a_step_that_ends_inside_keeps_infinities_apart(worker, tokens, dtype):
+    """k of 48 and 1040: the last 32-row step repeats 16 rows, and an infinite weight among them must not become NaN.  With and without a norm (of
+    ones: ones), the projections' own activations and given ones; SiLU(8) is nearly 8, so that h is finite but for its infinite channels."""
+    hidden, inter = 48, 1040
+    x, gamma = torch.ones(tokens, hidden, dtype=dtype, device="cuda"), torch.ones(1, hidden, device="cuda")
+    wg = torch.full((hidden, inter), 8.0 / hidden, dtype=dtype, device="cuda")
+    wd = torch.full((inter, hidden), 1.0 / inter, dtype=dtype, device="cuda")
+    wu_inf, wd_inf = wg.clone(), wd.clone()
+    wu_inf[-32, 3] = wd_inf[-32, 0] = wd_inf[-1, -1] = float("inf")
+    out = torch.zeros(tokens, hidden, dtype=torch.float32, device="cuda")
+    worker.set_option("gemm_narrow", -1)
+    try:
+        for fuse in (0, 7):
+            worker.set_option("skinny_fuse", fuse)
+            for program, gamma_arg, eps in ((runtime.ffn_swiglu, (), ()), (runtime.ffn_block, (gamma,), (1e-6,))):
+                with worker.register(program) as h:
+                    def call(wu, wd):
+                        out.fill_(float("nan"))
+                        h(x, *gamma_arg, wg, wu, wd, out, *eps)
+                        worker.sync()
+                        return out.clone()
+
+                    assert bool(call(wg, wd).isfinite().all())
+                    got = call(wg, wd_inf)
+                    assert bool((got[:, 0] == float("inf")).all()) and bool((got[:, -1] == float("inf")).all()) and bool(got[:, 1:-1].isfinite().all())
+                    assert bool((call(wu_inf, wd) == float("inf")).all())
+    finally:
+        worker.set_option("gemm_narrow", 0)
+        worker.set_option("skinny_fuse", 7)
+
+
 def test_replays_of_a_captured_layer(worker):
     """Recorded after one eager call, replayed between eager calls that use the same scratch."""
     d = workloads.decoder_layer_inputs(batch=1, hidden=2048, num_heads=16, kv_head_num=4, intermediate=5632, context_lens=[700], seed=3, device="cuda")
