@@ -276,8 +276,10 @@ extern "C" int pto_hip_ffn_swiglu(const void* x, const float* gamma, const void*
       return ffn_stream(x, gamma, w_gate, w_up, w_down, out, tokens, hidden, intermediate, eps, dtype, out_dtype, rows, st);
   }
 
-  const size_t xn_bytes = gamma ? ((size_t)tokens * hidden * eb + 255) / 256 * 256 : 0;
-  const size_t h_bytes = (size_t)tokens * intermediate * eb;
+  // (up to 32 rows one call sizes the scratch for all of them, as the skinny form's does: it cannot grow under capture)
+  const size_t rows = sixteen ? std::max(tokens, kSkinnyMaxTokens) : tokens;
+  const size_t xn_bytes = gamma ? (rows * hidden * eb + 255) / 256 * 256 : 0;
+  const size_t h_bytes = rows * intermediate * eb;
   void* ws = nullptr;
   int rc = workspace(xn_bytes + h_bytes, &ws);
   if (rc) return rc;

@@ -10,7 +10,7 @@ import pytest
 import torch
 
 from pypto_amd import workloads
-from pypto_amd.runtime import decoder_layer_decode, ffn_block, paged_attention, projection
+from pypto_amd.runtime import decoder_layer_decode, ffn_block, ffn_swiglu, paged_attention, projection
 
 pytestmark = pytest.mark.gpu
 
@@ -119,6 +119,36 @@ def test_a_skinny_projection_sizes_its_scratch_for_every_batch(worker):
         h(x, w, out)
     worker.sync()
     assert worker.get_option("workspace_bytes") == sized
+
+
+@pytest.mark.parametrize("hidden,inter", [(512, 1024), (512, 3520), (40, 96)])  # narrow tiles; skinny projections; no k for those
+@pytest.mark.parametrize("norm", [False, True])
+def test_an_ffn_call_sizes_its_scratch_for_up_to_32_tokens(worker, hidden, inter, norm):
+    """One eager call of one token, then a capture of 32 of the same block: whichever form its products take."""
+    _without_scratch(worker)
+    f = workloads.ffn_inputs(tokens=32, hidden=hidden, intermediate=inter, with_norm=norm, seed=hidden, device="cuda")
+
+    def call(h, tokens, out, **kw):
+        h(f.x[:tokens], *((f.gamma,) if norm else ()), f.w_gate, f.w_up, f.w_down, out, *((f.eps,) if norm else ()), **kw)
+
+    got = torch.full_like(f.out, float("nan"))
+    stream = torch.cuda.Stream()
+    with worker.register(ffn_block if norm else ffn_swiglu) as h:
+        call(h, 1, f.out[:1])
+        worker.sync()
+        held = worker.get_option("workspace_bytes")
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=stream):
+            call(h, 32, got, stream=stream.cuda_stream)
+        assert worker.get_option("workspace_bytes") == held
+        call(h, 32, f.out)
+        worker.sync()
+        for _ in range(3):
+            got.fill_(float("nan"))
+            graph.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(got, f.out)
+            call(h, 1, torch.empty_like(f.out[:1]))
 
 
 def _without_scratch(worker):
