@@ -119,6 +119,7 @@ def test_a_step_that_ends_inside_keeps_infinities_apart(worker, tokens, hidden, 
 def test_replays_of_a_captured_block(worker):
     """Recorded after one eager call; every replay, between eager calls that use the same scratch, gives its result."""
     small = workloads.ffn_inputs(tokens=40, hidden=4096, intermediate=11008, seed=1, device="cuda")
+    torch.cuda.synchronize()  # the inputs are made on another stream than the call's
     with worker.register(runtime.ffn_block) as h:
         stream = torch.cuda.Stream()
         with torch.cuda.stream(stream):
