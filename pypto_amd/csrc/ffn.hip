@@ -168,14 +168,17 @@ int ffn_skinny(const void* x, const float* gamma, const void* w_gate, const void
   return PTO_HIP_OK;
 }
 
+// Scratch of ffn_stream: whole groups of 16 rows of the activations and of h.
+size_t stream_xn_bytes(int rows, int64_t hidden) { return ((size_t)rows * hidden * 2 + 255) / 256 * 256; }
+size_t stream_bytes(int rows, int64_t hidden, int64_t intermediate) { return stream_xn_bytes(rows, hidden) + (size_t)rows * intermediate * 2; }
+
 int ffn_stream(const void* x, const float* gamma, const void* w_gate, const void* w_up, const void* w_down, void* out, int64_t tokens,
                int64_t hidden, int64_t intermediate, float eps, int dtype, int out_dtype, int rows, hipStream_t st) {
   using namespace pto_hip;
-  const size_t xn_bytes = ((size_t)rows * hidden * 2 + 255) / 256 * 256;
   void* ws = nullptr;
-  int rc = workspace(xn_bytes + (size_t)rows * intermediate * 2, &ws);
+  int rc = workspace(stream_bytes(rows, hidden, intermediate), &ws);
   if (rc) return rc;
-  void* h = reinterpret_cast<char*>(ws) + xn_bytes;
+  void* h = reinterpret_cast<char*>(ws) + stream_xn_bytes(rows, hidden);
   rc = gamma ? rms_norm_blocked(x, gamma, ws, tokens, hidden, eps, dtype, st, rows) : rows_blocked(x, ws, tokens, hidden, st, rows);
   if (rc) return rc;
   W8Partials parts{};
@@ -270,9 +273,10 @@ extern "C" int pto_hip_ffn_swiglu(const void* x, const float* gamma, const void*
     return ffn_skinny(x, gamma, w_gate, w_up, w_down, out, tokens, hidden, intermediate, eps, dtype, out_dtype, st);
 
   // Some tens of tokens: the block streams its weights, from activations that the norm (or a copy) and the pair's finish leave in blocked form.
+  // (not where that would have to grow the scratch under capture: the tiled GEMM needs less)
   if (sixteen && ((uintptr_t)x | (uintptr_t)gamma | (uintptr_t)out) % 16 == 0 && (out_dtype == PTO_HIP_FP32 || out_dtype == dtype)) {
     const int rows = stream_rows_for(tokens, hidden, intermediate, w_gate, w_up, true, st);
-    if (rows && (!gamma || rms_norm_blocked_fits(tokens, hidden, rows)) && stream_rows_for(tokens, intermediate, hidden, w_down, nullptr, true, st))
+    if (rows && (stream_bytes(rows, hidden, intermediate) <= ctx().workspace_bytes || !stream_capturing(st)) && (!gamma || rms_norm_blocked_fits(tokens, hidden, rows)) && stream_rows_for(tokens, intermediate, hidden, w_down, nullptr, true, st))
       return ffn_stream(x, gamma, w_gate, w_up, w_down, out, tokens, hidden, intermediate, eps, dtype, out_dtype, rows, st);
   }
 

@@ -40,18 +40,25 @@ int layer_large_batch(const PtoHipDecoderLayerArgs* a, int rope_w, void* stream)
   const bool vec = ((uintptr_t)a->hidden_states | (uintptr_t)a->gamma_in | (uintptr_t)a->gamma_post) % 16 == 0;
   hipStream_t st = (hipStream_t)stream;
   // Rows of the blocked layout of the activations in front of a projection that streams its weights; 0: rows, and the tiled GEMM.
-  const int qkv_rows = vec ? stream_rows_for(b, h, qkv_n, a->wqkv_q, nullptr, w16, st) : 0;
-  const int o_rows = stream_rows_for(b, hq * d, h, a->wo_q, nullptr, w16, st);
-  const int gu_rows = stream_rows_for(b, h, inter, a->wg_q, a->wu_q, w16, st);
-  const int down_rows = gu_rows ? stream_rows_for(b, inter, h, a->wd_q, nullptr, w16, st) : 0;
+  int qkv_rows = vec ? stream_rows_for(b, h, qkv_n, a->wqkv_q, nullptr, w16, st) : 0;
+  int o_rows = stream_rows_for(b, hq * d, h, a->wo_q, nullptr, w16, st);
+  int gu_rows = stream_rows_for(b, h, inter, a->wg_q, a->wu_q, w16, st);
+  int down_rows = gu_rows ? stream_rows_for(b, inter, h, a->wd_q, nullptr, w16, st) : 0;
   const bool fused_norm = w8a16_finish_norm_fits(h);
-  const size_t rows16 = std::max<int64_t>(b, std::max(std::max(qkv_rows, o_rows), std::max(gu_rows, down_rows)));
-  const size_t sz_normed = up(rows16 * h * 2), sz_qkv = up((size_t)b * std::max(qkv_n, h) * 4),  // also holds an unsplit o_proj product
-               sz_q = up((size_t)b * hq * d * 2), sz_attn = up((size_t)b * hq * d * 4),
-               sz_attn16 = up(rows16 * hq * d * 2), sz_resid = up((size_t)b * h * 4),
-               sz_h = up(rows16 * inter * 2);
+  const size_t sz_qkv = up((size_t)b * std::max(qkv_n, h) * 4),  // also holds an unsplit o_proj product
+               sz_q = up((size_t)b * hq * d * 2), sz_attn = up((size_t)b * hq * d * 4), sz_resid = up((size_t)b * h * 4);
+  size_t sz_normed = 0, sz_attn16 = 0, sz_h = 0;
+  auto total = [&] {
+    const size_t rows16 = std::max<int64_t>(b, std::max(std::max(qkv_rows, o_rows), std::max(gu_rows, down_rows)));
+    sz_normed = up(rows16 * h * 2);
+    sz_attn16 = up(rows16 * hq * d * 2);
+    sz_h = up(rows16 * inter * 2);
+    return sz_normed + sz_qkv + sz_q + sz_attn + sz_attn16 + sz_resid + sz_normed + sz_h;
+  };
+  // The blocked layout's whole groups of 16 rows take more room, which cannot be made under capture.
+  if (total() > ctx().layer_ws_bytes && stream_capturing(st)) qkv_rows = o_rows = gu_rows = down_rows = 0;
   void* lws = nullptr;
-  int rc = layer_workspace(sz_normed + sz_qkv + sz_q + sz_attn + sz_attn16 + sz_resid + sz_normed + sz_h, &lws);
+  int rc = layer_workspace(total(), &lws);
   if (rc) return rc;
   char* w = reinterpret_cast<char*>(lws);
   void* normed = w;              w += sz_normed;
