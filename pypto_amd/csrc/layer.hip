@@ -41,10 +41,13 @@ int layer_large_batch(const PtoHipDecoderLayerArgs* a, int rope_w, void* stream)
   hipStream_t st = (hipStream_t)stream;
   // Rows of the blocked layout of the activations in front of a projection that streams its weights; 0: rows, and the tiled GEMM.
   int qkv_rows = vec ? stream_rows_for(b, h, qkv_n, a->wqkv_q, nullptr, w16, st) : 0;
-  int o_rows = stream_rows_for(b, hq * d, h, a->wo_q, nullptr, w16, st);
-  int gu_rows = stream_rows_for(b, h, inter, a->wg_q, a->wu_q, w16, st);
-  int down_rows = gu_rows ? stream_rows_for(b, inter, h, a->wd_q, nullptr, w16, st) : 0;
+  // (misaligned scales, residuals and results stay with the entry points of the tiled form, which refuse them)
   const bool fused_norm = w8a16_finish_norm_fits(h);
+  const bool o_vec = fused_norm || ((uintptr_t)a->wo_s | (uintptr_t)a->hidden_states) % 16 == 0;
+  const bool gu_vec = ((uintptr_t)a->wg_s | (uintptr_t)a->wu_s) % 16 == 0, down_vec = ((uintptr_t)a->wd_s | (uintptr_t)a->out) % 16 == 0;
+  int o_rows = o_vec ? stream_rows_for(b, hq * d, h, a->wo_q, nullptr, w16, st) : 0;
+  int gu_rows = gu_vec ? stream_rows_for(b, h, inter, a->wg_q, a->wu_q, w16, st) : 0;
+  int down_rows = gu_rows && down_vec ? stream_rows_for(b, inter, h, a->wd_q, nullptr, w16, st) : 0;
   const size_t sz_qkv = up((size_t)b * std::max(qkv_n, h) * 4),  // also holds an unsplit o_proj product
                sz_q = up((size_t)b * hq * d * 2), sz_attn = up((size_t)b * hq * d * 4), sz_resid = up((size_t)b * h * 4);
   size_t sz_normed = 0, sz_attn16 = 0, sz_h = 0;

@@ -1,10 +1,12 @@
 """Projections of 33 to 96 rows that stream their weights (stream_rows.h), inside decoder layers and FFN blocks."""
 
+import ctypes as C
+
 import pytest
 import torch
 
 import oracle
-from pypto_amd import runtime, workloads
+from pypto_amd import _lib, runtime, workloads
 
 pytestmark = pytest.mark.gpu
 
@@ -137,3 +139,44 @@ def test_replays_of_a_captured_block(worker):
                 assert torch.equal(small.out, want)
                 h(small.x, small.gamma, small.w_gate, small.w_up, small.w_down, torch.empty_like(small.out), small.eps, stream=stream.cuda_stream)
                 stream.synchronize()
+
+
+class _LayerArgs(C.Structure):
+    """PtoHipDecoderLayerArgs (programs refuse misaligned tensors by themselves, callers of the C interface do not)."""
+
+    POINTERS = ("hidden_states seq_lens block_table key_cache value_cache rope_cos rope_sin gamma_in gamma_post wqkv_q wqkv_s wo_q wo_s wg_q wg_s "
+                "wu_q wu_s wd_q wd_s out").split()
+    SIZES = "batch hidden num_heads kv_head_num head_dim intermediate block_size max_num_blocks_per_req max_pos pool_rows".split()
+    _fields_ = ([(n, C.c_void_p) for n in POINTERS] + [(n, C.c_int64) for n in SIZES] + [("eps", C.c_float)] +
+                [(n, C.c_int32) for n in ("dtype", "kv_dtype", "rope_table_width")] + [("k_scale", C.c_void_p), ("v_scale", C.c_void_p)])
+
+
+# the o projection with its finish and norm in one kernel (whose scale may start anywhere), and apart
+@pytest.mark.parametrize("hidden,name", [(512, "wg_s"), (512, "wu_s"), (512, "wd_s"), (512, "out"), (8208, "wo_s"), (8208, "hidden_states")])
+def test_a_streamed_layer_refuses_what_the_tiled_one_refuses(worker, hidden, name):
+    """An operand that starts four bytes off a 16-byte boundary: the same refusal in both forms, and none where all are aligned."""
+    d = workloads.decoder_layer_inputs(batch=40, hidden=hidden, num_heads=2, kv_head_num=1, intermediate=1040, block_size=64, context=50, seed=1,
+                                       device="cuda", int8_weights=True, weight_std=None)
+    tensors = dict(zip(_LayerArgs.POINTERS, d.args()))
+    t = tensors[name]
+    moved = torch.cat([t.flatten()[:4 // t.element_size()], t.flatten()])[4 // t.element_size():]
+    assert moved.data_ptr() % 16 == 4
+    lib, said = _lib.load(), []
+
+    def call(**kw):
+        a = _LayerArgs(**{n: t.data_ptr() for n, t in {**tensors, **kw}.items()}, batch=40, hidden=hidden, num_heads=2, kv_head_num=1, head_dim=128,
+                       intermediate=1040, block_size=64, max_num_blocks_per_req=d.block_table.numel() // 40, max_pos=d.rope_cos.shape[0],
+                       pool_rows=d.key_cache.shape[0], eps=d.eps, dtype=runtime._dtype_code(torch.bfloat16))
+        _lib.check(lib.pto_hip_decoder_layer_decode(C.byref(a), None))
+
+    try:
+        for stream in (0, 2):
+            worker.set_option("gemm_stream", stream)
+            call()
+            with pytest.raises(ValueError, match="misaligned") as refused:
+                call(**{name: moved})
+            worker.sync()
+            said.append(str(refused.value))
+    finally:
+        worker.set_option("gemm_stream", 1)
+    assert said[0] == said[1]
