@@ -46,11 +46,19 @@ bool narrow_not_skinny(int64_t k, int64_t n, bool dual) {
          pto_hip::narrow_beats_skinny(k, n, dual);
 }
 
+// A result [m, n] laid over the operand x [m, k] it is made from.  In the small-call form one workgroup would write what another has still to read; the
+// skinny form writes behind a launch that has read everything.
+bool in_place(const void* x, const void* out, int64_t m, int64_t k, int64_t n, int out_dtype) {
+  const uintptr_t x0 = (uintptr_t)x, x1 = x0 + (uintptr_t)m * k * 2, c0 = (uintptr_t)out, c1 = c0 + (uintptr_t)m * n * pto_hip::dtype_bytes(out_dtype);
+  return c0 < x1 && x0 < c1;
+}
+
 // Tile of the small-call form for a product with 16-bit weights, 0 for the tiled GEMM.  A forced tile form, height or split
 // count asks for the tiled GEMM.  Whoever sums the slabs of partials_out spares that product its finish launch.
-int narrow_tile(const GemmParams& p, bool dual) {
+int narrow_tile(const GemmParams& p, bool dual, int out_dtype) {
   const pto_hip::Context& cx = pto_hip::ctx();
   if (cx.gemm_variant != 0 || cx.gemm_splits != 0 || cx.gemm_quad_rows != 0 || cx.gemm_narrow < 0 || p.k < kNarrowMinK) return 0;
+  if (in_place(p.a, p.c, p.m, p.k, p.n, out_dtype)) return 0;
   if (cx.gemm_narrow > 0) return (int)cx.gemm_narrow;
   int height = 0, splits = 1;
   double us = pto_hip::choose_quad(p.m, p.n, p.k, dual, cx.num_cu, 0, &height, &splits);
@@ -62,7 +70,7 @@ int narrow_tile(const GemmParams& p, bool dual) {
 template <bool DUAL>
 int launch_typed(const GemmParams& p, int dtype, int out_dtype, hipStream_t st) {
   const bool built = dtype == out_dtype || (!DUAL && out_dtype == PTO_HIP_FP32);
-  if (const int tile = !p.scale0 && built ? narrow_tile(p, DUAL) : 0) {
+  if (const int tile = !p.scale0 && built ? narrow_tile(p, DUAL, out_dtype) : 0) {
     if (p.partials_out) *p.partials_out = pto_hip::finished_slab(reinterpret_cast<const float*>(p.c));
     if (DUAL) return dtype == PTO_HIP_BF16 ? pto_hip::narrow_dual_bf16(p, tile, st) : pto_hip::narrow_dual_fp16(p, tile, st);
     return dtype == PTO_HIP_BF16 ? pto_hip::narrow_single_bf16(p, tile, out_dtype, st)
@@ -426,7 +434,7 @@ extern "C" int pto_hip_projection(const void* x, const void* w, const void* resi
   PTO_CHECK_ARG(((uintptr_t)x | (uintptr_t)w | (uintptr_t)out | (uintptr_t)residual) % 16 == 0,
                 "projection: operand pointers must be 16-byte aligned");
   hipStream_t st = (hipStream_t)stream;
-  if (m <= kSkinnyMaxTokens && ctx().gemm_variant == 0 && k % 16 == 0 && k >= 32 && !narrow_not_skinny(k, n, false)) {
+  if (m <= kSkinnyMaxTokens && ctx().gemm_variant == 0 && k % 16 == 0 && k >= 32 && (in_place(x, out, m, k, n, out_dtype) || !narrow_not_skinny(k, n, false))) {
     W8Partials parts{};
     int rc = w8a16_partials(x, false, w, nullptr, m, k, n, dtype, st, &parts, true);
     if (rc) return rc;
@@ -467,7 +475,7 @@ extern "C" int pto_hip_gate_up_swiglu(const void* x, const void* w_gate, const v
   PTO_CHECK_ARG(((uintptr_t)x | (uintptr_t)w_gate | (uintptr_t)w_up | (uintptr_t)out) % 16 == 0,
                 "gate_up_swiglu: operand pointers must be 16-byte aligned");
   hipStream_t st = (hipStream_t)stream;
-  if (m <= kSkinnyMaxTokens && ctx().gemm_variant == 0 && k % 16 == 0 && k >= 32 && !narrow_not_skinny(k, n, true)) {
+  if (m <= kSkinnyMaxTokens && ctx().gemm_variant == 0 && k % 16 == 0 && k >= 32 && (in_place(x, out, m, k, n, dtype) || !narrow_not_skinny(k, n, true))) {
     W8Partials parts{};
     int rc = w8a16_partials(x, false, w_gate, w_up, m, k, n, dtype, st, &parts, true);
     if (rc) return rc;

@@ -88,3 +88,27 @@ def test_small_block_against_the_tiled_and_skinny_forms(worker, tokens):
     finally:
         worker.set_option("gemm_narrow", 0)
     assert ((got[0] - got[1]).norm() / got[1].norm()).item() < 2.0 ** -9
+
+
+@pytest.mark.parametrize("k,n", [(512, 512), (1024, 256)])
+@pytest.mark.parametrize("m", [1, 17, 32])
+@pytest.mark.parametrize("program", [projection, gate_up_swiglu])
+def test_a_result_laid_over_its_operand(worker, m, k, n, program):
+    """Up to 32 rows a result may lie where the activations do: the small-call form would write them while other workgroups still read, so
+    such a call takes the form with a finish of its own, and has its bits."""
+    g = torch.Generator(device="cuda").manual_seed(m + n)
+    x = (torch.randn((m, k), generator=g, device="cuda") / k ** 0.5).to(torch.bfloat16)
+    w = tuple(torch.randn((k, n), generator=g, device="cuda").to(torch.bfloat16) for _ in range(1 if program is projection else 2))
+    with worker.register(program) as h:
+        want = torch.zeros((m, n), dtype=torch.bfloat16, device="cuda")
+        worker.set_option("gemm_narrow", -1)
+        try:
+            h(x, *w, want)
+        finally:
+            worker.set_option("gemm_narrow", 0)
+        for _ in range(8):
+            buf = x.clone()
+            over = buf.flatten()[:m * n].view(m, n)
+            h(buf, *w, over)
+            worker.sync()
+            assert torch.equal(over, want)
