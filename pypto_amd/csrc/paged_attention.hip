@@ -1617,7 +1617,7 @@ void attention_tuning_last(int64_t* cap, int64_t* wg, int64_t* ordered) {
   *cap = *wg = *ordered = -1;
   if (!g_last_tuned) return;
   tune_harvest(*g_last_tuned);  // readings that have arrived since the last launch
-  if (g_last_tuned->chosen < 0) return;
+  if (g_last_tuned->settled < g_last_tuned->cands.size()) return;  // a round is not over: what it started from may not stay
   *cap = g_last_tuned->cands[g_last_tuned->chosen].cap;
   *wg = g_last_tuned->cands[g_last_tuned->chosen].wg ? 1 : 0;
   *ordered = g_last_tuned->cands[g_last_tuned->chosen].ordered ? 1 : 0;

@@ -40,3 +40,27 @@ def test_by_length_or_as_they_come(worker, batch, heads, kv_heads, head_dim, blo
         worker.set_option("attn_order", -1)
     assert bool(got[0].isfinite().all())
     assert torch.equal(got[0], got[1]) and torch.equal(got[0], got[2])
+
+
+@pytest.mark.parametrize("e4m3", [False, True])
+def test_the_choice_reads_as_settled_only_once_it_stays(worker, e4m3):
+    """Four or five shapes are measured four times each, then two or three by length: -1 until all of it is over, and no change afterwards."""
+    lens = [random.Random(i).randint(200, 3000) for i in range(64)]
+    a = workloads.paged_attention_inputs(batch=64, num_heads=32, kv_head_num=8, head_dim=128, block_size=64, ctx_range=(1, 3000), context_lens=lens,
+                                         fp8_kv=e4m3, seed=5, device="cuda")
+    worker.set_option("attn_autotune", 0)  # forget what earlier tests settled
+    worker.set_option("attn_autotune", 1)
+    names = ("attn_tuned_waves_per_cu", "attn_tuned_workgroup_form", "attn_tuned_order")
+    said, outs = [], []
+    with worker.register(paged_attention) as h:
+        for _ in range(80):
+            a.out.fill_(float("nan"))
+            h(*a.args())
+            worker.sync()
+            said.append(tuple(worker.get_option(n) for n in names))
+            outs.append(a.out.clone())
+    measured = said.count((-1, -1, -1))
+    assert (4 + 2) * 4 - 1 <= measured <= (5 + 3) * 4
+    assert said[measured] == said[-1] and all(v >= 0 for v in said[-1])
+    assert all(s == said[0] for s in said[:measured]) and all(s == said[-1] for s in said[measured:])
+    assert all(torch.equal(o, outs[0]) for o in outs)
