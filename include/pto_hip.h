@@ -580,13 +580,15 @@ PTO_HIP_API int pto_hip_backend_handler_query(const char* hook, int32_t arg, cha
  *                               0 = by estimate (256 under variant 7, default), 64, 128, 192, 256
  *  "gemm_narrow"                products with 16-bit weights in tiles of 16 to 64 rows x 32 or 64 channels, one launch
  *                               each: 0 = where estimated faster than the tiled GEMM, and up to 32 rows for at most
- *                               1.6 million weights (default), -1 = never, 1..4 = always, with that tile
+ *                               1.6 million weights (default), -1 = never, 1..4 = always, with that tile, but for
+ *                               decoder layers of up to 32 sequences and results laid over their activations
  *                               ("gemm_variant", "gemm_quad_rows" or "gemm_splits" other than 0 switch it off).
- *                               e4m3 products likewise, tiles of 16 x 16, 32 x 32 and 64 x 32 (4 counts as 3)
+ *                               e4m3 products likewise, tiles of 16 x 16, 32 x 32 and 64 x 32 (4 counts as 3),
+ *                               switched off by "gemm_variant" and "gemm_splits"
  *  "gemm_stream"                projections of 33 to 96 rows inside a decoder layer or an FFN block that
  *                               stream their weights into registers: 1 = where measured ahead of the tiled GEMM
  *                               (default), 0 = never, 2 = whenever shapes allow ("gemm_variant", "gemm_quad_rows"
- *                               or "gemm_splits" other than 0 switch it off)
+ *                               or "gemm_splits" other than 0 switch it off, and 16-bit weights a "gemm_narrow" of 1..4)
  *  "gemm_splits"                k splits of the tiled GEMMs: 0 = by shape (default), 1..16 = as given
  *                               when k allows (16-bit and int8 weights: each split at least four 64-row
  *                               k tiles; e4m3: at least one tile of 128 codes), under every "gemm_variant"

@@ -43,7 +43,7 @@ constexpr int kNarrowMinK = 32;
 // Products of up to kSkinnyMaxTokens rows that take the small-call form instead of the skinny one (every k of a block's at least 32).
 bool narrow_not_skinny(int64_t k, int64_t n, bool dual) {
   return pto_hip::ctx().gemm_narrow >= 0 && pto_hip::ctx().gemm_splits == 0 && pto_hip::ctx().gemm_quad_rows == 0 && k >= kNarrowMinK &&
-         pto_hip::narrow_beats_skinny(k, n, dual);
+         (pto_hip::ctx().gemm_narrow > 0 || pto_hip::narrow_beats_skinny(k, n, dual));
 }
 
 // A result [m, n] laid over the operand x [m, k] it is made from.  In the small-call form one workgroup would write what another has still to read; the

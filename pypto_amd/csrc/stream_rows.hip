@@ -18,6 +18,7 @@ int stream_splits(int64_t k, int64_t n, int mats) {
 int stream_rows_for(int64_t m, int64_t k, int64_t n, const void* wq0, const void* wq1, bool w16, hipStream_t st) {
   const int mats = wq1 ? 2 : 1;
   if (ctx().gemm_stream == 0 || ctx().gemm_variant != 0 || ctx().gemm_splits != 0 || ctx().gemm_quad_rows != 0) return 0;
+  if (w16 && ctx().gemm_narrow > 0) return 0;  // a tile of the small-call form is asked for
   if (k % 8 != 0 || k < 32 || n % 8 != 0 || (n + 127) / 128 * mats > ctx().num_cu || ((uintptr_t)wq0 | (uintptr_t)wq1) % 16 != 0) return 0;
   if (m <= kW8MaxM || m > kStreamRowsMax || (ctx().gemm_stream == 1 && !stream_rows_ahead(m, k, n, mats == 2, w16))) return 0;
   void* area = nullptr;

@@ -112,3 +112,28 @@ def test_a_result_laid_over_its_operand(worker, m, k, n, program):
             h(buf, *w, over)
             worker.sync()
             assert torch.equal(over, want)
+
+
+@pytest.mark.parametrize("program,m,more,k,n", [(projection, 8, 40, 2048, 1024), (gate_up_swiglu, 8, 40, 1024, 1024), (ffn_block, 8, 100, 1024, 1024),
+                                                (ffn_block, 40, 100, 4096, 11008)])
+def test_a_tile_asked_for_is_taken_whatever_the_rows(worker, program, m, more, k, n):
+    """Shapes that the skinny form (up to 32 rows) and the streams (33 to 96) have by default: with a tile forced, a row has the bits that it has
+    in a call of more rows, which only the small-call form gives."""
+    from pypto_amd import workloads
+    f = workloads.ffn_inputs(tokens=more, hidden=k, intermediate=n, out_dtype=torch.float32, seed=m, device="cuda")
+    weights = {projection: (f.w_gate,), gate_up_swiglu: (f.w_gate, f.w_up), ffn_block: (f.w_gate, f.w_up, f.w_down)}[program]
+    width, out_dtype = (k if program is ffn_block else n), torch.bfloat16 if program is gate_up_swiglu else torch.float32
+    got = {}
+    try:
+        for tile in (0, 3):
+            worker.set_option("gemm_narrow", tile)
+            for rows in (m, more):
+                out = torch.full((rows, width), float("nan"), dtype=out_dtype, device="cuda")
+                with worker.register(program) as h:
+                    h(*((f.x[:rows], f.gamma) if program is ffn_block else (f.x[:rows],)), *weights, out, *((f.eps,) if program is ffn_block else ()))
+                worker.sync()
+                got[tile, rows] = out
+    finally:
+        worker.set_option("gemm_narrow", 0)
+    assert torch.equal(got[3, m], got[3, more][:m])
+    assert not torch.equal(got[3, m], got[0, m])
