@@ -111,15 +111,6 @@ __device__ __forceinline__ int slab_count(const SlabMap& s, int splits, int mat,
   const unsigned first = (unsigned)(mat * s.slabs + (ch >> s.shift)) * s.ks;
   return (int)(((first + s.ks) * s.wgs - 1) / s.units - ((first + 1) * s.wgs - 1) / s.units) + 1;
 }
-// Row a workgroup takes where one writes a row of the blocked layout [K/8][rows][8]: its 128-byte lines are eight rows' pieces, and
-// eight rows whose workgroups run on one XCD (workgroup id mod 8) meet in that XCD's L2.  A permutation of 0 .. rows - 1; rows 0, for up to
-// 32 rows, where nothing is gained: as they come.
-__device__ __forceinline__ int blocked_row(int id, int rows) {
-  if (rows == 0) return id;
-  const int base = id & ~63, groups = min(rows - base, 64) >> 3;  // groups of eight rows among the next 64
-  if (groups == 0 || id - base >= groups * 8) return id;
-  return base + (id - base) % groups * 8 + (id - base) / groups;
-}
 // fp32 partial sums of a projection: element (s, m, n) of projection i is part[i][s * slab_stride + m * N + n] for
 // s below slab_count(map, splits, i, n).  The skinny kernels write [M, N] slabs into the shared workspace; the
 // tiled GEMM writes [M, N] slabs into its own scratch area (or, with one split, the finished product into the

@@ -8,6 +8,7 @@
 #include <hip/hip_runtime.h>
 
 #include "common.h"
+#include "launch_choice.h"
 
 namespace {
 

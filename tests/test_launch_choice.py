@@ -25,6 +25,7 @@ extern "C" int64_t partition_align_shape(int64_t pairs, int64_t max_ctx, int64_t
 extern "C" int64_t e4m3_partition(int64_t pairs, int64_t max_ctx, int64_t bytes_per_part, int64_t scratch, int64_t plain) {
   return pto_hip::attn_e4m3_partition_tokens(pairs, max_ctx, 256, 8, bytes_per_part, scratch, plain);
 }
+extern "C" int blocked_row(int id, int rows) { return pto_hip::blocked_row(id, rows); }
 """
 
 
@@ -181,3 +182,16 @@ def test_e4m3_partitions_stay_where_the_cus_are_full(choice, pairs, tokens, spli
 def test_tile_choice_on_ragged_columns_is_not_the_form_that_spills(choice, m, n, k, want):
     """Single passes that measured 27 to 39 % behind the best pair on 256-row tiles."""
     assert _quad(choice, m, n, k, False) == want
+
+
+def test_rows_of_one_line_are_written_from_few_xcds(choice):
+    """Rows of the blocked layout by workgroup: a permutation, and the eight rows of a line on as few XCDs (id mod 8) as their number allows."""
+    for rows in range(33, 200):
+        row = [choice.blocked_row(i, rows) for i in range(rows)]
+        assert sorted(row) == list(range(rows)), rows
+        for base in range(0, rows, 64):
+            groups = min(rows - base, 64) // 8
+            for g in range(groups):
+                lines = {i % 8 for i in range(rows) if base + 8 * g <= row[i] < base + 8 * g + 8}
+                assert len(lines) <= -(-8 // groups) + (8 % groups != 0), (rows, base, g)
+    assert [choice.blocked_row(i, 0) for i in range(32)] == list(range(32))
