@@ -241,10 +241,11 @@ size_t fused_lds(const SkinnyPlan& q, int64_t m) {
 // The launch saved is 2 to 5 us of a chain of ten; what is made instead is made by every workgroup, so it pays while a thread's part is
 // held in registers at once, one round trip to the caches (decoder layer, us, one / two rows, separate launch -> made here):
 // kNorm, up to 4 rows: 4096 wide int8 71.9 / 75.1 -> 70.4 / 73.1, 2048 wide 48.5 / 49.9 -> 46.8 / 48.3.
-// kSwiglu: 5632 -> 2048 channels (352 k rows a share) 48.5 / 49.9 -> 46.9 / 48.6; 14336 -> 4096 (1792) 55.2 -> 54.4 in one round trip, but 75.1 -> 76.7
-// for two rows in two; 20032 -> 8192 (5008) 142.9 -> 144.0.
-// kMerge: a head a wavefront (32 heads, 4096 wide) 71.9 -> 69.7, two 75.1 -> 75.0, three (40 heads, 8192 wide) 142.9 -> 145.4; 63 partitions, a loop
-// past the 32 held, 38.3 -> 42.6.
+// kSwiglu, up to two quads of channels a thread, 2048 values a share: 5632 -> 2048 channels (352 k rows a share) 48.5 / 49.9 -> 46.9 / 48.6; 14336 -> 4096
+// (1792) for one row 67.8 -> 66.9, 16-bit 98.1 -> 97.8, block of one token 64.2 -> 63.8; but 75.1 -> 76.7 for two rows, in two round trips;
+// 20032 -> 8192 (5008) 142.9 -> 144.0.
+// kMerge: a head a wavefront (32 heads, 4096 wide) 71.9 -> 69.7, two 75.1 -> 75.0, three (40 heads, 8192 wide) 142.9 -> 145.4.  More than the
+// kMergeHeld partitions of a row keep their merge launch: 63 of them, in a loop past those held, 38.3 -> 42.6.
 bool skinny_fuses(ProjectionSource::Kind kind, int64_t m, int64_t k, int64_t n, const void* wq0, const void* wq1, bool w16, int64_t head_dim) {
   const Context& cx = ctx();
   if (!(cx.skinny_fuse >> (kind - 1) & 1) || cx.w8a16_nt == 0 || m > kSkinnyFusedRows || k % 16 != 0 || k < kStep) return false;
@@ -253,7 +254,7 @@ bool skinny_fuses(ProjectionSource::Kind kind, int64_t m, int64_t k, int64_t n, 
   const int64_t share = ((int64_t)q.ks + q.per_slab - 1) / q.per_slab * kStep;
   switch (kind) {
     case ProjectionSource::kNorm: return k <= 8 * 256 * kNormVecs && share + (k % kStep ? kStep : 0) <= 8 * 256 * kNormOwn;
-    case ProjectionSource::kSwiglu: return m * share <= 1536;
+    case ProjectionSource::kSwiglu: return m * share <= kSwigluQuads * 4 * kWaves * 64;
     case ProjectionSource::kMerge: {
       const bool whole = q.ks % q.per_slab == 0 && share % head_dim == 0;
       return m * (whole ? share / head_dim : share / head_dim + 2) <= kWaves;

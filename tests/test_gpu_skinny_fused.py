@@ -36,7 +36,7 @@ def _same(a, b):
 # to 40 and more (which keeps its merge launch); an empty sequence beside long ones; 8 and 16 codes a lane.  The calls are not measured: a
 # measured call keeps its merge launch.  takes: the sources that the dispatch takes
 @pytest.mark.parametrize("batch,hidden,heads,kv_heads,head_dim,inter,block,lens,int8,e4m3,wide,takes", [
-    (1, 4096, 32, 8, 128, 14336, 128, [2049], True, False, 1, 5), (2, 1040, 8, 2, 128, 2064, 64, [1, 700], True, False, 1, 7),
+    (1, 4096, 32, 8, 128, 14336, 128, [2049], True, False, 1, 7), (2, 1040, 8, 2, 128, 2064, 64, [1, 700], True, False, 1, 7),
     (4, 1040, 8, 1, 128, 2064, 64, [0, 33, 1300, 2500], False, False, 1, 3), (3, 512, 4, 4, 256, 1040, 128, [400, 0, 3000], False, False, 1, 7),
     (1, 2048, 8, 2, 256, 4096, 64, [1111], True, True, 1, 7), (4, 2048, 16, 4, 128, 5632, 128, [600, 599, 1, 128], False, False, 1, 3),
     (2, 2048, 16, 4, 128, 5632, 128, [600, 5000], True, True, 2, 3), (1, 48, 2, 1, 128, 80, 16, [17], True, False, 1, 3),
@@ -89,7 +89,7 @@ def test_measured_and_settled_calls_have_the_same_bits(worker, hidden, heads, le
     assert all(torch.equal(o, outs[0]) for o in outs)
 
 
-@pytest.mark.parametrize("tokens,hidden,inter", [(1, 4096, 11008), (2, 1040, 4112), (3, 2048, 5632), (4, 1024, 3072), (4, 8192, 2048), (1, 48, 40000),
+@pytest.mark.parametrize("tokens,hidden,inter", [(1, 4096, 11008), (2, 1040, 4112), (3, 2048, 5632), (4, 1024, 3072), (4, 8192, 2048), (1, 48, 40000), (1, 4096, 16384), (2, 4096, 16384),
                                                  (1, 2496, 8448), (2, 2560, 8448)])  # the pair's channels have two or three partial sums
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 def test_ffn_block_has_the_bits_of_separate_launches(worker, tokens, hidden, inter, dtype):
