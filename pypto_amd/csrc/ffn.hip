@@ -62,9 +62,12 @@ int narrow_tile(const GemmParams& p, bool dual, int out_dtype) {
   if (cx.gemm_narrow > 0) return (int)cx.gemm_narrow;
   int height = 0, splits = 1;
   double us = pto_hip::choose_quad(p.m, p.n, p.k, dual, cx.num_cu, 0, &height, &splits);
-  if (splits > 1 && p.partials_out) us -= 2.95;
+  if (splits > 1 && p.partials_out) {
+    us -= 2.95;
+    splits = 1;
+  }
   if (p.m <= kSkinnyMaxTokens && pto_hip::narrow_beats_skinny(p.k, p.n, dual)) us = 1e9;
-  return pto_hip::choose_narrow(p.m, p.n, p.k, dual, cx.num_cu, us);
+  return pto_hip::choose_narrow(p.m, p.n, p.k, dual, cx.num_cu, us, splits);
 }
 
 template <bool DUAL>

@@ -99,12 +99,18 @@ inline double choose_quad(int m, int n, int k, bool dual, int64_t num_cu, int fo
 // the last term, 1.3 us per MB of a single product's activations: without it blocks of 333 to 1000 rows lost up to 17 % (768 x 2560 at 768 rows 25.7
 // -> 30.2 us, 1024 x 3072 at 640 30.3 -> 35.4).  With it, over 110 blocks of 64 to 1300 rows of
 // ten shapes, 512 x 1024 to 1280 x 4096: 1.13 times as fast as the tiled form, five slower, by 2 to 4 %.
+// Three corrections from 470 blocks of 33 to 1400 rows, 512 to 2300 wide, channels in eights and in 64s (kernel traces, products one by one): a
+// single tiled product with two or three k splits takes 2 us less than choose_quad says; rows that are no multiple of 64 channels put every
+// piece of a pair's weights on a line more, 0.005 us a KB; and 64 x 64 tiles wait for a pair's weights beyond 8 MB, 0.3 us a MB.  Blocks slower than
+// on the tiled form alone by more than 1 %: 23 -> none (65 rows of 1216 x 4408 31.1 -> 28.0 us, 195 of 1096 x 3680 35.0 -> 31.2, 232 of 1152 x
+// 4032 32.3 -> 30.2, 733 of 1024 x 2176 31.8 -> 30.5).
 // Up to 32 rows a product in the skinny form streams its weights once, in two launches; this form is ahead up to 1.6 million weights
 // (us, skinny -> this, 1 / 32 rows: 512 x 1024 pair 6.1 / 7.3 -> 4.2 / 4.5, 1024 x 1024 5.7 / 7.3 -> 4.1 / 4.7, 2048 x 768 6.1 / 7.5 ->
 // 5.6 / 6.8; but 768 x 2048 pair 7.0 / 8.4 -> 7.7 / 7.7, 1024 x 2048 pair 7.0 / 8.6 -> 9.3 / 9.5).
 inline bool narrow_beats_skinny(int64_t k, int64_t n, bool dual) { return k * n * (dual ? 2 : 1) <= 1600000; }
 
-inline int choose_narrow(int64_t m, int64_t n, int64_t k, bool dual, int64_t num_cu, double tiled_us) {
+// splits: of k, with which the tiled form would run.
+inline int choose_narrow(int64_t m, int64_t n, int64_t k, bool dual, int64_t num_cu, double tiled_us, int splits = 1) {
   struct Tile {
     int rows, channels;
     double us[2], round[2], mb[2];  // of a single product and of a pair
@@ -113,14 +119,17 @@ inline int choose_narrow(int64_t m, int64_t n, int64_t k, bool dual, int64_t num
                                      {32, 32, {2.33, 2.22}, {0.0201, 0.0226}, {0.313, 0.274}},
                                      {32, 64, {1.83, 1.67}, {0.0226, 0.0257}, {0.070, 0.084}},
                                      {64, 64, {2.80, 2.77}, {0.0191, 0.0275}, {0.165, 0.0}}};
-  double best = (1.112 * tiled_us + 2.05) * 0.95;
+  double best = (1.112 * tiled_us + 2.05 - (!dual && (splits == 2 || splits == 3) ? 1.9 : 0.0)) * 0.95;
   int tile = 0;
   for (int i = 0; i < 4; ++i) {
     const Tile& t = kTiles[i];
     const int64_t wgs = ((m + t.rows - 1) / t.rows) * ((n + t.channels - 1) / t.channels);
     const double kb = (double)k * 2.0 * (t.channels * (dual ? 2 : 1) + t.rows) * 1e-3;
-    const double us = t.us[dual] + t.round[dual] * (double)((wgs + num_cu - 1) / num_cu) * kb + t.mb[dual] * (double)k * n * (dual ? 2 : 1) * 2e-6 +
-                      (dual ? 0.0 : 1.3 * (double)m * k * 2e-6);
+    const double weights_mb = (double)k * n * (dual ? 2 : 1) * 2e-6;
+    const double round = t.round[dual] + (dual && n % 64 != 0 ? 0.005 : 0.0);
+    double us = t.us[dual] + round * (double)((wgs + num_cu - 1) / num_cu) * kb + t.mb[dual] * weights_mb;
+    if (!dual) us += 1.3 * (double)m * k * 2e-6;
+    else if (i == 3) us += 0.3 * std::max(weights_mb - 8.0, 0.0);
     if (us < best) {
       best = us;
       tile = i + 1;

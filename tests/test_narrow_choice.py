@@ -13,6 +13,11 @@ extern "C" int choose_narrow(int m, int n, int k, int dual) {
   int height = 0, splits = 0;
   return pto_hip::choose_narrow(m, n, k, dual != 0, 256, pto_hip::choose_quad(m, n, k, dual != 0, 256, 0, &height, &splits));
 }
+extern "C" int choose_narrow_splits(int m, int n, int k, int dual) {
+  int height = 0, splits = 0;
+  const double us = pto_hip::choose_quad(m, n, k, dual != 0, 256, 0, &height, &splits);
+  return pto_hip::choose_narrow(m, n, k, dual != 0, 256, us, splits);
+}
 extern "C" int choose_narrow8(int m, int n, int k, int dual, double tiled_us) { return pto_hip::choose_narrow8(m, n, k, dual != 0, 256, tiled_us); }
 extern "C" int beats_skinny(int64_t k, int64_t n, int dual) { return pto_hip::narrow_beats_skinny(k, n, dual != 0); }
 """
@@ -42,6 +47,15 @@ def test_large_products_keep_the_tiled_form(choice):
     for m, n, k, dual in ((1024, 2048, 1024, 1), (512, 3584, 1024, 1), (96, 1536, 4096, 0), (256, 2048, 5632, 0), (40, 14336, 4096, 1),
                           (333, 14336, 4096, 1), (2048, 11008, 4096, 1), (2048, 4096, 11008, 0), (1 << 20, 8192, 8192, 0)):
         assert choice.choose_narrow(m, n, k, dual) == 0, (m, n, k, dual)
+
+
+def test_products_that_measured_slower_in_a_block_keep_the_tiled_form(choice):
+    """Ragged channels of a pair, a pair's weights beyond 8 MB, a tiled single product of two or three k splits."""
+    for m, n, k, dual in ((65, 4408, 1216, 1), (195, 3680, 1096, 1), (114, 3672, 936, 1), (36, 3928, 1008, 1), (208, 3904, 1216, 1), (232, 4032, 1152, 1),
+                          (299, 3264, 1088, 1), (733, 1024, 2176, 0), (894, 768, 1664, 0), (984, 768, 1856, 0)):
+        assert choice.choose_narrow_splits(m, n, k, dual) == 0, (m, n, k, dual)
+    for m, n, k, dual in ((128, 1024, 512, 1), (128, 512, 1024, 0), (512, 2048, 1024, 1), (931, 832, 1664, 0), (120, 3264, 896, 1), (262, 680, 2408, 0)):
+        assert choice.choose_narrow_splits(m, n, k, dual) > 0, (m, n, k, dual)
 
 
 def test_up_to_32_rows_only_small_weights(choice):
