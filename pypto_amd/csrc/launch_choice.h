@@ -175,9 +175,24 @@ inline int choose_narrow8(int64_t m, int64_t n, int64_t k, bool dual, int64_t nu
 // and 60 million up, with few slabs a channel (13824 x 5120 3 / 3 / 2 / 2, 16384 x 8192 7 / 5 / 4 / 3; 14336 x 4096 lost 0 to 2).
 // Few k, up to 64 rows (layers with these projections tiled -> streamed, k split in both, 36 / 48 / 64 rows, us gained): hidden 1024 5 / 4 / 2,
 // 1280 4 / 3 / 0, 1536 4 / 2 / -1, 1792 2 / 1 / 0, 2048 2 / 1 / 0, 2304 2 / 1 / 0, 3072 3 / 2 / 2, 3584 8 / 9 / 8.
+// A pair of more slabs than half the CUs has no k split, and the fewer slabs beyond, the more CUs have none while the launch lasts as long as with 256.  Up to
+// 2/3 of the CUs such pairs lose against the tiled GEMM: with 16-bit weights 1 to 7 us (36 / 48 / 57 / 64 / 80 / 96 rows of 4096 x 8960 3 / 4 / 5 / 4 / 4 / 4, 4992 x 9472 3 /
+// 4 / 6 / 4 / 2 / 2, 52 of 3200 x 9216 3), unless the down projection streams as well, which only a streamed pair leaves its activations to (4096 x 9984 gains 4 / 5 /
+// 3 / 3 / 0 / 0 in both), or k is below 2560 (45 x 2112 x 8320 7 gained); with int8 above 48 rows up to 0.6 of the CUs and above 64 rows up to 2/3 (4992 x 8960
+// 1 and 1 gained, 3 / 3 / 5 / 5 lost, 4096 x 10496 7 / 7 / 2 / 4 gained, 2 / 1 lost), but not with a last slab that is no whole 128 channels, which the
+// tiled int8 GEMM is slower with (65 to 96 rows of 4224 x 9664 gain 6 to 9).
 constexpr int kStreamRowsMax = 96;
-inline bool stream_rows_ahead(int64_t m, int64_t k, int64_t n, bool dual, bool w16) {
-  const int64_t weights = k * n * (dual ? 2 : 1);
+// k splits of a streamed projection: what the CUs hold of its 128-channel slabs, of at least eight 32-row steps each.
+inline int stream_splits(int64_t k, int64_t n, bool dual, int64_t num_cu) {
+  const int64_t slabs = (n + 127) / 128 * (dual ? 2 : 1), ks = (k + 31) / 32;
+  return (int)std::max<int64_t>(1, std::min<int64_t>(num_cu / slabs, ks / 8));
+}
+inline bool stream_rows_ahead(int64_t m, int64_t k, int64_t n, bool dual, bool w16, int64_t num_cu) {
+  const int64_t weights = k * n * (dual ? 2 : 1), slabs = (n + 127) / 128 * (dual ? 2 : 1);
+  if (dual && 2 * slabs > num_cu && 3 * slabs < 2 * num_cu) {
+    if (w16 && k >= 2560 && !(weights >= 80000000 && n >= 2 * k)) return false;
+    if (!w16 && n % 128 == 0 && m > 48 && (m > 64 || 5 * slabs < 3 * num_cu)) return false;
+  }
   if (w16) return dual ? weights >= 30000000 : weights >= 40000000 && k >= 2 * n;
   if (dual) return weights >= 80000000 || (m <= 64 && k <= (m <= 48 ? 1536 : 1280));
   return (m <= 64 && k <= 4096 && (m <= 48 || k <= 1280 || k >= 3072)) || (n >= 5120 && weights >= 60000000 && k >= 2 * n);

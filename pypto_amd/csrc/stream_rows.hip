@@ -8,21 +8,14 @@ namespace pto_hip {
 int stream_rows_w8(const stream::StreamParams& p, bool bf16, hipStream_t st);
 int stream_rows_w16(const stream::StreamParams& p, bool bf16, hipStream_t st);
 
-namespace {
-int stream_splits(int64_t k, int64_t n, int mats) {
-  const int64_t slabs = (n + 127) / 128 * mats, ks = (k + 31) / 32;
-  return (int)std::max<int64_t>(1, std::min<int64_t>(ctx().num_cu / slabs, ks / 8));
-}
-}  // namespace
-
 int stream_rows_for(int64_t m, int64_t k, int64_t n, const void* wq0, const void* wq1, bool w16, hipStream_t st) {
   const int mats = wq1 ? 2 : 1;
   if (ctx().gemm_stream == 0 || ctx().gemm_variant != 0 || ctx().gemm_splits != 0 || ctx().gemm_quad_rows != 0) return 0;
   if (w16 && ctx().gemm_narrow > 0) return 0;  // a tile of the small-call form is asked for
   if (k % 8 != 0 || k < 32 || n % 8 != 0 || (n + 127) / 128 * mats > ctx().num_cu || ((uintptr_t)wq0 | (uintptr_t)wq1) % 16 != 0) return 0;
-  if (m <= kW8MaxM || m > kStreamRowsMax || (ctx().gemm_stream == 1 && !stream_rows_ahead(m, k, n, mats == 2, w16))) return 0;
+  if (m <= kW8MaxM || m > kStreamRowsMax || (ctx().gemm_stream == 1 && !stream_rows_ahead(m, k, n, mats == 2, w16, ctx().num_cu))) return 0;
   void* area = nullptr;
-  if (gemm_slabs((size_t)stream_splits(k, n, mats) * mats * m * n * sizeof(float), st, &area) || !area) return 0;
+  if (gemm_slabs((size_t)stream_splits(k, n, mats == 2, ctx().num_cu) * mats * m * n * sizeof(float), st, &area) || !area) return 0;
   return (int)((m + 15) / 16 * 16);
 }
 
@@ -39,7 +32,7 @@ int stream_partials(const void* x, int x_rows, const void* wq0, const void* wq1,
   p.mats = wq1 ? 2 : 1;
   p.slabs = (int)((n + 127) / 128);
   p.ks = (int)((k + 31) / 32);
-  p.splits = stream_splits(k, n, p.mats);
+  p.splits = stream_splits(k, n, p.mats == 2, ctx().num_cu);
   void* area = nullptr;
   int rc = gemm_slabs((size_t)p.splits * p.mats * m * n * sizeof(float), st, &area);
   if (rc) return rc;

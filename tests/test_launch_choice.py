@@ -26,6 +26,8 @@ extern "C" int64_t e4m3_partition(int64_t pairs, int64_t max_ctx, int64_t bytes_
   return pto_hip::attn_e4m3_partition_tokens(pairs, max_ctx, 256, 8, bytes_per_part, scratch, plain);
 }
 extern "C" int blocked_row(int id, int rows) { return pto_hip::blocked_row(id, rows); }
+extern "C" int stream_ahead(int m, int k, int n, int dual, int w16) { return pto_hip::stream_rows_ahead(m, k, n, dual != 0, w16 != 0, 256); }
+extern "C" int stream_splits(int k, int n, int dual) { return pto_hip::stream_splits(k, n, dual != 0, 256); }
 """
 
 
@@ -195,3 +197,21 @@ def test_rows_of_one_line_are_written_from_few_xcds(choice):
                 lines = {i % 8 for i in range(rows) if base + 8 * g <= row[i] < base + 8 * g + 8}
                 assert len(lines) <= -(-8 // groups) + (8 % groups != 0), (rows, base, g)
     assert [choice.blocked_row(i, 0) for i in range(32)] == list(range(32))
+
+
+# (rows, k, channels, 16-bit): behind the tiled GEMM with 129 to 170 slabs of 128 channels and no k split
+@pytest.mark.parametrize("m,k,n,w16", [(36, 4096, 8960, 1), (57, 4992, 9472, 1), (52, 3200, 9216, 1), (96, 3072, 10496, 1), (64, 3456, 8640, 1),
+                                       (57, 4288, 9600, 0), (64, 4992, 9728, 0), (80, 4096, 10496, 0), (96, 4992, 8960, 0), (65, 4480, 10880, 0)])
+def test_pairs_that_leave_a_third_of_the_cus_idle_do_not_stream(choice, m, k, n, w16):
+    assert not choice.stream_ahead(m, k, n, 1, w16)
+
+
+# two k splits; from 171 slabs on; the down projection streams too; few k; int8 of up to 48 rows; a last slab that is not whole
+@pytest.mark.parametrize("m,k,n,w16", [(64, 4992, 8192, 1), (64, 4992, 8192, 0), (96, 4096, 11008, 1), (96, 4096, 11008, 0), (48, 4096, 9984, 1),
+                                       (54, 3840, 10624, 1), (45, 2112, 8320, 1), (48, 4992, 8960, 0), (64, 4096, 9984, 0), (96, 4224, 9664, 0)])
+def test_pairs_that_stay_streamed(choice, m, k, n, w16):
+    assert choice.stream_ahead(m, k, n, 1, w16)
+
+
+def test_streamed_k_splits_fill_the_cus(choice):
+    assert [choice.stream_splits(4992, n, 1) for n in (8192, 8320, 5504, 1024)] == [2, 1, 2, 16] and choice.stream_splits(256, 1024, 0) == 1
