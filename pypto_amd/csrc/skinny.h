@@ -48,6 +48,7 @@ struct GemvParams {
   int per_wg, extra;    // units / workgroups and its remainder (see SlabMap)
   int mapped;           // 0: a workgroup per slab
   int per_slab;         // workgroups of a slab (fused form)
+  int wgs;              // workgroups; gridDim.x lies behind src, two lines of arguments further (0.03 us a launch)
   ProjectionSource src; // unless kGiven
 };
 
@@ -174,7 +175,7 @@ __global__ __launch_bounds__(kWaves * 64) __attribute__((amdgpu_waves_per_eu(1, 
   const int c = lane & 15, kg = lane >> 4;
 
   // this workgroup's units, and a cursor over them in rounds of kWaves steps of one slab
-  const int wg = blockIdx.x, wgs = gridDim.x;
+  const int wg = blockIdx.x, wgs = p.wgs;
   const int u_begin = wg * p.per_wg + wg * p.extra / wgs, u_end = (wg + 1) * p.per_wg + (wg + 1) * p.extra / wgs;
   struct Cursor {
     int slab, step, end;  // the round's first step and the end of its run

@@ -285,6 +285,7 @@ int w8a16_partials(const void* x, bool x_blocked, const void* wq0, const void* w
   p.extra = (int)(q.units % q.wgs);
   p.mapped = q.mapped ? 1 : 0;
   p.per_slab = q.per_slab;
+  p.wgs = (int)q.wgs;
   out->map = q.mapped ? SlabMap{(unsigned)q.units, (unsigned)q.wgs, (unsigned)q.ks, q.wide ? 8 : 7, q.slabs} : SlabMap{};
   out->splits = q.splits;
   // scratch for 32 rows whatever m: a call sized once fits every smaller and larger batch of the shape, also under capture
