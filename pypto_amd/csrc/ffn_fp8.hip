@@ -575,8 +575,11 @@ int launch_tiles(Params& p, bool sums_on_the_way, hipStream_t st) {
       }
     }
     // Small calls in narrow tiles, one launch.  The estimate's 3 us for the launch that sums the slabs do not count against a caller that has one anyway.
+    // (not a result laid over its own activations: one workgroup would write what another has still to read)
     const int64_t narrow = pto_hip::ctx().gemm_narrow;
-    if (can_split && forced == 0 && narrow >= 0) {
+    const uintptr_t a0 = (uintptr_t)p.a, c0 = (uintptr_t)p.c;
+    const bool in_place = c0 < a0 + (uintptr_t)p.m * p.lda && a0 < c0 + (uintptr_t)p.m * p.ldc * sizeof(OutT);
+    if (can_split && forced == 0 && narrow >= 0 && !in_place) {
       const double tiled_us = best - (sums_on_the_way && splits > 1 ? 3.0 : 0.0);
       const int tile = narrow > 0 ? (int)std::min<int64_t>(narrow, 3) : pto_hip::choose_narrow8(p.m, p.n, p.k, DUAL, num_cu, tiled_us);
       if (tile > 0) {

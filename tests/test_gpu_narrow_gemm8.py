@@ -82,3 +82,27 @@ def test_error_is_no_larger_than_the_tiled_form(worker, m, k, n):
     finally:
         worker.set_option("gemm_narrow", 0)
     assert max(err[1], err[2], err[3]) <= 1.1 * err[-1], err
+
+
+@pytest.mark.parametrize("m,k,n,dual", [(1, 512, 256, False), (17, 512, 256, False), (32, 4096, 256, False), (8, 4096, 2048, False),
+                                        (17, 256, 128, True), (8, 2048, 512, True)])
+def test_a_result_laid_over_its_codes(worker, m, k, n, dual):
+    """A product whose tiled form has one tile of channels, or k splits that are summed behind it, may write its result over its codes; the
+    small-call form would write them while other workgroups still read.  Such a call has the tiled form's bits."""
+    lib = _lib.load()
+    g = torch.Generator().manual_seed(m + n)
+    codes = lambda rows: _codes(rows, k, torch.randn((rows, k), generator=g))
+    x, w, u = codes(m), codes(n), codes(n) if dual else None
+    sx, sw, su = (torch.rand(rows, generator=g).cuda() * 0.05 + 0.01 for rows in (m, n, n))
+    program = lib.pto_hip_gate_up_swiglu_fp8 if dual else lib.pto_hip_projection_fp8
+    weights = (w.data_ptr(), sw.data_ptr()) + ((u.data_ptr(), su.data_ptr()) if dual else ())
+    try:
+        worker.set_option("gemm_narrow", -1)
+        want = _run(lib, x, sx, w, sw, u, su, m, k, n, torch.bfloat16)
+    finally:
+        worker.set_option("gemm_narrow", 0)
+    for _ in range(8):
+        buf = x.clone().flatten()
+        _lib.check(program(buf.data_ptr(), sx.data_ptr(), *weights, buf.data_ptr(), m, k, n, _dtype_code(torch.bfloat16), 0))
+        torch.cuda.synchronize()
+        assert torch.equal(buf[:m * n * 2].view(torch.bfloat16).view(m, n), want)
