@@ -175,6 +175,11 @@ inline int choose_narrow8(int64_t m, int64_t n, int64_t k, bool dual, int64_t nu
 // and 60 million up, with few slabs a channel (13824 x 5120 3 / 3 / 2 / 2, 16384 x 8192 7 / 5 / 4 / 3; 14336 x 4096 lost 0 to 2).
 // Few k, up to 64 rows (layers with these projections tiled -> streamed, k split in both, 36 / 48 / 64 rows, us gained): hidden 1024 5 / 4 / 2,
 // 1280 4 / 3 / 0, 1536 4 / 2 / -1, 1792 2 / 1 / 0, 2048 2 / 1 / 0, 2304 2 / 1 / 0, 3072 3 / 2 / 2, 3584 8 / 9 / 8.
+// Why k from 1280 to 3072 stays tiled above 48 rows: the two are level there, or streams behind, where a product has whole tiles of 256 channels and as
+// many k splits streamed as tiled, k / 256 (layers, tiled -> streamed, us: 64 rows of 2048 67.1 -> 67.2, of 2304 70.6 -> 70.6; 61 of 1856 with 4608 q/k/v
+// channels 76.7 -> 77.7, 60 of 2368 with 1536 73.4 -> 73.7).  Few k leave the tiled form few splits and most CUs idle; many k give it more of them than
+// the CUs hold of the streamed form's, and so more partial sums (64 rows of 3072 87.8 -> 84.3, of 4096 107.1 -> 102.1).  Streams would also be ahead in between where n ends
+// inside a tile or the CUs hold fewer streamed splits (60 rows of 2112 with 1152 q/k/v channels 69.0 -> 67.2, 58 of 2688 with 4608 96.4 -> 93.2): not used.
 // A pair of more slabs than half the CUs has no k split, and the fewer slabs beyond, the more CUs have none while the launch lasts as long as with 256.  Up to
 // 2/3 of the CUs such pairs lose against the tiled GEMM: with 16-bit weights 1 to 7 us (36 / 48 / 57 / 64 / 80 / 96 rows of 4096 x 8960 3 / 4 / 5 / 4 / 4 / 4, 4992 x 9472 3 /
 // 4 / 6 / 4 / 2 / 2, 52 of 3200 x 9216 3), unless the down projection streams as well, which only a streamed pair leaves its activations to (4096 x 9984 gains 4 / 5 /
